@@ -33,3 +33,37 @@ def test_cdist_tiles(n_a, n_b, dim, offset):
     assert (got[n_a * n_b:] == -7.0).all()  # nothing past the end
     ref = O.cdist(a, b)
     np.testing.assert_allclose(got[:n_a * n_b].reshape(n_a, n_b), ref, rtol=2.0**-24 + 2.0**-40, atol=0)
+
+
+def order_key(x):
+    """The total order of the scatter's maximum: floats by value, -0.0 below +0.0, NaNs beyond the infinities."""
+    b = np.ascontiguousarray(x).view(np.int32).astype(np.int64)
+    return np.where(b < 0, -(b & 0x7FFFFFFF) - 1, b)
+
+
+@pytest.mark.parametrize("n_row,n_in,n_out,offset", [(1, 1, 1, 0), (3, 7, 2, 1), (5, 1023, 40, 2), (2, 1025, 1, 3),
+                                                     (3, 8193, 700, 1), (16, 70_001, 3000, 0), (2, 0, 5, 0)])
+@pytest.mark.parametrize("fill", ["low", "mid", "special"])
+def test_edge_max_reduce_edges(n_row, n_in, n_out, offset, fill):
+    """Chunk edges, rows off the 16-byte grid, nodes shared by many and by neighbouring values, fills below, among and
+    above the values, and infinities, signed zeros and NaNs on both sides.  A maximum: bit for bit."""
+    r = np.random.default_rng(n_in)
+    xe = r.normal(size=(n_row, n_in)).astype(np.float32)
+    vy = np.full(n_row, {"low": -np.inf, "mid": 0.5, "special": 0.0}[fill], np.float32)
+    if fill == "special":
+        special = np.array([0.0, -0.0, np.inf, -np.inf, np.nan, -np.nan], np.float32)
+        xe[:, :] = np.where(r.random(xe.shape) < 0.02, r.choice(special, xe.shape), xe)
+        vy[:] = r.choice(special, n_row)
+        xe.reshape(-1)[:2] = -0.0
+    nodes = (r.integers(0, n_out, n_in) // 3 * 3 if n_in % 2 else np.sort(r.integers(0, n_out, n_in))).astype(np.int32)
+    x = torch.empty(n_row * n_in + 4, device="cuda")
+    x[offset:offset + n_row * n_in] = dev(xe.reshape(-1))
+    out = torch.full((n_row * n_out + 8,), 3.0, device="cuda")
+    ac.EdgeMaxReduce2_t(n_in, n_out, n_row, dev(vy), x.data_ptr() + 4 * offset, out, dev(nodes))
+    torch.cuda.synchronize()
+    key = np.repeat(order_key(vy)[:, None], n_out, axis=1)
+    for i in range(n_row):
+        np.maximum.at(key[i], nodes, order_key(xe[i]))
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(order_key(got[:n_row * n_out]).reshape(n_row, n_out), key)
+    assert (got[n_row * n_out:] == 3.0).all()
