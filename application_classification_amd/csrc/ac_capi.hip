@@ -186,10 +186,6 @@ struct ac_ctx {
   DevBuf<int> csc_eid;
   DevBuf<Run> runs_in, runs_out;
   DevBuf<Split> splits_in, splits_out;
-  // The plain walk's fixup work: chunks of at most kFixChunk pieces of a split vertex ({v, first piece, count, out
-  // partial or -1}) and the vertices of several chunks ({v, first partial, count}).
-  DevBuf<Split> fix_chunks, fix_multi;
-  int nfix_chunks = 0, nfix_multi = 0, nfix_parts = 0;
   std::vector<Run> h_runs_in;
   std::vector<int> h_run_src0;  // first (least) source of each in-edge run
   // Internal vertex order: vertices with in- and out-edges, in-edges only, out-edges only, then isolated ones, each
@@ -242,8 +238,8 @@ struct ac_ctx {
   bool use_mfma_cdist = true;  // feature distances on FP64 matrix cores (GEMM form, cancellation-guarded)
   DevBuf<double> cd_scratch;   // the matrix-core operands of the pattern features
   DevBuf<float> bmin;      // [bundles][Qs] least cost per bundle and pattern edge
+  DevBuf<int> bstate;      // [bundles] launch_walk_max
   DevBuf<double> carry_in, carry_out;
-  DevBuf<float> fix_part;  // [nfix_parts][Qs]
   DevBuf<QPart> qpart;
   DevBuf<Lse> ppart, lpart;
   DevBuf<QStat> qstat;  // [3][Q]: prep state, then by iteration parity
@@ -459,20 +455,6 @@ static int set_data(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int64_
   int slin = 0, slout = 0;
   build_runs(in_off, nV, rin, sin, slin);
   build_runs(sord_off, (int64_t)sord.size(), rout, sout, slout, sord.data(), false);
-  std::vector<Split> fch, fms;
-  int nparts = 0;
-  for (const Split& S : sin) {
-    const int nch = (S.count + ac::kFixChunk - 1) / ac::kFixChunk;
-    if (nch == 1) {
-      fch.push_back(Split{S.v, S.first, S.count, -1});
-      continue;
-    }
-    fms.push_back(Split{S.v, nparts, nch, 0});
-    for (int c = 0; c < nch; ++c)
-      fch.push_back(Split{S.v, S.first + c * ac::kFixChunk, std::min(ac::kFixChunk, S.count - c * ac::kFixChunk),
-                          nparts + c});
-    nparts += nch;
-  }
 
   ctx->has_data = false;
   hipStream_t st = ctx->stream;
@@ -486,11 +468,6 @@ static int set_data(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int64_
   HIPCHK(ctx, ctx->runs_out.upload(rout.data(), rout.size(), st));
   HIPCHK(ctx, ctx->splits_in.upload(sin.data(), sin.size(), st));
   HIPCHK(ctx, ctx->splits_out.upload(sout.data(), sout.size(), st));
-  HIPCHK(ctx, ctx->fix_chunks.upload(fch.data(), fch.size(), st));
-  HIPCHK(ctx, ctx->fix_multi.upload(fms.data(), fms.size(), st));
-  ctx->nfix_chunks = (int)fch.size();
-  ctx->nfix_multi = (int)fms.size();
-  ctx->nfix_parts = nparts;
   ctx->dn = nV;
   ctx->max_outdeg = max_outdeg;
   ctx->n_iso = n_iso;
@@ -739,7 +716,6 @@ static int ensure_work(ac_ctx* ctx) {
   HIPCHK(ctx, ctx->VR.alloc((size_t)(n * ctx->VRs)));
   HIPCHK(ctx, ctx->OUT.alloc((size_t)(n * P)));
   HIPCHK(ctx, ctx->carry_in.alloc((size_t)std::max(1, ctx->nslots_in) * Qs));
-  HIPCHK(ctx, ctx->fix_part.alloc((size_t)std::max(1, ctx->nfix_parts) * Qs));
   HIPCHK(ctx, ctx->carry_out.alloc((size_t)std::max(1, ctx->nslots_out) * Qs * 2));
   HIPCHK(ctx, ctx->qpart.alloc((size_t)(ctx->nb_vertex + 1) * std::max(1, Q)));
   HIPCHK(ctx, ctx->ppart.alloc((size_t)(ctx->nb_vertex_c + 1) * P));
@@ -849,10 +825,14 @@ static int ensure_tape(ac_ctx* ctx, int n_iter) {
   return AC_OK;
 }
 
-// Combines the split vertices' pieces of a plain (non-recording) walk.
-static void launch_fixup32(ac_ctx* ctx, hipStream_t st) {
-  ac::launch_walk_max_fixup32(ctx->nfix_chunks, ctx->fix_chunks.p, ctx->nfix_multi, ctx->fix_multi.p, ctx->carry_in.p,
-                              ctx->Qs, ctx->fix_part.p, ctx->FMaxN.p, st);
+// The split vertices' rows of the live FMaxN, reset before a plain (non-recording) walk.
+static ac::SplitRows split_rows(ac_ctx* ctx) {
+  ac::SplitRows r;
+  r.nsplit = ctx->nsplit_in;
+  r.splits = ctx->splits_in.p;
+  r.Qs = ctx->Qs;
+  r.FMaxN = ctx->FMaxN.p;
+  return r;
 }
 
 // Prep (src/main.cu:107-148), between events ev[0] and ev[1].
@@ -873,6 +853,7 @@ static int enqueue_prep(ac_ctx* ctx) {
   double* cds_e = ctx->use_mfma_cdist ? ctx->cd_scratch.p + vsd : nullptr;
   if (Q > 0) {
     HIPCHK(ctx, ctx->bmin.alloc((size_t)std::max<int64_t>(1, ctx->bs->nbundles) * Qs));
+    HIPCHK(ctx, ctx->bstate.alloc((size_t)std::max<int64_t>(1, ctx->bs->nbundles)));
     if (ctx->pack_costs) HIPCHK(ctx, ctx->bpack.alloc((size_t)std::max<int64_t>(1, ctx->bs->nbundles)));
     if (ctx->pack_costs) HIPCHK(ctx, ctx->CEp.alloc((size_t)std::max<int64_t>(1, ctx->bs->brows * (Qs / 4) * 3)));
   }
@@ -924,23 +905,22 @@ static int enqueue_prep(ac_ctx* ctx) {
       HIPCHK(ctx, hipMemcpyAsync(ctx->lse_ce.p, empty.data(), sizeof(Lse2) * Q, hipMemcpyHostToDevice, st));
       HIPCHK(ctx, hipStreamSynchronize(st));
     }
-    ac::launch_prep_scalars(P, Q, ctx->d_ps.p, ctx->d_pd.p, ctx->lse_cv.p, ctx->lse_ce.p, qs_prep, st);
+    const bool tape = ctx->tape_K > 0;
+    ac::launch_prep_scalars(P, Q, ctx->d_ps.p, ctx->d_pd.p, ctx->lse_cv.p, ctx->lse_ce.p, qs_prep, st,
+                            tape ? ac::SplitRows() : split_rows(ctx));
     HIPCHK(ctx, hipStreamWaitEvent(st, ctx->xev[3], 0));
     ctx->costs_packed = false;
     // The prep's max over in-edges of -CE reads every cost row once, so it also writes the 24-bit codes of the
     // bundles that pack (one pass over CE instead of a separate packing pass).
-    const bool tape = ctx->tape_K > 0;
     ac::launch_walk_max(ctx->bs->nbundles, ctx->bs->bundles.p, ctx->bs->gslot.p, ctx->bs->bsrc.p, ctx->bs->bdst.p,
                         ctx->CE.p, nullptr, ctx->VRs, Q, Qs, qs_prep, ctx->FMaxN.p, ctx->carry_in.p,
                         walk_batch_of(ctx), st, tape ? ctx->FA0.p : nullptr, tape ? ctx->carg_in.p : nullptr,
                         nullptr, nullptr, ctx->pack_costs ? ctx->bpack.p : nullptr,
-                        ctx->pack_costs ? ctx->CEp.p : nullptr);
+                        ctx->pack_costs ? ctx->CEp.p : nullptr, ctx->bstate.p);
     ctx->costs_packed = ctx->pack_costs;
     if (tape)
       ac::launch_walk_max_fixup(ctx->nsplit_in, ctx->splits_in.p, ctx->carry_in.p, Q, Qs, qs_prep, ctx->FMaxN.p, st,
                                 ctx->carg_in.p, ctx->FA0.p);
-    else
-      launch_fixup32(ctx, st);
     if (tape) {
       // Rows of the minimum-cost out-edge of every (v, q) (the RMax argmax), for the adjoint.
       ac::launch_fill_int(ctx->AO.p, n * Qs, INT32_MAX, st);
@@ -993,10 +973,10 @@ static ac::VertexArgs vertex_args(ac_ctx* ctx) {
 }
 
 // One iteration (src/main.cu:160-245) reading the scalars of state `qs_state`, writing those of the new state into
-// the parity slot of `it`.  Kernels only (no copies or fills), so it can be captured into a graph.  FA (nullable):
-// the walk also records its argmax rows there (the split vertices' pieces are then combined with theirs); the maxima
-// are the same as a plain walk's, bit for bit.
-static int enqueue_iteration(ac_ctx* ctx, ac::VertexArgs& va, int it, const QStat*& qs_state, int* FA = nullptr) {
+// the parity slot of `it`.  Kernels only (no copies or fills), so it can be captured into a graph.  The split
+// vertices' rows are reset beside the reduction (after pass A, their last reader, and before the walk, whose pieces
+// raise them): combining the pieces in two launches of their own took 9.5 us per iteration.
+static int enqueue_iteration(ac_ctx* ctx, ac::VertexArgs& va, int it, const QStat*& qs_state) {
   hipStream_t st = ctx->stream;
   const int P = ctx->P, Q = ctx->Q, Qs = ctx->Qs;
   QStat* qs_new = ctx->qstat.p + (1 + (it & 1)) * std::max(1, Q);
@@ -1008,21 +988,16 @@ static int enqueue_iteration(ac_ctx* ctx, ac::VertexArgs& va, int it, const QSta
       Range r("step1+step3+step4a");  // VF, VR; VFmax, RE's normaliser, RMax; VRmax, FE's normaliser
       ac::launch_vertex(ac::kModeA, va, ctx->nb_vertex, st);
       MARK(AC_STAGE_VERTEX_A);
-      ac::launch_reduce_q(ctx->nb_vertex + 1, Q, ctx->qpart.p, qs_new, st, cnull_of(ctx));
+      ac::launch_reduce_q(ctx->nb_vertex + 1, Q, ctx->qpart.p, qs_new, st, cnull_of(ctx), split_rows(ctx));
       MARK(AC_STAGE_REDUCE_A);
     }
     Range r("step2+step4b+step4c");  // FE messages, normalised, scatter-max by destination
     ac::launch_walk_max(ctx->bs->nbundles, ctx->bs->bundles.p, ctx->bs->gslot.p, ctx->bs->bsrc.p, ctx->bs->bdst.p,
                         ctx->CE.p, ctx->VR.p, ctx->VRs, Q, Qs, qs_new, ctx->FMaxN.p, ctx->carry_in.p,
-                        walk_batch_of(ctx), st, FA, FA ? ctx->carg_in.p : nullptr, ctx->prune ? ctx->bmin.p : nullptr,
-                        ctx->costs_packed ? ctx->CEp.p : nullptr, ctx->costs_packed ? ctx->bpack.p : nullptr);
+                        walk_batch_of(ctx), st, nullptr, nullptr, ctx->prune ? ctx->bmin.p : nullptr,
+                        ctx->costs_packed ? ctx->CEp.p : nullptr, ctx->costs_packed ? ctx->bpack.p : nullptr, nullptr,
+                        ctx->bstate.p);
     MARK(AC_STAGE_EDGE_WALK);
-    if (FA)
-      ac::launch_walk_max_fixup(ctx->nsplit_in, ctx->splits_in.p, ctx->carry_in.p, Q, Qs, qs_new, ctx->FMaxN.p, st,
-                                ctx->carg_in.p, FA);
-    else
-      launch_fixup32(ctx, st);
-    MARK(AC_STAGE_WALK_FIXUP);
     qs_state = qs_new;
   }
   va.first = 0;

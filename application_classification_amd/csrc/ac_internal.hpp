@@ -61,6 +61,13 @@ struct Run {
 struct Split {
   int v, first, count, pad;
 };
+// The split vertices' FMaxN rows, set to -inf before a plain walk raises them piece by piece (nsplit 0: none).
+struct SplitRows {
+  int nsplit = 0;
+  const Split* splits = nullptr;
+  int Qs = 4;
+  float* FMaxN = nullptr;
+};
 // G runs walked side by side by one wave: rows [base, base + len * G) of CE / bsrc / bdst; len is a multiple of
 // the walk's batch size.
 struct Bundle {
@@ -113,7 +120,8 @@ size_t cdist_scratch_doubles(int Kstore, int dim);
 void launch_col_lse_neg(int64_t n, int P, const float* X, Lse* part, int nblocks, hipStream_t st);
 void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStream_t st);
 // cnull (nullptr: off): per pattern edge, the PNNL Cnull term subtracted from both fills of the new state.
-void launch_reduce_q(int nparts, int Q, const QPart* part, QStat* out, hipStream_t st, const double* cnull = nullptr);
+void launch_reduce_q(int nparts, int Q, const QPart* part, QStat* out, hipStream_t st, const double* cnull = nullptr,
+                     const SplitRows& rows = SplitRows());
 // Per column p of the n rows X[n][P]: IsoCol{LSE of -X, min X and its lowest row + base}; partial buffers of
 // nparts * P entries each.
 void launch_iso_cols(int64_t n, int P, const float* X, int base, Lse* lpart, float* pv, int* pi, int nparts,
@@ -122,7 +130,7 @@ void launch_iso_cols(int64_t n, int P, const float* X, int base, Lse* lpart, flo
 void launch_bundle_min(int64_t nbundles, const Bundle* bundles, const float* CE, int Q, int Qs, float* bmin,
                        unsigned* bpack, hipStream_t st);
 void launch_prep_scalars(int P, int Q, const int* ps, const int* pd, const Lse2* cv, const Lse2* ce, QStat* qs,
-                         hipStream_t st);
+                         hipStream_t st, const SplitRows& rows = SplitRows());
 void launch_fill(float* p, int64_t count, float value, hipStream_t st);
 void launch_fill_slots(float* A, float* B, int64_t nslots, int64_t stride, int64_t a0, int64_t al, int64_t b0,
                        int64_t bl, int64_t c0, int64_t cl, hipStream_t st);
@@ -133,18 +141,17 @@ void launch_walk_src_fixup(int nsplit, const Split* splits, const double* carry,
 void launch_build_bundles(int64_t nbundles, const Bundle* bundles, const int* brun, const Run* runs, const int2* sd,
                           const int* eid, int G, int* bsrc, int* bdst, int* beid, int* rowmap, hipStream_t st);
 void launch_remap_ks(int64_t m, const int2* ks, const int* rowmap, int2* out, hipStream_t st);
+// bstate (nullable; one int per bundle): 0 while the bundle's FMaxN rows are known to hold -inf, so that a pruned walk
+// writes them once and not on every iteration; a walk that reads every edge sets it.  Only where the iterations write
+// one FMaxN in place.
 // CEp / bpack (launch_bundle_min): the walk reads the packed rows of the bundles whose base is nonzero.  CEp_out /
 // bpack (the prep walk, no pruning): the walk reads the FP32 rows and writes those bundles' packed rows to CEp_out.
 void launch_walk_max(int64_t nbundles, const Bundle* bundles, const int* gslot, const int* bsrc, const int* bdst,
                      const float* CE, const float* VR, int VRs, int Q, int Qs, const QStat* qs, float* FMaxN,
                      double* carry, int B, hipStream_t st, int* FA = nullptr, int* carg = nullptr,
                      const float* bmin = nullptr, const unsigned* CEp = nullptr, const unsigned* bpack = nullptr,
-                     unsigned* CEp_out = nullptr);
-// Plain-path fixup (FP32 normalised pieces): chunks of at most kFixChunk pieces, then the vertices of several
-// chunks from their partials (part: one [Qs] row per partial).
-constexpr int kFixChunk = 16;
-void launch_walk_max_fixup32(int nchunk, const Split* chunks, int nms, const Split* ms, const double* carry, int Qs,
-                             float* part, float* FMaxN, hipStream_t st);
+                     unsigned* CEp_out = nullptr, int* bstate = nullptr);
+// Taped walks (FA): the pieces' FP64 maxima and rows, combined one wave per split vertex.
 void launch_walk_max_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, const QStat* qs,
                            float* FMaxN, hipStream_t st, const int* carg = nullptr, int* FA = nullptr);
 void launch_vertex(int mode, const VertexArgs& a, int nblocks, hipStream_t st);

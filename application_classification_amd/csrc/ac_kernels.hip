@@ -524,12 +524,34 @@ void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStre
   hipLaunchKernelGGL(k_reduce_lse, dim3(ncol), dim3(256), 0, st, nparts, ncol, part, out);
 }
 
+// FMaxN rows of the split vertices to -inf, over nblocks blocks: the walk's pieces of a split vertex then raise its row
+// with atomic maxima.
+__device__ __forceinline__ void reset_split_rows(int block, int nblocks, int nsplit, const Split* __restrict__ splits,
+                                                 int Qs, float* __restrict__ FMaxN) {
+  const int L4 = Qs / 4;
+  const int64_t total = (int64_t)nsplit * L4;
+  for (int64_t i = (int64_t)block * blockDim.x + threadIdx.x; i < total; i += (int64_t)nblocks * blockDim.x) {
+    const int s = (int)(i / L4), j = (int)(i - (int64_t)s * L4);
+    reinterpret_cast<f4v*>(FMaxN)[(int64_t)splits[s].v * L4 + j] = f4v{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+  }
+}
+
+// Blocks that reset nsplit rows: four 16-byte stores a thread, at most 256 blocks.
+static int reset_blocks(int nsplit, int Qs) {
+  return (int)std::min<int64_t>(256, ((int64_t)nsplit * (Qs / 4) + 1023) / 1024);
+}
+
 // cnull != nullptr: the iteration's fills are lowered by the PNNL Cnull term, fillF = max VR - cnull[q] and
 // fillR = max VF - cnull[q] (test.py:148-149; cnull <= 0, so the fills rise and the pruning bound below, which assumes
 // the unraised fill, stays valid).
 __global__ __launch_bounds__(256) void k_reduce_q(int nparts, int Q, const QPart* __restrict__ part,
-                                                  const double* __restrict__ cnull, QStat* __restrict__ out) {
+                                                  const double* __restrict__ cnull, QStat* __restrict__ out,
+                                                  SplitRows rows) {
   __shared__ QPart red[256];
+  if ((int)blockIdx.x >= Q) {  // the blocks after the Q reducing ones
+    reset_split_rows(blockIdx.x - Q, gridDim.x - Q, rows.nsplit, rows.splits, rows.Qs, rows.FMaxN);
+    return;
+  }
   const int q = blockIdx.x, t = threadIdx.x;
   const QPart empty{-kInf, -kInf, lse_empty(), lse_empty(), -1, -1};
   QPart s = empty;
@@ -570,9 +592,11 @@ __global__ __launch_bounds__(256) void k_reduce_q(int nparts, int Q, const QPart
   }
 }
 
-void launch_reduce_q(int nparts, int Q, const QPart* part, QStat* out, hipStream_t st, const double* cnull) {
+void launch_reduce_q(int nparts, int Q, const QPart* part, QStat* out, hipStream_t st, const double* cnull,
+                     const SplitRows& rows) {
   if (Q == 0) return;
-  hipLaunchKernelGGL(k_reduce_q, dim3(Q), dim3(256), 0, st, nparts, Q, part, cnull, out);
+  hipLaunchKernelGGL(k_reduce_q, dim3(Q + reset_blocks(rows.nsplit, rows.Qs)), dim3(256), 0, st, nparts, Q, part, cnull,
+                     out, rows);
 }
 
 // Isolated-vertex columns: one pass over X[n][P] giving per-block partials of LSE(-X) and of (min X, lowest row).
@@ -666,17 +690,23 @@ void launch_iso_cols(int64_t n, int P, const float* X, int base, Lse* lpart, flo
 // Scalars of the prep state (src/main.cu:116-146): MU0 = LSM(-CV), RE0 = FE0 = LSM(-CE).  The column maximum of
 // MU0 sits at the minimum cost, where (x - m) = 0, so max_v MU0[v][p] = -log1p(t_p).
 __global__ void k_prep_scalars(int Q, const int* __restrict__ ps, const int* __restrict__ pd,
-                               const Lse2* __restrict__ cv, const Lse2* __restrict__ ce, QStat* __restrict__ qs) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+                               const Lse2* __restrict__ cv, const Lse2* __restrict__ ce, QStat* __restrict__ qs,
+                               SplitRows rows) {
+  if (blockIdx.x > 0) {
+    reset_split_rows(blockIdx.x - 1, gridDim.x - 1, rows.nsplit, rows.splits, rows.Qs, rows.FMaxN);
+    return;
+  }
+  const int q = threadIdx.x;  // Q <= 256
   if (q >= Q) return;
   qs[q] = QStat{-cv[ps[q]].l, -cv[pd[q]].l, ce[q].m, ce[q].l, ce[q].m, ce[q].l, -1, -1, kInf};
 }
 
 void launch_prep_scalars(int P, int Q, const int* ps, const int* pd, const Lse2* cv, const Lse2* ce, QStat* qs,
-                         hipStream_t st) {
+                         hipStream_t st, const SplitRows& rows) {
   (void)P;
   if (Q == 0) return;
-  hipLaunchKernelGGL(k_prep_scalars, dim3((Q + 255) / 256), dim3(256), 0, st, Q, ps, pd, cv, ce, qs);
+  hipLaunchKernelGGL(k_prep_scalars, dim3(1 + reset_blocks(rows.nsplit, rows.Qs)), dim3(256), 0, st, Q, ps, pd, cv, ce,
+                     qs, rows);
 }
 
 __global__ void k_fill(float* __restrict__ p, int64_t count, float value) {
@@ -884,6 +914,16 @@ int walk_batch() {
   return 4;  // measured at R-MAT 22 with packed costs and runs of 128 edges
 }
 
+// Float maximum by integer atomics, exact and independent of order: floats of positive sign order like signed ints,
+// those of negative sign inversely to their unsigned bit patterns.  A NaN wins whatever its sign.
+__device__ __forceinline__ void atomic_raise(float* addr, float v) {
+  if (v != v) v = __uint_as_float(0x7FC00000u);
+  if (signbit(v))
+    atomicMin(reinterpret_cast<unsigned*>(addr), __float_as_uint(v));
+  else
+    atomicMax(reinterpret_cast<int*>(addr), __float_as_int(v));
+}
+
 // kArg: also records, per (v, q), the row of the in-edge attaining the maximum (the first one in walk order on
 // ties; -1 if none) into FA[v][Qs], and per carry slot into carg, for the adjoint's max-subgradient routing.
 // kPrune (bmin != nullptr): exact pruning, per bundle and per lane (below).
@@ -897,7 +937,7 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_max(int64_t nbundles, const
                                                          int* __restrict__ carg, const float* __restrict__ bmin,
                                                          const unsigned* __restrict__ CEp,
                                                          const unsigned* __restrict__ bpack,
-                                                         unsigned* __restrict__ CEpo) {
+                                                         unsigned* __restrict__ CEpo, int* __restrict__ bstate) {
   const int L4 = Qs / 4, G = 64 / L4, VR4s = VRs / 4;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane / L4, j = lane - g * L4;
@@ -905,6 +945,8 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_max(int64_t nbundles, const
   if (g >= G || b >= nbundles) return;
   const Bundle Bd = bundles[b];
   const int slot = gslot[b * G + g];
+  // bstate (nullable): whether the bundle's FMaxN rows may hold anything but -inf.
+  const int written = kPrune && bstate ? bstate[b] : 1;
   // Exact pruning: an edge whose cost is at or above its pattern edge's bound cannot raise FMax above the fill, so a
   // term that is -inf instead gives the same FMax (the fill wins, as it would have).  A wave with no live lane skips
   // its bundle and writes -inf rows; a dead lane (none of its four pattern edges has a cost below the bound in this
@@ -921,17 +963,17 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_max(int64_t nbundles, const
       if (slot >= 0 && kArg) {
         double* o = carry + (int64_t)slot * Qs + 4 * j;
         o[0] = o[1] = o[2] = o[3] = -kInf;
-      } else if (slot >= 0) {
-        reinterpret_cast<f4v*>(carry)[(int64_t)slot * L4 + j] = f4v{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-      } else {
+      } else if (slot < 0 && written) {  // (a piece leaves its split vertex's row, reset to -inf, alone)
         const int v0 = bdst[Bd.base + g], v1 = bdst[Bd.base + (int64_t)(Bd.len - 1) * G + g];
         const float4 ninf = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
         if (v0 >= 0)
           for (int v = v0; v <= v1; ++v) reinterpret_cast<float4*>(FMaxN)[(int64_t)v * L4 + j] = ninf;
       }
+      if (bstate && written && lane == 0) bstate[b] = 0;
       return;
     }
   }
+  if (bstate && lane == 0 && (!kPrune || !written)) bstate[b] = 1;
   // log sum_e exp(FE[q][e]) as one FP64 value (its FP64 rounding is far below the FP32 rounding of the result).
   double sl[4];
 #pragma unroll
@@ -1085,10 +1127,12 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_max(int64_t nbundles, const
     o[3] = mx3;
     reinterpret_cast<int4*>(carg)[(int64_t)slot * L4 + j] = make_int4(a0, a1, a2, a3);
   } else if (slot >= 0) {
-    // A piece of a split vertex: its maximum, normalised and rounded like a finished row.  Rounding is monotone,
-    // so the maximum over the pieces of the rounded values is the rounded maximum (exact).
-    reinterpret_cast<f4v*>(carry)[(int64_t)slot * L4 + j] = f4v{(float)(mx0 - sl[0]), (float)(mx1 - sl[1]),
-                                                                (float)(mx2 - sl[2]), (float)(mx3 - sl[3])};
+    // A piece of a split vertex: its maximum, normalised and rounded like a finished row, raises the row.  Rounding
+    // is monotone, so the maximum over the pieces of the rounded values is the rounded maximum (exact, in any order).
+    const float o[4] = {(float)(mx0 - sl[0]), (float)(mx1 - sl[1]), (float)(mx2 - sl[2]), (float)(mx3 - sl[3])};
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (4 * j + u < Q && o[u] != -INFINITY) atomic_raise(FMaxN + (int64_t)cur * Qs + 4 * j + u, o[u]);
   } else if (cur >= 0) {
     AC_WK_EMIT(cur);
   }
@@ -1100,22 +1144,22 @@ static void launch_walk_max_t(int B, int nb, hipStream_t st, int64_t nbundles, c
                               const int* gslot, const int* bsrc, const int* bdst, const float* CE, const float* VR,
                               int VRs, int Q, int Qs, const QStat* qs, float* FMaxN, double* carry, int* FA,
                               int* carg, const float* bmin, const unsigned* CEp, const unsigned* bpack,
-                              unsigned* CEpo) {
+                              unsigned* CEpo, int* bstate) {
   switch (B) {
     case 1:
       hipLaunchKernelGGL((k_walk_max<kWithVR, 1, kArg, kPrune>), dim3(nb), dim3(kWalkBlock), 0, st, nbundles,
                          bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs, FMaxN, carry, FA, carg, bmin, CEp, bpack,
-                         CEpo);
+                         CEpo, bstate);
       break;
     case 4:
       hipLaunchKernelGGL((k_walk_max<kWithVR, 4, kArg, kPrune>), dim3(nb), dim3(kWalkBlock), 0, st, nbundles,
                          bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs, FMaxN, carry, FA, carg, bmin, CEp, bpack,
-                         CEpo);
+                         CEpo, bstate);
       break;
     default:
       hipLaunchKernelGGL((k_walk_max<kWithVR, 2, kArg, kPrune>), dim3(nb), dim3(kWalkBlock), 0, st, nbundles,
                          bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs, FMaxN, carry, FA, carg, bmin, CEp, bpack,
-                         CEpo);
+                         CEpo, bstate);
       break;
   }
 }
@@ -1125,35 +1169,35 @@ static void launch_walk_max_p(int B, int nb, hipStream_t st, int64_t nbundles, c
                               const int* gslot, const int* bsrc, const int* bdst, const float* CE, const float* VR,
                               int VRs, int Q, int Qs, const QStat* qs, float* FMaxN, double* carry, int* FA,
                               int* carg, const float* bmin, const unsigned* CEp, const unsigned* bpack,
-                              unsigned* CEpo) {
+                              unsigned* CEpo, int* bstate) {
   if (bmin)
     launch_walk_max_t<kWithVR, kArg, true>(B, nb, st, nbundles, bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs,
-                                           FMaxN, carry, FA, carg, bmin, CEp, bpack, CEpo);
+                                           FMaxN, carry, FA, carg, bmin, CEp, bpack, CEpo, bstate);
   else
     launch_walk_max_t<kWithVR, kArg, false>(B, nb, st, nbundles, bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs,
-                                            FMaxN, carry, FA, carg, bmin, CEp, bpack, CEpo);
+                                            FMaxN, carry, FA, carg, bmin, CEp, bpack, CEpo, bstate);
 }
 
 void launch_walk_max(int64_t nbundles, const Bundle* bundles, const int* gslot, const int* bsrc, const int* bdst,
                      const float* CE, const float* VR, int VRs, int Q, int Qs, const QStat* qs, float* FMaxN,
                      double* carry, int B, hipStream_t st, int* FA, int* carg, const float* bmin,
-                     const unsigned* CEp, const unsigned* bpack, unsigned* CEp_out) {
+                     const unsigned* CEp, const unsigned* bpack, unsigned* CEp_out, int* bstate) {
   if (nbundles == 0) return;
   const int nb = (int)((nbundles + kWalkBlock / 64 - 1) / (kWalkBlock / 64));
   if (!bpack) CEp = CEp_out = nullptr;
   if (CEp_out) CEp = nullptr;  // packing on the way: the walk reads the FP32 rows
   if (VR && FA)
     launch_walk_max_p<true, true>(B, nb, st, nbundles, bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs, FMaxN,
-                                  carry, FA, carg, bmin, CEp, bpack, CEp_out);
+                                  carry, FA, carg, bmin, CEp, bpack, CEp_out, bstate);
   else if (VR)
     launch_walk_max_p<true, false>(B, nb, st, nbundles, bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs, FMaxN,
-                                   carry, FA, carg, bmin, CEp, bpack, CEp_out);
+                                   carry, FA, carg, bmin, CEp, bpack, CEp_out, bstate);
   else if (FA)
     launch_walk_max_p<false, true>(B, nb, st, nbundles, bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs, FMaxN,
-                                   carry, FA, carg, bmin, CEp, bpack, CEp_out);
+                                   carry, FA, carg, bmin, CEp, bpack, CEp_out, bstate);
   else
     launch_walk_max_p<false, false>(B, nb, st, nbundles, bundles, gslot, bsrc, bdst, CE, VR, VRs, Q, Qs, qs, FMaxN,
-                                    carry, FA, carg, bmin, CEp, bpack, CEp_out);
+                                    carry, FA, carg, bmin, CEp, bpack, CEp_out, bstate);
 }
 
 // The base of a bundle's 24-bit cost codes from its least and largest cost bit patterns over columns q < Q, +inf
@@ -1341,80 +1385,6 @@ __global__ __launch_bounds__(256) void k_walk_max_fixup(int nsplit, const Split*
     reinterpret_cast<float4*>(FMaxN)[(int64_t)S.v * L4 + j] = out;
     if (carg) reinterpret_cast<int4*>(FA)[(int64_t)S.v * L4 + j] = make_int4(oarg[0], oarg[1], oarg[2], oarg[3]);
   }
-}
-
-// Plain path: the pieces hold normalised FP32 maxima, and their maximum is exact in any order.  Pieces are grouped
-// into chunks of at most kFixChunk (Split{v, first piece, count, out}); one group of Qs/4 lanes takes a chunk with
-// all its loads in flight and writes the vertex's row (out < 0) or chunk partial `out`; vertices of several chunks
-// (MSplit{v, first partial, count}) are then finished from their partials, one wave each.
-__global__ __launch_bounds__(256) void k_fix_chunks(int nchunk, const Split* __restrict__ chunks,
-                                                    const f4v* __restrict__ carry, int Qs, f4v* __restrict__ part,
-                                                    f4v* __restrict__ FMaxN) {
-  const int lane = threadIdx.x & 63;
-  const int L4 = Qs / 4, G = 64 / L4;
-  const int g = lane / L4, j = lane - g * L4;
-  if (g >= G) return;
-  const int64_t ngroups = (int64_t)gridDim.x * (blockDim.x / 64) * G;
-  for (int64_t ci = ((int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6)) * G + g; ci < nchunk;
-       ci += ngroups) {
-    const Split C = chunks[ci];
-    const f4v* c = carry + (int64_t)C.first * L4 + j;
-    f4v x[kFixChunk];
-#pragma unroll
-    for (int k = 0; k < kFixChunk; ++k)
-      x[k] = k < C.count ? c[(int64_t)k * L4] : f4v{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
-    f4v m = x[0];
-#pragma unroll
-    for (int k = 1; k < kFixChunk; ++k)
-      m = f4v{fmaxf(m.x, x[k].x), fmaxf(m.y, x[k].y), fmaxf(m.z, x[k].z), fmaxf(m.w, x[k].w)};
-    if (C.pad < 0)
-      FMaxN[(int64_t)C.v * L4 + j] = m;
-    else
-      part[(int64_t)C.pad * L4 + j] = m;
-  }
-}
-
-__global__ __launch_bounds__(256) void k_fix_multi(int nms, const Split* __restrict__ ms, const f4v* __restrict__ part,
-                                                   int Qs, f4v* __restrict__ FMaxN) {
-  const int lane = threadIdx.x & 63;
-  const int L4 = Qs / 4, G = 64 / L4;
-  const int g = lane / L4, j = lane - g * L4;
-  const int64_t w = (int64_t)blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
-  if (w >= nms) return;
-  const Split M = ms[w];
-  f4v m0 = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}, m1 = m0;
-  if (g < G) {
-    int c = g;
-    for (; c + G < M.count; c += 2 * G) {
-      const f4v a = part[(int64_t)(M.first + c) * L4 + j], b = part[(int64_t)(M.first + c + G) * L4 + j];
-      m0 = f4v{fmaxf(m0.x, a.x), fmaxf(m0.y, a.y), fmaxf(m0.z, a.z), fmaxf(m0.w, a.w)};
-      m1 = f4v{fmaxf(m1.x, b.x), fmaxf(m1.y, b.y), fmaxf(m1.z, b.z), fmaxf(m1.w, b.w)};
-    }
-    if (c < M.count) {
-      const f4v a = part[(int64_t)(M.first + c) * L4 + j];
-      m0 = f4v{fmaxf(m0.x, a.x), fmaxf(m0.y, a.y), fmaxf(m0.z, a.z), fmaxf(m0.w, a.w)};
-    }
-  }
-  f4v m = {fmaxf(m0.x, m1.x), fmaxf(m0.y, m1.y), fmaxf(m0.z, m1.z), fmaxf(m0.w, m1.w)};
-  // Across the groups: lane (0, j) gathers lanes (gg, j).
-  for (int gg = 1; gg < G; ++gg) {
-    const int src = gg * L4 + j;
-    const f4v o = {__shfl(m.x, src, 64), __shfl(m.y, src, 64), __shfl(m.z, src, 64), __shfl(m.w, src, 64)};
-    m = f4v{fmaxf(m.x, o.x), fmaxf(m.y, o.y), fmaxf(m.z, o.z), fmaxf(m.w, o.w)};
-  }
-  if (g == 0) FMaxN[(int64_t)M.v * L4 + j] = m;
-}
-
-void launch_walk_max_fixup32(int nchunk, const Split* chunks, int nms, const Split* ms, const double* carry, int Qs,
-                             float* part, float* FMaxN, hipStream_t st) {
-  if (nchunk == 0) return;
-  const int G = 64 / (Qs / 4);
-  const int blocks = (int)std::min<int64_t>(((int64_t)nchunk + 4 * G - 1) / (4 * G), 8192);
-  hipLaunchKernelGGL(k_fix_chunks, dim3(blocks), dim3(256), 0, st, nchunk, chunks, reinterpret_cast<const f4v*>(carry),
-                     Qs, reinterpret_cast<f4v*>(part), reinterpret_cast<f4v*>(FMaxN));
-  if (nms > 0)
-    hipLaunchKernelGGL(k_fix_multi, dim3((nms + 3) / 4), dim3(256), 0, st, nms, ms, reinterpret_cast<const f4v*>(part),
-                       Qs, reinterpret_cast<f4v*>(FMaxN));
 }
 
 void launch_walk_max_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, const QStat* qs,

@@ -165,7 +165,7 @@ void* ac_stream(ac_ctx* ctx);
 #define AC_STAGE_VERTEX_A 1    /* VF / VR, column maxima, edge log-sum-exps (steps 1, 3a, 4a)                 */
 #define AC_STAGE_REDUCE_A 2    /* combine the per-block partials of stage 1                                   */
 #define AC_STAGE_EDGE_WALK 3   /* destination maxima over the data edges (steps 2, 4b, 4c)                    */
-#define AC_STAGE_WALK_FIXUP 4  /* combine the pieces of vertices with very long in-edge lists                 */
+#define AC_STAGE_WALK_FIXUP 4  /* combine the pieces of vertices with very long in-edge lists (taped runs)     */
 #define AC_STAGE_VERTEX_C 5    /* MU column log-sum-exp (step 5)                                               */
 #define AC_STAGE_REDUCE_C 6    /* combine the per-block partials of stage 5                                   */
 #define AC_STAGE_OUTPUT 7      /* normalised MU written in dn x pn order (src/main.cu:247)                     */
