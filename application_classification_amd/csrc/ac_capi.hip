@@ -689,7 +689,7 @@ static int ensure_work(ac_ctx* ctx) {
   if (std::equal(key, key + 5, ctx->work_key)) return AC_OK;
   const int64_t n = ctx->dn;
   const int P = ctx->P, Q = ctx->Q, Qs = ctx->Qs;
-  ctx->VT = ac::vertex_tile(P, Q);
+  ctx->VT = ac::vertex_tile(ctx->n_act, P, Q);
   const int64_t ntiles = (std::max<int64_t>(ctx->n_act, 1) + ctx->VT - 1) / ctx->VT;
   {
     ac::VertexArgs va{};

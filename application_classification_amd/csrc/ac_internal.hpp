@@ -97,15 +97,15 @@ struct VertexArgs {
   // >= o_end have no out-edge (VFm = -inf, minCEo = +inf, lsO = 0).
   int64_t f_end, o_lo, o_hi, o_end;
   const IsoCol* iso;    // [P] isolated vertices' columns (nullptr: none); modes A and C write their share as the
-                        // extra partial slot gridDim.x
+                        // extra partial slot after those of the tile blocks
   const int* ps;
   const int* pd;
   const int* inc_off;  // [P + 1]
   const int* inc;      // incidence of each pattern vertex: (q << 1) | (1 if RMax term else 0), ascending q
   const QStat* qs;     // scalars that finish FMax / RMax of the state being read
   const Lse2* pst;     // log-sum-exp of each MU column
-  QPart* qpart;        // [gridDim + 1][Q]
-  Lse* ppart;          // [gridDim + 1][P]
+  QPart* qpart;        // [tile blocks + 1][Q]
+  Lse* ppart;          // [tile blocks + 1][P]
   int first;           // MU = LSM(-CV): the prep state, no FMax / RMax terms
   int track_arg;       // mode A: record the vertices of the column maxima (QStat vF / vR)
 };
@@ -163,6 +163,6 @@ void launch_copy_cols(int64_t n, int P, int c0, int ncol, const float* src, floa
 int walk_blocks(int64_t nruns, int Qs);
 int walk_groups(int Qs);  // runs per bundle: 64 / (Qs / 4)
 int walk_batch();         // default steps per batch of the bundle walk: 1, 2 or 4 (bundle lengths are multiples of it)
-int vertex_tile(int P, int Q);
+int vertex_tile(int64_t n, int P, int Q);  // rows per tile for n vertices
 
 }  // namespace ac

@@ -458,12 +458,35 @@ void launch_cdist(int64_t nrows, const int* idx, const float* feats, int dim, co
   }
 }
 
+// Merge of a block's per-thread accumulators by column: thread t holds s of column t % C, C <= NT, threads
+// t >= rows * C none.  Thread c < C gets column c's, its rows summed in order.  sh: (rows + 1) * C doubles.
+__device__ __forceinline__ Lse block_columns_lse(const Lse& s, int C, int rows, double* sh) {
+  const int t = threadIdx.x;
+  const bool active = t < rows * C;
+  if (active) sh[t] = s.m;
+  __syncthreads();
+  Lse acc = lse_empty();
+  if (t < C) {
+    for (int r = 0; r < rows; ++r) acc.m = fmax(acc.m, sh[r * C + t]);
+    sh[rows * C + t] = acc.m;
+  }
+  __syncthreads();
+  const double x = active ? lse_rescaled(s, sh[rows * C + t % C]) : 0.0;
+  if (active) sh[t] = x;
+  __syncthreads();
+  if (t < C) {
+    bool seen = false;
+    for (int r = 0; r < rows; ++r) lse_sum_step(acc.t, seen, sh[r * C + t]);
+  }
+  return acc;
+}
+
 // ---------------------------------------------------------------------------------------------------------------
 // Column log-sum-exp of -X over the n rows of X[n][P] (the prep's LSM(-CV) normaliser, src/main.cu:117).
 
 __global__ __launch_bounds__(256) void k_col_lse_neg(int64_t n, int P, const float* __restrict__ X,
                                                      Lse* __restrict__ part) {
-  __shared__ Lse red[256];
+  __shared__ double red[512];
   const int t = threadIdx.x;
   const int RP = 256 / P;
   const bool active = t < RP * P;
@@ -472,51 +495,54 @@ __global__ __launch_bounds__(256) void k_col_lse_neg(int64_t n, int P, const flo
   if (active)
     for (int64_t v = (int64_t)blockIdx.x * RP + t / P; v < n; v += (int64_t)gridDim.x * RP)
       lse_add(acc, -(double)X[v * P + p]);
-  red[t] = acc;
-  __syncthreads();
-  if (t < P) {
-    Lse s = lse_empty();
-    for (int r = 0; r < RP; ++r) s = lse_merge(s, red[r * P + t]);
-    part[(int64_t)blockIdx.x * P + t] = s;
-  }
+  const Lse s = block_columns_lse(acc, P, RP, red);
+  if (t < P) part[(int64_t)blockIdx.x * P + t] = s;
 }
 
 void launch_col_lse_neg(int64_t n, int P, const float* X, Lse* part, int nblocks, hipStream_t st) {
   hipLaunchKernelGGL(k_col_lse_neg, dim3(nblocks), dim3(256), 0, st, n, P, X, part);
 }
 
-// Partials a thread of a fixed-order reduction loads before merging them: one memory round trip per batch rather
-// than one per partial (and per field).  Slots past the last partial load the last partial (an in-bounds address)
-// and then hold the empty partial, whose merge is an exact identity, so the merge sequence is the same for every
-// batch size.
-constexpr int kRedBatchLse = 8, kRedBatchQ = 4;
+// Partials a thread of a fixed-order reduction holds in registers, all loaded at once: kRed* x 256 partials take one
+// memory round trip and one exponential each.  Further ones are merged into them one by one.  Slots past the last
+// partial load the last partial (an in-bounds address) and then hold the empty one.
+constexpr int kRedLse = 8, kRedQ = 5;
 
 // Reduce per-block partials [nparts][ncol] column by column in a fixed order (deterministic).
 __global__ __launch_bounds__(256) void k_reduce_lse(int nparts, int ncol, const Lse* __restrict__ part,
                                                     Lse2* __restrict__ out) {
-  __shared__ Lse red[256];
+  __shared__ double red[8];
   const int c = blockIdx.x, t = threadIdx.x;
-  Lse s = lse_empty();
-  for (int b0 = t; b0 < nparts; b0 += 256 * kRedBatchLse) {
-    Lse v[kRedBatchLse];
+  Lse v[kRedLse];
 #pragma unroll
-    for (int u = 0; u < kRedBatchLse; ++u) {
+  for (int u = 0; u < kRedLse; ++u) {
+    const int b = t + u * 256;
+    v[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * ncol + c];
+  }
+#pragma unroll
+  for (int u = 0; u < kRedLse; ++u)
+    if (t + u * 256 >= nparts) v[u] = lse_empty();
+  for (int b0 = 256 * kRedLse + t; b0 < nparts; b0 += 256 * kRedLse) {
+    Lse w[kRedLse];
+#pragma unroll
+    for (int u = 0; u < kRedLse; ++u) {
       const int b = b0 + u * 256;
-      v[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * ncol + c];
+      w[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * ncol + c];
     }
 #pragma unroll
-    for (int u = 0; u < kRedBatchLse; ++u)
-      if (b0 + u * 256 >= nparts) v[u].m = -kInf;
+    for (int u = 0; u < kRedLse; ++u)
+      if (b0 + u * 256 < nparts) v[u] = lse_merge(v[u], w[u]);
+  }
+  double m = v[0].m;
 #pragma unroll
-    for (int u = 0; u < kRedBatchLse; ++u) s = lse_merge(s, v[u]);
-  }
-  red[t] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) red[t] = lse_merge(red[t], red[t + w]);
-    __syncthreads();
-  }
-  if (t == 0) out[c] = Lse2{red[0].m, log1p(red[0].t)};
+  for (int u = 1; u < kRedLse; ++u) m = fmax(m, v[u].m);
+  const double M = block_max<256>(m, red);
+  double sum = 0.0;
+  bool seen = false;
+#pragma unroll
+  for (int u = 0; u < kRedLse; ++u) lse_sum_step(sum, seen, lse_rescaled(v[u], M));
+  sum = block_lse_sum<256>(sum, seen, red);
+  if (t == 0) out[c] = Lse2{M, log1p(sum)};
 }
 
 void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStream_t st) {
@@ -547,39 +573,72 @@ static int reset_blocks(int nsplit, int Qs) {
 __global__ __launch_bounds__(256) void k_reduce_q(int nparts, int Q, const QPart* __restrict__ part,
                                                   const double* __restrict__ cnull, QStat* __restrict__ out,
                                                   SplitRows rows) {
-  __shared__ QPart red[256];
+  __shared__ double red[8], redv[8];
+  __shared__ int redi[8];
   if ((int)blockIdx.x >= Q) {  // the blocks after the Q reducing ones
     reset_split_rows(blockIdx.x - Q, gridDim.x - Q, rows.nsplit, rows.splits, rows.Qs, rows.FMaxN);
     return;
   }
   const int q = blockIdx.x, t = threadIdx.x;
   const QPart empty{-kInf, -kInf, lse_empty(), lse_empty(), -1, -1};
-  QPart s = empty;
-  for (int b0 = t; b0 < nparts; b0 += 256 * kRedBatchQ) {
-    QPart v[kRedBatchQ];
+  QPart v[kRedQ];
 #pragma unroll
-    for (int u = 0; u < kRedBatchQ; ++u) {
+  for (int u = 0; u < kRedQ; ++u) {
+    const int b = t + u * 256;
+    v[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * Q + q];
+  }
+#pragma unroll
+  for (int u = 0; u < kRedQ; ++u)
+    if (t + u * 256 >= nparts) v[u] = empty;
+  for (int b0 = 256 * kRedQ + t; b0 < nparts; b0 += 256 * kRedQ) {
+    QPart w[kRedQ];
+#pragma unroll
+    for (int u = 0; u < kRedQ; ++u) {
       const int b = b0 + u * 256;
-      v[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * Q + q];
+      w[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * Q + q];
     }
 #pragma unroll
-    for (int u = 0; u < kRedBatchQ; ++u)
-      if (b0 + u * 256 >= nparts) v[u] = empty;
-#pragma unroll
-    for (int u = 0; u < kRedBatchQ; ++u) qpart_merge(s, v[u]);
+    for (int u = 0; u < kRedQ; ++u)
+      if (b0 + u * 256 < nparts) qpart_merge(v[u], w[u]);
   }
-  red[t] = s;
+  QPart s = v[0];
+#pragma unroll
+  for (int u = 1; u < kRedQ; ++u) {
+    argmax_merge(s.vfmax, s.avf, v[u].vfmax, v[u].avf);
+    argmax_merge(s.vrmax, s.avr, v[u].vrmax, v[u].avr);
+    s.re.m = fmax(s.re.m, v[u].re.m);
+    s.fe.m = fmax(s.fe.m, v[u].fe.m);
+  }
+  s.re.m = block_max<256>(s.re.m, red);
+  s.fe.m = block_max<256>(s.fe.m, red);
+  s.re.t = s.fe.t = 0.0;
+  bool ore = false, ofe = false;
+#pragma unroll
+  for (int u = 0; u < kRedQ; ++u) {
+    lse_sum_step(s.re.t, ore, lse_rescaled(v[u].re, s.re.m));
+    lse_sum_step(s.fe.t, ofe, lse_rescaled(v[u].fe, s.fe.m));
+  }
+  s.re.t = block_lse_sum<256>(s.re.t, ore, red);
+  s.fe.t = block_lse_sum<256>(s.fe.t, ofe, redv);
+  // The maxima with their vertices (ties: the lowest, in any order).
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    argmax_merge(s.vfmax, s.avf, __shfl_xor(s.vfmax, o, 64), __shfl_xor(s.avf, o, 64));
+    argmax_merge(s.vrmax, s.avr, __shfl_xor(s.vrmax, o, 64), __shfl_xor(s.avr, o, 64));
+  }
+  __syncthreads();  // red and redv read
+  if ((t & 63) == 0) {
+    const int w = t >> 6;
+    red[w] = s.vfmax, red[4 + w] = s.vrmax;
+    redi[w] = s.avf, redi[4 + w] = s.avr;
+  }
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) {
-      QPart a = red[t];
-      qpart_merge(a, red[t + w]);
-      red[t] = a;
-    }
-    __syncthreads();
-  }
   if (t == 0) {
-    const QPart r = red[0];
+    for (int w = 1; w < 4; ++w) {
+      argmax_merge(s.vfmax, s.avf, red[w], redi[w]);
+      argmax_merge(s.vrmax, s.avr, red[4 + w], redi[4 + w]);
+    }
+    const QPart r = s;
     // Edge pruning bound.  An edge term is (VR[src] - CE) - LSE_FE with VR[src] <= fillF (rounded to FP32 once),
     // so it cannot exceed fillF when CE + LSE_FE >= 2^-22 (|fillF| + |CE| + |LSE_FE|); cthr = -LSE_FE plus four
     // times that margin (a cost near the bound has |CE| ~ |LSE_FE|; a larger one clears it by itself).
@@ -602,7 +661,7 @@ void launch_reduce_q(int nparts, int Q, const QPart* part, QStat* out, hipStream
 // Isolated-vertex columns: one pass over X[n][P] giving per-block partials of LSE(-X) and of (min X, lowest row).
 __global__ __launch_bounds__(256) void k_iso_cols(int64_t n, int P, const float* __restrict__ X, Lse* __restrict__ lpart,
                                                   float* __restrict__ pv, int* __restrict__ pi) {
-  __shared__ Lse red[256];
+  __shared__ double red[512];
   __shared__ float rv[256];
   __shared__ int ri[256];
   const int t = threadIdx.x, RP = 256 / P;
@@ -620,14 +679,11 @@ __global__ __launch_bounds__(256) void k_iso_cols(int64_t n, int P, const float*
         bi = (int)v;
       }
     }
-  red[t] = acc;
   rv[t] = best;
   ri[t] = bi;
-  __syncthreads();
+  const Lse s = block_columns_lse(acc, P, RP, red);
   if (t < P) {
-    Lse s = lse_empty();
     for (int r = 0; r < RP; ++r) {
-      s = lse_merge(s, red[r * P + t]);
       const float x = rv[r * P + t];
       const int xi = ri[r * P + t];
       if (x < best || (x == best && xi < bi)) {
@@ -645,7 +701,7 @@ __global__ __launch_bounds__(256) void k_iso_cols(int64_t n, int P, const float*
 __global__ __launch_bounds__(256) void k_iso_final(int nparts, int P, int base, const Lse* __restrict__ lpart,
                                                    const float* __restrict__ pv, const int* __restrict__ pi,
                                                    IsoCol* __restrict__ out) {
-  __shared__ Lse rs[256];
+  __shared__ double rs[8];
   __shared__ float rv[256];
   __shared__ int ri[256];
   const int p = blockIdx.x, t = threadIdx.x;
@@ -661,13 +717,15 @@ __global__ __launch_bounds__(256) void k_iso_final(int nparts, int P, int base, 
       bi = xi;
     }
   }
-  rs[t] = s;
   rv[t] = best;
   ri[t] = bi;
-  __syncthreads();
+  const double M = block_max<256>(s.m, rs);
+  double sum = 0.0;
+  bool seen = false;
+  lse_sum_step(sum, seen, lse_rescaled(s, M));
+  sum = block_lse_sum<256>(sum, seen, rs);
   for (int w = 128; w > 0; w >>= 1) {
     if (t < w) {
-      rs[t] = lse_merge(rs[t], rs[t + w]);
       if (rv[t + w] < rv[t] || (rv[t + w] == rv[t] && ri[t + w] < ri[t])) {
         rv[t] = rv[t + w];
         ri[t] = ri[t + w];
@@ -677,7 +735,7 @@ __global__ __launch_bounds__(256) void k_iso_final(int nparts, int P, int base, 
   }
   // A column whose isolated costs are all +inf has no finite share: treat it as empty.
   if (t == 0)
-    out[p] = ri[0] == INT_MAX ? IsoCol{-kInf, 0.0, INFINITY, -1} : IsoCol{rs[0].m, rs[0].t, rv[0], base + ri[0]};
+    out[p] = ri[0] == INT_MAX ? IsoCol{-kInf, 0.0, INFINITY, -1} : IsoCol{M, sum, rv[0], base + ri[0]};
 }
 
 void launch_iso_cols(int64_t n, int P, const float* X, int base, Lse* lpart, float* pv, int* pi, int nparts,
@@ -764,7 +822,7 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
                                                          int Q, int Qs, float* __restrict__ minCEo,
                                                          float* __restrict__ lsO, float* __restrict__ VFm,
                                                          double* __restrict__ carry, Lse* __restrict__ gpart) {
-  __shared__ Lse red[kWalkBlock * 4];
+  __shared__ double red[kWalkBlock * 4 + 256];
   const int L4 = Qs / 4, G = 64 / L4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int g = lane / L4, j = lane - g * L4;
@@ -827,15 +885,28 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
       emit(cur);
     }
   }
-  // Block partial of the global log-sum-exp, merged in a fixed (wave, group) order per pattern edge.
+  // Block partial of the global log-sum-exp, per pattern edge in a fixed (wave, group) order: the groups' maxima, then
+  // every group's share of the largest, then their sum.
+  const int slots = (kWalkBlock / 64) * G, sl = wave * G + g;  // [slots][Qs], then the maxima [Qs]
+  if (g < G)
 #pragma unroll
-  for (int c = 0; c < 4; ++c) red[threadIdx.x * 4 + c] = glob[c];
+    for (int c = 0; c < 4; ++c) red[sl * Qs + 4 * j + c] = glob[c].m;
+  __syncthreads();
+  double* mx = red + kWalkBlock * 4;
+  for (int q = threadIdx.x; q < Qs; q += kWalkBlock) {
+    double m = -kInf;
+    for (int i = 0; i < slots; ++i) m = fmax(m, red[i * Qs + q]);
+    mx[q] = m;
+  }
+  __syncthreads();
+  if (g < G)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) red[sl * Qs + 4 * j + c] = lse_rescaled(glob[c], mx[4 * j + c]);
   __syncthreads();
   for (int q = threadIdx.x; q < Q; q += kWalkBlock) {
-    const int jj = q >> 2, c = q & 3;
-    Lse acc = lse_empty();
-    for (int w = 0; w < kWalkBlock / 64; ++w)
-      for (int gg = 0; gg < G; ++gg) acc = lse_merge(acc, red[(w * 64 + gg * L4 + jj) * 4 + c]);
+    Lse acc{mx[q], 0.0};
+    bool seen = false;
+    for (int i = 0; i < slots; ++i) lse_sum_step(acc.t, seen, red[i * Qs + q]);
     gpart[(int64_t)blockIdx.x * Q + q] = acc;
   }
 }
@@ -1395,17 +1466,25 @@ void launch_walk_max_fixup(int nsplit, const Split* splits, const double* carry,
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Vertex passes.  A block takes tiles of VT (<= 64) consecutive vertices.  The tile's rows of FMaxN and VFm (and,
-// in mode A, of minCEo and lsO), contiguous in HBM, and of CV are staged in LDS as FP32, into rows padded to an odd
-// stride; the next tile's rows are loaded into registers (coalesced float4 loads) while the current tile is
-// computed, so the loads of one tile overlap the arithmetic of the previous one.
-//   p-phase : wave w handles pattern vertices p = w, w + 4, ...; lane r is tile row r, so the pattern's incidence
-//             structure is wave-uniform (no divergence).  MU_pre = -CV + sum over the incidences of p in ascending q
-//             (FMax term before RMax term; src/ac.hxx:164-170 made deterministic), FMax = max(fillF, FMaxN),
-//             RMax = max(fillR, VFm - LSE_RE).  Mode A keeps MU = MU_pre - LSE_MU in LDS (FP64), mode OUT writes it
-//             in dn x pn order, mode C reduces the column's log-sum-exp across the wave.
+// Vertex passes.  A block takes tiles of VT (a power of two, <= 64) consecutive vertices.  The tile's rows of FMaxN and
+// VFm (and, in mode A, of minCEo and lsO), contiguous in HBM, and of CV are staged in LDS as FP32, into rows padded to an
+// odd stride; the next tile's rows are loaded into registers (coalesced float4 loads) while the current tile is
+// computed, so the loads of one tile overlap the arithmetic of the previous one.  Each thread's LDS positions are the
+// same in every tile and are kept in registers: forming them took ten integer divisions per thread and tile.
+//   p-phase : a lane per (tile row, pattern vertex), VT lanes to a pattern vertex: a wave handles 64 / VT of them at a
+//             time.  MU_pre = -CV + sum over the incidences of p in ascending q (FMax term before RMax term;
+//             src/ac.hxx:164-170 made deterministic), FMax = max(fillF, FMaxN), RMax = max(fillR, VFm - LSE_RE).
+//             Mode A keeps MU = MU_pre - LSE_MU in LDS (FP64), mode OUT writes it in dn x pn order, mode C accumulates
+//             the column's log-sum-exp per lane.
 //   q-phase : (mode A) a thread per (q, row): VF = MU[pd] - FMax, VR = MU[ps] - RMax (src/main.cu:165-176), stored
 //             with coalesced writes, and the per-q maxima / edge log-sum-exps accumulated in registers.
+// At R-MAT 22 (64-row tiles) passes A and C are bound by their streams; on small graphs, and with patterns whose rows
+// fill a tile with few vertices, by the chain through one block: its tables, its tiles one after the other, the merge
+// of its partials.  Hence short tiles where there are few (vertex_tile), lanes shared among pattern vertices, and
+// merges that take one exponential however many partials they merge.  Passes A / C per launch, before (a wave per
+// pattern vertex whatever the tile's height, isolated vertices on block 0's way, serial merges) and now: 1,000 vertices
+// with a 10/12 pattern 20.0 / 8.5 -> 11.0 / 6.2 us; 50,001 with 40/70 48.9 / 44.4 -> 32.3 / 23.8 us; R-MAT 16 slabs of
+// 128 pattern edges 98.5 / 108.3 -> 67.7 / 30.6 us; R-MAT 20 with 16/24 105.7 / 58.9 -> 104.5 / 48.0 us.
 
 constexpr int kVTMax = 64;
 // Staged tile limits: VT * Qs <= 2048 and VT * P <= 2048 floats, for every block size NT (256 or 512).
@@ -1423,19 +1502,24 @@ static size_t vertex_lds_bytes(int mode, int VT, int P, int Q, int Qs) {
   size_t b = (size_t)(2 * P) * sizeof(double);                               // MU normalisers
   b += (size_t)(2 * Q + 1) * sizeof(IncRec);                                 // incidence records (+ one pad)
   if (mode != kModeC) b += (size_t)(P + 1) * VT * sizeof(double);            // MU
-  if (mode == kModeC) b += (size_t)P * sizeof(Lse);                          // column accumulators
   const int nst = mode == kModeA ? 4 : 2;                                    // staged [VT][Qs] arrays
   b += (size_t)VT * (nst * (Qs + 1) + (P + 1)) * sizeof(float);              // staged rows
+  b += (size_t)(P + 1) * sizeof(int);                                        // incidence offsets
   if (mode == kModeOut) b += (size_t)VT * sizeof(int);                       // the tile's caller ids
   return (b + 15) / 16 * 16;
 }
 
-int vertex_tile(int P, int Q) {
+// Tiles wanted at least: two for each of the 256 CUs.
+constexpr int kTilesWanted = 512;
+
+int vertex_tile(int64_t n, int P, int Q) {
   const int Qs = std::max(4, (Q + 3) / 4 * 4);
   int vt = kVTMax;
   if (const char* e = std::getenv("AC_VERTEX_TILE")) {  // tuning override: rows per tile, 8, 16, 32 or 64
     const int v = std::atoi(e);
     if (v == 8 || v == 16 || v == 32 || v == 64) vt = v;
+  } else {
+    while (vt > 8 && (n + vt - 1) / vt < kTilesWanted) vt /= 2;
   }
   while (vt > 4 && (vertex_lds_bytes(kModeA, vt, P, Q, Qs) > 65536 || vt * Qs > kTileFloats ||
                     vt * P > kTileFloats))
@@ -1443,158 +1527,91 @@ int vertex_tile(int P, int Q) {
   return vt;
 }
 
-// log-sum-exp of one value per lane over the wave (-inf lanes contribute nothing); fixed butterfly order.
-__device__ __forceinline__ Lse wave_lse(double x) {
-  double m = x;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
-  if (m == -kInf) return lse_empty();
-  const unsigned long long at_max = __ballot(x == m);
-  const int first = __ffsll((long long)at_max) - 1;
-  double e = ((int)(threadIdx.x & 63) == first) ? 0.0 : (double)__expf((float)(x - m));
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
-  return Lse{m, e};
-}
-
-// Butterfly merge of one log-sum-exp accumulator per lane over the wave (fixed order; lane 0's result is used).
-__device__ __forceinline__ Lse wave_lse_merge(Lse s) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const Lse w{__shfl_xor(s.m, o, 64), __shfl_xor(s.t, o, 64)};
-    s = lse_merge(s, w);
-  }
-  return s;
-}
-
 // Read-only inputs seen through the constant address space: loads at wave-uniform indexes become scalar loads, and
 // branches on their values scalar branches.
 typedef const __attribute__((address_space(4))) int cint_t;
 
-// The isolated vertices' share, in closed form (block 0 of a vertex pass writes it as one extra partial).  Their
-// FMaxN = VFm = -inf rows make MU_pre = -CV + K_p, K_p the sum of the fills of p's incidences (in the vertex pass's
-// own operation sequence), so MU is largest at the least-cost isolated vertex and the column log-sum-exp is
+// The isolated vertices' share, in closed form (a block of a vertex pass of its own writes it as one extra partial).
+// Their FMaxN = VFm = -inf rows make MU_pre = -CV + K_p, K_p the sum of the fills of p's incidences (in the vertex
+// pass's own operation sequence), so MU is largest at the least-cost isolated vertex and the column log-sum-exp is
 // LSE(-CV) + K_p.  They have no out-edges: no edge terms.
-__device__ double iso_kp(const VertexArgs& a, int p, bool sums, double acc) {
+__device__ double iso_kp(const IncRec* recs, const int* ioff, int p, bool sums, double acc) {
   if (sums)
-    for (int k = a.inc_off[p]; k < a.inc_off[p + 1]; ++k) {
-      const int code = a.inc[k], qq = code >> 1;
-      acc += (code & 1) ? fmax(a.qs[qq].fillR, -kInf) : fmax(a.qs[qq].fillF, (double)(-INFINITY));
-    }
+    for (int k = ioff[p]; k < ioff[p + 1]; ++k) acc += fmax(recs[k].fill, -kInf);
   return acc;
 }
 
-__device__ QPart iso_qpart(const VertexArgs& a, int q) {
+__device__ QPart iso_qpart(const VertexArgs& a, const IncRec* recs, const int* ioff, int q) {
   QPart w{-kInf, -kInf, lse_empty(), lse_empty(), -1, -1};
   if (!a.iso) return w;
   const int pd = a.pd[q], ps = a.ps[q];
-  const double fm = fmax(a.qs[q].fillF, (double)(-INFINITY)), rm = fmax(a.qs[q].fillR, -kInf);
+  const double fm = fmax(a.qs[q].fillF, -kInf), rm = fmax(a.qs[q].fillR, -kInf);
   if (a.iso[pd].vmin >= 0) {
-    const double mu = (iso_kp(a, pd, !a.first, -(double)a.iso[pd].cmin) - a.pst[pd].m) - a.pst[pd].l;
+    const double mu = (iso_kp(recs, ioff, pd, !a.first, -(double)a.iso[pd].cmin) - a.pst[pd].m) - a.pst[pd].l;
     w.vfmax = mu - fm;
     if (w.vfmax > -kInf) w.avf = a.iso[pd].vmin;  // as in the vertex pass, -inf records no vertex
   }
   if (a.iso[ps].vmin >= 0) {
-    const double mu = (iso_kp(a, ps, !a.first, -(double)a.iso[ps].cmin) - a.pst[ps].m) - a.pst[ps].l;
+    const double mu = (iso_kp(recs, ioff, ps, !a.first, -(double)a.iso[ps].cmin) - a.pst[ps].m) - a.pst[ps].l;
     w.vrmax = mu - rm;
     if (w.vrmax > -kInf) w.avr = a.iso[ps].vmin;
   }
   return w;
 }
 
-__device__ Lse iso_lse(const VertexArgs& a, int p) {
+__device__ Lse iso_lse(const VertexArgs& a, const IncRec* recs, const int* ioff, int p) {
   if (!a.iso || a.iso[p].vmin < 0) return lse_empty();
-  const double m = iso_kp(a, p, !a.first, a.iso[p].m);
+  const double m = iso_kp(recs, ioff, p, !a.first, a.iso[p].m);
   return m > -kInf ? Lse{m, a.iso[p].t} : lse_empty();
 }
 
-// NT threads per block (kVW = NT / 64 waves).  kPW > 0 (mode C with P <= kVW * kPW): each lane accumulates its rows' log-sum-exp of its wave's kPW pattern vertices
-// in registers over all tiles, merged across the wave once at the end.  kPW == 0: one wave-level reduction per tile.
+constexpr int kPW = 4;  // mode C: pattern vertices per lane; VT * P <= kTileFloats = kPW * 512 covers every P
+
+// NT threads per block (kVW = NT / 64 waves); block 0 of modes A and C writes the isolated vertices' partial (slot nb),
+// the other nb blocks take the tiles.
+// kFull: VT == 64, so a wave handles one pattern vertex at a time and its incidence structure is wave-uniform.
 // kArgMax (mode A): also track the vertices of the column maxima (the adjoint's tape needs them).
 // kPFC: CV values each thread prefetches per tile (VT * P <= NT * kPFC); fewer registers allow more resident waves.
-template <int kMode, int kPW, bool kArgMax, int NT, int kPFC = kTileFloats / NT>
+template <int kMode, bool kFull, bool kArgMax, int NT, int kPFC = kTileFloats / NT>
 __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
   constexpr int kVW = NT / 64, kPF4 = kTileFloats / 4 / NT;
-  constexpr bool kA = kMode == kModeA;
+  constexpr bool kA = kMode == kModeA, kC = kMode == kModeC;
   constexpr bool kRows = kMode == kModeOut || kMode == kModeMU;  // MU tile staged, written back row by row
   extern __shared__ double lds[];
-  const int Q = a.Q, P = a.P, Qs = a.Qs, VT = a.VT;
+  const int Q = a.Q, P = a.P, Qs = a.Qs, VT = kFull ? 64 : a.VT;
   const int ldq = Qs + 1, ldp = P + 1;
   double* pmu = lds;                                   // [2][P]: m, l of LSE_MU
   IncRec* recs = reinterpret_cast<IncRec*>(pmu + 2 * P);  // [2Q + 1] incidence records, inc order
   double* MUs = reinterpret_cast<double*>(recs + 2 * Q + 1);  // [VT][P + 1] (modes A, OUT, MU)
   const int ldm = P + 1;
-  Lse* lacc = reinterpret_cast<Lse*>(MUs + (kA || kRows ? ldm * VT : 0));    // [P] (mode C)
-  float* Fs = reinterpret_cast<float*>(lacc + (kMode == kModeC ? P : 0));    // [VT][ldq] FMaxN
+  float* Fs = reinterpret_cast<float*>(MUs + (kC ? 0 : ldm * VT));  // [VT][ldq] FMaxN
   float* Vs = Fs + VT * ldq;                           // [VT][ldq] VFm
   float* Ms = Vs + VT * ldq;                           // [VT][ldq] minCEo (mode A)
   float* Ls = Ms + (kA ? VT * ldq : 0);                // [VT][ldq] lsO (mode A)
   float* Cs = Ls + (kA ? VT * ldq : 0);                // [VT][ldp] CV
-  int* Prow = reinterpret_cast<int*>(Cs + VT * ldp);   // [VT] caller id of each tile row (mode OUT)
+  int* ioff = reinterpret_cast<int*>(Cs + VT * ldp);   // [P + 1] incidence offsets
+  int* Prow = ioff + P + 1;                            // [VT] caller id of each tile row (mode OUT)
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const bool sums = !a.first;
   cint_t* const c_incoff = (cint_t*)a.inc_off;
-
-  for (int k = t; k <= 2 * Q; k += NT) {
-    IncRec r{-kInf, 0.0, 0.0, 0, 0};  // k = 2Q: read ahead of the last incidence, never used
-    if (k < 2 * Q) {
-      const int code = a.inc[k], qq = code >> 1;
-      const QStat x = a.qs[qq];
-      r = (code & 1) ? IncRec{x.fillR, x.mRE, x.lRE, VT * ldq + qq, 0} : IncRec{x.fillF, 0.0, 0.0, qq, 0};
-    }
-    recs[k] = r;
-  }
-  for (int i = t; i < P; i += NT) {
-    if (kMode != kModeC) {
-      pmu[i] = a.pst[i].m;
-      pmu[P + i] = a.pst[i].l;
-    } else {
-      lacc[i] = lse_empty();
-    }
-  }
-
-  // Block 0 also writes the isolated vertices' partial, after the blocks' own ones (slot gridDim.x).
-  if (blockIdx.x == 0) {
-    if (kMode == kModeA)
-      for (int i = t; i < Q; i += NT) a.qpart[(int64_t)gridDim.x * Q + i] = iso_qpart(a, i);
-    else if (kMode == kModeC)
-      for (int i = t; i < P; i += NT) a.ppart[(int64_t)gridDim.x * P + i] = iso_lse(a, i);
-  }
-
-  const int RQ = Q > 0 ? NT / Q : 0;
-  const bool qthread = t < RQ * Q;
-  const int q = qthread ? t % Q : 0, rq = qthread ? t / Q : 0;
-  // Read once: loads inside the tile loop would follow the loop's stores (possible aliases) and wait for every
-  // outstanding load, the next tile's prefetch included.
-  const int q_ps = kA && qthread ? a.ps[q] : 0, q_pd = kA && qthread ? a.pd[q] : 0;
-  // The thread's pattern edge's fills and RE normaliser, in registers for the whole pass: an LDS table of them would
-  // take pass A (VT = 64, 24 pattern edges) just past the 40 KB that lets four blocks share a CU.
-  double fF = 0.0, fR = 0.0, mR = 0.0, lR = 0.0;
-  if (kA && qthread) {
-    const QStat x = a.qs[q];
-    fF = x.fillF, fR = x.fillR, mR = x.mRE, lR = x.lRE;
-  }
-  double vfmax = -kInf, vrmax = -kInf;
-  int avf = -1, avr = -1;
-  Lse lre = lse_empty(), lfe = lse_empty();
+  const bool iso_block = (kA || kC) && blockIdx.x == 0;
+  const int64_t G = (kA || kC) ? gridDim.x - 1 : gridDim.x;  // tile blocks
+  const int64_t blk = (kA || kC) ? (int64_t)blockIdx.x - 1 : blockIdx.x;
+  const int64_t ntiles = (a.n + VT - 1) / VT;
 
   const f4v* F4 = reinterpret_cast<const f4v*>(a.FMaxN);
   const f4v* V4 = reinterpret_cast<const f4v*>(a.VFm);
   const f4v* M4 = reinterpret_cast<const f4v*>(a.minCEo);
   const f4v* L4v = reinterpret_cast<const f4v*>(a.lsO);
-  const int64_t ntiles = (a.n + VT - 1) / VT;
   const int64_t L4q = Qs / 4, f_end4 = a.f_end * L4q, o_lo4 = a.o_lo * L4q, o_hi4 = a.o_hi * L4q,
                 o_end4 = a.o_end * L4q;
-  Lse pacc[kPW > 0 ? kPW : 1];
-#pragma unroll
-  for (int pi = 0; pi < (kPW > 0 ? kPW : 1); ++pi) pacc[pi] = lse_empty();
   typedef f4v PfSet[4][kPF4];  // FMaxN, VFm (and in pass A minCEo, lsO)
-  PfSet pfA;
-  float pcA[kPFC];
-  int ppA = 0;  // mode OUT: the caller id of tile row t
-  // Loads of a tile into one register set; indexes past the tile are clamped to its last element (loaded, never
+  PfSet pf;
+  float pc[kPFC];
+  int pp = 0;  // mode OUT: the caller id of tile row t
+  // Loads of a tile into the register set; indexes past the tile are clamped to its last element (loaded, never
   // used).
-  auto prefetch = [&](int64_t tl, PfSet& pf, float (&pc)[kPFC], int& pp) __attribute__((always_inline)) {
+  auto prefetch = [&](int64_t tl) __attribute__((always_inline)) {
     const int64_t v0_ = tl * VT;
     const int nv_ = (int)((a.n - v0_) < VT ? (a.n - v0_) : VT);
     const int last4_ = nv_ * Qs / 4 - 1, lastc_ = nv_ * P - 1;
@@ -1614,20 +1631,81 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
     for (int k = 0; k < kPFC; ++k) pc[k] = a.CV[bc_ + min(t + k * NT, lastc_)];
     if (kMode == kModeOut && a.perm) pp = a.perm[v0_ + min(t, nv_ - 1)];
   };
-  const int64_t G = gridDim.x;
-  // One tile: stage its register set in LDS, refill the set with the block's next tile, compute.
-  auto run_tile = [&](int64_t tile, PfSet& pf, float (&pc)[kPFC], int& pp) __attribute__((always_inline)) {
+  if (!iso_block && blk < ntiles) prefetch(blk);  // in flight while the tables are built
+
+  for (int k = t; k <= 2 * Q; k += NT) {
+    IncRec r{-kInf, 0.0, 0.0, 0, 0};  // k = 2Q: read ahead of the last incidence, never used
+    if (k < 2 * Q) {
+      const int code = a.inc[k], qq = code >> 1;
+      const QStat x = a.qs[qq];
+      r = (code & 1) ? IncRec{x.fillR, x.mRE, x.lRE, VT * ldq + qq, 0} : IncRec{x.fillF, 0.0, 0.0, qq, 0};
+    }
+    recs[k] = r;
+  }
+  for (int i = t; i <= P; i += NT) ioff[i] = a.inc_off[i];
+  if (!kC)
+    for (int i = t; i < P; i += NT) {
+      pmu[i] = a.pst[i].m;
+      pmu[P + i] = a.pst[i].l;
+    }
+  if (iso_block) {
+    __syncthreads();
+    if (kA)
+      for (int i = t; i < Q; i += NT) a.qpart[G * Q + i] = iso_qpart(a, recs, ioff, i);
+    else
+      for (int i = t; i < P; i += NT) a.ppart[G * P + i] = iso_lse(a, recs, ioff, i);
+    return;
+  }
+
+  // This thread's LDS positions of its staged values: element i = t + k NT of the tile goes to row i / width, column
+  // i % width of the padded rows (below 2^16, two to a register).
+  unsigned off4 = 0, offc[(kPFC + 1) / 2];
+#pragma unroll
+  for (int k = 0; k < kPF4; ++k) {
+    const int e = 4 * (t + k * NT), r = e / Qs;
+    off4 |= (unsigned)(r * ldq + e - r * Qs) << (16 * k);
+  }
+#pragma unroll
+  for (int k = 0; k < kPFC; ++k) {
+    const int i = t + k * NT, r = i / P;
+    const unsigned o = (unsigned)(r * ldp + i - r * P) & 0xFFFFu;
+    offc[k / 2] = k & 1 ? offc[k / 2] | (o << 16) : o;
+  }
+
+  const int RQ = Q > 0 ? NT / Q : 0;
+  const bool qthread = t < RQ * Q;
+  const int q = qthread ? t % Q : 0, rq = qthread ? t / Q : 0;
+  // Read once: loads inside the tile loop would follow the loop's stores (possible aliases) and wait for every
+  // outstanding load, the next tile's prefetch included.
+  const int q_ps = kA && qthread ? a.ps[q] : 0, q_pd = kA && qthread ? a.pd[q] : 0;
+  // The thread's pattern edge's fills and RE normaliser, in registers for the whole pass: an LDS table of them would
+  // take pass A (VT = 64, 24 pattern edges) just past the 40 KB that lets four blocks share a CU.
+  double fF = 0.0, fR = 0.0, mR = 0.0, lR = 0.0;
+  if (kA && qthread) {
+    const QStat x = a.qs[q];
+    fF = x.fillF, fR = x.fillR, mR = x.mRE, lR = x.lRE;
+  }
+  double vfmax = -kInf, vrmax = -kInf;
+  int avf = -1, avr = -1;
+  Lse lre = lse_empty(), lfe = lse_empty();
+
+  Lse pacc[kPW];
+#pragma unroll
+  for (int pi = 0; pi < kPW; ++pi) pacc[pi] = lse_empty();
+  // Lane -> (tile row, one of the wave's pattern vertices); psweep pattern vertices per step of the block.
+  const int prow = kFull ? lane : lane & (VT - 1);
+  const int pfirst = kFull ? wave : wave * (64 / VT) + lane / VT, psweep = kFull ? kVW : kVW * (64 / VT);
+
+  for (int64_t tile = blk; tile < ntiles; tile += G) {
     const int64_t v0 = tile * VT;
     const int nv = (int)((a.n - v0) < VT ? (a.n - v0) : VT);
     __syncthreads();  // tables written (first tile) / previous tile consumed
     {
       const int cnt4 = nv * Qs / 4, cntc = nv * P;
 #pragma unroll
-      for (int k = 0; k < kPF4; ++k) {
-        const int i = t + k * NT;
-        if (i < cnt4) {
-          const int e = 4 * i, r = e / Qs, c = e - r * Qs;
-          const int o = r * ldq + c;
+      for (int k = 0; k < kPF4; ++k)
+        if (t + k * NT < cnt4) {
+          const int o = (off4 >> (16 * k)) & 0xFFFF;
 #pragma unroll
           for (int u = 0; u < 4; ++u) {
             Fs[o + u] = pf[0][k][u];
@@ -1638,66 +1716,40 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
             }
           }
         }
-      }
 #pragma unroll
-      for (int k = 0; k < kPFC; ++k) {
-        const int i = t + k * NT;
-        if (i < cntc) {
-          const int r = i / P, c = i - r * P;
-          Cs[r * ldp + c] = pc[k];
-        }
-      }
+      for (int k = 0; k < kPFC; ++k)
+        if (t + k * NT < cntc) Cs[(offc[k / 2] >> (16 * (k & 1))) & 0xFFFF] = pc[k];
       if (kMode == kModeOut && a.perm && t < nv) Prow[t] = pp;
     }
     __syncthreads();
-    if (tile + G < ntiles) prefetch(tile + G, pf, pc, pp);
-    // p-phase: wave-uniform pattern vertex, lane = tile row.
-    // MU_pre of row `r` and pattern vertex `p` (-inf for rows past the tile).
-#define AC_VX_MU_PRE(X, P_, R_)                                                                              \
-    {                                                                                                      \
-      X = -kInf;                                                                                           \
-      if ((R_) < nv) {                                                                                     \
-        double acc_ = -(double)Cs[(R_) * ldp + (P_)];                                                      \
-        if (sums) {                                                                                        \
-          const int k1_ = c_incoff[(P_) + 1];                                                              \
-          int k_ = c_incoff[P_];                                                                           \
-          IncRec rc_ = recs[k_];                                                                           \
-          for (; k_ < k1_; ++k_) {                                                                         \
-            const IncRec nx_ = recs[k_ + 1]; /* in flight while this term is formed */                     \
-            const float x_ = Fs[(R_) * ldq + rc_.col];                                                     \
-            const double d_ = ((double)x_ - rc_.m) - rc_.l;                                                \
-            acc_ += fmax(rc_.fill, x_ == -INFINITY ? -kInf : d_);                                          \
-            rc_ = nx_;                                                                                     \
-          }                                                                                                \
-        }                                                                                                  \
-        X = acc_;                                                                                          \
-      }                                                                                                    \
-    }
-    if (kMode == kModeC && kPW > 0) {
+    if (tile + G < ntiles) prefetch(tile + G);
+    // p-phase.  MU_pre of row prow and pattern vertex p.
+    auto mu_pre = [&](int p) __attribute__((always_inline)) {
+      double acc = -(double)Cs[prow * ldp + p];
+      if (sums) {
+        const int k1 = kFull ? c_incoff[p + 1] : ioff[p + 1];
+        int k = kFull ? c_incoff[p] : ioff[p];
+        IncRec rc = recs[k];
+        for (; k < k1; ++k) {
+          const IncRec nx = recs[k + 1];  // in flight while this term is formed
+          const float x = Fs[prow * ldq + rc.col];
+          const double d = ((double)x - rc.m) - rc.l;
+          acc += fmax(rc.fill, x == -INFINITY ? -kInf : d);
+          rc = nx;
+        }
+      }
+      return acc;
+    };
+    if (kC) {
 #pragma unroll
       for (int pi = 0; pi < kPW; ++pi) {
-        const int p = wave + kVW * pi;
-        if (p < P) {
-          double x;
-          AC_VX_MU_PRE(x, p, lane);
-          lse_add(pacc[pi], x);
-        }
+        const int p = pfirst + psweep * pi;
+        if (p < P) lse_add(pacc[pi], prow < nv ? mu_pre(p) : -kInf);
       }
     } else {
-      for (int p = wave; p < P; p += kVW) {
-        const int r = lane;
-        double x;
-        AC_VX_MU_PRE(x, p, r);
-        if (kMode == kModeC) {
-          const Lse w = wave_lse(x);
-          if (lane == 0) lacc[p] = lse_merge(lacc[p], w);
-        } else if (r < nv) {
-          const double mu = (x - pmu[p]) - pmu[P + p];
-          MUs[r * ldm + p] = mu;
-        }
-      }
+      for (int p = pfirst; p < P; p += psweep)
+        if (prow < nv) MUs[prow * ldm + p] = (mu_pre(p) - pmu[p]) - pmu[P + p];
     }
-#undef AC_VX_MU_PRE
     if (kRows) {
       // The tile's rows go out whole: consecutive threads write consecutive columns of a row.
       __syncthreads();
@@ -1748,32 +1800,53 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
         }
       }
     }
-  };
-  int64_t tile = blockIdx.x;
-  if (tile < ntiles) prefetch(tile, pfA, pcA, ppA);
-  for (; tile < ntiles; tile += G) run_tile(tile, pfA, pcA, ppA);
+  }
   __syncthreads();
 
-  // Block partials, merged in a fixed order.
-  if (kMode == kModeA) {
+  // Block partials, merged in a fixed order: the maxima first, then every accumulator rescaled to them at once (one
+  // exponential each, in parallel), then the sum.
+  if (kA) {
     QPart* red = reinterpret_cast<QPart*>(lds);
     if (qthread) red[rq * Q + q] = QPart{vfmax, vrmax, lre, lfe, avf, avr};
     __syncthreads();
-    if (t < Q) {
-      QPart acc{-kInf, -kInf, lse_empty(), lse_empty(), -1, -1};
-      for (int r = 0; r < RQ; ++r) qpart_merge(acc, red[r * Q + t]);
-      a.qpart[(int64_t)blockIdx.x * Q + t] = acc;
-    }
-  } else if (kMode == kModeC) {
-    if (kPW > 0) {
-#pragma unroll
-      for (int pi = 0; pi < kPW; ++pi) {
-        const int p = wave + kVW * pi;
-        const Lse w = wave_lse_merge(pacc[pi]);
-        if (p < P && lane == 0) a.ppart[(int64_t)blockIdx.x * P + p] = w;
+    QPart acc{-kInf, -kInf, lse_empty(), lse_empty(), -1, -1};
+    if (t < Q)
+      for (int r = 0; r < RQ; ++r) {
+        const QPart x = red[r * Q + t];
+        argmax_merge(acc.vfmax, acc.avf, x.vfmax, x.avf);
+        argmax_merge(acc.vrmax, acc.avr, x.vrmax, x.avr);
+        acc.re.m = fmax(acc.re.m, x.re.m);
+        acc.fe.m = fmax(acc.fe.m, x.fe.m);
       }
-    } else {
-      for (int i = t; i < P; i += NT) a.ppart[(int64_t)blockIdx.x * P + i] = lacc[i];
+    __syncthreads();  // every field of red read
+    double* Mx = lds;                // [2][Q] the maxima
+    double* Ts = Mx + 2 * Q;         // [2][RQ][Q] the rescaled sums
+    if (t < Q) {
+      Mx[t] = acc.re.m;
+      Mx[Q + t] = acc.fe.m;
+    }
+    __syncthreads();
+    if (qthread) {
+      Ts[t] = lse_rescaled(lre, Mx[q]);
+      Ts[RQ * Q + t] = lse_rescaled(lfe, Mx[Q + q]);
+    }
+    __syncthreads();
+    if (t < Q) {
+      // (each rescaled term counts its own maximum; the overall one is left out again)
+      acc.re.t = acc.fe.t = 0.0;
+      bool ore = false, ofe = false;
+      for (int r = 0; r < RQ; ++r) {
+        lse_sum_step(acc.re.t, ore, Ts[r * Q + t]);
+        lse_sum_step(acc.fe.t, ofe, Ts[RQ * Q + r * Q + t]);
+      }
+      a.qpart[blk * Q + t] = acc;
+    }
+  } else if (kC) {
+#pragma unroll
+    for (int pi = 0; pi < kPW; ++pi) {
+      const int p = pfirst + psweep * pi;
+      const Lse w = lanes_lse_merge(pacc[pi], VT);
+      if (p < P && prow == 0) a.ppart[blk * P + p] = w;
     }
   }
 }
@@ -1786,24 +1859,27 @@ static bool short_cv(const VertexArgs& a) { return a.VT * a.P <= kNA * 4; }
 
 typedef void (*VertexKernel)(VertexArgs);
 
+template <bool kFull>
+static VertexKernel vertex_kernel_t(int mode, const VertexArgs& a) {
+  switch (mode) {
+    case kModeA:
+      if (a.track_arg) return short_cv(a) ? k_vertex<kModeA, kFull, true, kNA, 4> : k_vertex<kModeA, kFull, true, kNA>;
+      return short_cv(a) ? k_vertex<kModeA, kFull, false, kNA, 4> : k_vertex<kModeA, kFull, false, kNA>;
+    case kModeC:
+      return k_vertex<kModeC, kFull, false, kNO>;
+    case kModeMU:
+      return k_vertex<kModeMU, kFull, false, kNO>;
+    default:
+      return k_vertex<kModeOut, kFull, false, kNO>;
+  }
+}
+
 // The kernel a pass launches, its block size and dynamic LDS bytes.
 static VertexKernel vertex_kernel(int mode, const VertexArgs& a, int* nt, size_t* lds) {
   const size_t tiles = vertex_lds_bytes(mode, a.VT, a.P, a.Q, a.Qs);
   *nt = mode == kModeA ? kNA : kNO;
   *lds = mode == kModeA ? std::max(tiles, sizeof(QPart) * kNA) : tiles;
-  switch (mode) {
-    case kModeA:
-      if (a.track_arg) return short_cv(a) ? k_vertex<kModeA, 0, true, kNA, 4> : k_vertex<kModeA, 0, true, kNA>;
-      return short_cv(a) ? k_vertex<kModeA, 0, false, kNA, 4> : k_vertex<kModeA, 0, false, kNA>;
-    case kModeC:
-      if (a.P <= 4 * (kNO / 64)) return k_vertex<kModeC, 4, false, kNO>;
-      if (a.P <= 8 * (kNO / 64)) return k_vertex<kModeC, 8, false, kNO>;
-      return k_vertex<kModeC, 0, false, kNO>;
-    case kModeMU:
-      return k_vertex<kModeMU, 0, false, kNO>;
-    default:
-      return k_vertex<kModeOut, 0, false, kNO>;
-  }
+  return a.VT == 64 ? vertex_kernel_t<true>(mode, a) : vertex_kernel_t<false>(mode, a);
 }
 
 void launch_vertex(int mode, const VertexArgs& a, int nblocks, hipStream_t st) {
@@ -1812,10 +1888,12 @@ void launch_vertex(int mode, const VertexArgs& a, int nblocks, hipStream_t st) {
   const VertexKernel k = vertex_kernel(mode, a, &nt, &lds);
   VertexArgs arg = a;
   void* args[] = {&arg};
-  (void)hipLaunchKernel(reinterpret_cast<const void*>(k), dim3(nblocks), dim3(nt), args, lds, st);
+  const int extra = mode == kModeA || mode == kModeC ? 1 : 0;  // the isolated vertices' block
+  (void)hipLaunchKernel(reinterpret_cast<const void*>(k), dim3(nblocks + extra), dim3(nt), args, lds, st);
 }
 
-// Blocks of a vertex pass resident at once on the device (CUs x blocks per CU at the pass's registers and LDS).
+// Tile blocks of a vertex pass resident at once on the device (CUs x blocks per CU at the pass's registers and LDS,
+// less the isolated vertices' block).
 int vertex_resident_blocks(int mode, const VertexArgs& a) {
   int dev = 0, cus = 0, per = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
@@ -1826,7 +1904,8 @@ int vertex_resident_blocks(int mode, const VertexArgs& a) {
   const VertexKernel k = vertex_kernel(mode, a, &nt, &lds);
   const hipError_t e =
       hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void*>(k), nt, lds);
-  return e == hipSuccess ? cus * std::max(per, 1) : 0;
+  const int extra = mode == kModeA || mode == kModeC ? 1 : 0;
+  return e == hipSuccess ? cus * std::max(per, 1) - extra : 0;
 }
 
 // Columns [c0, c0 + ncol) of src[n][P] into dst[n][ncol].

@@ -1,0 +1,42 @@
+"""The matcher at the sizes where its kernels' tiles, lane groups and merges change, against the FP64 oracle at the
+reference's own tolerance (validate.py:7)."""
+import numpy as np
+import pytest
+
+from application_classification_amd import workloads as W
+from application_classification_amd.matcher import Matcher
+from oracle import oracle as O
+from tests.conftest import allclose_report
+
+pytestmark = pytest.mark.gpu
+
+
+def g64(g):
+    return O.Graph64.of(g.vfeat, g.efeat, g.src, g.dst)
+
+
+def random_graph(n, m, dv, de, seed):
+    r = np.random.default_rng(seed)
+    return W.Graph(r.normal(size=(n, dv)).astype(np.float32), r.normal(size=(m, de)).astype(np.float32),
+                   r.integers(0, n, m).astype(np.int32), r.integers(0, n, m).astype(np.int32))
+
+
+def check(data, patt, n_iter=3):
+    with Matcher(0) as m:
+        m.set_data(data)
+        m.set_pattern(patt)
+        mu = m.run(n_iter)
+    bad, ratio = allclose_report(mu, O.run(g64(data), g64(patt), n_iter=n_iter))
+    print(f"dn={data.num_nodes} de={data.num_edges} pn={patt.num_nodes} pe={patt.num_edges}: max err/tol {ratio:.4f}", flush=True)
+    assert bad == 0, ratio
+
+
+@pytest.mark.parametrize("n,m,pn,pe", [
+    (2, 1, 1, 1), (9, 30, 1, 3), (64, 200, 2, 1),            # a few rows, one pattern vertex or edge
+    (4095, 9000, 5, 3), (4097, 5000, 17, 65),                # 8- and 16-row tiles, some vertices isolated
+    (20_000, 90_000, 33, 20), (70_000, 90_000, 9, 24),       # 32- and 64-row tiles; a full block of partials
+    (500, 3000, 256, 256), (1200, 2500, 3, 256), (900, 4000, 255, 64),  # the widest patterns
+])
+def test_vertex_pass_tiles(n, m, pn, pe):
+    """Multigraphs with self-loops and isolated vertices; the tile height follows the vertex count and the pattern."""
+    check(random_graph(n, m, 4, 5, n), random_graph(pn, pe, 4, 5, pn + pe))
