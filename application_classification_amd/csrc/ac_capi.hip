@@ -41,14 +41,18 @@ struct Range {
   Range& operator=(const Range&) = delete;
 };
 
-// Edges per run of an edge walk (a tuning knob, AC_RUN_EDGES).  Vertices whose edge list is longer are split into
-// pieces of this length.
-int run_edges() {
+// Edges per run of an edge walk in a graph of nE edges (AC_RUN_EDGES overrides it).  Vertices whose edge list is longer
+// are split into pieces of this length.  A run is walked step by step by one group of lanes, so short runs spread a small
+// graph over the chip, while long ones take fewer bundle headers and leave fewer pieces.  us per call at 8 / 16 / 32 /
+// 64 / 128: 20 K edges 611 / 644 / 692 / 765 / 910; 242 K edges 2283 / 1964 / 1864 / 1974 / 2380; 0.9 M edges 8356 / 6596
+// / 5960 / 5774 / 5876; 3.9 M edges 3341 / 2954 / 2783 / 2786 / 2888; 16 M edges (device time) 10340 / 8277 / 7396 / 7010
+// / 7087.
+int run_edges(int64_t nE) {
   if (const char* e = std::getenv("AC_RUN_EDGES")) {
     const int v = std::atoi(e);
     if (v >= 4 && v <= 4096) return v;
   }
-  return 128;  // measured at R-MAT 22 against 48-512 (with walk batch 4)
+  return nE <= 50'000 ? 8 : nE <= 120'000 ? 16 : nE <= 500'000 ? 32 : nE <= 10'000'000 ? 64 : 128;
 }
 
 int round8(int x) { return (x + 7) / 8 * 8; }
@@ -129,7 +133,7 @@ struct DevBuf {
 // destination by one at each new vertex); the CSR walk reads each edge's source and takes any order.
 void build_runs(const std::vector<int64_t>& off, int64_t n, std::vector<Run>& runs, std::vector<Split>& splits,
                 int& nslots, const int* vid = nullptr, bool consecutive = true) {
-  const int kRunEdges = run_edges();
+  const int kRunEdges = run_edges(off[n]);
   runs.clear();
   splits.clear();
   nslots = 0;

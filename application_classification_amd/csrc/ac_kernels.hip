@@ -830,24 +830,33 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
   Lse glob[4] = {lse_empty(), lse_empty(), lse_empty(), lse_empty()};
   if (g < G && r < nruns) {
     const Run R = runs[r];
-    Lse s[4] = {lse_empty(), lse_empty(), lse_empty(), lse_empty()};
+    // The open vertex's least cost and the sum of exp(least - cost) over its other edges.  The difference of two floats
+    // rounded to FP32 is the argument of the FP32 exponential whether it is formed in FP32 or in FP64; the sum is FP64.
+    float mn[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
+    double tt[4] = {0.0, 0.0, 0.0, 0.0};
+    auto add = [&](int c, float x) {
+      const float d = mn[c] - x;  // > 0: a new least cost, the old ones rescaled to it
+      float e = __expf(-fabsf(d));
+      e = x == INFINITY ? 0.f : e;  // (and exp(-inf) = 0 where x is the first finite cost)
+      tt[c] = d > 0.f ? fma(tt[c], (double)e, (double)e) : tt[c] + (double)e;
+      mn[c] = fminf(mn[c], x);
+    };
     int cur = ks[R.kb].y;
     // A finished source vertex.  It runs at vertex changes, which differ between the wave's runs, so each costs the
     // whole wave: its log1p and the merge into the block partial take FP32 transcendentals (lsO is stored in FP32;
-    // the merge's exponential has the precision of lse_add's terms).
+    // the merge's exponential has the precision of the sum's terms).
     auto emit = [&](int v) {
-      float4 mn, ls, vf;
-      mn.x = (float)(-s[0].m), mn.y = (float)(-s[1].m), mn.z = (float)(-s[2].m), mn.w = (float)(-s[3].m);
-      ls.x = log1pf((float)s[0].t), ls.y = log1pf((float)s[1].t), ls.z = log1pf((float)s[2].t);
-      ls.w = log1pf((float)s[3].t);
-      vf.x = (float)s[0].m, vf.y = (float)s[1].m, vf.z = (float)s[2].m, vf.w = (float)s[3].m;
-      reinterpret_cast<float4*>(minCEo)[(int64_t)v * L4 + j] = mn;
+      float4 ls;
+      ls.x = log1pf((float)tt[0]), ls.y = log1pf((float)tt[1]), ls.z = log1pf((float)tt[2]);
+      ls.w = log1pf((float)tt[3]);
+      reinterpret_cast<float4*>(minCEo)[(int64_t)v * L4 + j] = make_float4(mn[0], mn[1], mn[2], mn[3]);
       reinterpret_cast<float4*>(lsO)[(int64_t)v * L4 + j] = ls;
-      reinterpret_cast<float4*>(VFm)[(int64_t)v * L4 + j] = vf;
+      reinterpret_cast<float4*>(VFm)[(int64_t)v * L4 + j] = make_float4(-mn[0], -mn[1], -mn[2], -mn[3]);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        glob[c] = lse_merge_fast(glob[c], s[c]);
-        s[c] = lse_empty();
+        glob[c] = lse_merge_fast(glob[c], Lse{-(double)mn[c], tt[c]});
+        mn[c] = INFINITY;
+        tt[c] = 0.0;
       }
     };
     // Steps in batches of kSrcBatch: the batch's (row, vertex) pairs, then its cost rows, are loaded together (two
@@ -868,18 +877,19 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
           emit(cur);
           cur = e[u].y;
         }
-        lse_add(s[0], -(double)c[u].x);
-        lse_add(s[1], -(double)c[u].y);
-        lse_add(s[2], -(double)c[u].z);
-        lse_add(s[3], -(double)c[u].w);
+        add(0, c[u].x);
+        add(1, c[u].y);
+        add(2, c[u].z);
+        add(3, c[u].w);
       }
     }
     if (R.slot >= 0) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        carry[((int64_t)R.slot * Qs + 4 * j + c) * 2 + 0] = s[c].m;
-        carry[((int64_t)R.slot * Qs + 4 * j + c) * 2 + 1] = s[c].t;
-        glob[c] = lse_merge_fast(glob[c], s[c]);
+        const Lse s{-(double)mn[c], tt[c]};
+        carry[((int64_t)R.slot * Qs + 4 * j + c) * 2 + 0] = s.m;
+        carry[((int64_t)R.slot * Qs + 4 * j + c) * 2 + 1] = s.t;
+        glob[c] = lse_merge_fast(glob[c], s);
       }
     } else {
       emit(cur);
@@ -918,39 +928,58 @@ void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float
 }
 
 // One wave per split vertex: groups of Qs/4 lanes take its pieces round-robin (lane j owns pattern edges
-// 4j..4j+3), then the groups' results are merged in group order through LDS.  Deterministic.
+// 4j..4j+3), first for the largest maximum, then for the pieces' shares of it, whose exponentials do not wait for each
+// other; the groups' results are combined in group order through LDS.  Deterministic.
 __global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split* __restrict__ splits,
                                                         const double* __restrict__ carry, int Q, int Qs,
                                                         float* __restrict__ minCEo, float* __restrict__ lsO,
                                                         float* __restrict__ VFm) {
-  __shared__ Lse red[4][64][4];
+  __shared__ double red[4][64][4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int L4 = Qs / 4, G = 64 / L4;
   const int g = lane / L4, j = lane - g * L4;
   const int sidx = blockIdx.x * 4 + wave;
   const bool active = sidx < nsplit && g < G;
-  Lse s[4] = {lse_empty(), lse_empty(), lse_empty(), lse_empty()};
   Split S{0, 0, 0, 0};
   if (sidx < nsplit) S = splits[sidx];
+  const double* base = carry + ((int64_t)S.first * Qs + 4 * j) * 2;
+  double M[4] = {-kInf, -kInf, -kInf, -kInf}, sum[4] = {0.0, 0.0, 0.0, 0.0};
+  bool seen[4] = {false, false, false, false};
   if (active)
-    for (int c = g; c < S.count; c += G) {
-      const double* o = carry + ((int64_t)(S.first + c) * Qs + 4 * j) * 2;
+#pragma unroll 4
+    for (int c = g; c < S.count; c += G)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) s[u] = lse_merge(s[u], Lse{o[2 * u], o[2 * u + 1]});
-    }
+      for (int u = 0; u < 4; ++u) M[u] = fmax(M[u], base[(int64_t)c * Qs * 2 + 2 * u]);
 #pragma unroll
-  for (int u = 0; u < 4; ++u) red[wave][lane][u] = s[u];
+  for (int u = 0; u < 4; ++u) red[wave][lane][u] = M[u];
+  __syncthreads();
+  if (active)
+    for (int gg = 0; gg < G; ++gg)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) M[u] = fmax(M[u], red[wave][gg * L4 + j][u]);
+  if (active)
+#pragma unroll 4
+    for (int c = g; c < S.count; c += G)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double* o = base + (int64_t)c * Qs * 2 + 2 * u;
+        lse_sum_step(sum[u], seen[u], lse_rescaled(Lse{o[0], o[1]}, M[u]));
+      }
+  __syncthreads();  // the maxima are read
+#pragma unroll
+  for (int u = 0; u < 4; ++u) red[wave][lane][u] = seen[u] ? -sum[u] : sum[u];  // a share of the group (lse_sum_step)
   __syncthreads();
   if (sidx < nsplit && g == 0) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      Lse acc = lse_empty();
-      for (int gg = 0; gg < G; ++gg) acc = lse_merge(acc, red[wave][gg * L4 + j][u]);
+      double t = 0.0;
+      bool any = false;
+      for (int gg = 0; gg < G; ++gg) lse_sum_step(t, any, red[wave][gg * L4 + j][u]);
       const int q = 4 * j + u;
       const int64_t o = (int64_t)S.v * Qs + q;
-      minCEo[o] = q < Q ? (float)(-acc.m) : 0.f;
-      lsO[o] = q < Q ? (float)log1p(acc.t) : 0.f;
-      VFm[o] = q < Q ? (float)acc.m : 0.f;
+      minCEo[o] = q < Q ? (float)(-M[u]) : 0.f;
+      lsO[o] = q < Q ? (float)log1p(t) : 0.f;
+      VFm[o] = q < Q ? (float)M[u] : 0.f;
     }
   }
 }
@@ -1300,16 +1329,22 @@ __global__ __launch_bounds__(kWalkBlock) void k_bundle_min(int64_t nbundles, con
   if (g < G && b < nbundles) {
     const Bundle Bd = bundles[b];
     const f4v* ce = reinterpret_cast<const f4v*>(CE) + (Bd.base + g) * L4 + j;
-    for (int s = 0; s < Bd.len; ++s) {
-      const f4v c = __builtin_nontemporal_load(ce + (int64_t)s * G * L4);
-      m = f4v{fminf(m[0], c[0]), fminf(m[1], c[1]), fminf(m[2], c[2]), fminf(m[3], c[3])};
-      if (bpack) {
+    // Eight rows in flight (past the end: the last one again), where a row at a time waited for each.
+    for (int s0 = 0; s0 < Bd.len; s0 += 8) {
+      f4v c[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const unsigned x = __float_as_uint(c[u]);
-          if (4 * j + u < Q && x != 0x7F800000u) {
-            lo = min(lo, x);
-            hi = max(hi, x);
+      for (int s = 0; s < 8; ++s) c[s] = __builtin_nontemporal_load(ce + (int64_t)min(s0 + s, Bd.len - 1) * G * L4);
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        m = f4v{fminf(m[0], c[s][0]), fminf(m[1], c[s][1]), fminf(m[2], c[s][2]), fminf(m[3], c[s][3])};
+        if (bpack) {
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const unsigned x = __float_as_uint(c[s][u]);
+            if (4 * j + u < Q && x != 0x7F800000u) {
+              lo = min(lo, x);
+              hi = max(hi, x);
+            }
           }
         }
       }

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from application_classification_amd import workloads as W
-from application_classification_amd.matcher import Matcher
+from application_classification_amd.matcher import AC_OPT_PRUNE, Matcher
 from oracle import oracle as O
 from tests.conftest import allclose_report
 
@@ -40,3 +40,25 @@ def check(data, patt, n_iter=3):
 def test_vertex_pass_tiles(n, m, pn, pe):
     """Multigraphs with self-loops and isolated vertices; the tile height follows the vertex count and the pattern."""
     check(random_graph(n, m, 4, 5, n), random_graph(pn, pe, 4, 5, pn + pe))
+
+
+@pytest.mark.parametrize("run_edges", [4, 8, 16, 32, 64, 128])
+@pytest.mark.parametrize("prune", [0, 1])
+def test_run_lengths(run_edges, prune, monkeypatch):
+    """Every run length the edge count can select, on a graph with hubs of both kinds, one to hundreds of pieces: the
+    pieces' atomic maxima over several iterations (each resetting the rows), pruned bundles included."""
+    monkeypatch.setenv("AC_RUN_EDGES", str(run_edges))
+    r = np.random.default_rng(run_edges)
+    n, hub_in, hub_out = 1500, 900, 400
+    src = np.concatenate([r.integers(0, n, 6000), r.integers(0, n, hub_in), np.full(hub_out, 7), r.integers(0, n, 130)])
+    dst = np.concatenate([r.integers(0, n, 6000), np.full(hub_in, 3), r.integers(0, n, hub_out), np.full(130, 4)])
+    data = W.Graph(r.normal(size=(n, 6)).astype(np.float32), r.normal(size=(len(src), 6)).astype(np.float32),
+                   src.astype(np.int32), dst.astype(np.int32))
+    patt = W.planted_pattern(data, 7, 10, 1)
+    with Matcher(0) as m:
+        m.set_option(AC_OPT_PRUNE, prune)
+        m.set_data(data)
+        m.set_pattern(patt)
+        for n_iter in (0, 1, 7):
+            bad, ratio = allclose_report(m.run(n_iter), O.run(g64(data), g64(patt), n_iter=n_iter))
+            assert bad == 0, (n_iter, ratio)
