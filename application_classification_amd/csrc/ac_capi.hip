@@ -191,7 +191,7 @@ struct ac_ctx {
   DevBuf<Run> runs_in, runs_out;
   DevBuf<Split> splits_in, splits_out;
   std::vector<Run> h_runs_in;
-  std::vector<int> h_run_src0;  // first (least) source of each in-edge run
+  std::vector<int> h_run_order;  // the in-edge runs, longest first, ties by first (least) source, then by position
   // Internal vertex order: vertices with in- and out-edges, in-edges only, out-edges only, then isolated ones, each
   // class in ascending caller order.  perm maps an internal vertex to the caller's; the vertex passes stream the
   // first n_act = dn - n_iso rows only.
@@ -487,8 +487,25 @@ static int set_data(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int64_
   ctx->nsplit_out = (int)sout.size();
   ctx->nslots_in = slin;
   ctx->nslots_out = slout;
-  ctx->h_run_src0.resize(rin.size());
-  for (size_t i = 0; i < rin.size(); ++i) ctx->h_run_src0[i] = csc_sd[rin[i].kb].x;
+  {
+    // A radix sort: by first source, 2^11 values a pass, then by decreasing length, every pass stable.
+    const size_t nr = rin.size();
+    std::vector<int> from(nr), to(nr), cnt;
+    for (size_t i = 0; i < nr; ++i) from[i] = (int)i;
+    auto pass = [&](int nkeys, auto key) {
+      cnt.assign((size_t)nkeys + 1, 0);
+      for (size_t i = 0; i < nr; ++i) ++cnt[(size_t)key(from[i]) + 1];
+      for (int k = 0; k < nkeys; ++k) cnt[k + 1] += cnt[k];
+      for (size_t i = 0; i < nr; ++i) to[(size_t)cnt[key(from[i])]++] = from[i];
+      from.swap(to);
+    };
+    for (int shift = 0; shift < 32 && ((nV - 1) >> shift) > 0; shift += 11)
+      pass(1 << 11, [&](int i) { return (csc_sd[rin[i].kb].x >> shift) & 2047; });
+    int longest = 0;
+    for (const Run& r : rin) longest = std::max(longest, r.ke - r.kb);
+    pass(longest + 1, [&](int i) { return longest - (rin[i].ke - rin[i].kb); });
+    ctx->h_run_order = std::move(from);
+  }
   ctx->h_runs_in = std::move(rin);
   ctx->bsets.clear();  // bundle layouts follow the graph, not only its sizes
   ctx->bs = nullptr;
@@ -619,13 +636,7 @@ static int select_bundles(ac_ctx* ctx) {
     }
   const std::vector<Run>& R = ctx->h_runs_in;
   const int64_t nr = (int64_t)R.size();
-  std::vector<int> order(nr);
-  for (int64_t i = 0; i < nr; ++i) order[i] = (int)i;
-  const std::vector<int>& S0 = ctx->h_run_src0;
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-    const int la = R[a].ke - R[a].kb, lb = R[b].ke - R[b].kb;
-    return la > lb || (la == lb && S0[a] < S0[b]);
-  });
+  const std::vector<int>& order = ctx->h_run_order;
   const int64_t nb = (nr + G - 1) / G;
   std::vector<Bundle> bun(nb);
   std::vector<int> brun((size_t)std::max<int64_t>(1, nb * G), -1), gslot((size_t)std::max<int64_t>(1, nb * G), -1);
