@@ -18,6 +18,7 @@
 #include "ac_adjoint.hpp"
 #include "ac_host.hpp"
 #include "ac_internal.hpp"
+#include "ac_select.hpp"
 
 using ac::Lse;
 using ac::Lse2;
@@ -274,6 +275,12 @@ struct ac_ctx {
   DevBuf<float> gERsum;               // per (vertex, pattern edge), gE_R summed over the steps back
   DevBuf<double> cD, colsum, bpart, red4, cq, opart, osum, MUd;
   DevBuf<int> api;
+
+  // Selection of the best candidates (ac_select.hpp): one buffer per kind, and the flag, indexes and values that go to
+  // the host together, in one copy: {flag, idx [P][k], val [P][k]}.
+  DevBuf<unsigned> sel_u32;
+  DevBuf<unsigned long long> sel_keys;
+  DevBuf<int> sel_out;
 
   // Batched scoring: the patterns (host copies, concatenated), where each one's result lives in `bout`, and the
   // statistics of the last batched run.
@@ -1203,12 +1210,55 @@ extern "C" int ac_get_mu(ac_ctx* ctx, float* host_out) {
   return AC_OK;
 }
 
+// Each pattern vertex's k best data vertices on the device, if the sizes suit it: out = {idx [P][k], val [P][k]}.
+// *done is left false where the caller has to select on the host (sizes, a NaN, more ties than fit).
+static int select_topk(ac_ctx* ctx, int k, std::vector<int>& out, bool* done) {
+  *done = false;
+  if (!ctx->have_result) return ctx->fail(AC_ERR_STATE, "ac_get_mu: no result; call ac_run first");
+  const int P = ctx->P;
+  const ac::SelShape sh = ac::sel_shape(ctx->dn, P, k);
+  if (sh.chunks == 0) return AC_OK;
+  HIPCHK(ctx, hipSetDevice(ctx->device));
+  hipStream_t st = ctx->stream;
+  const size_t np = (size_t)P, nk = np * (size_t)k;
+  if (ctx->sel_u32.alloc(np * (size_t)sh.chunks + 2 * np) != hipSuccess ||
+      ctx->sel_keys.alloc(np * ac::kSelCap) != hipSuccess || ctx->sel_out.alloc(1 + 2 * nk) != hipSuccess) {
+    (void)hipGetLastError();  // no device memory to spare: the host path needs none
+    return AC_OK;
+  }
+  unsigned* u = ctx->sel_u32.p;
+  int* o = ctx->sel_out.p;
+  const ac::SelBufs b{u,          u + np * sh.chunks, reinterpret_cast<int*>(u + np * sh.chunks + np), ctx->sel_keys.p, o + 1,
+                      reinterpret_cast<float*>(o + 1 + nk), o};
+  HIPCHK(ctx, hipMemsetAsync(o, 0, sizeof(int), st));
+  ac::launch_select(ctx->dn, P, k, sh, ctx->OUT.p, b, st);
+  HIPCHK(ctx, hipGetLastError());
+  out.resize(1 + 2 * nk);
+  HIPCHK(ctx, hipMemcpyAsync(out.data(), o, out.size() * sizeof(int), hipMemcpyDeviceToHost, st));
+  HIPCHK(ctx, hipStreamSynchronize(st));
+  *done = out[0] == 0;
+  return AC_OK;
+}
+
 extern "C" int ac_get_match(ac_ctx* ctx, float log_tau, uint8_t* host_out) {
   if (!ctx || !host_out) return ctx ? ctx->fail(AC_ERR_ARG, "ac_get_match: null output") : AC_ERR_ARG;
   const int64_t n = ctx->dn;
   const int P = ctx->P;
+  std::vector<int> sel;
+  bool done = false;
+  int rc = select_topk(ctx, 1, sel, &done);
+  if (rc != AC_OK) return rc;
+  if (done) {
+    std::memset(host_out, 0, (size_t)(n * P));
+    for (int p = 0; p < P; ++p) {
+      float best;
+      std::memcpy(&best, &sel[1 + P + p], sizeof(float));
+      host_out[(int64_t)sel[1 + p] * P + p] = best >= log_tau ? 2 : 1;
+    }
+    return AC_OK;
+  }
   std::vector<float> mu((size_t)(n * P));
-  int rc = ac_get_mu(ctx, mu.data());
+  rc = ac_get_mu(ctx, mu.data());
   if (rc != AC_OK) return rc;
   std::vector<int64_t> arg(P, 0);
   for (int64_t v = 1; v < n; ++v)
@@ -1225,8 +1275,18 @@ extern "C" int ac_get_topk(ac_ctx* ctx, int k, int32_t* idx_out, float* val_out)
     return ctx->fail(AC_ERR_ARG, "ac_get_topk: need 1 <= k <= number of data vertices");
   const int64_t n = ctx->dn;
   const int P = ctx->P;
+  std::vector<int> sel;
+  bool done = false;
+  int rc = select_topk(ctx, k, sel, &done);
+  if (rc != AC_OK) return rc;
+  if (done) {
+    const size_t nk = (size_t)P * (size_t)k;
+    std::memcpy(idx_out, sel.data() + 1, nk * sizeof(int32_t));
+    if (val_out) std::memcpy(val_out, sel.data() + 1 + nk, nk * sizeof(float));
+    return AC_OK;
+  }
   std::vector<float> mu((size_t)(n * P));
-  int rc = ac_get_mu(ctx, mu.data());
+  rc = ac_get_mu(ctx, mu.data());
   if (rc != AC_OK) return rc;
   // Per pattern vertex: the k best (value descending, vertex ascending on ties), by a bounded selection on the
   // calling thread (dn * pn comparisons, no worker threads).

@@ -62,3 +62,36 @@ def test_run_lengths(run_edges, prune, monkeypatch):
         for n_iter in (0, 1, 7):
             bad, ratio = allclose_report(m.run(n_iter), O.run(g64(data), g64(patt), n_iter=n_iter))
             assert bad == 0, (n_iter, ratio)
+
+
+@pytest.mark.parametrize("n,pn,k,kind", [
+    (70_000, 1, 1, "random"), (6554, 10, 3, "random"), (6553, 10, 3, "random"),  # one side and the other of the size rule
+    (40_000, 5, 512, "random"), (40_000, 5, 513, "random"), (300, 256, 75, "random"), (300, 256, 150, "random"),
+    (50_000, 7, 40, "groups"), (50_000, 3, 9, "equal"), (20_000, 12, 20_000, "random"), (30_000, 4, 5, "nan"),
+])
+def test_topk_and_match_selection(n, pn, k, kind):
+    """The k best of each column in order, ties by lower vertex: device and host selection, chunks of one row, values
+    shared by a few vertices (groups) and by more than the device keeps (equal), and NaN columns."""
+    data, patt = random_graph(n, 2 * n, 3, 2, n + k), random_graph(pn, pn, 3, 2, pn)
+    if kind == "groups":
+        data.vfeat[:] = data.vfeat[np.arange(n) % 900]
+    elif kind == "equal":
+        data.vfeat[:] = data.vfeat[0]
+    elif kind == "nan":
+        data.vfeat[n // 2] = np.nan
+    with Matcher(0) as m:
+        m.set_data(data)
+        m.set_pattern(patt)
+        mu = m.run(0)
+        idx, val = m.topk(k)
+        match = m.match(-8.0)
+    if kind == "nan":
+        assert np.isnan(mu).any()
+        return  # no order to hold: the calls return, as they did
+    want = np.stack([np.lexsort((np.arange(n), -mu[:, p]))[:k] for p in range(pn)])
+    np.testing.assert_array_equal(idx, want)
+    np.testing.assert_array_equal(val, np.take_along_axis(mu.T, want, axis=1))
+    best = mu.argmax(axis=0)
+    expect = np.zeros((n, pn), np.uint8)
+    expect[best, np.arange(pn)] = np.where(mu[best, np.arange(pn)] >= -8.0, 2, 1)
+    np.testing.assert_array_equal(match, expect)
