@@ -312,7 +312,9 @@ struct ac_ctx {
   };
   DevBuf<char> pat;
   Part<double> pf_v, pf_e;
-  Part<int> d_ps, d_pd, d_inc_off, d_inc;
+  Part<int> d_ps, d_pd, d_inc_off, d_inc, d_sum_off;
+  Part<int2> d_sums;
+  int nsum = 0;  // partial sums of the vertex passes
 
   // Work buffers.
   DevBuf<float> CE, CV, FMaxN, VFm, minCEo, lsO, VR, OUT;
@@ -351,7 +353,7 @@ struct ac_ctx {
   DevBuf<Lse2> pstat, lse_cv, lse_ce;
   DevBuf<IsoCol> iso;   // [P] the isolated vertices' columns of CV (when n_iso > 0)
   int nb_vertex = 0, nb_vertex_c = 0, nb_vertex_o = 0, nb_col = 0, nb_src = 0, VT = 0, VRs = 0;
-  int64_t work_key[5] = {-1, -1, -1, -1, -1};
+  int64_t work_key[6] = {-1, -1, -1, -1, -1, -1};
 
   bool have_result = false;
   int last_iters = 0;
@@ -666,7 +668,12 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
     if (bytes) std::memcpy(all.data() + at, v.data(), bytes);
     return at;
   };
-  const size_t o_v = part(pv), o_e = part(pe), o_s = part(ps_pad), o_d = part(pd_pad), o_o = part(inc_off), o_i = part(inc);
+  const int nsum = ac::vertex_sums((int)nV, inc_off.data(), nullptr, nullptr);
+  std::vector<int2> sums((size_t)std::max(1, nsum));
+  std::vector<int> sum_off(nV + 1);
+  (void)ac::vertex_sums((int)nV, inc_off.data(), sums.data(), sum_off.data());
+  const size_t o_v = part(pv), o_e = part(pe), o_s = part(ps_pad), o_d = part(pd_pad), o_o = part(inc_off),
+               o_i = part(inc), o_u = part(sums), o_f = part(sum_off);
   HIPCHK(ctx, ctx->pat.alloc(all.size()));
   if (ctx->stage.ready()) {
     HIPCHK(ctx, ctx->stage.to_device(ctx->pat.p, all.data(), all.size(), st));
@@ -680,6 +687,9 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
   ctx->d_pd.p = reinterpret_cast<int*>(ctx->pat.p + o_d);
   ctx->d_inc_off.p = reinterpret_cast<int*>(ctx->pat.p + o_o);
   ctx->d_inc.p = reinterpret_cast<int*>(ctx->pat.p + o_i);
+  ctx->d_sums.p = reinterpret_cast<int2*>(ctx->pat.p + o_u);
+  ctx->d_sum_off.p = reinterpret_cast<int*>(ctx->pat.p + o_f);
+  ctx->nsum = nsum;
   ctx->cnull_groups.assign({0, (int)nE});
   ctx->has_patt = true;
   ctx->have_result = false;
@@ -822,11 +832,11 @@ static int select_bundles(ac_ctx* ctx) {
 static int ensure_work(ac_ctx* ctx) {
   int rc = select_bundles(ctx);
   if (rc != AC_OK) return rc;
-  const int64_t key[5] = {ctx->dn, ctx->de, ctx->P, ctx->Q, ctx->bs->brows};
-  if (std::equal(key, key + 5, ctx->work_key)) return AC_OK;
+  const int64_t key[6] = {ctx->dn, ctx->de, ctx->P, ctx->Q, ctx->bs->brows, ctx->nsum};
+  if (std::equal(key, key + 6, ctx->work_key)) return AC_OK;
   const int64_t n = ctx->dn;
   const int P = ctx->P, Q = ctx->Q, Qs = ctx->Qs;
-  ctx->VT = ac::vertex_tile(ctx->n_act, P, Q);
+  ctx->VT = ac::vertex_tile(ctx->n_act, P, Q, ctx->nsum);
   const int64_t ntiles = (std::max<int64_t>(ctx->n_act, 1) + ctx->VT - 1) / ctx->VT;
   {
     ac::VertexArgs va{};
@@ -834,6 +844,7 @@ static int ensure_work(ac_ctx* ctx) {
     va.Q = Q;
     va.Qs = Qs;
     va.VT = ctx->VT;
+    va.nsum = ctx->nsum;
     const int64_t all_tiles = (n + ctx->VT - 1) / ctx->VT;
     ctx->nb_vertex = vertex_blocks("AC_VERTEX_BLOCKS", ac::vertex_resident_blocks(ac::kModeA, va), 1, ntiles);
     ctx->nb_vertex_c = vertex_blocks("AC_VERTEX_BLOCKS_C", ac::vertex_resident_blocks(ac::kModeC, va), 1, ntiles);
@@ -867,7 +878,7 @@ static int ensure_work(ac_ctx* ctx) {
   // Padding columns of the row-major [n][Qs] arrays are never read as data; keep them zero.
   HIPCHK(ctx, hipMemsetAsync(ctx->VR.p, 0, ctx->VR.n * sizeof(float), ctx->stream));
   HIPCHK(ctx, hipMemsetAsync(ctx->qstat.p, 0, ctx->qstat.n * sizeof(QStat), ctx->stream));
-  std::copy(key, key + 5, ctx->work_key);
+  std::copy(key, key + 6, ctx->work_key);
   return AC_OK;
 }
 
@@ -1103,6 +1114,9 @@ static ac::VertexArgs vertex_args(ac_ctx* ctx) {
   va.pd = ctx->d_pd.p;
   va.inc_off = ctx->d_inc_off.p;
   va.inc = ctx->d_inc.p;
+  va.sums = ctx->d_sums.p;
+  va.sum_off = ctx->d_sum_off.p;
+  va.nsum = ctx->nsum;
   va.pst = ctx->pstat.p;
   va.qpart = ctx->qpart.p;
   va.ppart = ctx->ppart.p;

@@ -102,10 +102,13 @@ struct VertexArgs {
   const int* pd;
   const int* inc_off;  // [P + 1]
   const int* inc;      // incidence of each pattern vertex: (q << 1) | (1 if RMax term else 0), ascending q
+  const int2* sums;    // [nsum] incidences [x, y) of each partial sum of the MU sums (vertex_sums)
+  const int* sum_off;  // [P + 1]
+  int nsum;
   const QStat* qs;     // scalars that finish FMax / RMax of the state being read
   const Lse2* pst;     // log-sum-exp of each MU column
-  QPart* qpart;        // [tile blocks + 1][Q]
-  Lse* ppart;          // [tile blocks + 1][P]
+  QPart* qpart;        // [Q][tile blocks + 1]
+  Lse* ppart;          // [P][tile blocks + 1]
   int first;           // MU = LSM(-CV): the prep state, no FMax / RMax terms
   int track_arg;       // mode A: record the vertices of the column maxima (QStat vF / vR)
 };
@@ -163,6 +166,9 @@ void launch_copy_cols(int64_t n, int P, int c0, int ncol, const float* src, floa
 int walk_blocks(int64_t nruns, int Qs);
 int walk_groups(int Qs);  // runs per bundle: 64 / (Qs / 4)
 int walk_batch();         // default steps per batch of the bundle walk: 1, 2 or 4 (bundle lengths are multiples of it)
-int vertex_tile(int64_t n, int P, int Q);  // rows per tile for n vertices
+int vertex_tile(int64_t n, int P, int Q, int nsum);  // rows per tile for n vertices
+// The partial sums of a pattern's MU sums: their incidence ranges and each pattern vertex's first one (either may be
+// null); returns their number.
+int vertex_sums(int P, const int* inc_off, int2* sums, int* off);
 
 }  // namespace ac

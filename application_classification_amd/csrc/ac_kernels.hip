@@ -496,7 +496,7 @@ __global__ __launch_bounds__(256) void k_col_lse_neg(int64_t n, int P, const flo
     for (int64_t v = (int64_t)blockIdx.x * RP + t / P; v < n; v += (int64_t)gridDim.x * RP)
       lse_add(acc, -(double)X[v * P + p]);
   const Lse s = block_columns_lse(acc, P, RP, red);
-  if (t < P) part[(int64_t)blockIdx.x * P + t] = s;
+  if (t < P) part[(int64_t)t * gridDim.x + blockIdx.x] = s;
 }
 
 void launch_col_lse_neg(int64_t n, int P, const float* X, Lse* part, int nblocks, hipStream_t st) {
@@ -508,26 +508,26 @@ void launch_col_lse_neg(int64_t n, int P, const float* X, Lse* part, int nblocks
 // partial load the last partial (an in-bounds address) and then hold the empty one.
 constexpr int kRedLse = 8, kRedQ = 5;
 
-// Reduce per-block partials [nparts][ncol] column by column in a fixed order (deterministic).
-__global__ __launch_bounds__(256) void k_reduce_lse(int nparts, int ncol, const Lse* __restrict__ part,
-                                                    Lse2* __restrict__ out) {
+// Reduce per-block partials [ncol][nparts] column by column in a fixed order (deterministic).  (A column's partials lie
+// together: by block, [nparts][ncol], every partial of a column was a line of its own.)
+__global__ __launch_bounds__(256) void k_reduce_lse(int nparts, const Lse* __restrict__ part, Lse2* __restrict__ out) {
   __shared__ double red[8];
   const int c = blockIdx.x, t = threadIdx.x;
   Lse v[kRedLse];
 #pragma unroll
   for (int u = 0; u < kRedLse; ++u) {
+    v[u] = lse_empty();
+    if (u * 256 >= nparts) continue;  // (the same for the whole block)
     const int b = t + u * 256;
-    v[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * ncol + c];
+    const Lse x = part[(int64_t)c * nparts + (b < nparts ? b : nparts - 1)];
+    if (b < nparts) v[u] = x;
   }
-#pragma unroll
-  for (int u = 0; u < kRedLse; ++u)
-    if (t + u * 256 >= nparts) v[u] = lse_empty();
   for (int b0 = 256 * kRedLse + t; b0 < nparts; b0 += 256 * kRedLse) {
     Lse w[kRedLse];
 #pragma unroll
     for (int u = 0; u < kRedLse; ++u) {
       const int b = b0 + u * 256;
-      w[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * ncol + c];
+      w[u] = part[(int64_t)c * nparts + (b < nparts ? b : nparts - 1)];
     }
 #pragma unroll
     for (int u = 0; u < kRedLse; ++u)
@@ -540,14 +540,15 @@ __global__ __launch_bounds__(256) void k_reduce_lse(int nparts, int ncol, const 
   double sum = 0.0;
   bool seen = false;
 #pragma unroll
-  for (int u = 0; u < kRedLse; ++u) lse_sum_step(sum, seen, lse_rescaled(v[u], M));
+  for (int u = 0; u < kRedLse; ++u)
+    if (u * 256 < nparts) lse_sum_step(sum, seen, lse_rescaled(v[u], M));
   sum = block_lse_sum<256>(sum, seen, red);
   if (t == 0) out[c] = Lse2{M, log1p(sum)};
 }
 
 void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStream_t st) {
   if (ncol == 0) return;
-  hipLaunchKernelGGL(k_reduce_lse, dim3(ncol), dim3(256), 0, st, nparts, ncol, part, out);
+  hipLaunchKernelGGL(k_reduce_lse, dim3(ncol), dim3(256), 0, st, nparts, part, out);
 }
 
 // FMaxN rows of the split vertices to -inf, over nblocks blocks: the walk's pieces of a split vertex then raise its row
@@ -570,91 +571,120 @@ static int reset_blocks(int nsplit, int Qs) {
 // cnull != nullptr: the iteration's fills are lowered by the PNNL Cnull term, fillF = max VR - cnull[q] and
 // fillR = max VF - cnull[q] (test.py:148-149; cnull <= 0, so the fills rise and the pruning bound below, which assumes
 // the unraised fill, stays valid).
-__global__ __launch_bounds__(256) void k_reduce_q(int nparts, int Q, const QPart* __restrict__ part,
-                                                  const double* __restrict__ cnull, QStat* __restrict__ out,
-                                                  SplitRows rows) {
-  __shared__ double red[8], redv[8];
-  __shared__ int redi[8];
+// Four groups of 256 threads, one for each of RE's log-sum-exp, FE's, max VF and max VR, side by side (one group taking
+// them in turn, partials of a column a line each: 7.4-12 us; now 5.2-7.3 us).
+__global__ __launch_bounds__(1024) void k_reduce_q(int nparts, int Q, const QPart* __restrict__ part,
+                                                   const double* __restrict__ cnull, QStat* __restrict__ out,
+                                                   SplitRows rows) {
   if ((int)blockIdx.x >= Q) {  // the blocks after the Q reducing ones
     reset_split_rows(blockIdx.x - Q, gridDim.x - Q, rows.nsplit, rows.splits, rows.Qs, rows.FMaxN);
     return;
   }
-  const int q = blockIdx.x, t = threadIdx.x;
-  const QPart empty{-kInf, -kInf, lse_empty(), lse_empty(), -1, -1};
-  QPart v[kRedQ];
-#pragma unroll
-  for (int u = 0; u < kRedQ; ++u) {
-    const int b = t + u * 256;
-    v[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * Q + q];
-  }
-#pragma unroll
-  for (int u = 0; u < kRedQ; ++u)
-    if (t + u * 256 >= nparts) v[u] = empty;
-  for (int b0 = 256 * kRedQ + t; b0 < nparts; b0 += 256 * kRedQ) {
-    QPart w[kRedQ];
+  __shared__ double sm[4][4], ss[4][4];
+  __shared__ int sa[4][4];
+  const int q = blockIdx.x, t = threadIdx.x & 255, lane = t & 63, w = t >> 6;
+  const int job = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+  double m = -kInf, sum = 0.0;
+  int arg = -1;
+  bool seen = false;
+  const QPart* pq = part + (int64_t)q * nparts;
+  if (job < 2) {
+    Lse v[kRedQ];
 #pragma unroll
     for (int u = 0; u < kRedQ; ++u) {
-      const int b = b0 + u * 256;
-      w[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * Q + q];
+      v[u] = lse_empty();
+      if (u * 256 >= nparts) continue;  // (the same for the whole block)
+      const int b = t + u * 256;
+      const QPart* p = pq + (b < nparts ? b : nparts - 1);
+      const Lse x = job == 0 ? p->re : p->fe;
+      if (b < nparts) v[u] = x;
     }
+    for (int b0 = 256 * kRedQ + t; b0 < nparts; b0 += 256 * kRedQ)
+#pragma unroll
+      for (int u = 0; u < kRedQ; ++u) {
+        const int b = b0 + u * 256;
+        if (b < nparts) v[u] = lse_merge(v[u], job == 0 ? pq[b].re : pq[b].fe);
+      }
+#pragma unroll
+    for (int u = 0; u < kRedQ; ++u) m = fmax(m, v[u].m);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o, 64));
+    if (lane == 0) sm[job][w] = m;
+    __syncthreads();
+    m = fmax(fmax(sm[job][0], sm[job][1]), fmax(sm[job][2], sm[job][3]));
 #pragma unroll
     for (int u = 0; u < kRedQ; ++u)
-      if (b0 + u * 256 < nparts) qpart_merge(v[u], w[u]);
-  }
-  QPart s = v[0];
+      if (u * 256 < nparts) lse_sum_step(sum, seen, lse_rescaled(v[u], m));
+    const unsigned long long holders = __ballot(seen);
+    if (seen && lane != __ffsll((long long)holders) - 1) sum += 1.0;
 #pragma unroll
-  for (int u = 1; u < kRedQ; ++u) {
-    argmax_merge(s.vfmax, s.avf, v[u].vfmax, v[u].avf);
-    argmax_merge(s.vrmax, s.avr, v[u].vrmax, v[u].avr);
-    s.re.m = fmax(s.re.m, v[u].re.m);
-    s.fe.m = fmax(s.fe.m, v[u].fe.m);
-  }
-  s.re.m = block_max<256>(s.re.m, red);
-  s.fe.m = block_max<256>(s.fe.m, red);
-  s.re.t = s.fe.t = 0.0;
-  bool ore = false, ofe = false;
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    if (lane == 0) {
+      ss[job][w] = sum;
+      sa[job][w] = holders != 0;
+    }
+  } else {
+    for (int b0 = t; b0 < nparts; b0 += 256 * kRedQ) {
+      double x[kRedQ];
+      int a[kRedQ];
 #pragma unroll
-  for (int u = 0; u < kRedQ; ++u) {
-    lse_sum_step(s.re.t, ore, lse_rescaled(v[u].re, s.re.m));
-    lse_sum_step(s.fe.t, ofe, lse_rescaled(v[u].fe, s.fe.m));
-  }
-  s.re.t = block_lse_sum<256>(s.re.t, ore, red);
-  s.fe.t = block_lse_sum<256>(s.fe.t, ofe, redv);
-  // The maxima with their vertices (ties: the lowest, in any order).
+      for (int u = 0; u < kRedQ; ++u) {
+        const int b = b0 + u * 256;
+        const QPart* p = pq + (b < nparts ? b : nparts - 1);  // (past the end: the last one again)
+        x[u] = job == 2 ? p->vfmax : p->vrmax;
+        a[u] = job == 2 ? p->avf : p->avr;
+      }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    argmax_merge(s.vfmax, s.avf, __shfl_xor(s.vfmax, o, 64), __shfl_xor(s.avf, o, 64));
-    argmax_merge(s.vrmax, s.avr, __shfl_xor(s.vrmax, o, 64), __shfl_xor(s.avr, o, 64));
-  }
-  __syncthreads();  // red and redv read
-  if ((t & 63) == 0) {
-    const int w = t >> 6;
-    red[w] = s.vfmax, red[4 + w] = s.vrmax;
-    redi[w] = s.avf, redi[4 + w] = s.avr;
+      for (int u = 0; u < kRedQ; ++u) argmax_merge(m, arg, x[u], a[u]);
+    }
+    // Ties: the lowest vertex, in any order.
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) argmax_merge(m, arg, __shfl_xor(m, o, 64), __shfl_xor(arg, o, 64));
+    if (lane == 0) {
+      sm[job][w] = m;
+      sa[job][w] = arg;
+    }
+    __syncthreads();
   }
   __syncthreads();
   if (t == 0) {
-    for (int w = 1; w < 4; ++w) {
-      argmax_merge(s.vfmax, s.avf, red[w], redi[w]);
-      argmax_merge(s.vrmax, s.avr, red[4 + w], redi[4 + w]);
+    if (job < 2) {
+      sum = ss[job][0];
+      bool any = sa[job][0] != 0;
+      for (int i = 1; i < 4; ++i) {
+        sum += ss[job][i];
+        if (sa[job][i]) {
+          if (any) sum += 1.0;
+          any = true;
+        }
+      }
+      ss[job][0] = sum;
+      sm[job][1] = log1p(sum);
+    } else {
+      for (int i = 1; i < 4; ++i) argmax_merge(m, arg, sm[job][i], sa[job][i]);
+      sa[job][0] = arg;
     }
-    const QPart r = s;
+    sm[job][0] = m;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const double vfmax = sm[2][0], vrmax = sm[3][0];
     // Edge pruning bound.  An edge term is (VR[src] - CE) - LSE_FE with VR[src] <= fillF (rounded to FP32 once),
     // so it cannot exceed fillF when CE + LSE_FE >= 2^-22 (|fillF| + |CE| + |LSE_FE|); cthr = -LSE_FE plus four
     // times that margin (a cost near the bound has |CE| ~ |LSE_FE|; a larger one clears it by itself).
-    const double fF = r.vrmax, sl = r.fe.m + log1p(r.fe.t);
+    const double fF = vrmax, sl = sm[1][0] + sm[1][1];
     double cthr = kInf;
     if (fF > -kInf && fF < kInf && sl > -kInf && sl < kInf)
       cthr = -sl + 0x1p-20 * (fabs(fF) + 2.0 * fabs(sl) + 1.0);
-    const double fillF = cnull ? r.vrmax - cnull[q] : r.vrmax, fillR = cnull ? r.vfmax - cnull[q] : r.vfmax;
-    out[q] = QStat{fillF, fillR, r.re.m, log1p(r.re.t), r.fe.m, log1p(r.fe.t), r.avr, r.avf, cthr};
+    const double fillF = cnull ? vrmax - cnull[q] : vrmax, fillR = cnull ? vfmax - cnull[q] : vfmax;
+    out[q] = QStat{fillF, fillR, sm[0][0], sm[0][1], sm[1][0], sm[1][1], sa[3][0], sa[2][0], cthr};
   }
 }
 
 void launch_reduce_q(int nparts, int Q, const QPart* part, QStat* out, hipStream_t st, const double* cnull,
                      const SplitRows& rows) {
   if (Q == 0) return;
-  hipLaunchKernelGGL(k_reduce_q, dim3(Q + reset_blocks(rows.nsplit, rows.Qs)), dim3(256), 0, st, nparts, Q, part, cnull,
+  hipLaunchKernelGGL(k_reduce_q, dim3(Q + reset_blocks(rows.nsplit, rows.Qs)), dim3(1024), 0, st, nparts, Q, part, cnull,
                      out, rows);
 }
 
@@ -917,7 +947,7 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
     Lse acc{mx[q], 0.0};
     bool seen = false;
     for (int i = 0; i < slots; ++i) lse_sum_step(acc.t, seen, red[i * Qs + q]);
-    gpart[(int64_t)blockIdx.x * Q + q] = acc;
+    gpart[(int64_t)q * gridDim.x + blockIdx.x] = acc;
   }
 }
 
@@ -1517,9 +1547,9 @@ void launch_walk_max_fixup(int nsplit, const Split* splits, const double* carry,
 // fill a tile with few vertices, by the chain through one block: its tables, its tiles one after the other, the merge
 // of its partials.  Hence short tiles where there are few (vertex_tile), lanes shared among pattern vertices, and
 // merges that take one exponential however many partials they merge.  Passes A / C per launch, before (a wave per
-// pattern vertex whatever the tile's height, isolated vertices on block 0's way, serial merges) and now: 1,000 vertices
-// with a 10/12 pattern 20.0 / 8.5 -> 11.0 / 6.2 us; 50,001 with 40/70 48.9 / 44.4 -> 32.3 / 23.8 us; R-MAT 16 slabs of
-// 128 pattern edges 98.5 / 108.3 -> 67.7 / 30.6 us; R-MAT 20 with 16/24 105.7 / 58.9 -> 104.5 / 48.0 us.
+// pattern vertex whatever the tile's height, isolated vertices on block 0's way, serial merges, a term at a time) and
+// now: 1,000 vertices with a 10/12 pattern 20.0 / 8.5 -> 11.8 / 5.3 us; 50,001 with 40/70 48.9 / 44.4 -> 29.2 / 20.0 us;
+// R-MAT 16 slabs of 128 pattern edges 98.5 / 108.3 -> 50 / 35 us; R-MAT 20 with 16/24 105.7 / 58.9 -> 97 / 42 us.
 
 constexpr int kVTMax = 64;
 // Staged tile limits: VT * Qs <= 2048 and VT * P <= 2048 floats, for every block size NT (256 or 512).
@@ -1533,8 +1563,12 @@ struct IncRec {
   int col, pad;
 };
 
-static size_t vertex_lds_bytes(int mode, int VT, int P, int Q, int Qs) {
+// Partial sums of the MU sums (tiles of fewer than 64 rows): up to kTerms consecutive incidences of one pattern vertex.
+constexpr int kTerms = 4;
+
+static size_t vertex_lds_bytes(int mode, int VT, int P, int Q, int Qs, int nsum) {
   size_t b = (size_t)(2 * P) * sizeof(double);                               // MU normalisers
+  if (VT < 64) b += (size_t)nsum * (VT * sizeof(double) + sizeof(int2)) + (size_t)(P + 1) * sizeof(int);  // partial sums
   b += (size_t)(2 * Q + 1) * sizeof(IncRec);                                 // incidence records (+ one pad)
   if (mode != kModeC) b += (size_t)(P + 1) * VT * sizeof(double);            // MU
   const int nst = mode == kModeA ? 4 : 2;                                    // staged [VT][Qs] arrays
@@ -1544,10 +1578,21 @@ static size_t vertex_lds_bytes(int mode, int VT, int P, int Q, int Qs) {
   return (b + 15) / 16 * 16;
 }
 
-// Tiles wanted at least: two for each of the 256 CUs.
-constexpr int kTilesWanted = 512;
+// Tiles wanted at least: one for each of the 256 CUs.
+constexpr int kTilesWanted = 256;
 
-int vertex_tile(int64_t n, int P, int Q) {
+int vertex_sums(int P, const int* inc_off, int2* sums, int* off) {
+  int m = 0;
+  for (int p = 0; p < P; ++p) {
+    if (off) off[p] = m;
+    for (int k = inc_off[p]; k < inc_off[p + 1]; k += kTerms, ++m)
+      if (sums) sums[m] = make_int2(k, std::min(k + kTerms, inc_off[p + 1]));
+  }
+  if (off) off[P] = m;
+  return m;
+}
+
+int vertex_tile(int64_t n, int P, int Q, int nsum) {
   const int Qs = std::max(4, (Q + 3) / 4 * 4);
   int vt = kVTMax;
   if (const char* e = std::getenv("AC_VERTEX_TILE")) {  // tuning override: rows per tile, 8, 16, 32 or 64
@@ -1556,7 +1601,7 @@ int vertex_tile(int64_t n, int P, int Q) {
   } else {
     while (vt > 8 && (n + vt - 1) / vt < kTilesWanted) vt /= 2;
   }
-  while (vt > 4 && (vertex_lds_bytes(kModeA, vt, P, Q, Qs) > 65536 || vt * Qs > kTileFloats ||
+  while (vt > 4 && (vertex_lds_bytes(kModeA, vt, P, Q, Qs, nsum) > 65536 || vt * Qs > kTileFloats ||
                     vt * P > kTileFloats))
     vt /= 2;
   return vt;
@@ -1570,9 +1615,14 @@ typedef const __attribute__((address_space(4))) int cint_t;
 // Their FMaxN = VFm = -inf rows make MU_pre = -CV + K_p, K_p the sum of the fills of p's incidences (in the vertex
 // pass's own operation sequence), so MU is largest at the least-cost isolated vertex and the column log-sum-exp is
 // LSE(-CV) + K_p.  They have no out-edges: no edge terms.
-__device__ double iso_kp(const IncRec* recs, const int* ioff, int p, bool sums, double acc) {
-  if (sums)
-    for (int k = ioff[p]; k < ioff[p + 1]; ++k) acc += fmax(recs[k].fill, -kInf);
+__device__ double iso_kp(const VertexArgs& a, const IncRec* recs, const int* ioff, int p, double acc) {
+  if (a.first) return acc;
+  const int step = a.VT == 64 ? 1 : kTerms;
+  for (int k = ioff[p]; k < ioff[p + 1]; k += step) {
+    double s = fmax(recs[k].fill, -kInf);
+    for (int u = 1; u < step && k + u < ioff[p + 1]; ++u) s += fmax(recs[k + u].fill, -kInf);
+    acc += s;
+  }
   return acc;
 }
 
@@ -1582,12 +1632,12 @@ __device__ QPart iso_qpart(const VertexArgs& a, const IncRec* recs, const int* i
   const int pd = a.pd[q], ps = a.ps[q];
   const double fm = fmax(a.qs[q].fillF, -kInf), rm = fmax(a.qs[q].fillR, -kInf);
   if (a.iso[pd].vmin >= 0) {
-    const double mu = (iso_kp(recs, ioff, pd, !a.first, -(double)a.iso[pd].cmin) - a.pst[pd].m) - a.pst[pd].l;
+    const double mu = (iso_kp(a, recs, ioff, pd, -(double)a.iso[pd].cmin) - a.pst[pd].m) - a.pst[pd].l;
     w.vfmax = mu - fm;
     if (w.vfmax > -kInf) w.avf = a.iso[pd].vmin;  // as in the vertex pass, -inf records no vertex
   }
   if (a.iso[ps].vmin >= 0) {
-    const double mu = (iso_kp(recs, ioff, ps, !a.first, -(double)a.iso[ps].cmin) - a.pst[ps].m) - a.pst[ps].l;
+    const double mu = (iso_kp(a, recs, ioff, ps, -(double)a.iso[ps].cmin) - a.pst[ps].m) - a.pst[ps].l;
     w.vrmax = mu - rm;
     if (w.vrmax > -kInf) w.avr = a.iso[ps].vmin;
   }
@@ -1596,7 +1646,7 @@ __device__ QPart iso_qpart(const VertexArgs& a, const IncRec* recs, const int* i
 
 __device__ Lse iso_lse(const VertexArgs& a, const IncRec* recs, const int* ioff, int p) {
   if (!a.iso || a.iso[p].vmin < 0) return lse_empty();
-  const double m = iso_kp(recs, ioff, p, !a.first, a.iso[p].m);
+  const double m = iso_kp(a, recs, ioff, p, a.iso[p].m);
   return m > -kInf ? Lse{m, a.iso[p].t} : lse_empty();
 }
 
@@ -1608,8 +1658,8 @@ constexpr int kPW = 4;  // mode C: pattern vertices per lane; VT * P <= kTileFlo
 // kArgMax (mode A): also track the vertices of the column maxima (the adjoint's tape needs them).
 // kPFC: CV values each thread prefetches per tile (VT * P <= NT * kPFC); fewer registers allow more resident waves.
 template <int kMode, bool kFull, bool kArgMax, int NT, int kPFC = kTileFloats / NT>
-__global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
-  constexpr int kVW = NT / 64, kPF4 = kTileFloats / 4 / NT;
+__global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void k_vertex(VertexArgs a) {
+  constexpr int kVW = NT / 64, kPF4 = kTileFloats / 4 / NT, kUnroll = kMode == kModeA ? 2 : 4;
   constexpr bool kA = kMode == kModeA, kC = kMode == kModeC;
   constexpr bool kRows = kMode == kModeOut || kMode == kModeMU;  // MU tile staged, written back row by row
   extern __shared__ double lds[];
@@ -1617,15 +1667,19 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
   const int ldq = Qs + 1, ldp = P + 1;
   double* pmu = lds;                                   // [2][P]: m, l of LSE_MU
   IncRec* recs = reinterpret_cast<IncRec*>(pmu + 2 * P);  // [2Q + 1] incidence records, inc order
-  double* MUs = reinterpret_cast<double*>(recs + 2 * Q + 1);  // [VT][P + 1] (modes A, OUT, MU)
+  const int nsum = kFull ? 0 : a.nsum;
+  double* Ps = reinterpret_cast<double*>(recs + 2 * Q + 1);  // [nsum][VT] partial sums (tiles of fewer than 64 rows)
+  double* MUs = Ps + nsum * VT;                        // [VT][P + 1] (modes A, OUT, MU)
   const int ldm = P + 1;
-  float* Fs = reinterpret_cast<float*>(MUs + (kC ? 0 : ldm * VT));  // [VT][ldq] FMaxN
+  int2* tasks = reinterpret_cast<int2*>(MUs + (kC ? 0 : ldm * VT));  // [nsum] incidences [x, y) of each partial sum
+  float* Fs = reinterpret_cast<float*>(tasks + nsum);  // [VT][ldq] FMaxN
   float* Vs = Fs + VT * ldq;                           // [VT][ldq] VFm
   float* Ms = Vs + VT * ldq;                           // [VT][ldq] minCEo (mode A)
   float* Ls = Ms + (kA ? VT * ldq : 0);                // [VT][ldq] lsO (mode A)
   float* Cs = Ls + (kA ? VT * ldq : 0);                // [VT][ldp] CV
   int* ioff = reinterpret_cast<int*>(Cs + VT * ldp);   // [P + 1] incidence offsets
-  int* Prow = ioff + P + 1;                            // [VT] caller id of each tile row (mode OUT)
+  int* soff = ioff + P + 1;                            // [P + 1] first partial sum of each pattern vertex
+  int* Prow = soff + (kFull ? 0 : P + 1);              // [VT] caller id of each tile row (mode OUT)
   const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const bool sums = !a.first;
   cint_t* const c_incoff = (cint_t*)a.inc_off;
@@ -1678,6 +1732,10 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
     recs[k] = r;
   }
   for (int i = t; i <= P; i += NT) ioff[i] = a.inc_off[i];
+  if (!kFull) {
+    for (int i = t; i < nsum; i += NT) tasks[i] = a.sums[i];
+    for (int i = t; i <= P; i += NT) soff[i] = a.sum_off[i];
+  }
   if (!kC)
     for (int i = t; i < P; i += NT) {
       pmu[i] = a.pst[i].m;
@@ -1686,9 +1744,9 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
   if (iso_block) {
     __syncthreads();
     if (kA)
-      for (int i = t; i < Q; i += NT) a.qpart[G * Q + i] = iso_qpart(a, recs, ioff, i);
+      for (int i = t; i < Q; i += NT) a.qpart[i * (G + 1) + G] = iso_qpart(a, recs, ioff, i);
     else
-      for (int i = t; i < P; i += NT) a.ppart[G * P + i] = iso_lse(a, recs, ioff, i);
+      for (int i = t; i < P; i += NT) a.ppart[i * (G + 1) + G] = iso_lse(a, recs, ioff, i);
     return;
   }
 
@@ -1758,26 +1816,67 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
     }
     __syncthreads();
     if (tile + G < ntiles) prefetch(tile + G);
-    // p-phase.  MU_pre of row prow and pattern vertex p.
+    // One incidence's term in tile row prow.
+    auto term = [&](const IncRec& rc, float x) __attribute__((always_inline)) {
+      const double d = ((double)x - rc.m) - rc.l;
+      return fmax(rc.fill, x == -INFINITY ? -kInf : d);
+    };
+    // p-phase.  Tiles of fewer than 64 rows form the sums in two steps, so that a pattern vertex with many incidences
+    // (a hub) is spread over the block: kTerms incidences per lane, then the partial sums in order.
+    if (!kFull && sums) {
+      for (int v = pfirst; v < nsum; v += psweep)
+        if (prow < nv) {
+          const int2 ks = tasks[v];
+          IncRec rc[kTerms];
+          float x[kTerms];
+#pragma unroll
+          for (int u = 0; u < kTerms; ++u) rc[u] = recs[min(ks.x + u, ks.y - 1)];
+#pragma unroll
+          for (int u = 0; u < kTerms; ++u) x[u] = Fs[prow * ldq + rc[u].col];
+          double s = term(rc[0], x[0]);
+#pragma unroll
+          for (int u = 1; u < kTerms; ++u)
+            if (ks.x + u < ks.y) s += term(rc[u], x[u]);
+          Ps[v * VT + prow] = s;
+        }
+      __syncthreads();
+    }
+    // MU_pre of row prow and pattern vertex p.
     auto mu_pre = [&](int p) __attribute__((always_inline)) {
       double acc = -(double)Cs[prow * ldp + p];
-      if (sums) {
-        const int k1 = kFull ? c_incoff[p + 1] : ioff[p + 1];
-        int k = kFull ? c_incoff[p] : ioff[p];
-        IncRec rc = recs[k];
-        for (; k < k1; ++k) {
-          const IncRec nx = recs[k + 1];  // in flight while this term is formed
-          const float x = Fs[prow * ldq + rc.col];
-          const double d = ((double)x - rc.m) - rc.l;
-          acc += fmax(rc.fill, x == -INFINITY ? -kInf : d);
-          rc = nx;
-        }
+      if (!sums) return acc;
+      if (!kFull) {
+        const int v1 = soff[p + 1];
+#pragma unroll 4
+        for (int v = soff[p]; v < v1; ++v) acc += Ps[v * VT + prow];
+        return acc;
+      }
+      // kUnroll terms at a time, their LDS reads all in flight; the sum is taken in order.  (A term by itself waits for
+      // its record, then for its value: about 200 cycles.)
+      const int k1 = c_incoff[p + 1];
+      int k = c_incoff[p];
+      for (; k + kUnroll <= k1; k += kUnroll) {
+        IncRec rc[kUnroll];
+        float x[kUnroll];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) rc[u] = recs[k + u];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) x[u] = Fs[prow * ldq + rc[u].col];
+#pragma unroll
+        for (int u = 0; u < kUnroll; ++u) acc += term(rc[u], x[u]);
+      }
+      IncRec rc = recs[k];
+      for (; k < k1; ++k) {
+        const IncRec nx = recs[k + 1];  // in flight while this term is formed
+        acc += term(rc, Fs[prow * ldq + rc.col]);
+        rc = nx;
       }
       return acc;
     };
     if (kC) {
 #pragma unroll
       for (int pi = 0; pi < kPW; ++pi) {
+        if (psweep * pi >= P) break;
         const int p = pfirst + psweep * pi;
         if (p < P) lse_add(pacc[pi], prow < nv ? mu_pre(p) : -kInf);
       }
@@ -1874,14 +1973,15 @@ __global__ __launch_bounds__(NT) void k_vertex(VertexArgs a) {
         lse_sum_step(acc.re.t, ore, Ts[r * Q + t]);
         lse_sum_step(acc.fe.t, ofe, Ts[RQ * Q + r * Q + t]);
       }
-      a.qpart[blk * Q + t] = acc;
+      a.qpart[t * (G + 1) + blk] = acc;
     }
   } else if (kC) {
 #pragma unroll
     for (int pi = 0; pi < kPW; ++pi) {
+      if (psweep * pi >= P) break;
       const int p = pfirst + psweep * pi;
       const Lse w = lanes_lse_merge(pacc[pi], VT);
-      if (p < P && prow == 0) a.ppart[blk * P + p] = w;
+      if (p < P && prow == 0) a.ppart[p * (G + 1) + blk] = w;
     }
   }
 }
@@ -1911,7 +2011,7 @@ static VertexKernel vertex_kernel_t(int mode, const VertexArgs& a) {
 
 // The kernel a pass launches, its block size and dynamic LDS bytes.
 static VertexKernel vertex_kernel(int mode, const VertexArgs& a, int* nt, size_t* lds) {
-  const size_t tiles = vertex_lds_bytes(mode, a.VT, a.P, a.Q, a.Qs);
+  const size_t tiles = vertex_lds_bytes(mode, a.VT, a.P, a.Q, a.Qs, a.nsum);
   *nt = mode == kModeA ? kNA : kNO;
   *lds = mode == kModeA ? std::max(tiles, sizeof(QPart) * kNA) : tiles;
   return a.VT == 64 ? vertex_kernel_t<true>(mode, a) : vertex_kernel_t<false>(mode, a);
