@@ -343,12 +343,11 @@ struct ac_ctx {
   DevBuf<unsigned> CEp;    // [rows * Qs * 3 / 4] packed costs of the bundles whose base is nonzero
   DevBuf<unsigned> bpack;  // [bundles] base of a bundle's codes, 0 = FP32 rows
   bool use_mfma_cdist = true;  // feature distances on FP64 matrix cores (GEMM form, cancellation-guarded)
-  DevBuf<double> cd_scratch;   // the matrix-core operands of the pattern features
   DevBuf<float> bmin;      // [bundles][Qs] least cost per bundle and pattern edge
   DevBuf<int> bstate;      // [bundles] launch_walk_max
   DevBuf<double> carry_in, carry_out;
   DevBuf<QPart> qpart;
-  DevBuf<Lse> ppart, lpart;
+  DevBuf<Lse> ppart, lpart, spart;  // spart: the per-source statistics', which run beside the vertex side's lpart
   DevBuf<QStat> qstat;  // [3][Q]: prep state, then by iteration parity
   DevBuf<Lse2> pstat, lse_cv, lse_ce;
   DevBuf<IsoCol> iso;   // [P] the isolated vertices' columns of CV (when n_iso > 0)
@@ -853,7 +852,6 @@ static int ensure_work(ac_ctx* ctx) {
   }
   ctx->nb_col = (int)std::min<int64_t>((n + 255) / 256, 1024);
   ctx->nb_src = std::max(1, ac::walk_blocks(ctx->nruns_out, Qs));
-  const int nb_l = std::max(ctx->nb_col, ctx->nb_src);
   HIPCHK(ctx, ctx->CE.alloc((size_t)std::max<int64_t>(1, ctx->bs->brows * Qs)));
   HIPCHK(ctx, ctx->CV.alloc((size_t)(n * P)));
   HIPCHK(ctx, ctx->FMaxN.alloc((size_t)(n * Qs)));
@@ -867,7 +865,8 @@ static int ensure_work(ac_ctx* ctx) {
   HIPCHK(ctx, ctx->carry_out.alloc((size_t)std::max(1, ctx->nslots_out) * Qs * 2));
   HIPCHK(ctx, ctx->qpart.alloc((size_t)(ctx->nb_vertex + 1) * std::max(1, Q)));
   HIPCHK(ctx, ctx->ppart.alloc((size_t)(ctx->nb_vertex_c + 1) * P));
-  HIPCHK(ctx, ctx->lpart.alloc((size_t)nb_l * std::max(P, std::max(Q, 1))));
+  HIPCHK(ctx, ctx->lpart.alloc((size_t)ctx->nb_col * P));
+  HIPCHK(ctx, ctx->spart.alloc((size_t)ctx->nb_src * std::max(Q, 1)));
   HIPCHK(ctx, ctx->qstat.alloc((size_t)3 * std::max(1, Q)));
   HIPCHK(ctx, ctx->pstat.alloc((size_t)P));
   HIPCHK(ctx, ctx->lse_cv.alloc((size_t)P));
@@ -994,11 +993,6 @@ static int enqueue_prep(ac_ctx* ctx) {
   HIPCHK(ctx, hipEventRecord(ctx->ev[0], st));
   MARK(-1);
   // ---- prep (src/main.cu:107-148)
-  // Vertex and edge distances run at the same time, so each has its own pattern operands.
-  const size_t vsd = ac::cdist_scratch_doubles(P, (int)ctx->dV), esd = ac::cdist_scratch_doubles(Qs, (int)ctx->dE);
-  HIPCHK(ctx, ctx->cd_scratch.alloc(std::max<size_t>(1, vsd + esd)));
-  double* cds_v = ctx->use_mfma_cdist ? ctx->cd_scratch.p : nullptr;
-  double* cds_e = ctx->use_mfma_cdist ? ctx->cd_scratch.p + vsd : nullptr;
   if (Q > 0) {
     HIPCHK(ctx, ctx->bmin.alloc((size_t)std::max<int64_t>(1, ctx->bs->nbundles) * Qs));
     HIPCHK(ctx, ctx->bstate.alloc((size_t)std::max<int64_t>(1, ctx->bs->nbundles)));
@@ -1007,33 +1001,27 @@ static int enqueue_prep(ac_ctx* ctx) {
   }
   // The vertex side (distances, column statistics, isolated columns) and the constant rows of the per-vertex arrays
   // go to the second stream, beside the edge distances on the first; the first waits for them (xev[1]) before the
-  // per-source statistics, which reuse the partial buffer, and the prep scalars, which read lse_cv.
+  // prep scalars, which read lse_cv.
   hipStream_t ax = ctx->aux;
   HIPCHK(ctx, hipEventRecord(ctx->xev[0], st));
   HIPCHK(ctx, hipStreamWaitEvent(ax, ctx->xev[0], 0));
   ac::launch_cdist(n, ctx->d_perm.p, ctx->vfeat.p, (int)ctx->dV, ctx->pf_v.p, P, round8(P), P, ctx->CV.p, P,
-                   ctx->has_wv ? ctx->wv.p : nullptr, cds_v, ax);
+                   ctx->has_wv ? ctx->wv.p : nullptr, ctx->use_mfma_cdist, ax);
   ac::launch_col_lse_neg(n, P, ctx->CV.p, ctx->lpart.p, ctx->nb_col, ax);
-  ac::launch_reduce_lse(ctx->nb_col, P, ctx->lpart.p, ctx->lse_cv.p, ax);
+  ac::launch_reduce_lse(ctx->nb_col, P, ctx->lpart.p, ctx->lse_cv.p, ax, ctx->pstat.p);
   if (ctx->n_iso > 0)
     ac::launch_iso_cols(ctx->n_iso, P, ctx->CV.p + ctx->n_act * P, (int)ctx->n_act, ctx->lpart.p, ctx->apv.p,
                         ctx->api.p, std::min(ctx->nb_col, 256), ctx->iso.p, ax);
-  HIPCHK(ctx, hipMemcpyAsync(ctx->pstat.p, ctx->lse_cv.p, sizeof(Lse2) * P, hipMemcpyDeviceToDevice, ax));
   if (Q > 0) {
     // Only the constant rows: the per-source statistics write every row of a vertex with out-edges, and the prep
     // walk every row of a vertex with in-edges (internal order: both, in-edges only, out-edges only, isolated).
     const int64_t in_lo = ctx->n_both, in_hi = ctx->n_both + ctx->n_inonly, iso = ctx->n_act;
-    for (const auto& r : {std::make_pair(in_lo, in_hi), std::make_pair(iso, n)}) {
-      ac::launch_fill(ctx->minCEo.p + r.first * Qs, (r.second - r.first) * Qs, INFINITY, ax);
-      ac::launch_fill(ctx->lsO.p + r.first * Qs, (r.second - r.first) * Qs, 0.f, ax);
-      ac::launch_fill(ctx->VFm.p + r.first * Qs, (r.second - r.first) * Qs, -INFINITY, ax);
-    }
-    ac::launch_fill(ctx->FMaxN.p + in_hi * Qs, (n - in_hi) * Qs, -INFINITY, ax);
+    ac::launch_fill_const(n, Qs, in_lo, in_hi, iso, in_hi, ctx->minCEo.p, ctx->lsO.p, ctx->VFm.p, ctx->FMaxN.p, ax);
   }
   HIPCHK(ctx, hipEventRecord(ctx->xev[1], ax));
   if (Q > 0) {
     ac::launch_cdist(ctx->bs->brows, ctx->bs->beid.p, ctx->efeat.p, (int)ctx->dE, ctx->pf_e.p, Q, round8(Q), Qs, ctx->CE.p,
-                     Qs, ctx->has_we ? ctx->we.p : nullptr, cds_e, st);
+                     Qs, ctx->has_we ? ctx->we.p : nullptr, ctx->use_mfma_cdist, st);
     // The bundle minima (a stream over CE) on the second stream, beside the per-source statistics (a gather over
     // CE, bound by its own instruction chains); the first stream waits for them (xev[3]) before the prep walk.
     HIPCHK(ctx, hipEventRecord(ctx->xev[2], st));
@@ -1041,18 +1029,18 @@ static int enqueue_prep(ac_ctx* ctx) {
     ac::launch_bundle_min(ctx->bs->nbundles, ctx->bs->bundles.p, ctx->CE.p, Q, Qs, ctx->bmin.p,
                           ctx->pack_costs ? ctx->bpack.p : nullptr, ax);
     HIPCHK(ctx, hipEventRecord(ctx->xev[3], ax));
-    HIPCHK(ctx, hipStreamWaitEvent(st, ctx->xev[1], 0));
     if (ctx->nruns_out > 0) {
       ac::launch_walk_src(ctx->nruns_out, ctx->runs_out.p, ctx->bs->csr_kb.p, ctx->CE.p, Q, Qs, ctx->minCEo.p,
-                          ctx->lsO.p, ctx->VFm.p, ctx->carry_out.p, ctx->lpart.p, ctx->nb_src, st);
+                          ctx->lsO.p, ctx->VFm.p, ctx->carry_out.p, ctx->spart.p, ctx->nb_src, st);
       ac::launch_walk_src_fixup(ctx->nsplit_out, ctx->splits_out.p, ctx->carry_out.p, Q, Qs, ctx->minCEo.p,
                                 ctx->lsO.p, ctx->VFm.p, st);
-      ac::launch_reduce_lse(ctx->nb_src, Q, ctx->lpart.p, ctx->lse_ce.p, st);
+      ac::launch_reduce_lse(ctx->nb_src, Q, ctx->spart.p, ctx->lse_ce.p, st);
     } else {
       std::vector<Lse2> empty(Q, Lse2{-std::numeric_limits<double>::infinity(), 0.0});
       HIPCHK(ctx, hipMemcpyAsync(ctx->lse_ce.p, empty.data(), sizeof(Lse2) * Q, hipMemcpyHostToDevice, st));
       HIPCHK(ctx, hipStreamSynchronize(st));
     }
+    HIPCHK(ctx, hipStreamWaitEvent(st, ctx->xev[1], 0));
     const bool tape = ctx->tape_K > 0;
     ac::launch_prep_scalars(P, Q, ctx->d_ps.p, ctx->d_pd.p, ctx->lse_cv.p, ctx->lse_ce.p, qs_prep, st,
                             tape ? ac::SplitRows() : split_rows(ctx));

@@ -116,12 +116,11 @@ struct VertexArgs {
 enum VertexMode { kModeA = 0, kModeC = 1, kModeOut = 2, kModeMU = 3 };  // kModeMU: MU in FP64 into mu_out
 
 // Launchers (ac_kernels.hip).  All asynchronous on `st`.
-// scratch (may be null: no matrix-core path): cdist_scratch_doubles(Kstore, dim) doubles.
+// mfma: the matrix-core path, where the widths allow it.
 void launch_cdist(int64_t nrows, const int* idx, const float* feats, int dim, const double* pat, int K, int Kp,
-                  int Kstore, float* out, int out_stride, const double* w, double* scratch, hipStream_t st);
-size_t cdist_scratch_doubles(int Kstore, int dim);
+                  int Kstore, float* out, int out_stride, const double* w, bool mfma, hipStream_t st);
 void launch_col_lse_neg(int64_t n, int P, const float* X, Lse* part, int nblocks, hipStream_t st);
-void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStream_t st);
+void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStream_t st, Lse2* out2 = nullptr);
 // cnull (nullptr: off): per pattern edge, the PNNL Cnull term subtracted from both fills of the new state.
 void launch_reduce_q(int nparts, int Q, const QPart* part, QStat* out, hipStream_t st, const double* cnull = nullptr,
                      const SplitRows& rows = SplitRows());
@@ -134,7 +133,8 @@ void launch_bundle_min(int64_t nbundles, const Bundle* bundles, const float* CE,
                        unsigned* bpack, hipStream_t st);
 void launch_prep_scalars(int P, int Q, const int* ps, const int* pd, const Lse2* cv, const Lse2* ce, QStat* qs,
                          hipStream_t st, const SplitRows& rows = SplitRows());
-void launch_fill(float* p, int64_t count, float value, hipStream_t st);
+void launch_fill_const(int64_t n, int w, int64_t a0, int64_t a1, int64_t b0, int64_t f0, float* minC, float* ls,
+                       float* vfm, float* fmaxn, hipStream_t st);
 void launch_fill_slots(float* A, float* B, int64_t nslots, int64_t stride, int64_t a0, int64_t al, int64_t b0,
                        int64_t bl, int64_t c0, int64_t cl, hipStream_t st);
 void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float* CE, int Q, int Qs, float* minCEo,

@@ -152,7 +152,7 @@ __device__ __forceinline__ int mfma_col(int m) { return 4 * (m & 3) + (m >> 2); 
 
 // LDS position of pattern operand e = c * 4 D4 + d (pattern column c = 16 pt + mfma_col(m), feature d = D4 kk + s2):
 // the layout [pt][s2][kk][m], so that product step s2 of tile pt reads 64 consecutive doubles across the wave (lane
-// 16 kk + m), one conflict-free LDS access.  In the layout of patm itself the 64 lanes' operands lie 128 or 512
+// 16 kk + m), one conflict-free LDS access.  In the natural [column][feature] layout the 64 lanes' operands lie 128 or 512
 // bytes apart, all in one bank pair, and each access is serialised.
 __device__ __forceinline__ int lds_operand(int e, int D4) {
   const int c = e / (4 * D4), d = e - c * (4 * D4);
@@ -173,21 +173,42 @@ __device__ __forceinline__ float sqrt_rn(float x) { return sqrt_rn_fix(x, __buil
 template <int D4, bool kIdx, bool kW, bool kVec>
 __global__ __launch_bounds__(256, D4 <= 16 ? 3 : 1) void k_cdist_mfma(int64_t nrows, const int* __restrict__ idx,
                                                     const float* __restrict__ feats, int dim,
-                                                    const double* __restrict__ patm, const double* __restrict__ pp,
                                                     const double* __restrict__ w, const double* __restrict__ pat,
                                                     int K, int Kstore, float* __restrict__ out, int out_stride) {
-  // LDS: npt * 16 * 4 D4 pattern operands (the block's copy of patm, laid out by lds_operand), [4 D4] weights,
-  // [npt * 16] pattern norms.
+  // LDS: npt * 16 * 4 D4 pattern operands -2 w_d p_c[d] (zero past dim and past K, laid out by lds_operand; the factor is
+  // exact), [4 D4] weights, [npt * 16] pattern norms sum_d w_d p_c[d]^2.  Every block forms them from the pattern's
+  // features: a kernel of their own took 5-25 us before each distance launch.
   extern __shared__ double bsh[];
   const int lane = threadIdx.x & 63, i = lane & 15, kk = lane >> 4;
   const int64_t nw = (int64_t)gridDim.x * 4, step = nw * 16;
   const int npt = (Kstore + 15) / 16;
   double* wsh = bsh + npt * 16 * 4 * D4;
   double* psh = wsh + 4 * D4;
-  for (int e = threadIdx.x; e < npt * 16 * 4 * D4; e += 256) bsh[lds_operand(e, D4)] = patm[e];
+  const int K8 = (K + 7) / 8 * 8;  // columns of pat
+  if (dim < 4 * D4 || K8 < npt * 16) {
+    for (int e = threadIdx.x; e < npt * 16 * 4 * D4; e += 256) bsh[e] = 0.0;
+    __syncthreads();
+  }
+  for (int e = threadIdx.x; e < K8 * dim; e += 256) {  // in the order of pat
+    const int cd = e >> 3, cg = cd / dim, d = cd - cg * dim, c = 8 * cg + (e & 7);
+    const double pv = pat[e];
+    bsh[lds_operand(c * 4 * D4 + d, D4)] = -2.0 * (kW ? w[d] * pv : pv);
+  }
   if (kW)
     for (int d = threadIdx.x; d < 4 * D4; d += 256) wsh[d] = d < dim ? w[d] : 0.0;
-  for (int c = threadIdx.x; c < npt * 16; c += 256) psh[c] = pp[c];
+  // Norms: a wave per 16 columns, four lanes to a column.
+  for (int pt = threadIdx.x >> 6; pt < npt; pt += 4) {
+    const int c = 16 * pt + i;
+    double s = 0.0;
+    if (c < K)
+      for (int d = kk; d < dim; d += 4) {
+        const double pv = pat[((int64_t)(c >> 3) * dim + d) * 8 + (c & 7)];
+        s = fma(kW ? w[d] * pv : pv, pv, s);
+      }
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (kk == 0) psh[c] = s;
+  }
   __syncthreads();
   // Without kVec the features past dim are zeroed at conversion (lim of this lane's chunk exist).  Rows that do not
   // exist are not zeroed: their loads read row 0 and their outputs are +inf regardless.
@@ -341,38 +362,12 @@ __global__ __launch_bounds__(256, D4 <= 16 ? 3 : 1) void k_cdist_mfma(int64_t nr
   }
 }
 
-// MFMA operands of the patterns: patm[c][4 D4] = -2 w_d p_c[d] (zero past dim or past K), pp[c] = sum_d w_d p_c[d]^2.
-// The factor -2 is exact.
-__global__ void k_build_patm(int K, int Kp16, int dim, int D4, const double* __restrict__ pat,
-                             const double* __restrict__ w, double* __restrict__ patm, double* __restrict__ pp) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= Kp16) return;
-  double s2 = 0.0;
-  for (int d = 0; d < 4 * D4; ++d) {
-    double v = 0.0;
-    if (c < K && d < dim) {
-      const double pv = pat[((int64_t)(c / 8) * dim + d) * 8 + c % 8];
-      const double wd = w ? w[d] : 1.0;
-      v = wd * pv;
-      s2 += v * pv;
-    }
-    patm[(int64_t)c * (4 * D4) + d] = -2.0 * v;
-  }
-  pp[c] = s2;
-}
-
 int cdist_mfma_d4(int dim) {
   if (dim <= 16) return 4;
   if (dim <= 32) return 8;
   if (dim <= 64) return 16;
   if (dim <= 128) return 32;
   return 0;
-}
-
-size_t cdist_scratch_doubles(int K, int dim) {
-  const int D4 = cdist_mfma_d4(dim);
-  const int Kp16 = (K + 15) / 16 * 16;
-  return D4 ? (size_t)Kp16 * (4 * D4 + 1) : 0;
 }
 
 // Fallback for feature widths too large to stage: one thread per output element, rows read from global memory.
@@ -396,31 +391,31 @@ __global__ void k_cdist_direct(int64_t nrows, const int* __restrict__ idx, const
 }
 
 void launch_cdist(int64_t nrows, const int* idx, const float* feats, int dim, const double* pat, int K, int Kp,
-                  int Kstore, float* out, int out_stride, const double* w, double* scratch, hipStream_t st) {
+                  int Kstore, float* out, int out_stride, const double* w, bool mfma, hipStream_t st) {
   if (nrows == 0 || Kstore == 0) return;
   const int D4 = cdist_mfma_d4(dim);
   // The pattern operands, weights and norms are staged in LDS: up to 64 KB.
-  if (scratch && D4 && dim > 0 &&
+  if (mfma && D4 && dim > 0 &&
       ((size_t)((Kstore + 15) / 16 * 16 + 1) * 4 * D4 + (Kstore + 15) / 16 * 16) * sizeof(double) <= 65536) {
     const int Kp16 = (Kstore + 15) / 16 * 16;
-    double* patm = scratch;
-    double* pp = scratch + (size_t)Kp16 * 4 * D4;
-    hipLaunchKernelGGL(k_build_patm, dim3((Kp16 + 63) / 64), dim3(64), 0, st, K, Kp16, dim, D4, pat, w, patm, pp);
-    const int blocks = (int)std::min<int64_t>((nrows + 63) / 64, 8192);
+    // Three blocks a CU, resident at once, so that the operands are formed once per CU slot (the prep of R-MAT 20 with 24
+    // columns of 64 features, and of R-MAT 16 slabs with 128 columns: 3.62 ms and 819 us at 8192 blocks, 3.75 / 767 at
+    // 3072, 3.59 / 761 at 1024, 3.48 / 786 at 768).
+    const int blocks = (int)std::min<int64_t>((nrows + 63) / 64, 768);
     const size_t lds = ((size_t)(Kp16 + 1) * 4 * D4 + Kp16) * sizeof(double);  // operands, weights, norms
 #define AC_CD_MFMA_V(N, V)                                                                                        \
   if (idx && w)                                                                                                   \
     hipLaunchKernelGGL((k_cdist_mfma<N, true, true, V>), dim3(blocks), dim3(256), lds, st, nrows, idx, feats, dim, \
-                       patm, pp, w, pat, K, Kstore, out, out_stride);                                             \
+                       w, pat, K, Kstore, out, out_stride);                                             \
   else if (idx)                                                                                                   \
     hipLaunchKernelGGL((k_cdist_mfma<N, true, false, V>), dim3(blocks), dim3(256), lds, st, nrows, idx, feats,     \
-                       dim, patm, pp, w, pat, K, Kstore, out, out_stride);                                        \
+                       dim, w, pat, K, Kstore, out, out_stride);                                        \
   else if (w)                                                                                                     \
     hipLaunchKernelGGL((k_cdist_mfma<N, false, true, V>), dim3(blocks), dim3(256), lds, st, nrows, idx, feats,     \
-                       dim, patm, pp, w, pat, K, Kstore, out, out_stride);                                        \
+                       dim, w, pat, K, Kstore, out, out_stride);                                        \
   else                                                                                                            \
     hipLaunchKernelGGL((k_cdist_mfma<N, false, false, V>), dim3(blocks), dim3(256), lds, st, nrows, idx, feats,    \
-                       dim, patm, pp, w, pat, K, Kstore, out, out_stride);
+                       dim, w, pat, K, Kstore, out, out_stride);
 #define AC_CD_MFMA(N)                \
   case N:                            \
     if (dim == 4 * N) {              \
@@ -510,7 +505,8 @@ constexpr int kRedLse = 8, kRedQ = 5;
 
 // Reduce per-block partials [ncol][nparts] column by column in a fixed order (deterministic).  (A column's partials lie
 // together: by block, [nparts][ncol], every partial of a column was a line of its own.)
-__global__ __launch_bounds__(256) void k_reduce_lse(int nparts, const Lse* __restrict__ part, Lse2* __restrict__ out) {
+__global__ __launch_bounds__(256) void k_reduce_lse(int nparts, const Lse* __restrict__ part, Lse2* __restrict__ out,
+                                                    Lse2* __restrict__ out2) {
   __shared__ double red[8];
   const int c = blockIdx.x, t = threadIdx.x;
   Lse v[kRedLse];
@@ -543,12 +539,15 @@ __global__ __launch_bounds__(256) void k_reduce_lse(int nparts, const Lse* __res
   for (int u = 0; u < kRedLse; ++u)
     if (u * 256 < nparts) lse_sum_step(sum, seen, lse_rescaled(v[u], M));
   sum = block_lse_sum<256>(sum, seen, red);
-  if (t == 0) out[c] = Lse2{M, log1p(sum)};
+  if (t == 0) {
+    out[c] = Lse2{M, log1p(sum)};
+    if (out2) out2[c] = Lse2{M, log1p(sum)};
+  }
 }
 
-void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStream_t st) {
+void launch_reduce_lse(int nparts, int ncol, const Lse* part, Lse2* out, hipStream_t st, Lse2* out2) {
   if (ncol == 0) return;
-  hipLaunchKernelGGL(k_reduce_lse, dim3(ncol), dim3(256), 0, st, nparts, part, out);
+  hipLaunchKernelGGL(k_reduce_lse, dim3(ncol), dim3(256), 0, st, nparts, part, out, out2);
 }
 
 // FMaxN rows of the split vertices to -inf, over nblocks blocks: the walk's pieces of a split vertex then raise its row
@@ -797,15 +796,29 @@ void launch_prep_scalars(int P, int Q, const int* ps, const int* pd, const Lse2*
                      qs, rows);
 }
 
-__global__ void k_fill(float* __restrict__ p, int64_t count, float value) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = value;
+// The constant rows of the per-vertex arrays [n][w], in one launch: rows [a0, a1) and [b0, n) of minC (+inf), ls (0) and
+// vfm (-inf), rows [f0, n) of fmaxn (-inf).
+__global__ void k_fill_const(int64_t n, int w, int64_t a0, int64_t a1, int64_t b0, int64_t f0, float* __restrict__ minC,
+                             float* __restrict__ ls, float* __restrict__ vfm, float* __restrict__ fmaxn) {
+  const int64_t la = (a1 - a0) * w, lo = la + (n - b0) * w, total = lo + (n - f0) * w;
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    if (i < lo) {
+      const int64_t o = i < la ? a0 * w + i : b0 * w + (i - la);
+      minC[o] = INFINITY;
+      ls[o] = 0.f;
+      vfm[o] = -INFINITY;
+    } else {
+      fmaxn[f0 * w + (i - lo)] = -INFINITY;
+    }
+  }
 }
 
-void launch_fill(float* p, int64_t count, float value, hipStream_t st) {
-  if (count == 0) return;
-  int blocks = (int)std::min<int64_t>((count + 255) / 256, 1 << 16);
-  hipLaunchKernelGGL(k_fill, dim3(blocks), dim3(256), 0, st, p, count, value);
+void launch_fill_const(int64_t n, int w, int64_t a0, int64_t a1, int64_t b0, int64_t f0, float* minC, float* ls,
+                       float* vfm, float* fmaxn, hipStream_t st) {
+  const int64_t total = ((a1 - a0) + (n - b0) + (n - f0)) * w;
+  if (total == 0) return;
+  const int blocks = (int)std::min<int64_t>((total + 1023) / 1024, 1 << 14);
+  hipLaunchKernelGGL(k_fill_const, dim3(blocks), dim3(256), 0, st, n, w, a0, a1, b0, f0, minC, ls, vfm, fmaxn);
 }
 
 // -inf into three ranges of each of nslots slots (stride `stride` floats): [a0, a0 + al) of A, and [b0, b0 + bl) and
@@ -983,8 +996,9 @@ __global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split*
 #pragma unroll
   for (int u = 0; u < 4; ++u) red[wave][lane][u] = M[u];
   __syncthreads();
+  const int used = min(G, S.count);  // groups that have a piece
   if (active)
-    for (int gg = 0; gg < G; ++gg)
+    for (int gg = 0; gg < used; ++gg)
 #pragma unroll
       for (int u = 0; u < 4; ++u) M[u] = fmax(M[u], red[wave][gg * L4 + j][u]);
   if (active)
@@ -1004,7 +1018,7 @@ __global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split*
     for (int u = 0; u < 4; ++u) {
       double t = 0.0;
       bool any = false;
-      for (int gg = 0; gg < G; ++gg) lse_sum_step(t, any, red[wave][gg * L4 + j][u]);
+      for (int gg = 0; gg < used; ++gg) lse_sum_step(t, any, red[wave][gg * L4 + j][u]);
       const int q = 4 * j + u;
       const int64_t o = (int64_t)S.v * Qs + q;
       minCEo[o] = q < Q ? (float)(-M[u]) : 0.f;
