@@ -76,17 +76,16 @@ __global__ __launch_bounds__(256) void k_colsum(int64_t n, int C, const float* _
   if (t < C) {
     double a = 0.0;
     for (int r = 0; r < RC; ++r) a += red[r * C + t];
-    part[(int64_t)blockIdx.x * C + t] = a;
+    part[(int64_t)t * gridDim.x + blockIdx.x] = a;
   }
 }
 
-// out[c] = sum over parts of part[b][c]: a block takes CB = min(C, 32) columns and 256 / CB lanes per column, lane l
-// summing parts l, l + L, ... in order, the lanes then summed in order (deterministic).
-__global__ __launch_bounds__(256) void k_sum_parts(int nparts, int C, const double* __restrict__ part,
+// out[c] = sum over parts of part[b * sb + c * sc].
+__global__ __launch_bounds__(256) void k_sum_parts(int nparts, int64_t sb, int64_t sc, const double* __restrict__ part,
                                                    double* __restrict__ out) {
   // One block per column: lane l sums partials l, l + 256, ... in order (eight loads in flight before the adds), then
   // a fixed tree over the lanes.  The order is the same on every call.
-  __shared__ double red[256];
+  __shared__ double red[4];
   const int t = threadIdx.x, c = blockIdx.x;
   double a = 0.0;
   for (int b0 = t; b0 < nparts; b0 += 8 * 256) {
@@ -94,19 +93,17 @@ __global__ __launch_bounds__(256) void k_sum_parts(int nparts, int C, const doub
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int b = b0 + u * 256;
-      v[u] = part[(int64_t)(b < nparts ? b : nparts - 1) * C + c];
+      v[u] = part[(b < nparts ? b : nparts - 1) * sb + c * sc];
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (b0 + u * 256 < nparts) a += v[u];
   }
-  red[t] = a;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+  if ((t & 63) == 0) red[t >> 6] = a;
   __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (t < w) red[t] += red[t + w];
-    __syncthreads();
-  }
-  if (t == 0) out[c] = red[0];
+  if (t == 0) out[c] = ((red[0] + red[1]) + red[2]) + red[3];
 }
 
 // Log-softmax Jacobian of MU = LSM_v(Z): gMU <- gZ = gMU - exp(MU) colsum(gMU); gCV -= gZ.
@@ -123,7 +120,7 @@ __global__ __launch_bounds__(256) void k_bwd_out(int64_t total, int P, const dou
 // Max-subgradient routing of FMax / RMax of state S (thread per (v, q), q fixed per thread).  gF = -gVF + gZ[pd]
 // (with_gz), gR = -gVR + gZ[ps], where gVF / gVR are the next state's (the step processed before this one; zero at the
 // first): the gradients of this state's FMax / RMax through the next step's inputs.  The edge term takes the
-// gradient where it is strictly above the fill.  Per-block partials part[b][4][Q]: sum gE_F, sum gE_R, fill gradient
+// gradient where it is strictly above the fill.  Per-block partials part[4][Q][blocks]: sum gE_F, sum gE_R, fill gradient
 // of fillF, of fillR.  gmax (nullable) receives the largest |gE_F| (as float bits, an atomic maximum: exact and
 // order-free), which sets the fixed-point scale of the FMax edge terms' source sums.  gERsum (nullable) accumulates
 // gE_R per (v, q) over the steps: the RMax rows AO are the same in every step, so their edge terms are applied once.
@@ -172,7 +169,7 @@ __global__ __launch_bounds__(256) void k_bwd_route(BwdGraph G, BwdState S, const
     for (int k = 0; k < 4; ++k) {
       double a = 0.0;
       for (int r = 0; r < RQ; ++r) a += red[r * Q + t][k];
-      part[((int64_t)blockIdx.x * 4 + k) * Q + t] = a;
+      part[((int64_t)k * Q + t) * gridDim.x + blockIdx.x] = a;
     }
 }
 
@@ -257,7 +254,7 @@ __global__ __launch_bounds__(256) void k_bwd_in(BwdGraph G, BwdState S, const do
 //   1. gVR[v][q] += gVRfix[v][q] 2^-k, the fixed-point sums of the step's FMax edge terms (where nonzero; the
 //      accumulator is cleared for the next step), staged with gVF in LDS;
 //   2. gMU[v][p] = sum over the incidences of p (ascending q) of gVF (q ends at p) or gVR (q starts at p);
-//   3. per-block partial column sums of gMU in FP64, vertices in order: part[b][p].
+//   3. per-block partial column sums of gMU in FP64, vertices in order: part[p][b].
 // The input state's FMax / RMax gradients are -gVF / -gVR, which k_bwd_route of the next step back reads directly.
 __global__ __launch_bounds__(256) void k_bwd_vtx(BwdGraph G, float* __restrict__ gVR, const float* __restrict__ gVF,
                                                  unsigned long long* __restrict__ gVRfix,
@@ -305,7 +302,7 @@ __global__ __launch_bounds__(256) void k_bwd_vtx(BwdGraph G, float* __restrict__
     if (t < P)
       for (int vl = 0; vl < nv; ++vl) col += (double)tM[vl * P + t];
   }
-  if (t < P) part[(int64_t)blockIdx.x * P + t] = col;
+  if (t < P) part[(int64_t)t * gridDim.x + blockIdx.x] = col;
 }
 
 // Fill subgradients of the prep state go to the argmax of MU0 = LSM(-CV) of the source / destination pattern vertex:
@@ -317,19 +314,6 @@ __global__ void k_bwd_prep_fill(BwdGraph G, const double* __restrict__ red4, con
     const int ps = G.ps[q], pd = G.pd[q];
     gMU[(int64_t)am0[ps] * G.P + ps] += (float)red4[2 * G.Q + q];
     gMU[(int64_t)am0[pd] * G.P + pd] += (float)red4[3 * G.Q + q];
-  }
-}
-
-// Rows of the minimum cost among out-edges: AO[src][q] = lowest CE row whose cost equals minCEo[src][q] (CSR order
-// pairs {row, src}); AO starts at INT_MAX.
-__global__ void k_argmin_out(int64_t m, int Q, int Qs, const int2* __restrict__ ks, const float* __restrict__ CE,
-                             const float* __restrict__ minCEo, int* __restrict__ AO) {
-  const int64_t total = m * Q;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t k = i / Q;
-    const int q = (int)(i - k * Q);
-    const int2 e = ks[k];
-    if (CE[(int64_t)e.x * Qs + q] == minCEo[(int64_t)e.y * Qs + q]) atomicMin(&AO[(int64_t)e.y * Qs + q], e.x);
   }
 }
 
@@ -368,13 +352,15 @@ __global__ __launch_bounds__(256) void k_col_argmin(int64_t n, int P, const floa
   }
 }
 
-__global__ void k_col_argmin_final(int nparts, int P, const float* __restrict__ pv, const int* __restrict__ pi,
-                                   int* __restrict__ am) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= P) return;
+// One block per column: the least of its blocks' minima, the lowest row on ties.
+__global__ __launch_bounds__(256) void k_col_argmin_final(int nparts, int P, const float* __restrict__ pv,
+                                                          const int* __restrict__ pi, int* __restrict__ am) {
+  __shared__ float rv[256];
+  __shared__ int ri[256];
+  const int p = blockIdx.x, t = threadIdx.x;
   float best = INFINITY;
-  int bi = 0;
-  for (int b = 0; b < nparts; ++b) {
+  int bi = INT_MAX;
+  for (int b = t; b < nparts; b += 256) {
     const float x = pv[(int64_t)b * P + p];
     const int xi = pi[(int64_t)b * P + p];
     if (x < best || (x == best && xi < bi)) {
@@ -382,27 +368,48 @@ __global__ void k_col_argmin_final(int nparts, int P, const float* __restrict__ 
       bi = xi;
     }
   }
-  am[p] = bi;
+  rv[t] = best;
+  ri[t] = bi;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (t < w && (rv[t + w] < rv[t] || (rv[t + w] == rv[t] && ri[t + w] < ri[t]))) {
+      rv[t] = rv[t + w];
+      ri[t] = ri[t + w];
+    }
+    __syncthreads();
+  }
+  if (t == 0) am[p] = ri[0] == INT_MAX ? 0 : ri[0];
 }
 
 // Edge-cost gradients divided by twice the cost: G[row][q] = (gCE + (cD[src] + cq) exp(-CE)) / (2 CE), 0 for
 // padding rows and zero costs (d sqrt(s) / ds is unbounded at 0; such a pair contributes nothing here).
-__global__ void k_bwd_edge_coef(int64_t nrows, int Q, int Qs, const int* __restrict__ beid, const int* __restrict__ bsrc,
-                                const float* __restrict__ CE, const double* __restrict__ cD,
-                                const double* __restrict__ cq, float* __restrict__ G) {
-  const int64_t total = nrows * Qs;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t row = i / Qs;
-    const int q = (int)(i - row * Qs);
-    float out = 0.f;
-    if (q < Q && beid[row] >= 0) {
-      const double ce = (double)CE[i];
-      if (ce > 0.0 && ce != kInf) {
-        const double g = (double)G[i] + (cD[(int64_t)(bsrc[row] & ~kNewVertex) * Qs + q] + cq[q]) * exp(-ce);
-        out = (float)(g / (2.0 * ce));
+// A group of Qs/4 lanes per row, four pattern edges to a lane: 16- and 32-byte accesses, no index division per element.
+__global__ __launch_bounds__(256) void k_bwd_edge_coef(int64_t nrows, int Q, int Qs, const int* __restrict__ beid,
+                                                       const int* __restrict__ bsrc, const float* __restrict__ CE,
+                                                       const double* __restrict__ cD, const double* __restrict__ cq,
+                                                       float* __restrict__ G) {
+  const int L4 = Qs / 4, R = 256 / L4, r = threadIdx.x / L4, j = threadIdx.x - r * L4;
+  if (r >= R) return;
+  double c[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) c[u] = 4 * j + u < Q ? cq[4 * j + u] : 0.0;
+  for (int64_t row = (int64_t)blockIdx.x * R + r; row < nrows; row += (int64_t)gridDim.x * R) {
+    const int64_t o = row * L4 + j;
+    f4v out = {0.f, 0.f, 0.f, 0.f};
+    if (beid[row] >= 0) {
+      const f4v ce4 = reinterpret_cast<const f4v*>(CE)[o], g4 = reinterpret_cast<const f4v*>(G)[o];
+      const double4 d4 = reinterpret_cast<const double4*>(cD)[(int64_t)(bsrc[row] & ~kNewVertex) * L4 + j];
+      const double dd[4] = {d4.x, d4.y, d4.z, d4.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const double ce = (double)ce4[u];
+        if (4 * j + u < Q && ce > 0.0 && ce != kInf) {
+          const double g = (double)g4[u] + (dd[u] + c[u]) * exp(-ce);
+          out[u] = (float)(g / (2.0 * ce));
+        }
       }
     }
-    G[i] = out;
+    reinterpret_cast<f4v*>(G)[o] = out;
   }
 }
 
@@ -558,32 +565,22 @@ __global__ __launch_bounds__(256) void k_outer_mfma(int64_t nrows, const int* __
     }
 }
 
-__global__ void k_fill_int(int* __restrict__ p, int64_t count, int value) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-    p[i] = value;
-}
-
 // ---------------------------------------------------------------------------------------------------------------
 // Launchers.
 
 static int grid_for(int64_t total) { return (int)std::max<int64_t>(1, std::min<int64_t>((total + 255) / 256, 1 << 15)); }
 
-void launch_fill_int(int* p, int64_t count, int value, hipStream_t st) {
-  if (count == 0) return;
-  hipLaunchKernelGGL(k_fill_int, dim3(grid_for(count)), dim3(256), 0, st, p, count, value);
-}
-
-static int sum_blocks(int C) { return std::max(1, C); }
-
-void launch_sum_parts(int nparts, int C, const double* part, double* out, hipStream_t st) {
+// by_column: partials [C][nparts] (a column's together: whole lines to a block), else [nparts][C].
+void launch_sum_parts(int nparts, int C, const double* part, double* out, bool by_column, hipStream_t st) {
   if (C == 0) return;
-  hipLaunchKernelGGL(k_sum_parts, dim3(sum_blocks(C)), dim3(256), 0, st, nparts, C, part, out);
+  hipLaunchKernelGGL(k_sum_parts, dim3(C), dim3(256), 0, st, nparts, by_column ? (int64_t)1 : (int64_t)C,
+                     by_column ? (int64_t)nparts : (int64_t)1, part, out);
 }
 
 void launch_colsum(int64_t n, int C, const float* X, double* part, int nparts, double* out, hipStream_t st) {
   if (C == 0) return;
   hipLaunchKernelGGL(k_colsum, dim3(nparts), dim3(256), 0, st, n, C, X, part);
-  hipLaunchKernelGGL(k_sum_parts, dim3(sum_blocks(C)), dim3(256), 0, st, nparts, C, part, out);
+  launch_sum_parts(nparts, C, part, out, true, st);
 }
 
 void launch_bwd_out(const BwdGraph& G, const double* MU, const double* colsum, float* gMU, float* gCV, hipStream_t st) {
@@ -596,7 +593,7 @@ void launch_bwd_route(const BwdGraph& G, const BwdState& S, const float* gZ, int
   if (G.Q == 0) return;
   hipLaunchKernelGGL(k_bwd_route, dim3(nparts), dim3(256), 0, st, G, S, gZ, with_gz, gVF, gVR, gEF, gER, gmax, gERsum,
                      part);
-  hipLaunchKernelGGL(k_sum_parts, dim3(sum_blocks(4 * G.Q)), dim3(256), 0, st, nparts, 4 * G.Q, part, red4);
+  launch_sum_parts(nparts, 4 * G.Q, part, red4, true, st);
 }
 
 void launch_bwd_in(const BwdGraph& G, const BwdState& S, const double* MU, const QStat* qs1, const double* red4,
@@ -656,21 +653,15 @@ void launch_bwd_prep_fill(const BwdGraph& G, const double* red4, const int* am0,
   hipLaunchKernelGGL(k_bwd_prep_fill, dim3(1), dim3(64), 0, st, G, red4, am0, gMU);
 }
 
-void launch_argmin_out(int64_t m, int Q, int Qs, const int2* ks, const float* CE, const float* minCEo, int* AO,
-                       hipStream_t st) {
-  if (m == 0 || Q == 0) return;
-  hipLaunchKernelGGL(k_argmin_out, dim3(grid_for(m * Q)), dim3(256), 0, st, m, Q, Qs, ks, CE, minCEo, AO);
-}
-
 void launch_col_argmin(int64_t n, int P, const float* CV, float* pv, int* pi, int nparts, int* am, hipStream_t st) {
   hipLaunchKernelGGL(k_col_argmin, dim3(nparts), dim3(256), 0, st, n, P, CV, pv, pi);
-  hipLaunchKernelGGL(k_col_argmin_final, dim3((P + 255) / 256), dim3(256), 0, st, nparts, P, pv, pi, am);
+  hipLaunchKernelGGL(k_col_argmin_final, dim3(P), dim3(256), 0, st, nparts, P, pv, pi, am);
 }
 
 void launch_bwd_edge_coef(int64_t nrows, int Q, int Qs, const int* beid, const int* bsrc, const float* CE,
                           const double* cD, const double* cq, float* G, hipStream_t st) {
   if (nrows == 0) return;
-  hipLaunchKernelGGL(k_bwd_edge_coef, dim3(grid_for(nrows * Qs)), dim3(256), 0, st, nrows, Q, Qs, beid, bsrc, CE, cD,
+  hipLaunchKernelGGL(k_bwd_edge_coef, dim3(grid_for(nrows * (Qs / 4))), dim3(256), 0, st, nrows, Q, Qs, beid, bsrc, CE, cD,
                      cq, G);
 }
 

@@ -32,8 +32,7 @@ struct BwdState {
   int first;           // the prep state: MU = LSM(-CV), no FMax / RMax terms
 };
 
-void launch_fill_int(int* p, int64_t count, int value, hipStream_t st);
-void launch_sum_parts(int nparts, int C, const double* part, double* out, hipStream_t st);
+void launch_sum_parts(int nparts, int C, const double* part, double* out, bool by_column, hipStream_t st);
 void launch_colsum(int64_t n, int C, const float* X, double* part, int nparts, double* out, hipStream_t st);
 void launch_bwd_out(const BwdGraph& G, const double* MU, const double* colsum, float* gMU, float* gCV, hipStream_t st);
 // The FMax edge terms of one step back: the row FA[v][q] recorded for each (v, q) whose edge term carries gradient
@@ -70,8 +69,6 @@ int bwd_vtx_blocks(const BwdGraph& G);
 void launch_bwd_vtx(const BwdGraph& G, float* gVR, const float* gVF, unsigned long long* gVRfix, const unsigned* gmax,
                     float* gMU, double* part, hipStream_t st);
 void launch_bwd_prep_fill(const BwdGraph& G, const double* red4, const int* am0, float* gMU, hipStream_t st);
-void launch_argmin_out(int64_t m, int Q, int Qs, const int2* ks, const float* CE, const float* minCEo, int* AO,
-                       hipStream_t st);
 void launch_col_argmin(int64_t n, int P, const float* CV, float* pv, int* pi, int nparts, int* am, hipStream_t st);
 void launch_bwd_edge_coef(int64_t nrows, int Q, int Qs, const int* beid, const int* bsrc, const float* CE,
                           const double* cD, const double* cq, float* G, hipStream_t st);

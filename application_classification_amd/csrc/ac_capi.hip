@@ -364,7 +364,7 @@ struct ac_ctx {
   int tape_K = 0;
   bool tape_valid = false;
   int tape_iters = 0;
-  DevBuf<int> FA0, AO, am0, carg_in, tapeFA;
+  DevBuf<int> FA0, AO, am0, carg_in, carg_out, tapeFA;
   DevBuf<float> ckF, ckV, sgF, sgV;
   DevBuf<QStat> ckQ, sgQ;
   DevBuf<Lse2> ckP, sgP;
@@ -962,6 +962,7 @@ static int ensure_tape(ac_ctx* ctx, int n_iter) {
   HIPCHK(ctx, ctx->AO.alloc(nq));
   HIPCHK(ctx, ctx->am0.alloc(P));
   HIPCHK(ctx, ctx->carg_in.alloc((size_t)std::max(1, ctx->nslots_in) * ctx->Qs));
+  HIPCHK(ctx, ctx->carg_out.alloc((size_t)std::max(1, ctx->nslots_out) * ctx->Qs));
   HIPCHK(ctx, ctx->ckF.alloc(nck * nq));
   HIPCHK(ctx, ctx->ckV.alloc(nck * nq));
   HIPCHK(ctx, ctx->ckQ.alloc(nck * Q));
@@ -1029,11 +1030,15 @@ static int enqueue_prep(ac_ctx* ctx) {
     ac::launch_bundle_min(ctx->bs->nbundles, ctx->bs->bundles.p, ctx->CE.p, Q, Qs, ctx->bmin.p,
                           ctx->pack_costs ? ctx->bpack.p : nullptr, ax);
     HIPCHK(ctx, hipEventRecord(ctx->xev[3], ax));
+    const bool tape = ctx->tape_K > 0;
+    // With the tape: the row of the minimum-cost out-edge of every (v, q) too, the RMax argmax of every iteration.
+    int* const AO = tape ? ctx->AO.p : nullptr;
     if (ctx->nruns_out > 0) {
       ac::launch_walk_src(ctx->nruns_out, ctx->runs_out.p, ctx->bs->csr_kb.p, ctx->CE.p, Q, Qs, ctx->minCEo.p,
-                          ctx->lsO.p, ctx->VFm.p, ctx->carry_out.p, ctx->spart.p, ctx->nb_src, st);
+                          ctx->lsO.p, ctx->VFm.p, ctx->carry_out.p, ctx->spart.p, ctx->nb_src, st, AO,
+                          ctx->carg_out.p);
       ac::launch_walk_src_fixup(ctx->nsplit_out, ctx->splits_out.p, ctx->carry_out.p, Q, Qs, ctx->minCEo.p,
-                                ctx->lsO.p, ctx->VFm.p, st);
+                                ctx->lsO.p, ctx->VFm.p, st, ctx->carg_out.p, AO);
       ac::launch_reduce_lse(ctx->nb_src, Q, ctx->spart.p, ctx->lse_ce.p, st);
     } else {
       std::vector<Lse2> empty(Q, Lse2{-std::numeric_limits<double>::infinity(), 0.0});
@@ -1041,7 +1046,6 @@ static int enqueue_prep(ac_ctx* ctx) {
       HIPCHK(ctx, hipStreamSynchronize(st));
     }
     HIPCHK(ctx, hipStreamWaitEvent(st, ctx->xev[1], 0));
-    const bool tape = ctx->tape_K > 0;
     ac::launch_prep_scalars(P, Q, ctx->d_ps.p, ctx->d_pd.p, ctx->lse_cv.p, ctx->lse_ce.p, qs_prep, st,
                             tape ? ac::SplitRows() : split_rows(ctx));
     HIPCHK(ctx, hipStreamWaitEvent(st, ctx->xev[3], 0));
@@ -1057,15 +1061,10 @@ static int enqueue_prep(ac_ctx* ctx) {
     if (tape)
       ac::launch_walk_max_fixup(ctx->nsplit_in, ctx->splits_in.p, ctx->carry_in.p, Q, Qs, qs_prep, ctx->FMaxN.p, st,
                                 ctx->carg_in.p, ctx->FA0.p);
-    if (tape) {
-      // Rows of the minimum-cost out-edge of every (v, q) (the RMax argmax), for the adjoint.
-      ac::launch_fill_int(ctx->AO.p, n * Qs, INT32_MAX, st);
-      ac::launch_argmin_out(ctx->de, Q, Qs, ctx->bs->csr_kb.p, ctx->CE.p, ctx->minCEo.p, ctx->AO.p, st);
-    }
   }
   HIPCHK(ctx, hipStreamWaitEvent(st, ctx->xev[1], 0));  // (again, for Q = 0) everything of the second stream
   if (ctx->tape_K > 0) {
-    ac::launch_col_argmin(n, P, ctx->CV.p, ctx->apv.p, ctx->api.p, std::min(ctx->nb_col, 128), ctx->am0.p, st);
+    ac::launch_col_argmin(n, P, ctx->CV.p, ctx->apv.p, ctx->api.p, ctx->nb_col, ctx->am0.p, st);
     int rc = checkpoint(ctx, 0, qs_prep);
     if (rc != AC_OK) return rc;
   }
@@ -2079,7 +2078,7 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
       if (!have_mu) launch_mu(ctx, S1, st);
       // Column sums of gMU: from the previous step's vertex kernel, or (first step back) of the caller's gradient.
       if (have_mu)
-        ac::launch_sum_parts(ac::bwd_vtx_blocks(G), P, ctx->vpart.p, ctx->colsum.p, st);
+        ac::launch_sum_parts(ac::bwd_vtx_blocks(G), P, ctx->vpart.p, ctx->colsum.p, true, st);
       else
         ac::launch_colsum(n, P, ctx->gMU.p, ctx->bpart.p, nparts, ctx->colsum.p, st);
       ac::launch_bwd_out(G, ctx->MUd.p, ctx->colsum.p, ctx->gMU.p, ctx->gCV.p, st);
@@ -2131,7 +2130,7 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
     HIPCHK(ctx, ctx->opart.alloc((size_t)onp * w));
     HIPCHK(ctx, ctx->osum.alloc(w));
     ac::launch_outer_acc(n, ctx->d_perm.p, ctx->vfeat.p, dV, ctx->gCV.p, P, P, ctx->opart.p, onp, st);
-    ac::launch_sum_parts(onp, (int)w, ctx->opart.p, ctx->osum.p, st);
+    ac::launch_sum_parts(onp, (int)w, ctx->opart.p, ctx->osum.p, false, st);
     std::vector<double> sv(w);
     HIPCHK(ctx, hipMemcpyAsync(sv.data(), ctx->osum.p, w * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));
@@ -2144,7 +2143,7 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
     HIPCHK(ctx, ctx->opart.alloc((size_t)onp * w));
     HIPCHK(ctx, ctx->osum.alloc(w));
     ac::launch_outer_acc(brows, ctx->bs->beid.p, ctx->efeat.p, dE, ctx->gCE.p, Qs, Q, ctx->opart.p, onp, st);
-    ac::launch_sum_parts(onp, (int)w, ctx->opart.p, ctx->osum.p, st);
+    ac::launch_sum_parts(onp, (int)w, ctx->opart.p, ctx->osum.p, false, st);
     std::vector<double> se(w);
     HIPCHK(ctx, hipMemcpyAsync(se.data(), ctx->osum.p, w * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPCHK(ctx, hipStreamSynchronize(st));

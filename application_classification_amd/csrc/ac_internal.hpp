@@ -138,9 +138,10 @@ void launch_fill_const(int64_t n, int w, int64_t a0, int64_t a1, int64_t b0, int
 void launch_fill_slots(float* A, float* B, int64_t nslots, int64_t stride, int64_t a0, int64_t al, int64_t b0,
                        int64_t bl, int64_t c0, int64_t cl, hipStream_t st);
 void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float* CE, int Q, int Qs, float* minCEo,
-                     float* lsO, float* VFm, double* carry, Lse* gpart, int nblocks, hipStream_t st);
+                     float* lsO, float* VFm, double* carry, Lse* gpart, int nblocks, hipStream_t st, int* AO = nullptr,
+                     int* carg = nullptr);
 void launch_walk_src_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, float* minCEo,
-                           float* lsO, float* VFm, hipStream_t st);
+                           float* lsO, float* VFm, hipStream_t st, const int* carg = nullptr, int* AO = nullptr);
 void launch_build_bundles(int64_t nbundles, const Bundle* bundles, const int* brun, const Run* runs, const int2* sd,
                           const int* eid, int G, int* bsrc, int* bdst, int* beid, int* rowmap, hipStream_t st);
 void launch_remap_ks(int64_t m, const int2* ks, const int* rowmap, int2* out, hipStream_t st);

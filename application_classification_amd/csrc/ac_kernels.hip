@@ -860,11 +860,14 @@ int walk_blocks(int64_t nruns, int Qs) {
 // Source-side statistics of the edge costs (CSR walk): for every vertex v with out-edges and every q,
 //   minCEo[v][q] = min_e CE[e][q],  lsO[v][q] = log1p(sum_{other e} exp(minCEo - CE)),  VFm[v][q] = -minCEo
 // (VFm of the prep state: RE0 = -CE up to a per-q constant), and per-block partials of log sum_e exp(-CE[e][q]).
+// kArg: also the row of the least-cost out-edge of every (v, q), the lowest one on ties, into AO (pieces: into carg).
+template <bool kArg>
 __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Run* __restrict__ runs,
                                                          const int2* __restrict__ ks, const float* __restrict__ CE,
                                                          int Q, int Qs, float* __restrict__ minCEo,
                                                          float* __restrict__ lsO, float* __restrict__ VFm,
-                                                         double* __restrict__ carry, Lse* __restrict__ gpart) {
+                                                         double* __restrict__ carry, Lse* __restrict__ gpart,
+                                                         int* __restrict__ AO, int* __restrict__ carg) {
   __shared__ double red[kWalkBlock * 4 + 256];
   const int L4 = Qs / 4, G = 64 / L4;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -877,7 +880,9 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
     // rounded to FP32 is the argument of the FP32 exponential whether it is formed in FP32 or in FP64; the sum is FP64.
     float mn[4] = {INFINITY, INFINITY, INFINITY, INFINITY};
     double tt[4] = {0.0, 0.0, 0.0, 0.0};
-    auto add = [&](int c, float x) {
+    int ar[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX};
+    auto add = [&](int c, float x, int row) {
+      if (kArg && (x < mn[c] || (x == mn[c] && row < ar[c]))) ar[c] = row;
       const float d = mn[c] - x;  // > 0: a new least cost, the old ones rescaled to it
       float e = __expf(-fabsf(d));
       e = x == INFINITY ? 0.f : e;  // (and exp(-inf) = 0 where x is the first finite cost)
@@ -895,8 +900,10 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
       reinterpret_cast<float4*>(minCEo)[(int64_t)v * L4 + j] = make_float4(mn[0], mn[1], mn[2], mn[3]);
       reinterpret_cast<float4*>(lsO)[(int64_t)v * L4 + j] = ls;
       reinterpret_cast<float4*>(VFm)[(int64_t)v * L4 + j] = make_float4(-mn[0], -mn[1], -mn[2], -mn[3]);
+      if (kArg) reinterpret_cast<int4*>(AO)[(int64_t)v * L4 + j] = make_int4(ar[0], ar[1], ar[2], ar[3]);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
+        ar[c] = INT_MAX;
         glob[c] = lse_merge_fast(glob[c], Lse{-(double)mn[c], tt[c]});
         mn[c] = INFINITY;
         tt[c] = 0.0;
@@ -920,13 +927,14 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
           emit(cur);
           cur = e[u].y;
         }
-        add(0, c[u].x);
-        add(1, c[u].y);
-        add(2, c[u].z);
-        add(3, c[u].w);
+        add(0, c[u].x, e[u].x);
+        add(1, c[u].y, e[u].x);
+        add(2, c[u].z, e[u].x);
+        add(3, c[u].w, e[u].x);
       }
     }
     if (R.slot >= 0) {
+      if (kArg) reinterpret_cast<int4*>(carg)[(int64_t)R.slot * L4 + j] = make_int4(ar[0], ar[1], ar[2], ar[3]);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
         const Lse s{-(double)mn[c], tt[c]};
@@ -965,9 +973,14 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_src(int64_t nruns, const Ru
 }
 
 void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float* CE, int Q, int Qs, float* minCEo,
-                     float* lsO, float* VFm, double* carry, Lse* gpart, int nblocks, hipStream_t st) {
-  hipLaunchKernelGGL(k_walk_src, dim3(nblocks), dim3(kWalkBlock), 0, st, nruns, runs, ks, CE, Q, Qs, minCEo, lsO,
-                     VFm, carry, gpart);
+                     float* lsO, float* VFm, double* carry, Lse* gpart, int nblocks, hipStream_t st, int* AO,
+                     int* carg) {
+  if (AO)
+    hipLaunchKernelGGL(k_walk_src<true>, dim3(nblocks), dim3(kWalkBlock), 0, st, nruns, runs, ks, CE, Q, Qs, minCEo, lsO,
+                       VFm, carry, gpart, AO, carg);
+  else
+    hipLaunchKernelGGL(k_walk_src<false>, dim3(nblocks), dim3(kWalkBlock), 0, st, nruns, runs, ks, CE, Q, Qs, minCEo, lsO,
+                       VFm, carry, gpart, AO, carg);
 }
 
 // One wave per split vertex: groups of Qs/4 lanes take its pieces round-robin (lane j owns pattern edges
@@ -976,8 +989,10 @@ void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float
 __global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split* __restrict__ splits,
                                                         const double* __restrict__ carry, int Q, int Qs,
                                                         float* __restrict__ minCEo, float* __restrict__ lsO,
-                                                        float* __restrict__ VFm) {
+                                                        float* __restrict__ VFm, const int* __restrict__ carg,
+                                                        int* __restrict__ AO) {
   __shared__ double red[4][64][4];
+  __shared__ int rarg[4][64][4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int L4 = Qs / 4, G = 64 / L4;
   const int g = lane / L4, j = lane - g * L4;
@@ -1001,17 +1016,22 @@ __global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split*
     for (int gg = 0; gg < used; ++gg)
 #pragma unroll
       for (int u = 0; u < 4; ++u) M[u] = fmax(M[u], red[wave][gg * L4 + j][u]);
+  int ar[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX};  // with AO: the lowest row of the pieces that hold the least cost
   if (active)
 #pragma unroll 4
     for (int c = g; c < S.count; c += G)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const double* o = base + (int64_t)c * Qs * 2 + 2 * u;
+        if (AO && o[0] == M[u]) ar[u] = min(ar[u], carg[(int64_t)(S.first + c) * Qs + 4 * j + u]);
         lse_sum_step(sum[u], seen[u], lse_rescaled(Lse{o[0], o[1]}, M[u]));
       }
   __syncthreads();  // the maxima are read
 #pragma unroll
-  for (int u = 0; u < 4; ++u) red[wave][lane][u] = seen[u] ? -sum[u] : sum[u];  // a share of the group (lse_sum_step)
+  for (int u = 0; u < 4; ++u) {
+    red[wave][lane][u] = seen[u] ? -sum[u] : sum[u];  // a share of the group (lse_sum_step)
+    rarg[wave][lane][u] = ar[u];
+  }
   __syncthreads();
   if (sidx < nsplit && g == 0) {
 #pragma unroll
@@ -1024,15 +1044,20 @@ __global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split*
       minCEo[o] = q < Q ? (float)(-M[u]) : 0.f;
       lsO[o] = q < Q ? (float)log1p(t) : 0.f;
       VFm[o] = q < Q ? (float)M[u] : 0.f;
+      if (AO) {
+        int a = INT_MAX;
+        for (int gg = 0; gg < used; ++gg) a = min(a, rarg[wave][gg * L4 + j][u]);
+        AO[o] = a;
+      }
     }
   }
 }
 
 void launch_walk_src_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, float* minCEo,
-                           float* lsO, float* VFm, hipStream_t st) {
+                           float* lsO, float* VFm, hipStream_t st, const int* carg, int* AO) {
   if (nsplit == 0) return;
   hipLaunchKernelGGL(k_walk_src_fixup, dim3((unsigned)((nsplit + 3) / 4)), dim3(256), 0, st, nsplit, splits, carry,
-                     Q, Qs, minCEo, lsO, VFm);
+                     Q, Qs, minCEo, lsO, VFm, carg, AO);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1494,6 +1519,7 @@ __global__ __launch_bounds__(256) void k_walk_max_fixup(int nsplit, const Split*
   Split S{0, 0, 0, 0};
   if (sidx < nsplit) S = splits[sidx];
   if (active)
+#pragma unroll 4
     for (int c = g; c < S.count; c += G) {
       const double4 o = *reinterpret_cast<const double4*>(carry + (int64_t)(S.first + c) * Qs + 4 * j);
       const double ov[4] = {o.x, o.y, o.z, o.w};
@@ -1521,7 +1547,7 @@ __global__ __launch_bounds__(256) void k_walk_max_fixup(int nsplit, const Split*
     for (int u = 0; u < 4; ++u) {
       double acc = -kInf;
       int aa = -1;
-      for (int gg = 0; gg < G; ++gg)
+      for (int gg = 0; gg < min(G, S.count); ++gg)  // groups that have a piece
         if (red[wave][gg * L4 + j][u] > acc) {
           acc = red[wave][gg * L4 + j][u];
           aa = rarg[wave][gg * L4 + j][u];

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from application_classification_amd import workloads as W
-from application_classification_amd.matcher import AC_OPT_PRUNE, Matcher
+from application_classification_amd.matcher import AC_OPT_PRUNE, AC_OPT_TAPE, Matcher
 from oracle import oracle as O
 from tests.conftest import allclose_report
 
@@ -95,3 +95,32 @@ def test_topk_and_match_selection(n, pn, k, kind):
     expect = np.zeros((n, pn), np.uint8)
     expect[best, np.arange(pn)] = np.where(mu[best, np.arange(pn)] >= -8.0, 2, 1)
     np.testing.assert_array_equal(match, expect)
+
+
+@pytest.mark.parametrize("run_edges", [4, 16, 128])
+def test_gradients_do_not_depend_on_run_lengths(run_edges, monkeypatch):
+    """The recorded least-cost out-edges and argmax in-edges of hubs in one to hundreds of pieces, equal costs among
+    them: the gradients equal those of one piece per vertex to the rounding of the log-sum-exp merges (the forward
+    quantities differ by about 1e-7 of their size; 2e-5 allows for the sums over iterations and edges)."""
+    r = np.random.default_rng(5)
+    n = 700
+    src = np.concatenate([r.integers(0, n, 4000), r.integers(0, n, 600), np.full(600, 7)])
+    dst = np.concatenate([r.integers(0, n, 4000), np.full(600, 3), r.integers(0, n, 600)])
+    ef = r.normal(size=(len(src), 6)).astype(np.float32)
+    ef[-300:] = ef[-600:-300]  # equal costs among the hub's out-edges
+    data = W.Graph(r.normal(size=(n, 6)).astype(np.float32), ef, src.astype(np.int32), dst.astype(np.int32))
+    patt = W.planted_pattern(data, 6, 9, 2, sigma=0.3)
+    grad = np.zeros((n, 6), np.float32)
+    grad[patt.vmap, np.arange(6)] = -1.0 / 6
+
+    def run(L):
+        monkeypatch.setenv("AC_RUN_EDGES", str(L))
+        with Matcher(0) as m:
+            m.set_option(AC_OPT_TAPE, 1)
+            m.set_data(data)
+            m.set_pattern(patt)
+            m.run()
+            return m.backward(grad)
+
+    for got, want in zip(run(run_edges), run(4096)):
+        np.testing.assert_allclose(got, want, rtol=0, atol=2e-5 * np.abs(want).max())
