@@ -67,3 +67,97 @@ def test_edge_max_reduce_edges(n_row, n_in, n_out, offset, fill):
     got = out.cpu().numpy()
     np.testing.assert_array_equal(order_key(got[:n_row * n_out]).reshape(n_row, n_out), key)
     assert (got[n_row * n_out:] == 3.0).all()
+
+
+def at_offset(x, offset):
+    """x on the device, `offset` floats off an aligned start, and room behind it."""
+    buf = torch.full((x.size + 8,), 3.0, device="cuda")
+    buf[offset:offset + x.size] = dev(x.reshape(-1))
+    return buf, buf.data_ptr() + 4 * offset
+
+
+@pytest.mark.parametrize("n_row,n_col,offset", [(3, 1, 1), (2, 255, 0), (2, 257, 3), (3, 4096, 1), (2, 4097, 0),
+                                                (2, 32_768, 2), (3, 32_769, 1), (2, 70_001, 3)])
+def test_row_log_softmax_edges(n_row, n_col, offset):
+    """The one-launch and three-launch rows and their blocks' edges.  Each term is an FP32 exponential of a difference of
+    at most D: relative error (1 + D) 2^-23, which bounds the logarithm's; the result is rounded once."""
+    r = np.random.default_rng(n_col)
+    x = (r.normal(size=(n_row, n_col)) * 4).astype(np.float32)
+    if n_col > 1:
+        x[0, n_col // 2] = -np.inf
+        x[0, n_col - 1] = x[0].max()  # the maximum more than once
+    buf, ptr = at_offset(x, offset)
+    ac.RowSoftmax2(n_row, n_col, ptr)
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy()
+    assert (got[offset + x.size:] == 3.0).all() and (got[:offset] == 3.0).all()
+    ref = O.row_log_softmax(x.astype(np.float64))
+    spread = np.ptp(np.where(np.isfinite(x), x, 0.0))
+    np.testing.assert_allclose(got[offset:offset + x.size].reshape(x.shape), ref, rtol=2.0**-24,
+                               atol=(1 + spread) * 2.0**-23)
+
+
+@pytest.mark.parametrize("n_col", [300, 5000, 20_000, 40_000])
+def test_row_log_softmax_specials(n_col):
+    """One +inf takes the whole mass; two, a NaN, or nothing but -inf leave no number."""
+    x = np.random.default_rng(n_col).normal(size=(5, n_col)).astype(np.float32)
+    x[0, 7] = np.inf
+    x[1, [3, n_col - 1]] = np.inf
+    x[2, [4, n_col // 2]] = np.inf
+    x[3] = -np.inf
+    x[4, 9] = np.nan
+    buf, ptr = at_offset(x, 0)
+    ac.RowSoftmax2(5, n_col, ptr)
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy()[:x.size].reshape(x.shape)
+    assert np.isnan(got[0, 7]) and (np.delete(got[0], 7) == -np.inf).all()
+    assert np.isnan(got[1:]).all()
+
+
+@pytest.mark.parametrize("n_row,n_col,offset", [(1, 1, 0), (300, 3, 1), (3, 32_768, 1), (3, 32_769, 2), (2, 100_001, 3)])
+def test_row_max_edges(n_row, n_col, offset):
+    x = -np.abs(np.random.default_rng(n_col).normal(size=(n_row, n_col))).astype(np.float32) - 1.0
+    x[0, :] = -np.inf
+    buf, ptr = at_offset(x, offset)
+    out = torch.full((n_row + 4,), 3.0, device="cuda")
+    ac.RowMax2(n_row, n_col, ptr, out)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(out.cpu().numpy()[:n_row], x.max(axis=1))
+    assert (out.cpu().numpy()[n_row:] == 3.0).all()
+
+
+@pytest.mark.parametrize("n_in,n_out,P,Q,offset", [(8, 8, 3, 5, 0), (1028, 2052, 4, 70, 0), (1028, 2052, 4, 70, 1),
+                                                   (1027, 1030, 5, 130, 0), (4096, 1000, 2, 64, 0), (40, 44, 2, 700, 0),
+                                                   (7, 5, 3, 0, 0)])
+def test_compute_mu_edges(n_in, n_out, P, Q, offset):
+    """Both widths of access, columns on one side only, no pattern edge at all, loops, and more incident pattern edges
+    than one list holds.  FP64 sums in one order, rounded once: bit for bit."""
+    r = np.random.default_rng(Q)
+    cv, f, b = (r.normal(size=s).astype(np.float32) for s in ((P, n_out), (Q, n_in), (Q, n_in)))
+    src, dst = (r.integers(0, P, Q).astype(np.int32) for _ in range(2))
+    if Q:
+        src[0] = dst[0] = P - 1
+    keep = [at_offset(x, offset) for x in (cv, f, b)]
+    mu = torch.full((P * n_out + 8,), 3.0, device="cuda")
+    ac.ComputeMU2_t(n_in, Q, n_out, P, keep[0][1], keep[1][1], keep[2][1], dev(src), dev(dst),
+                    mu.data_ptr() + 4 * offset)
+    torch.cuda.synchronize()
+    ref = -cv.astype(np.float64)
+    n = min(n_in, n_out)
+    for q in range(Q):
+        ref[dst[q], :n] += f[q, :n]
+        ref[src[q], :n] += b[q, :n]
+    got = mu.cpu().numpy()
+    np.testing.assert_array_equal(got[offset:offset + P * n_out].reshape(P, n_out), ref.astype(np.float32))
+    assert (got[offset + P * n_out:] == 3.0).all() and (got[:offset] == 3.0).all()
+
+
+@pytest.mark.parametrize("n_rows,n_cols", [(1, 1), (64, 64), (63, 65), (3, 1000), (1000, 3), (16, 100_003), (70_001, 12)])
+def test_transpose_tiles(n_rows, n_cols):
+    x = np.arange(n_rows * n_cols, dtype=np.float32).reshape(n_rows, n_cols)
+    out = torch.full((x.size + 8,), -1.0, device="cuda")
+    ac.transpose(dev(x), out, n_rows, n_cols)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    np.testing.assert_array_equal(got[:x.size].reshape(n_cols, n_rows), x.T)
+    assert (got[x.size:] == -1.0).all()
