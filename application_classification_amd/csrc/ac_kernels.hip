@@ -1588,7 +1588,7 @@ void launch_walk_max_fixup(int nsplit, const Split* splits, const double* carry,
 // of its partials.  Hence short tiles where there are few (vertex_tile), lanes shared among pattern vertices, and
 // merges that take one exponential however many partials they merge.  Passes A / C per launch, before (a wave per
 // pattern vertex whatever the tile's height, isolated vertices on block 0's way, serial merges, a term at a time) and
-// now: 1,000 vertices with a 10/12 pattern 20.0 / 8.5 -> 11.8 / 5.3 us; 50,001 with 40/70 48.9 / 44.4 -> 29.2 / 20.0 us;
+// now: 1,000 vertices with a 10/12 pattern 20.0 / 8.5 -> 9.0 / 5.3 us; 50,001 with 40/70 48.9 / 44.4 -> 29.2 / 20.0 us;
 // R-MAT 16 slabs of 128 pattern edges 98.5 / 108.3 -> 50 / 35 us; R-MAT 20 with 16/24 105.7 / 58.9 -> 97 / 42 us.
 
 constexpr int kVTMax = 64;
@@ -1805,7 +1805,7 @@ __global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void
     offc[k / 2] = k & 1 ? offc[k / 2] | (o << 16) : o;
   }
 
-  const int RQ = Q > 0 ? NT / Q : 0;
+  const int RQ = Q > 0 ? min(NT / Q, VT) : 0;  // rows side by side (more would only lengthen the merge)
   const bool qthread = t < RQ * Q;
   const int q = qthread ? t % Q : 0, rq = qthread ? t / Q : 0;
   // Read once: loads inside the tile loop would follow the loop's stores (possible aliases) and wait for every
