@@ -673,7 +673,7 @@ extern "C" int ac_edge_max_reduce(int64_t n_col_in, int64_t n_col_out, int64_t n
     return bad("ac_edge_max_reduce: bad arguments");
   hipStream_t st = as_stream(stream);
   const int64_t fchunk = (n_col_out + 4095) / 4096;
-  if (n_col_out >= 4096 && n_row <= INT32_MAX / fchunk)
+  if (n_col_out >= 4096 && n_row > 0 && n_row <= INT32_MAX / fchunk)
     hipLaunchKernelGGL(k_stage_fill_long, dim3((unsigned)(n_row * fchunk)), dim3(kMaxBlock), 0, st, n_col_out, fchunk,
                        vymax, xmax);
   else if (n_row * n_col_out > 0)

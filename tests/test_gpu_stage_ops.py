@@ -42,7 +42,8 @@ def order_key(x):
 
 
 @pytest.mark.parametrize("n_row,n_in,n_out,offset", [(1, 1, 1, 0), (3, 7, 2, 1), (5, 1023, 40, 2), (2, 1025, 1, 3),
-                                                     (3, 8193, 700, 1), (16, 70_001, 3000, 0), (2, 0, 5, 0)])
+                                                     (3, 8193, 700, 1), (16, 70_001, 3000, 0), (2, 0, 5, 0),
+                                                     (3, 5, 4099, 1), (0, 5, 5000, 0)])
 @pytest.mark.parametrize("fill", ["low", "mid", "special"])
 def test_edge_max_reduce_edges(n_row, n_in, n_out, offset, fill):
     """Chunk edges, rows off the 16-byte grid, nodes shared by many and by neighbouring values, fills below, among and
