@@ -293,7 +293,8 @@ struct ac_ctx {
   DevBuf<int> d_perm;
   int64_t n_act = 0, n_iso = 0, n_both = 0, n_inonly = 0;
   int64_t nruns_in = 0, nruns_out = 0;
-  int nsplit_in = 0, nsplit_out = 0, nslots_in = 0, nslots_out = 0;
+  ac::SplitList list_in, list_out;
+  int nslots_in = 0, nslots_out = 0;
 
   // Per-dimension cdist weights (the adjoint's learnable feature metric); absent = the reference's cdist.
   bool has_wv = false, has_we = false;
@@ -578,8 +579,17 @@ static int set_data(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int64_
   HIPCHK(ctx, ctx->csc_eid.upload(csc_eid.data(), csc_eid.size(), st));
   HIPCHK(ctx, ctx->runs_in.upload(rin.data(), rin.size(), st));
   HIPCHK(ctx, ctx->runs_out.upload(rout.data(), rout.size(), st));
+  auto by_size = [](std::vector<Split>& s) {
+    const auto hubs = std::stable_partition(s.begin(), s.end(), [](const Split& x) { return x.count >= ac::kHubPieces; });
+    const auto few = std::stable_partition(hubs, s.end(), [](const Split& x) { return x.count > ac::kFewPieces; });
+    return ac::SplitList{(int)s.size(), (int)(hubs - s.begin()), (int)(s.end() - few), nullptr};
+  };
+  ctx->list_in = by_size(sin);
+  ctx->list_out = by_size(sout);
   HIPCHK(ctx, ctx->splits_in.upload(sin.data(), sin.size(), st));
   HIPCHK(ctx, ctx->splits_out.upload(sout.data(), sout.size(), st));
+  ctx->list_in.splits = ctx->splits_in.p;
+  ctx->list_out.splits = ctx->splits_out.p;
   ctx->dn = nV;
   ctx->max_outdeg = max_outdeg;
   ctx->n_iso = n_iso;
@@ -591,8 +601,6 @@ static int set_data(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int64_
   ctx->dE = dE;
   ctx->nruns_in = (int64_t)rin.size();
   ctx->nruns_out = (int64_t)rout.size();
-  ctx->nsplit_in = (int)sin.size();
-  ctx->nsplit_out = (int)sout.size();
   ctx->nslots_in = slin;
   ctx->nslots_out = slout;
   {
@@ -976,7 +984,7 @@ static int ensure_tape(ac_ctx* ctx, int n_iter) {
 // The split vertices' rows of the live FMaxN, reset before a plain (non-recording) walk.
 static ac::SplitRows split_rows(ac_ctx* ctx) {
   ac::SplitRows r;
-  r.nsplit = ctx->nsplit_in;
+  r.nsplit = ctx->list_in.n;
   r.splits = ctx->splits_in.p;
   r.Qs = ctx->Qs;
   r.FMaxN = ctx->FMaxN.p;
@@ -1037,7 +1045,7 @@ static int enqueue_prep(ac_ctx* ctx) {
       ac::launch_walk_src(ctx->nruns_out, ctx->runs_out.p, ctx->bs->csr_kb.p, ctx->CE.p, Q, Qs, ctx->minCEo.p,
                           ctx->lsO.p, ctx->VFm.p, ctx->carry_out.p, ctx->spart.p, ctx->nb_src, st, AO,
                           ctx->carg_out.p);
-      ac::launch_walk_src_fixup(ctx->nsplit_out, ctx->splits_out.p, ctx->carry_out.p, Q, Qs, ctx->minCEo.p,
+      ac::launch_walk_src_fixup(ctx->list_out, ctx->carry_out.p, Q, Qs, ctx->minCEo.p,
                                 ctx->lsO.p, ctx->VFm.p, st, ctx->carg_out.p, AO);
       ac::launch_reduce_lse(ctx->nb_src, Q, ctx->spart.p, ctx->lse_ce.p, st);
     } else {
@@ -1059,7 +1067,7 @@ static int enqueue_prep(ac_ctx* ctx) {
                         ctx->pack_costs ? ctx->CEp.p : nullptr, ctx->bstate.p);
     ctx->costs_packed = ctx->pack_costs;
     if (tape)
-      ac::launch_walk_max_fixup(ctx->nsplit_in, ctx->splits_in.p, ctx->carry_in.p, Q, Qs, qs_prep, ctx->FMaxN.p, st,
+      ac::launch_walk_max_fixup(ctx->list_in, ctx->carry_in.p, Q, Qs, qs_prep, ctx->FMaxN.p, st,
                                 ctx->carg_in.p, ctx->FA0.p);
   }
   HIPCHK(ctx, hipStreamWaitEvent(st, ctx->xev[1], 0));  // (again, for Q = 0) everything of the second stream
@@ -1894,7 +1902,7 @@ static int recompute_iteration(ac_ctx* ctx, int it, const StateBufs& In, const S
                         st, FA, ctx->carg_in.p, ctx->prune ? ctx->bmin.p : nullptr,
                         ctx->costs_packed ? ctx->CEp.p : nullptr, ctx->costs_packed ? ctx->bpack.p : nullptr);
     MARK(AC_STAGE_EDGE_WALK);
-    ac::launch_walk_max_fixup(ctx->nsplit_in, ctx->splits_in.p, ctx->carry_in.p, Q, Qs, Out.qs, Out.F, st,
+    ac::launch_walk_max_fixup(ctx->list_in, ctx->carry_in.p, Q, Qs, Out.qs, Out.F, st,
                               ctx->carg_in.p, FA);
     MARK(AC_STAGE_WALK_FIXUP);
   } else {

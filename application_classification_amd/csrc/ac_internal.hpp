@@ -61,6 +61,12 @@ struct Run {
 struct Split {
   int v, first, count, pad;
 };
+// The split vertices of one direction: first the nhub of at least kHubPieces pieces, last the nfew of at most kFewPieces.
+constexpr int kHubPieces = 32, kFewPieces = 4;
+struct SplitList {
+  int n = 0, nhub = 0, nfew = 0;
+  const Split* splits = nullptr;
+};
 // The split vertices' FMaxN rows, set to -inf before a plain walk raises them piece by piece (nsplit 0: none).
 struct SplitRows {
   int nsplit = 0;
@@ -140,7 +146,7 @@ void launch_fill_slots(float* A, float* B, int64_t nslots, int64_t stride, int64
 void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float* CE, int Q, int Qs, float* minCEo,
                      float* lsO, float* VFm, double* carry, Lse* gpart, int nblocks, hipStream_t st, int* AO = nullptr,
                      int* carg = nullptr);
-void launch_walk_src_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, float* minCEo,
+void launch_walk_src_fixup(const SplitList& L, const double* carry, int Q, int Qs, float* minCEo,
                            float* lsO, float* VFm, hipStream_t st, const int* carg = nullptr, int* AO = nullptr);
 void launch_build_bundles(int64_t nbundles, const Bundle* bundles, const int* brun, const Run* runs, const int2* sd,
                           const int* eid, int G, int* bsrc, int* bdst, int* beid, int* rowmap, hipStream_t st);
@@ -155,9 +161,9 @@ void launch_walk_max(int64_t nbundles, const Bundle* bundles, const int* gslot, 
                      double* carry, int B, hipStream_t st, int* FA = nullptr, int* carg = nullptr,
                      const float* bmin = nullptr, const unsigned* CEp = nullptr, const unsigned* bpack = nullptr,
                      unsigned* CEp_out = nullptr, int* bstate = nullptr);
-// Taped walks (FA): the pieces' FP64 maxima and rows, combined one wave per split vertex.
-void launch_walk_max_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, const QStat* qs,
-                           float* FMaxN, hipStream_t st, const int* carg = nullptr, int* FA = nullptr);
+// Taped walks (FA): the pieces' FP64 maxima and rows, combined per split vertex.
+void launch_walk_max_fixup(const SplitList& L, const double* carry, int Q, int Qs, const QStat* qs,
+                           float* FMaxN, hipStream_t st, const int* carg, int* FA);
 void launch_vertex(int mode, const VertexArgs& a, int nblocks, hipStream_t st);
 // Blocks of vertex pass `mode` resident at once on the current device (0 if unknown); a.VT/P/Q/Qs set its LDS.
 int vertex_resident_blocks(int mode, const VertexArgs& a);

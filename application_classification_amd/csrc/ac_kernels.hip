@@ -983,47 +983,112 @@ void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float
                        VFm, carry, gpart, AO, carg);
 }
 
-// One wave per split vertex: groups of Qs/4 lanes take its pieces round-robin (lane j owns pattern edges
-// 4j..4j+3), first for the largest maximum, then for the pieces' shares of it, whose exponentials do not wait for each
-// other; the groups' results are combined in group order through LDS.  Deterministic.
-__global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split* __restrict__ splits,
-                                                        const double* __restrict__ carry, int Q, int Qs,
-                                                        float* __restrict__ minCEo, float* __restrict__ lsO,
-                                                        float* __restrict__ VFm, const int* __restrict__ carg,
-                                                        int* __restrict__ AO) {
-  __shared__ double red[4][64][4];
-  __shared__ int rarg[4][64][4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int L4 = Qs / 4, G = 64 / L4;
-  const int g = lane / L4, j = lane - g * L4;
-  const int sidx = blockIdx.x * 4 + wave;
-  const bool active = sidx < nsplit && g < G;
-  Split S{0, 0, 0, 0};
-  if (sidx < nsplit) S = splits[sidx];
-  const double* base = carry + ((int64_t)S.first * Qs + 4 * j) * 2;
+// The split vertices' pieces combined: groups of Qs/4 lanes take a vertex's pieces round-robin (lane j owns pattern edges
+// 4j..4j+3), and their results are combined through LDS in a fixed order.  Bound by latency, a few dependent reads per
+// vertex, and by the hubs' chains, so the vertices of a list (hubs first, those of few pieces last) are taken in three
+// ways: a hub by all kFixWaves waves of a block, one of at most kFewPieces pieces by a thread per pattern edge, its pieces
+// all in flight (where a wave has as many groups, so that the pieces' order is that of the groups), the others by a wave.  A
+// wave for every vertex, before: R-MAT 18, 12/16 pattern, 48 us for the source side's sums and 15 us for the taped maxima;
+// now 26 and 10 us; 50,001 vertices, 40/70: 48 and 20 us for the sums.
+constexpr int kFixWaves = 8;
+struct FixTask {
+  Split S;
+  int g, j, w, W;  // the lane's group and place in it; the wave's place among the W that share the vertex
+  bool active, few;
+};
+__device__ __forceinline__ FixTask fix_task(const SplitList& L, int Qs) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, L4 = Qs / 4, G = 64 / L4;
+  const int nfew = G >= kFewPieces ? L.nfew : 0, nmid = L.n - L.nhub - nfew;
+  const int bmid = L.nhub + (nmid + kFixWaves - 1) / kFixWaves, b = blockIdx.x;
+  FixTask f;
+  f.g = lane / L4;
+  f.j = lane - f.g * L4;
+  f.W = b < L.nhub ? kFixWaves : 1;
+  f.w = b < L.nhub ? wave : 0;
+  f.few = b >= bmid;
+  int i = b < L.nhub ? b : L.nhub + (b - L.nhub) * kFixWaves + wave, end = L.n - nfew;
+  f.active = f.g < G;
+  if (f.few) {  // g: unused; j: the thread's pattern edge
+    const int e = (b - bmid) * (64 * kFixWaves) + threadIdx.x;
+    i = L.n - nfew + e / Qs;
+    end = L.n;
+    f.j = e - e / Qs * Qs;
+    f.active = true;
+  }
+  f.active = f.active && i < end;
+  f.S = f.active ? L.splits[i] : Split{0, 0, 0, 0};
+  return f;
+}
+static unsigned fix_blocks(const SplitList& L, int Qs) {
+  const int G = 64 / (Qs / 4), nfew = G >= kFewPieces ? L.nfew : 0, nmid = L.n - L.nhub - nfew;
+  return L.nhub + (nmid + kFixWaves - 1) / kFixWaves +
+         (int)(((int64_t)nfew * Qs + 64 * kFixWaves - 1) / (64 * kFixWaves));
+}
+
+// The largest maximum first, then the pieces' shares of it, whose exponentials do not wait for each other.
+__global__ __launch_bounds__(64 * kFixWaves) void k_walk_src_fixup(SplitList L,
+                                                                   const double* __restrict__ carry, int Q, int Qs,
+                                                                   float* __restrict__ minCEo, float* __restrict__ lsO,
+                                                                   float* __restrict__ VFm, const int* __restrict__ carg,
+                                                                   int* __restrict__ AO) {
+  __shared__ double red[kFixWaves][64][4];
+  __shared__ int rarg[kFixWaves][64][4];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, L4 = Qs / 4, G = 64 / L4;
+  const FixTask f = fix_task(L, Qs);
+  const int c0 = f.w * G + f.g, step = f.W * G, row = wave - f.w, j = f.j;  // row of red: the vertex's combined results
+  if (f.few) {
+    if (!f.active) return;
+    const double2* o = reinterpret_cast<const double2*>(carry) + (int64_t)f.S.first * Qs + j;
+    double2 x[kFewPieces];
+#pragma unroll
+    for (int c = 0; c < kFewPieces; ++c) x[c] = o[(int64_t)min(c, f.S.count - 1) * Qs];
+    double M = x[0].x, sum = 0.0;
+    bool any = false;
+    int a = INT_MAX;
+#pragma unroll
+    for (int c = 1; c < kFewPieces; ++c) M = fmax(M, x[c].x);  // (past the last piece: that piece again)
+#pragma unroll
+    for (int c = 0; c < kFewPieces; ++c)
+      if (c < f.S.count) {
+        if (AO && x[c].x == M) a = min(a, carg[(int64_t)(f.S.first + c) * Qs + j]);
+        lse_sum_step(sum, any, lse_rescaled(Lse{x[c].x, x[c].y}, M));
+      }
+    const int64_t at = (int64_t)f.S.v * Qs + j;
+    minCEo[at] = j < Q ? (float)(-M) : 0.f;
+    lsO[at] = j < Q ? (float)log1p(sum) : 0.f;
+    VFm[at] = j < Q ? (float)M : 0.f;
+    if (AO) AO[at] = a;
+    return;
+  }
+  const double* base = carry + ((int64_t)f.S.first * Qs + 4 * j) * 2;
   double M[4] = {-kInf, -kInf, -kInf, -kInf}, sum[4] = {0.0, 0.0, 0.0, 0.0};
   bool seen[4] = {false, false, false, false};
-  if (active)
+  if (f.active)
 #pragma unroll 4
-    for (int c = g; c < S.count; c += G)
+    for (int c = c0; c < f.S.count; c += step)
 #pragma unroll
       for (int u = 0; u < 4; ++u) M[u] = fmax(M[u], base[(int64_t)c * Qs * 2 + 2 * u]);
 #pragma unroll
   for (int u = 0; u < 4; ++u) red[wave][lane][u] = M[u];
   __syncthreads();
-  const int used = min(G, S.count);  // groups that have a piece
-  if (active)
+  const int used = min(G, f.S.count);  // groups that have a piece
+  if (f.W > 1) {
+    if (t < 256)
+      for (int w = 1; w < kFixWaves; ++w) red[0][t >> 2][t & 3] = fmax(red[0][t >> 2][t & 3], red[w][t >> 2][t & 3]);
+    __syncthreads();
+  }
+  if (f.active)
     for (int gg = 0; gg < used; ++gg)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) M[u] = fmax(M[u], red[wave][gg * L4 + j][u]);
+      for (int u = 0; u < 4; ++u) M[u] = fmax(M[u], red[row][gg * L4 + j][u]);
   int ar[4] = {INT_MAX, INT_MAX, INT_MAX, INT_MAX};  // with AO: the lowest row of the pieces that hold the least cost
-  if (active)
+  if (f.active)
 #pragma unroll 4
-    for (int c = g; c < S.count; c += G)
+    for (int c = c0; c < f.S.count; c += step)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const double* o = base + (int64_t)c * Qs * 2 + 2 * u;
-        if (AO && o[0] == M[u]) ar[u] = min(ar[u], carg[(int64_t)(S.first + c) * Qs + 4 * j + u]);
+        if (AO && o[0] == M[u]) ar[u] = min(ar[u], carg[(int64_t)(f.S.first + c) * Qs + 4 * j + u]);
         lse_sum_step(sum[u], seen[u], lse_rescaled(Lse{o[0], o[1]}, M[u]));
       }
   __syncthreads();  // the maxima are read
@@ -1033,31 +1098,44 @@ __global__ __launch_bounds__(256) void k_walk_src_fixup(int nsplit, const Split*
     rarg[wave][lane][u] = ar[u];
   }
   __syncthreads();
-  if (sidx < nsplit && g == 0) {
+  if (f.W > 1) {
+    if (t < 256) {
+      double x = 0.0;
+      bool any = false;
+      int a = INT_MAX;
+      for (int w = 0; w < kFixWaves; ++w) {
+        lse_sum_step(x, any, red[w][t >> 2][t & 3]);
+        a = min(a, rarg[w][t >> 2][t & 3]);
+      }
+      red[0][t >> 2][t & 3] = any ? -x : x;
+      rarg[0][t >> 2][t & 3] = a;
+    }
+    __syncthreads();
+  }
+  if (f.active && f.w == 0 && f.g == 0) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      double t = 0.0;
+      double x = 0.0;
       bool any = false;
-      for (int gg = 0; gg < used; ++gg) lse_sum_step(t, any, red[wave][gg * L4 + j][u]);
+      for (int gg = 0; gg < used; ++gg) lse_sum_step(x, any, red[row][gg * L4 + j][u]);
       const int q = 4 * j + u;
-      const int64_t o = (int64_t)S.v * Qs + q;
+      const int64_t o = (int64_t)f.S.v * Qs + q;
       minCEo[o] = q < Q ? (float)(-M[u]) : 0.f;
-      lsO[o] = q < Q ? (float)log1p(t) : 0.f;
+      lsO[o] = q < Q ? (float)log1p(x) : 0.f;
       VFm[o] = q < Q ? (float)M[u] : 0.f;
       if (AO) {
         int a = INT_MAX;
-        for (int gg = 0; gg < used; ++gg) a = min(a, rarg[wave][gg * L4 + j][u]);
+        for (int gg = 0; gg < used; ++gg) a = min(a, rarg[row][gg * L4 + j][u]);
         AO[o] = a;
       }
     }
   }
 }
 
-void launch_walk_src_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, float* minCEo,
+void launch_walk_src_fixup(const SplitList& L, const double* carry, int Q, int Qs, float* minCEo,
                            float* lsO, float* VFm, hipStream_t st, const int* carg, int* AO) {
-  if (nsplit == 0) return;
-  hipLaunchKernelGGL(k_walk_src_fixup, dim3((unsigned)((nsplit + 3) / 4)), dim3(256), 0, st, nsplit, splits, carry,
-                     Q, Qs, minCEo, lsO, VFm, carg, AO);
+  if (L.n == 0) return;
+  hipLaunchKernelGGL(k_walk_src_fixup, dim3(fix_blocks(L, Qs)), dim3(64 * kFixWaves), 0, st, L, carry, Q, Qs, minCEo, lsO, VFm, carg, AO);
 }
 
 // ---------------------------------------------------------------------------------------------------------------
@@ -1501,73 +1579,89 @@ void launch_remap_ks(int64_t m, const int2* ks, const int* rowmap, int2* out, hi
   hipLaunchKernelGGL(k_remap_ks, dim3(blocks), dim3(256), 0, st, m, ks, rowmap, out);
 }
 
-// One wave per split vertex, as k_walk_src_fixup.  With carg: the argmax row of the best piece (the first in merge
-// order on ties) into FA.
-__global__ __launch_bounds__(256) void k_walk_max_fixup(int nsplit, const Split* __restrict__ splits,
-                                                        const double* __restrict__ carry, int Q, int Qs,
-                                                        const QStat* __restrict__ qs, float* __restrict__ FMaxN,
-                                                        const int* __restrict__ carg, int* __restrict__ FA) {
-  __shared__ double red[4][64][4];
-  __shared__ int rarg[4][64][4];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int L4 = Qs / 4, G = 64 / L4;
-  const int g = lane / L4, j = lane - g * L4;
-  const int sidx = blockIdx.x * 4 + wave;
-  const bool active = sidx < nsplit && g < G;
+// The taped walks' pieces, as k_walk_src_fixup: the maxima, and the row of the best piece into FA.  Of equal pieces the
+// first of the lowest group counts, however many waves share the vertex.
+__global__ __launch_bounds__(64 * kFixWaves) void k_walk_max_fixup(SplitList L,
+                                                                   const double* __restrict__ carry, int Q, int Qs,
+                                                                   const QStat* __restrict__ qs,
+                                                                   float* __restrict__ FMaxN,
+                                                                   const int* __restrict__ carg, int* __restrict__ FA) {
+  __shared__ double red[kFixWaves][64][4];
+  __shared__ int rpiece[kFixWaves][64][4];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6, L4 = Qs / 4, G = 64 / L4;
+  const FixTask f = fix_task(L, Qs);
+  // Normalised as the walk normalises a vertex it finishes (one FP64 subtraction of mFE + lFE, rounded once), so a
+  // recording walk leaves the same FMaxN as a plain one, whose pieces are normalised that way.
+  auto finish = [&](int q, double m, int piece) {
+    const int64_t o = (int64_t)f.S.v * Qs + q;
+    FMaxN[o] = (float)(m - (q < Q ? qs[q].mFE + qs[q].lFE : 0.0));
+    FA[o] = piece < 0 ? -1 : carg[(int64_t)(f.S.first + piece) * Qs + q];
+  };
+  if (f.few) {
+    if (!f.active) return;
+    double o[kFewPieces], m = -kInf;
+    int a = -1;
+#pragma unroll
+    for (int c = 0; c < kFewPieces; ++c) o[c] = carry[(int64_t)(f.S.first + min(c, f.S.count - 1)) * Qs + f.j];
+#pragma unroll
+    for (int c = 0; c < kFewPieces; ++c)  // (past the last piece: that piece again, which changes nothing)
+      if (o[c] > m) m = o[c], a = c;
+    finish(f.j, m, a);
+    return;
+  }
   double mx[4] = {-kInf, -kInf, -kInf, -kInf};
-  int ag[4] = {-1, -1, -1, -1};
-  Split S{0, 0, 0, 0};
-  if (sidx < nsplit) S = splits[sidx];
-  if (active)
+  int at[4] = {-1, -1, -1, -1};
+  if (f.active)
 #pragma unroll 4
-    for (int c = g; c < S.count; c += G) {
-      const double4 o = *reinterpret_cast<const double4*>(carry + (int64_t)(S.first + c) * Qs + 4 * j);
+    for (int c = f.w * G + f.g; c < f.S.count; c += f.W * G) {
+      const double4 o = *reinterpret_cast<const double4*>(carry + (int64_t)(f.S.first + c) * Qs + 4 * f.j);
       const double ov[4] = {o.x, o.y, o.z, o.w};
-      int4 oa = make_int4(-1, -1, -1, -1);
-      if (carg) oa = reinterpret_cast<const int4*>(carg)[(int64_t)(S.first + c) * L4 + j];
-      const int oav[4] = {oa.x, oa.y, oa.z, oa.w};
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         if (ov[u] > mx[u]) {
           mx[u] = ov[u];
-          ag[u] = oav[u];
+          at[u] = c;
         }
     }
 #pragma unroll
   for (int u = 0; u < 4; ++u) {
     red[wave][lane][u] = mx[u];
-    rarg[wave][lane][u] = ag[u];
+    rpiece[wave][lane][u] = at[u];
   }
   __syncthreads();
-  if (sidx < nsplit && g == 0) {
-    float4 out;
-    float* po = reinterpret_cast<float*>(&out);
-    int oarg[4];
+  if (f.W > 1) {
+    if (t < 256) {
+      double m = red[0][t >> 2][t & 3];
+      int a = rpiece[0][t >> 2][t & 3];
+      for (int w = 1; w < kFixWaves; ++w) {
+        const double x = red[w][t >> 2][t & 3];
+        const int xa = rpiece[w][t >> 2][t & 3];
+        if (x > m || (x == m && xa < a)) m = x, a = xa;
+      }
+      red[0][t >> 2][t & 3] = m;
+      rpiece[0][t >> 2][t & 3] = a;
+    }
+    __syncthreads();
+  }
+  if (f.active && f.w == 0 && f.g == 0) {
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      double acc = -kInf;
-      int aa = -1;
-      for (int gg = 0; gg < min(G, S.count); ++gg)  // groups that have a piece
-        if (red[wave][gg * L4 + j][u] > acc) {
-          acc = red[wave][gg * L4 + j][u];
-          aa = rarg[wave][gg * L4 + j][u];
+      double m = -kInf;
+      int a = -1;
+      for (int gg = 0; gg < min(G, f.S.count); ++gg)  // groups that have a piece
+        if (red[wave][gg * L4 + f.j][u] > m) {
+          m = red[wave][gg * L4 + f.j][u];
+          a = rpiece[wave][gg * L4 + f.j][u];
         }
-      const int q = 4 * j + u;
-      // Normalised as the walk normalises a vertex it finishes (one FP64 subtraction of mFE + lFE, rounded once),
-      // so a recording walk leaves the same FMaxN as a plain one, whose pieces are normalised that way.
-      po[u] = (float)(acc - (q < Q ? qs[q].mFE + qs[q].lFE : 0.0));
-      oarg[u] = aa;
+      finish(4 * f.j + u, m, a);
     }
-    reinterpret_cast<float4*>(FMaxN)[(int64_t)S.v * L4 + j] = out;
-    if (carg) reinterpret_cast<int4*>(FA)[(int64_t)S.v * L4 + j] = make_int4(oarg[0], oarg[1], oarg[2], oarg[3]);
   }
 }
 
-void launch_walk_max_fixup(int nsplit, const Split* splits, const double* carry, int Q, int Qs, const QStat* qs,
+void launch_walk_max_fixup(const SplitList& L, const double* carry, int Q, int Qs, const QStat* qs,
                            float* FMaxN, hipStream_t st, const int* carg, int* FA) {
-  if (nsplit == 0) return;
-  hipLaunchKernelGGL(k_walk_max_fixup, dim3((unsigned)((nsplit + 3) / 4)), dim3(256), 0, st, nsplit, splits, carry,
-                     Q, Qs, qs, FMaxN, carg, FA);
+  if (L.n == 0) return;
+  hipLaunchKernelGGL(k_walk_max_fixup, dim3(fix_blocks(L, Qs)), dim3(64 * kFixWaves), 0, st, L, carry, Q, Qs, qs, FMaxN, carg, FA);
 }
 
 // ---------------------------------------------------------------------------------------------------------------

@@ -124,3 +124,29 @@ def test_gradients_do_not_depend_on_run_lengths(run_edges, monkeypatch):
 
     for got, want in zip(run(run_edges), run(4096)):
         np.testing.assert_allclose(got, want, rtol=0, atol=2e-5 * np.abs(want).max())
+
+
+@pytest.mark.parametrize("pe", [3, 70, 130, 250])
+@pytest.mark.parametrize("pieces", [3, 4, 5, 31, 32, 33, 300])
+def test_hub_pieces(pe, pieces, monkeypatch):
+    """Vertices at the piece counts where a group, a wave and a block take over, beside vertices of two and three
+    pieces, for patterns that leave a wave one group of lanes to many; recorded and plain walks agree bit for bit."""
+    monkeypatch.setenv("AC_RUN_EDGES", "4")
+    r = np.random.default_rng(pieces)
+    n, hub = 120, 4 * pieces
+    src = np.concatenate([r.integers(8, n, 900), r.integers(8, n, hub), np.full(hub, 5), r.integers(8, n, hub)])
+    dst = np.concatenate([r.integers(8, n, 900), np.full(hub, 3), r.integers(8, n, hub), np.full(hub, 4)])
+    data = W.Graph(r.normal(size=(n, 6)).astype(np.float32), r.normal(size=(len(src), 6)).astype(np.float32),
+                   src.astype(np.int32), dst.astype(np.int32))
+    patt = random_graph(9, pe, 6, 6, pe)
+    expect = O.run(g64(data), g64(patt), n_iter=4)
+    got = []
+    for tape in (0, 1):
+        with Matcher(0) as m:
+            m.set_option(AC_OPT_TAPE, tape)
+            m.set_data(data)
+            m.set_pattern(patt)
+            got.append(m.run(4))
+        bad, ratio = allclose_report(got[-1], expect)
+        assert bad == 0, (tape, ratio)
+    np.testing.assert_array_equal(got[0], got[1])
