@@ -31,35 +31,6 @@ namespace {
 constexpr double kInf = __builtin_huge_val();
 typedef float f4v __attribute__((ext_vector_type(4)));
 
-// MU[v][p] of a state: (Z - m) - l with Z = -CV + (first ? 0 : the incidence terms of p in ascending q, the FMax
-// term before the RMax term), exactly as the vertex pass evaluates it.
-__device__ __forceinline__ double mu_of(const BwdGraph& G, const BwdState& S, int64_t v, int p) {
-  double acc = -(double)G.CV[v * G.P + p];
-  if (!S.first)
-    for (int k = G.inc_off[p]; k < G.inc_off[p + 1]; ++k) {
-      const int code = G.inc[k];
-      const int q = code >> 1;
-      const QStat s = S.qs[q];
-      if (code & 1) {
-        const float vfm = S.VFm[v * G.Qs + q];
-        const double rn = vfm == -INFINITY ? -kInf : ((double)vfm - s.mRE) - s.lRE;
-        acc += fmax(s.fillR, rn);
-      } else {
-        acc += fmax(s.fillF, (double)S.FMaxN[v * G.Qs + q]);
-      }
-    }
-  return (acc - S.pst[p].m) - S.pst[p].l;
-}
-
-__device__ __forceinline__ double fmax_of(const BwdGraph& G, const BwdState& S, int64_t v, int q) {
-  return fmax(S.qs[q].fillF, (double)S.FMaxN[v * G.Qs + q]);
-}
-
-__device__ __forceinline__ double rn_of(const BwdGraph& G, const BwdState& S, int64_t v, int q) {
-  const float vfm = S.VFm[v * G.Qs + q];
-  return vfm == -INFINITY ? -kInf : ((double)vfm - S.qs[q].mRE) - S.qs[q].lRE;
-}
-
 }  // namespace
 
 // Column sums of X[n][C] (C <= 256): per-block partials in a fixed order.
@@ -117,43 +88,70 @@ __global__ __launch_bounds__(256) void k_bwd_out(int64_t total, int P, const dou
   }
 }
 
-// Max-subgradient routing of FMax / RMax of state S (thread per (v, q), q fixed per thread).  gF = -gVF + gZ[pd]
-// (with_gz), gR = -gVR + gZ[ps], where gVF / gVR are the next state's (the step processed before this one; zero at the
+// Max-subgradient routing of FMax / RMax of state S (thread per (v, q), q fixed per thread).  gF = -gVF + gZ[pd],
+// gR = -gVR + gZ[ps], where gVF / gVR are the next state's (the step processed before this one; zero at the
 // first): the gradients of this state's FMax / RMax through the next step's inputs.  The edge term takes the
 // gradient where it is strictly above the fill.  Per-block partials part[4][Q][blocks]: sum gE_F, sum gE_R, fill gradient
 // of fillF, of fillR.  gmax (nullable) receives the largest |gE_F| (as float bits, an atomic maximum: exact and
-// order-free), which sets the fixed-point scale of the FMax edge terms' source sums.  gERsum (nullable) accumulates
+// order-free), which sets the fixed-point scale of the FMax edge terms' source sums.  gERsum accumulates
 // gE_R per (v, q) over the steps: the RMax rows AO are the same in every step, so their edge terms are applied once.
-__global__ __launch_bounds__(256) void k_bwd_route(BwdGraph G, BwdState S, const float* __restrict__ gZ, int with_gz,
-                                                   const float* __restrict__ gVF, const float* __restrict__ gVR,
-                                                   float* __restrict__ gEF, float* __restrict__ gER,
-                                                   unsigned* __restrict__ gmax, float* __restrict__ gERsum,
-                                                   double* __restrict__ part) {
+// kOut: k_bwd_out's step for the rows of a tile first (T rows; T P <= kRouteTile), its gZ kept in LDS: gZ is read here
+// only, and in a launch of its own it was written and read back.  Isolated vertices have no edge terms (FMaxN and VFm hold
+// -inf), so their rows of S are not read, nor, with kOut, their zero rows of gEF and gER written.  Bound by its streams:
+// R-MAT 18 with 12/16, a step's two launches 43 us, now 33.
+constexpr int kRouteTile = 2048;
+template <bool kOut>
+__global__ __launch_bounds__(256) void k_bwd_route(BwdGraph G, BwdState S, const double* __restrict__ MU,
+                                                   const double* __restrict__ colsum, const float* __restrict__ gMU,
+                                                   float* __restrict__ gCV, const float* __restrict__ gVF,
+                                                   const float* __restrict__ gVR, float* __restrict__ gEF,
+                                                   float* __restrict__ gER, unsigned* __restrict__ gmax,
+                                                   float* __restrict__ gERsum, double* __restrict__ part, int T) {
   __shared__ double red[256][4];
+  __shared__ float gz[kOut ? kRouteTile : 1];
   __shared__ unsigned bmax;
-  const int t = threadIdx.x, Q = G.Q, RQ = 256 / Q;
+  const int t = threadIdx.x, Q = G.Q, P = G.P, RQ = 256 / Q;
   if (t == 0) bmax = 0u;
-  __syncthreads();
   const bool active = t < RQ * Q;
-  const int q = active ? t % Q : 0;
+  const int q = active ? t % Q : 0, rq = active ? t / Q : 0;
   double sF = 0.0, sR = 0.0, fF = 0.0, fR = 0.0;
   unsigned mx = 0u;
-  if (active) {
-    const int pdq = G.pd[q], psq = G.ps[q];
-    const double fillF = S.qs[q].fillF, fillR = S.qs[q].fillR;
-    for (int64_t v = (int64_t)blockIdx.x * RQ + t / Q; v < G.n; v += (int64_t)gridDim.x * RQ) {
-      const int64_t i = v * G.Qs + q;
-      float gF = -gVF[i], gR = -gVR[i];
-      if (with_gz) {
-        gF += gZ[v * G.P + pdq];
-        gR += gZ[v * G.P + psq];
+  const int pdq = G.pd[q], psq = G.ps[q];
+  const QStat s = S.qs[q];
+  for (int64_t v0 = (int64_t)blockIdx.x * T; v0 < G.n; v0 += (int64_t)gridDim.x * T) {
+    const int nv = (int)min((int64_t)T, G.n - v0);
+    __syncthreads();
+    if (kOut) {
+      for (int e = t; e < nv * P; e += 256) {
+        const int64_t i = v0 * P + e;
+        const float g = gMU[i] - __expf((float)MU[i]) * (float)colsum[e % P];
+        gz[e] = g;
+        gCV[i] -= g;
       }
-      const bool eF = (double)S.FMaxN[i] > fillF;
-      const bool eR = rn_of(G, S, v, q) > fillR;
+      __syncthreads();
+    }
+    if (!active) continue;
+#pragma unroll 2
+    for (int r = rq; r < nv; r += RQ) {
+      const int64_t i = (v0 + r) * G.Qs + q;
+      float gF = -gVF[i], gR = -gVR[i];
+      if (kOut) {
+        gF += gz[r * P + pdq];
+        gR += gz[r * P + psq];
+      }
+      if (v0 + r >= G.n_act) {
+        fF += gF;
+        fR += gR;
+        if (!kOut) gEF[i] = gER[i] = 0.f;
+        continue;
+      }
+      const float vfm = S.VFm[i];
+      const bool eF = (double)S.FMaxN[i] > s.fillF;
+      const bool eR = (vfm == -INFINITY ? -kInf : ((double)vfm - s.mRE) - s.lRE) > s.fillR;
       gEF[i] = eF ? gF : 0.f;
       gER[i] = eR ? gR : 0.f;
       if (eF) mx = max(mx, __float_as_uint(fabsf(gF)));
-      if (gERsum && eR && gR != 0.f) gERsum[i] += gR;
+      if (eR && gR != 0.f) gERsum[i] += gR;
       if (eF) sF += gF; else fF += gF;
       if (eR) sR += gR; else fR += gR;
     }
@@ -217,92 +215,133 @@ __global__ void k_bwd_fscatter(int64_t n, int Q, int Qs, const float* __restrict
 //   cD += S_F exp(VR - LSE_FE) + S_R exp(VF - LSE_RE)            (vertices with out-edges; FP64)
 // and the FMax edge terms of the step (fmax_edge_term; FE: the step's gE_F, argmax rows and fixed-point scale), whose
 // source sums go to gVRfix and are added to gVR by the vertex kernel that follows.
-__global__ __launch_bounds__(256) void k_bwd_in(BwdGraph G, BwdState S, const double* __restrict__ MU,
+// A thread keeps its pattern edge and takes kIn vertices at a time, all their loads in flight.  Isolated vertices have no
+// terms but those of the maxima's vertices.  Bound by its streams (14 values of 4 or 8 bytes per vertex and pattern edge)
+// and three FP64 exponentials: R-MAT 18 with 12/16 in 51 us (66 with a flat index
+// and the scalars read for every element; 57 with 8192 blocks, whose prologues follow each other).
+constexpr int kIn = 2;
+__global__ __launch_bounds__(256, 4) void k_bwd_in(BwdGraph G, BwdState S, const double* __restrict__ MU,
                                                 const QStat* __restrict__ qs1, const double* __restrict__ red4,
                                                 const float* __restrict__ gER, float* __restrict__ gVR,
                                                 float* __restrict__ gVF, double* __restrict__ cD, FmaxTerms FE) {
-  const int Q = G.Q;
-  const int64_t total = G.n * Q;
+  const int Q = G.Q, RQ = 256 / Q, t = threadIdx.x;
+  if (t >= RQ * Q) return;
   const double fscale = ldexp(1.0, fix_exponent(*FE.gmax, G.fix_shift));
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t v = i / Q;
-    const int q = (int)(i - v * Q);
-    const int64_t o = v * G.Qs + q;
-    const double VF = MU[v * G.P + G.pd[q]] - fmax_of(G, S, v, q);
-    const double VR = MU[v * G.P + G.ps[q]] - fmax(S.qs[q].fillR, rn_of(G, S, v, q));
-    const QStat s1 = qs1[q];
-    const double SF = red4[q], SR = red4[Q + q];
-    const float mo = G.minCEo[o];
-    double gvr = 0.0, gvf = (double)gER[o];
-    if (mo != INFINITY) {
-      const double eF = exp(VR - (s1.mFE + s1.lFE)), eR = exp(VF - (s1.mRE + s1.lRE));
-      const double wo = exp((double)G.lsO[o] - (double)mo);
-      gvr -= SF * eF * wo;
-      gvf -= SR * eR * wo;
-      cD[o] += SF * eF + SR * eR;
+  const int q = t % Q, pdq = G.pd[q], psq = G.ps[q];
+  const QStat s0 = S.qs[q], s1 = qs1[q];
+  const double SF = red4[q], SR = red4[Q + q], gfF = red4[2 * Q + q], gfR = red4[3 * Q + q];
+  const double lF = s1.mFE + s1.lFE, lR = s1.mRE + s1.lRE;
+  const int64_t step = (int64_t)gridDim.x * RQ;
+  for (int64_t v0 = (int64_t)blockIdx.x * RQ + t / Q; v0 < G.n; v0 += kIn * step) {
+    double muF[kIn], muR[kIn], cd[kIn];
+    float F[kIn], V[kIn], mo[kIn], ls[kIn], er[kIn], ge[kIn];
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) {
+      const int64_t v = v0 + u * step;
+      mo[u] = INFINITY;
+      er[u] = ge[u] = 0.f;
+      if (v < G.n_act) {
+        const int64_t o = v * G.Qs + q;
+        mo[u] = G.minCEo[o];
+        ls[u] = G.lsO[o];
+        muF[u] = MU[v * G.P + pdq];
+        muR[u] = MU[v * G.P + psq];
+        F[u] = S.FMaxN[o];
+        V[u] = S.VFm[o];
+        cd[u] = cD[o];
+        er[u] = gER[o];
+        ge[u] = FE.gEF[o];
+      }
     }
-    if (v == s1.vF) gvr += red4[2 * Q + q];
-    if (v == s1.vR) gvf += red4[3 * Q + q];
-    gVR[o] = (float)gvr;
-    gVF[o] = (float)gvf;
-    const float ge = FE.gEF[o];
-    if (ge != 0.f) fmax_edge_term(o, q, G.Qs, ge, FE.FA, FE.bsrc, FE.brows, FE.gCE, FE.gVRfix, fscale);
+#pragma unroll
+    for (int u = 0; u < kIn; ++u) {
+      const int64_t v = v0 + u * step;
+      if (v >= G.n) break;
+      const int64_t o = v * G.Qs + q;
+      double gvr = 0.0, gvf = (double)er[u];
+      if (mo[u] != INFINITY) {
+        const double VF = muF[u] - fmax(s0.fillF, (double)F[u]);
+        const double VR = muR[u] - fmax(s0.fillR, V[u] == -INFINITY ? -kInf : ((double)V[u] - s0.mRE) - s0.lRE);
+        const double eF = exp(VR - lF), eR = exp(VF - lR);
+        const double wo = exp((double)ls[u] - (double)mo[u]);
+        gvr -= SF * eF * wo;
+        gvf -= SR * eR * wo;
+        cD[o] = cd[u] + (SF * eF + SR * eR);
+      }
+      if (v == s1.vF) gvr += gfF;
+      if (v == s1.vR) gvf += gfR;
+      gVR[o] = (float)gvr;
+      gVF[o] = (float)gvf;
+      if (ge[u] != 0.f) fmax_edge_term(o, q, G.Qs, ge[u], FE.FA, FE.bsrc, FE.brows, FE.gCE, FE.gVRfix, fscale);
+    }
   }
 }
 
 // The vertex side of a step back, one tile of T vertices per block iteration:
 //   1. gVR[v][q] += gVRfix[v][q] 2^-k, the fixed-point sums of the step's FMax edge terms (where nonzero; the
-//      accumulator is cleared for the next step), staged with gVF in LDS;
-//   2. gMU[v][p] = sum over the incidences of p (ascending q) of gVF (q ends at p) or gVR (q starts at p);
-//   3. per-block partial column sums of gMU in FP64, vertices in order: part[p][b].
+//      accumulator is cleared for the next step), staged with gVF in LDS, four pattern edges to a thread;
+//   2. gMU[v][p] = sum over the incidences of p (ascending q) of gVF (q ends at p) or gVR (q starts at p), and the thread's
+//      (fixed p) part of the column sum of gMU, in FP64;
+//   3. per-block partial column sums: part[p][b].
 // The input state's FMax / RMax gradients are -gVF / -gVR, which k_bwd_route of the next step back reads directly.
+// Bound by its streams: R-MAT 18 with 12/16 in 22.4 us (26.7 with single values staged and a column's sum left to one
+// thread); by its tiles' latency on small graphs, hence
+// short ones there (1,000 vertices, 10/12: 7.1 -> 3.8 us).
 __global__ __launch_bounds__(256) void k_bwd_vtx(BwdGraph G, float* __restrict__ gVR, const float* __restrict__ gVF,
                                                  unsigned long long* __restrict__ gVRfix,
                                                  const unsigned* __restrict__ gmax, float* __restrict__ gMU,
                                                  double* __restrict__ part, int T) {
-  extern __shared__ float vsh[];  // [T][Qs] gVR, [T][Qs] gVF, [T][P] gMU, then the incidence lists
+  typedef unsigned long long u4v __attribute__((ext_vector_type(4)));
+  extern __shared__ float vsh[];  // [T][Qs] gVR, [T][Qs] gVF, then the incidence lists
+  __shared__ double cs[256];
   const int Qs = G.Qs, P = G.P, t = threadIdx.x;
   float* tR = vsh;
   float* tF = tR + T * Qs;
-  float* tM = tF + T * Qs;
-  int* ioff = reinterpret_cast<int*>(tM + T * P);
+  int* ioff = reinterpret_cast<int*>(tF + T * Qs);
   int* iinc = ioff + (P + 1);
   const int ninc = G.inc_off[P];
   for (int k = t; k <= P; k += 256) ioff[k] = G.inc_off[k];
   for (int k = t; k < ninc; k += 256) iinc[k] = G.inc[k];
   const double inv = ldexp(1.0, -fix_exponent(*gmax, G.fix_shift));
-  double col = 0.0;  // thread t < P: this block's partial sum of column t
-  __syncthreads();
+  const int64_t act4 = G.n_act * Qs / 4;  // isolated vertices are no edge's source
+  const int RP = 256 / P, p = t % P, rp = t / P;
+  double col = 0.0;
   for (int64_t v0 = (int64_t)blockIdx.x * T; v0 < G.n; v0 += (int64_t)gridDim.x * T) {
     const int nv = (int)min((int64_t)T, G.n - v0);
-    for (int e = t; e < nv * Qs; e += 256) {
-      const int64_t o = v0 * Qs + e;
-      float r = gVR[o];
-      const long long f = (long long)gVRfix[o];
-      if (f != 0) {
-        r = (float)((double)r + (double)f * inv);
-        gVR[o] = r;
-        gVRfix[o] = 0ull;
+    __syncthreads();  // the lists are written (first tile) / the last tile is read
+    for (int e = t; e < nv * Qs / 4; e += 256) {
+      const int64_t o = v0 * Qs / 4 + e;
+      f4v r = reinterpret_cast<const f4v*>(gVR)[o];
+      u4v f = {0, 0, 0, 0};
+      if (o < act4) f = reinterpret_cast<const u4v*>(gVRfix)[o];
+      reinterpret_cast<f4v*>(tF)[e] = reinterpret_cast<const f4v*>(gVF)[o];
+      if ((f[0] | f[1] | f[2] | f[3]) != 0) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (f[u] != 0) r[u] = (float)((double)r[u] + (double)(long long)f[u] * inv);
+        reinterpret_cast<f4v*>(gVR)[o] = r;
+        reinterpret_cast<u4v*>(gVRfix)[o] = u4v{0, 0, 0, 0};
       }
-      tR[e] = r;
-      tF[e] = gVF[o];
+      reinterpret_cast<f4v*>(tR)[e] = r;
     }
     __syncthreads();
-    for (int e = t; e < nv * P; e += 256) {
-      const int vl = e / P, p = e - vl * P;
-      float a = 0.f;
-      for (int k = ioff[p]; k < ioff[p + 1]; ++k) {
-        const int code = iinc[k];
-        a += (code & 1) ? tR[vl * Qs + (code >> 1)] : tF[vl * Qs + (code >> 1)];
+    if (rp < RP)
+      for (int vl = rp; vl < nv; vl += RP) {
+        float a = 0.f;
+        for (int k = ioff[p]; k < ioff[p + 1]; ++k) {
+          const int code = iinc[k];
+          a += (code & 1) ? tR[vl * Qs + (code >> 1)] : tF[vl * Qs + (code >> 1)];
+        }
+        gMU[(v0 + vl) * P + p] = a;
+        col += (double)a;
       }
-      tM[e] = a;
-      gMU[v0 * P + e] = a;
-    }
-    __syncthreads();
-    if (t < P)
-      for (int vl = 0; vl < nv; ++vl) col += (double)tM[vl * P + t];
   }
-  if (t < P) part[(int64_t)t * gridDim.x + blockIdx.x] = col;
+  cs[t] = col;
+  __syncthreads();
+  if (t < P) {
+    for (int r = 1; r < RP; ++r) col += cs[r * P + t];
+    part[(int64_t)t * gridDim.x + blockIdx.x] = col;
+  }
 }
 
 // Fill subgradients of the prep state go to the argmax of MU0 = LSM(-CV) of the source / destination pattern vertex:
@@ -587,19 +626,26 @@ void launch_bwd_out(const BwdGraph& G, const double* MU, const double* colsum, f
   hipLaunchKernelGGL(k_bwd_out, dim3(grid_for(G.n * G.P)), dim3(256), 0, st, G.n * G.P, G.P, MU, colsum, gMU, gCV);
 }
 
-void launch_bwd_route(const BwdGraph& G, const BwdState& S, const float* gZ, int with_gz, const float* gVF,
-                      const float* gVR, float* gEF, float* gER, unsigned* gmax, float* gERsum, double* part,
-                      int nparts, double* red4, hipStream_t st) {
-  if (G.Q == 0) return;
-  hipLaunchKernelGGL(k_bwd_route, dim3(nparts), dim3(256), 0, st, G, S, gZ, with_gz, gVF, gVR, gEF, gER, gmax, gERsum,
-                     part);
+void launch_bwd_route(const BwdGraph& G, const BwdState& S, const double* MU, const double* colsum, float* gMU,
+                      float* gCV, const float* gVF, const float* gVR, float* gEF, float* gER, unsigned* gmax,
+                      float* gERsum, double* part, int nparts, double* red4, hipStream_t st) {
+  if (G.Q == 0) {
+    if (MU) launch_bwd_out(G, MU, colsum, gMU, gCV, st);
+    return;
+  }
+  // Rows per tile: every block has one, as far as LDS holds it.
+  const int T = (int)std::min<int64_t>(std::max<int64_t>(16, (G.n + nparts - 1) / nparts), kRouteTile / G.P);
+  hipLaunchKernelGGL(MU ? k_bwd_route<true> : k_bwd_route<false>, dim3(nparts), dim3(256), 0, st, G, S, MU, colsum, gMU,
+                     gCV, gVF, gVR, gEF, gER, gmax, gERsum, part, T);
   launch_sum_parts(nparts, 4 * G.Q, part, red4, true, st);
 }
 
 void launch_bwd_in(const BwdGraph& G, const BwdState& S, const double* MU, const QStat* qs1, const double* red4,
                    const float* gER, float* gVR, float* gVF, double* cD, const FmaxTerms& FE, hipStream_t st) {
   if (G.Q == 0) return;
-  hipLaunchKernelGGL(k_bwd_in, dim3(grid_for(G.n * G.Q)), dim3(256), 0, st, G, S, MU, qs1, red4, gER, gVR, gVF, cD, FE);
+  const int64_t rows = kIn * (256 / G.Q);
+  const int nb = (int)std::min<int64_t>((G.n + rows - 1) / rows, 1024);  // resident at once: the prologue is paid once
+  hipLaunchKernelGGL(k_bwd_in, dim3(nb), dim3(256), 0, st, G, S, MU, qs1, red4, gER, gVR, gVF, cD, FE);
 }
 
 void launch_bwd_fscatter(const BwdGraph& G, const float* gEF, const int* FA, const int* bsrc, int64_t brows,
@@ -634,7 +680,10 @@ void launch_bwd_rterms(const BwdGraph& G, const float* gERsum, const int* AO, in
                      G.n, G.Q, G.Qs, gERsum, AO, brows, gCE);
 }
 
-int bwd_vtx_tile(const BwdGraph& G) { return std::max(1, std::min(64, 8192 / std::max(1, 2 * G.Qs + G.P))); }
+// Vertices per tile: as LDS holds (32 KB of rows), 64 at most, and fewer where that leaves CUs idle.
+static int bwd_vtx_tile(const BwdGraph& G) {
+  return (int)std::min<int64_t>(std::min(64, 4096 / std::max(1, G.Qs)), std::max<int64_t>(16, (G.n + 1023) / 1024));
+}
 
 int bwd_vtx_blocks(const BwdGraph& G) {
   const int T = bwd_vtx_tile(G);
@@ -644,7 +693,7 @@ int bwd_vtx_blocks(const BwdGraph& G) {
 void launch_bwd_vtx(const BwdGraph& G, float* gVR, const float* gVF, unsigned long long* gVRfix, const unsigned* gmax,
                     float* gMU, double* part, hipStream_t st) {
   const int T = bwd_vtx_tile(G), nb = bwd_vtx_blocks(G);
-  const size_t lds = (size_t)T * (2 * G.Qs + G.P) * sizeof(float) + (size_t)(G.P + 1 + 2 * G.Q) * sizeof(int);
+  const size_t lds = (size_t)T * 2 * G.Qs * sizeof(float) + (size_t)(G.P + 1 + 2 * G.Q) * sizeof(int);
   hipLaunchKernelGGL(k_bwd_vtx, dim3(nb), dim3(256), lds, st, G, gVR, gVF, gVRfix, gmax, gMU, part, T);
 }
 

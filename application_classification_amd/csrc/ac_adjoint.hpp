@@ -11,7 +11,7 @@ namespace ac {
 
 // The fixed inputs of the vertex side: costs, out-edge statistics and the pattern's incidence lists.
 struct BwdGraph {
-  int64_t n;
+  int64_t n, n_act;  // the vertices; those before the isolated ones
   int P, Q, Qs;
   const float* CV;      // [n][P]
   const float* minCEo;  // [n][Qs]
@@ -49,11 +49,12 @@ struct FmaxTerms {
 };
 
 // gVF / gVR: those of the next state (the previous step back; zeros at the first), whose negations are this state's
-// FMax / RMax gradients.  gmax (nullable, zero before): receives the largest |gE_F|; gERsum (nullable) accumulates
-// gE_R over the steps.
-void launch_bwd_route(const BwdGraph& G, const BwdState& S, const float* gZ, int with_gz, const float* gVF,
-                      const float* gVR, float* gEF, float* gER, unsigned* gmax, float* gERsum, double* part,
-                      int nparts, double* red4, hipStream_t st);
+// FMax / RMax gradients.  gmax (nullable, zero before): receives the largest |gE_F|; gERsum accumulates gE_R over the
+// steps.
+// MU (nullable; of the state S) with colsum: launch_bwd_out's step first, fused (gMU is left as it was where Q > 0).
+void launch_bwd_route(const BwdGraph& G, const BwdState& S, const double* MU, const double* colsum, float* gMU,
+                      float* gCV, const float* gVF, const float* gVR, float* gEF, float* gER, unsigned* gmax,
+                      float* gERsum, double* part, int nparts, double* red4, hipStream_t st);
 // Also the step's FMax edge terms FE.
 void launch_bwd_in(const BwdGraph& G, const BwdState& S, const double* MU, const QStat* qs1, const double* red4,
                    const float* gER, float* gVR, float* gVF, double* cD, const FmaxTerms& FE, hipStream_t st);

@@ -2004,7 +2004,7 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
   const int P = ctx->P, Q = ctx->Q, Qs = ctx->Qs, K = ctx->tape_K, n_iter = ctx->tape_iters;
   const int Q1 = std::max(1, Q);
   const size_t nq = (size_t)n * Qs, np = (size_t)n * P;
-  const int nparts = (int)std::max<int64_t>(1, std::min<int64_t>((n + 63) / 64, 2048));
+  const int nparts = (int)std::max<int64_t>(1, std::min<int64_t>((n + 15) / 16, 2048));
   const int64_t brows = ctx->bs->brows;
   // grad_mu is in the caller's vertex order; the adjoint works in the internal one.
   HIPCHK(ctx, ctx->gMUin.alloc(np));
@@ -2049,7 +2049,7 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
 
   int fix_shift = 0;
   while (((int64_t)1 << (23 + fix_shift)) < ctx->max_outdeg) ++fix_shift;
-  ac::BwdGraph G{n, P, Q, Qs, ctx->CV.p, ctx->minCEo.p, ctx->lsO.p, ctx->d_ps.p, ctx->d_pd.p, ctx->d_inc_off.p,
+  ac::BwdGraph G{n, ctx->n_act, P, Q, Qs, ctx->CV.p, ctx->minCEo.p, ctx->lsO.p, ctx->d_ps.p, ctx->d_pd.p, ctx->d_inc_off.p,
                  ctx->d_inc.p, fix_shift};
   HIPCHK(ctx, ctx->vpart.alloc((size_t)ac::bwd_vtx_blocks(G) * std::max(1, P)));
   // Segment states: state 0 is the checkpoint itself, states 1..K live in the segment buffers, whose constant rows
@@ -2089,10 +2089,9 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
         ac::launch_sum_parts(ac::bwd_vtx_blocks(G), P, ctx->vpart.p, ctx->colsum.p, true, st);
       else
         ac::launch_colsum(n, P, ctx->gMU.p, ctx->bpart.p, nparts, ctx->colsum.p, st);
-      ac::launch_bwd_out(G, ctx->MUd.p, ctx->colsum.p, ctx->gMU.p, ctx->gCV.p, st);
       unsigned* gmax = ctx->gmax.p + i;
-      ac::launch_bwd_route(G, S1, ctx->gMU.p, 1, ctx->gVF.p, ctx->gVR.p, ctx->gEF.p, ctx->gER.p, gmax, ctx->gERsum.p,
-                           ctx->bpart.p, nparts, ctx->red4.p, st);
+      ac::launch_bwd_route(G, S1, ctx->MUd.p, ctx->colsum.p, ctx->gMU.p, ctx->gCV.p, ctx->gVF.p, ctx->gVR.p, ctx->gEF.p,
+                           ctx->gER.p, gmax, ctx->gERsum.p, ctx->bpart.p, nparts, ctx->red4.p, st);
       launch_mu(ctx, S0, st);  // MU of the input state, reused by the next step back
       have_mu = true;
       if (Q == 0) HIPCHK(ctx, hipMemsetAsync(ctx->gVR.p, 0, nq * sizeof(float), st));
@@ -2108,7 +2107,7 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
   const ac::BwdState S0{ctx->ckF.p, ctx->ckV.p, ctx->ckQ.p, ctx->ckP.p, 1};
   std::vector<double> cq(Q1, 0.0);
   if (Q > 0) {
-    ac::launch_bwd_route(G, S0, nullptr, 0, ctx->gVF.p, ctx->gVR.p, ctx->gEF.p, ctx->gER.p, nullptr, ctx->gERsum.p,
+    ac::launch_bwd_route(G, S0, nullptr, nullptr, nullptr, nullptr, ctx->gVF.p, ctx->gVR.p, ctx->gEF.p, ctx->gER.p, nullptr, ctx->gERsum.p,
                          ctx->bpart.p, nparts, ctx->red4.p, st);
     ac::launch_bwd_fscatter(G, ctx->gEF.p, ctx->FA0.p, ctx->bs->bsrc.p, brows, ctx->gCE.p, st);
     ac::launch_bwd_rterms(G, ctx->gERsum.p, ctx->AO.p, brows, ctx->gCE.p, st);

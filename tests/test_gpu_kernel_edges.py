@@ -7,6 +7,7 @@ from application_classification_amd import workloads as W
 from application_classification_amd.matcher import AC_OPT_PRUNE, AC_OPT_TAPE, Matcher
 from oracle import oracle as O
 from tests.conftest import allclose_report
+from tests.test_gpu_adjoint import check_grad, fd_grad, gpu_grad, weights
 
 pytestmark = pytest.mark.gpu
 
@@ -150,3 +151,18 @@ def test_hub_pieces(pe, pieces, monkeypatch):
         bad, ratio = allclose_report(got[-1], expect)
         assert bad == 0, (tape, ratio)
     np.testing.assert_array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("n,m,pn,pe,K", [
+    (300, 900, 3, 200, 1), (2000, 500, 40, 1, 2), (1100, 3000, 256, 5, 1),  # many pattern edges, isolated vertices, many columns
+    (5, 9, 1, 1, 1), (17_000, 30_000, 7, 9, 3),                           # less than a tile; more tiles than 16 rows cover
+])
+def test_gradient_tiles(n, m, pn, pe, K):
+    """The adjoint's vertex kernels over their tiles and lane groups, against finite differences of the oracle."""
+    data = random_graph(n, m, 3, 3, n)
+    patt = random_graph(pn, pe, 3, 3, pn + pe)
+    patt.vmap = np.random.default_rng(pe).integers(0, n, pn)
+    wv, we = weights(2, 3, 3)
+    _, gv, ge = gpu_grad(data, patt, wv, we, 3, K=K)
+    fv, fe = fd_grad(g64(data), g64(patt), patt.vmap, wv.copy(), we.copy(), 3)
+    check_grad(np.concatenate([gv, ge]), np.concatenate([fv, fe]), f"dn={n} de={m} pn={pn} pe={pe}")
