@@ -461,14 +461,14 @@ __global__ void k_bwd_vertex_coef(int64_t total, const float* __restrict__ CV, f
 }
 
 // Outer-product sums over rows, for q < K, k < dim:  A[q][k] = sum_r G[r][q] x_r[k]^2,  B[q][k] = sum_r G[r][q]
-// x_r[k],  C[q] = sum_r G[r][q],  x_r = feats[idx ? idx[r] : r] (rows with idx < 0 skipped), one block partial each.
+// x_r[k],  C[q] = sum_r G[r][q],  x_r = feats[idx[r]] (rows with idx < 0 skipped), one block partial each.
 // For the (q, k) block [q0, q0 + 16 NQT) x [k0, k0 + 16 NKT) they are GEMMs over the rows on FP64 matrix cores
 // (v_mfma_f64_16x16x4f64, four rows per step).  A-operand lane
 // i + 16k holds G[row k][q0 + i], B-operand lane j + 16k holds x[row k][k0 + j] (or its square), and D[4r +
 // lane/16][lane%16] sits in register r.  Products of floats are exact in FP64; the sums are FP64.  The block's four
 // waves are summed in order.
 typedef double d4v __attribute__((ext_vector_type(4)));
-template <int NQT, int NKT, bool kIdx>
+template <int NQT, int NKT>
 __global__ __launch_bounds__(256) void k_outer_mfma(int64_t nrows, const int* __restrict__ idx,
                                                     const float* __restrict__ feats, int dim,
                                                     const float* __restrict__ G, int Gs, int K, int q0, int k0,
@@ -497,12 +497,12 @@ __global__ __launch_bounds__(256) void k_outer_mfma(int64_t nrows, const int* __
 #pragma unroll
     for (int h = 0; h < kOS; ++h) {
       const int64_t row = r0 + 4 * h + kr;
-      sv[h] = kIdx ? idx[row < nrows ? row : nrows - 1] : 0;
+      sv[h] = idx[row < nrows ? row : nrows - 1];
     }
   };
   auto src_of = [&](int64_t r0, int h, int raw) -> int64_t {
     const int64_t row = r0 + 4 * h + kr;
-    return row < nrows ? (kIdx ? (int64_t)raw : row) : -1;
+    return row < nrows ? (int64_t)raw : -1;
   };
   auto load = [&](int64_t r0) {
 #pragma unroll
@@ -545,7 +545,7 @@ __global__ __launch_bounds__(256) void k_outer_mfma(int64_t nrows, const int* __
 #pragma unroll
     for (int h = 0; h < kOS; ++h) {
       int raw = sid[h];
-      if (kIdx) asm volatile("" : "+v"(raw));  // an empty register barrier: the id is first needed here
+      asm volatile("" : "+v"(raw));  // an empty register barrier: the id is first needed here
       srcl[h] = src_of(r0 + stride, h, raw);
     }
     load(r0 + stride);
@@ -720,15 +720,25 @@ void launch_bwd_vertex_coef(int64_t total, const float* CV, float* G, hipStream_
 
 void launch_outer_acc(int64_t nrows, const int* idx, const float* feats, int dim, const float* G, int Gs, int K,
                       double* part, int nparts, hipStream_t st) {
-  // Matrix-core path in (q, k) blocks of 32 x 32 (each block of the grid covers every row once per launch).
-  for (int q0 = 0; q0 < K; q0 += 32)
-    for (int k0 = 0; k0 < dim; k0 += 32)
-      if (idx)
-        hipLaunchKernelGGL((k_outer_mfma<2, 2, true>), dim3(nparts), dim3(256), 0, st, nrows, idx, feats, dim, G, Gs,
-                           K, q0, k0, part);
+  // Blocks of at most 32 pattern columns, each covering every row once per launch: 32 features wide, or, where 16 columns
+  // are left (half the products of a 32-column block would be padding), up to 64, so that G is read once for them.  Bound by
+  // the products and the gathered rows: vertices and edges of a training step at R-MAT 18 (12/16, 32 features), 251 us
+  // together, 398 in 32-column blocks.  (The edges' coefficients formed in here instead of by k_bwd_edge_coef: 397 against
+  // 230 and 184 us, their FP64 exponentials waiting at this kernel's low occupancy.)
+  auto launch = [&](auto kernel, int q0, int k0) {
+    hipLaunchKernelGGL(kernel, dim3(nparts), dim3(256), 0, st, nrows, idx, feats, dim, G, Gs, K, q0, k0, part);
+  };
+  for (int q0 = 0; q0 < K; q0 += 32) {
+    const bool narrow = K - q0 <= 16;
+    for (int k0 = 0, w; k0 < dim; k0 += w) {
+      const int left = dim - k0;
+      w = left <= 16 ? 16 : left <= 32 || !narrow ? 32 : 64;
+      if (narrow)
+        launch(w == 16 ? k_outer_mfma<1, 1> : w == 32 ? k_outer_mfma<1, 2> : k_outer_mfma<1, 4>, q0, k0);
       else
-        hipLaunchKernelGGL((k_outer_mfma<2, 2, false>), dim3(nparts), dim3(256), 0, st, nrows, idx, feats, dim, G,
-                           Gs, K, q0, k0, part);
+        launch(w == 16 ? k_outer_mfma<2, 1> : k_outer_mfma<2, 2>, q0, k0);
+    }
+  }
 }
 
 }  // namespace ac

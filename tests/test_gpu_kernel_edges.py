@@ -153,16 +153,17 @@ def test_hub_pieces(pe, pieces, monkeypatch):
     np.testing.assert_array_equal(got[0], got[1])
 
 
-@pytest.mark.parametrize("n,m,pn,pe,K", [
-    (300, 900, 3, 200, 1), (2000, 500, 40, 1, 2), (1100, 3000, 256, 5, 1),  # many pattern edges, isolated vertices, many columns
-    (5, 9, 1, 1, 1), (17_000, 30_000, 7, 9, 3),                           # less than a tile; more tiles than 16 rows cover
+@pytest.mark.parametrize("n,m,pn,pe,K,dim", [
+    (300, 900, 3, 200, 1, 3), (2000, 500, 40, 1, 2, 3), (1100, 3000, 256, 5, 1, 3),  # edges, isolated vertices, columns
+    (5, 9, 1, 1, 1, 3), (17_000, 30_000, 7, 9, 3, 3),                 # less than a tile; more than 16 rows a block
+    (400, 900, 16, 17, 1, 17), (400, 900, 33, 48, 1, 33), (400, 900, 49, 16, 1, 65),  # blocks of columns and features
 ])
-def test_gradient_tiles(n, m, pn, pe, K):
-    """The adjoint's vertex kernels over their tiles and lane groups, against finite differences of the oracle."""
-    data = random_graph(n, m, 3, 3, n)
-    patt = random_graph(pn, pe, 3, 3, pn + pe)
+def test_gradient_tiles(n, m, pn, pe, K, dim):
+    """The adjoint's kernels over their tiles and lane groups, against finite differences of the oracle."""
+    data = random_graph(n, m, dim, dim, n)
+    patt = random_graph(pn, pe, dim, dim, pn + pe)
     patt.vmap = np.random.default_rng(pe).integers(0, n, pn)
-    wv, we = weights(2, 3, 3)
+    wv, we = weights(2, dim, dim)
     _, gv, ge = gpu_grad(data, patt, wv, we, 3, K=K)
     fv, fe = fd_grad(g64(data), g64(patt), patt.vmap, wv.copy(), we.copy(), 3)
-    check_grad(np.concatenate([gv, ge]), np.concatenate([fv, fe]), f"dn={n} de={m} pn={pn} pe={pe}")
+    check_grad(np.concatenate([gv, ge]), np.concatenate([fv, fe]), f"dn={n} de={m} pn={pn} pe={pe} dim={dim}")
