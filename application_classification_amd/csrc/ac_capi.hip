@@ -1105,6 +1105,9 @@ static ac::VertexArgs vertex_args(ac_ctx* ctx) {
   va.VR = ctx->VR.p;
   va.VRs = ctx->VRs;
   va.out = ctx->OUT.p;
+  va.c0 = va.q0 = 0;
+  va.ncol = ctx->P;
+  va.nq = ctx->Q;
   va.ps = ctx->d_ps.p;
   va.pd = ctx->d_pd.p;
   va.inc_off = ctx->d_inc_off.p;
@@ -1156,21 +1159,30 @@ static int enqueue_iteration(ac_ctx* ctx, ac::VertexArgs& va, int it, const QSta
   return AC_OK;
 }
 
-// Output of the current state (src/main.cu:247): MU[v][p] written directly in dn x pn order into OUT.
-static int enqueue_output(ac_ctx* ctx, ac::VertexArgs& va, int done, const QStat* qs_state) {
+// The output columns [c0, c0 + ncol), those of the pattern edges [q0, q0 + nq), after `t` iterations into dst[dn][ncol].
+struct Snapshot {
+  int t, c0, ncol, q0, nq;
+  float* dst;
+};
+
+// Output of the current state (src/main.cu:247): MU[v][p] written directly in dn x pn order into OUT, or S's columns into
+// S's rows (a batch's pattern: the whole slab's columns, then a copy of the pattern's, took 48 us a pattern at R-MAT
+// 16 with 32 of them, now 32).
+static int enqueue_output(ac_ctx* ctx, ac::VertexArgs& va, int done, const QStat* qs_state, const Snapshot* S = nullptr) {
   ac::VertexArgs vo = va;
   vo.n = ctx->dn;  // every row, isolated ones included, written to the caller's row
   vo.first = done == 0;
   vo.qs = qs_state;
+  if (S) {
+    vo.c0 = S->c0;
+    vo.ncol = S->ncol;
+    vo.q0 = S->q0;
+    vo.nq = S->nq;
+    vo.out = S->dst;
+  }
   ac::launch_vertex(ac::kModeOut, vo, ctx->nb_vertex_o, ctx->stream);
   return AC_OK;
 }
-
-// A copy of the output columns [c0, c0 + ncol) taken after `t` iterations into dst[dn][ncol].
-struct Snapshot {
-  int t, c0, ncol;
-  float* dst;
-};
 
 // Captured iteration pairs of one loop: one per parity of the pair's first iteration, because iteration `it`
 // reads the scalar slot that iteration it - 1 wrote (slot 1 + ((it - 1) & 1)) and writes slot 1 + (it & 1), and a
@@ -1208,10 +1220,8 @@ static int enqueue_loop(ac_ctx* ctx, int n_iter, const std::vector<Snapshot>& sn
   size_t si = 0;
   auto take = [&](int t) -> int {
     while (si < snaps.size() && snaps[si].t == t) {
-      const Snapshot& S = snaps[si++];
-      int rc = enqueue_output(ctx, va, t, qs_state);
+      const int rc = enqueue_output(ctx, va, t, qs_state, &snaps[si++]);
       if (rc != AC_OK) return rc;
-      ac::launch_copy_cols(ctx->dn, ctx->P, S.c0, S.ncol, ctx->OUT.p, S.dst, st);
     }
     return AC_OK;
   };
@@ -1743,7 +1753,7 @@ extern "C" int ac_batch_run(ac_ctx* ctx, const int32_t* n_iter) {
     int n_max = 0, sq = 0;
     for (size_t j = 0; j < members.size(); ++j) {
       const auto& B = ctx->bp[members[j]];
-      snaps.push_back(Snapshot{iters[members[j]], col0[j], B.P, ctx->bout.p + B.out_off});
+      snaps.push_back(Snapshot{iters[members[j]], col0[j], B.P, sq, B.Q, ctx->bout.p + B.out_off});
       n_max = std::max(n_max, iters[members[j]]);
       sq += B.Q;
       upd += ctx->de * B.Q * iters[members[j]];

@@ -96,7 +96,8 @@ struct VertexArgs {
   const float* lsO;     // [n][Qs] log1p(sum over other out-edges of exp(min - cost))
   float* VR;            // [n][VRs]
   int VRs;              // row stride of VR: a power of two up to 32 floats, else a multiple of 32 (whole lines)
-  float* out;           // [n][P]
+  float* out;           // mode OUT: [n][ncol], the columns [c0, c0 + ncol), whose pattern edges are [q0, q0 + nq)
+  int c0, ncol, q0, nq;
   double* mu_out;       // mode MU: [n][P] in internal vertex order
   const int* perm;      // mode OUT: internal row -> caller's row of `out` (nullptr: identity)
   // Constant rows, not read by mode A: rows >= f_end have no in-edge (FMaxN = -inf); rows in [o_lo, o_hi) and
@@ -169,7 +170,6 @@ void launch_vertex(int mode, const VertexArgs& a, int nblocks, hipStream_t st);
 int vertex_resident_blocks(int mode, const VertexArgs& a);
 // out[i][c] = in[perm[i]][c] for the n rows of ncol floats.
 void launch_gather_rows(int64_t n, int ncol, const int* perm, const float* in, float* out, hipStream_t st);
-void launch_copy_cols(int64_t n, int P, int c0, int ncol, const float* src, float* dst, hipStream_t st);
 int walk_blocks(int64_t nruns, int Qs);
 int walk_groups(int Qs);  // runs per bundle: 64 / (Qs / 4)
 int walk_batch();         // default steps per batch of the bundle walk: 1, 2 or 4 (bundle lengths are multiples of it)

@@ -1829,9 +1829,24 @@ __global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void
   const int64_t L4q = Qs / 4, f_end4 = a.f_end * L4q, o_lo4 = a.o_lo * L4q, o_hi4 = a.o_hi * L4q,
                 o_end4 = a.o_end * L4q;
   typedef f4v PfSet[4][kPF4];  // FMaxN, VFm (and in pass A minCEo, lsO)
-  PfSet pf;
-  float pc[kPFC];
+  PfSet pf = {};
+  float pc[kPFC] = {};
   int pp = 0;  // mode OUT: the caller id of tile row t
+  // Mode OUT of some columns: what they need of a row, the same in every tile (bit k: quadruple k; kPF4 + k: CV value k).
+  unsigned need = ~0u;
+  if (kMode == kModeOut && a.ncol < P) {
+    need = 0u;
+#pragma unroll
+    for (int k = 0; k < kPF4; ++k) {
+      const int col = 4 * (t + k * NT) % Qs;
+      if (col + 4 > a.q0 && col < a.q0 + a.nq) need |= 1u << k;
+    }
+#pragma unroll
+    for (int k = 0; k < kPFC; ++k) {
+      const int col = (t + k * NT) % P;
+      if (col >= a.c0 && col < a.c0 + a.ncol) need |= 1u << (kPF4 + k);
+    }
+  }
   // Loads of a tile into the register set; indexes past the tile are clamped to its last element (loaded, never
   // used).
   auto prefetch = [&](int64_t tl) __attribute__((always_inline)) {
@@ -1841,6 +1856,7 @@ __global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void
     const int64_t b4_ = v0_ * Qs / 4, bc_ = v0_ * P;
 #pragma unroll
     for (int k = 0; k < kPF4; ++k) {
+      if (kMode == kModeOut && !(need >> k & 1u)) continue;
       const int64_t g_ = b4_ + min(t + k * NT, last4_);
       const bool hasF_ = !kA || g_ < f_end4, hasO_ = !kA || g_ < o_lo4 || (g_ >= o_hi4 && g_ < o_end4);
       pf[0][k] = hasF_ ? F4[g_] : f4v{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
@@ -1851,7 +1867,8 @@ __global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void
       }
     }
 #pragma unroll
-    for (int k = 0; k < kPFC; ++k) pc[k] = a.CV[bc_ + min(t + k * NT, lastc_)];
+    for (int k = 0; k < kPFC; ++k)
+      if (kMode != kModeOut || (need >> (kPF4 + k) & 1u)) pc[k] = a.CV[bc_ + min(t + k * NT, lastc_)];
     if (kMode == kModeOut && a.perm) pp = a.perm[v0_ + min(t, nv_ - 1)];
   };
   if (!iso_block && blk < ntiles) prefetch(blk);  // in flight while the tables are built
@@ -1958,7 +1975,8 @@ __global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void
     // p-phase.  Tiles of fewer than 64 rows form the sums in two steps, so that a pattern vertex with many incidences
     // (a hub) is spread over the block: kTerms incidences per lane, then the partial sums in order.
     if (!kFull && sums) {
-      for (int v = pfirst; v < nsum; v += psweep)
+      const int v1 = kMode == kModeOut ? soff[a.c0 + a.ncol] : nsum;
+      for (int v = (kMode == kModeOut ? soff[a.c0] : 0) + pfirst; v < v1; v += psweep)
         if (prow < nv) {
           const int2 ks = tasks[v];
           IncRec rc[kTerms];
@@ -2015,18 +2033,20 @@ __global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void
         if (p < P) lse_add(pacc[pi], prow < nv ? mu_pre(p) : -kInf);
       }
     } else {
-      for (int p = pfirst; p < P; p += psweep)
+      const int p1 = kMode == kModeOut ? a.c0 + a.ncol : P;
+      for (int p = (kMode == kModeOut ? a.c0 : 0) + pfirst; p < p1; p += psweep)
         if (prow < nv) MUs[prow * ldm + p] = (mu_pre(p) - pmu[p]) - pmu[P + p];
     }
     if (kRows) {
       // The tile's rows go out whole: consecutive threads write consecutive columns of a row.
       __syncthreads();
-      for (int e = t; e < nv * P; e += NT) {
-        const int r = e / P, c = e - r * P;
+      const int w = kMode == kModeOut ? a.ncol : P;
+      for (int e = t; e < nv * w; e += NT) {
+        const int r = e / w, c = e - r * w;
         if (kMode == kModeMU)
           a.mu_out[(v0 + r) * P + c] = MUs[r * ldm + c];
         else
-          a.out[(int64_t)(a.perm ? Prow[r] : v0 + r) * P + c] = (float)MUs[r * ldm + c];
+          a.out[(int64_t)(a.perm ? Prow[r] : v0 + r) * w + c] = (float)MUs[r * ldm + a.c0 + c];
       }
     }
     if (kA) {
@@ -2177,15 +2197,6 @@ int vertex_resident_blocks(int mode, const VertexArgs& a) {
   return e == hipSuccess ? cus * std::max(per, 1) - extra : 0;
 }
 
-// Columns [c0, c0 + ncol) of src[n][P] into dst[n][ncol].
-__global__ void k_copy_cols(int64_t n, int P, int c0, int ncol, const float* __restrict__ src, float* __restrict__ dst) {
-  const int64_t total = n * ncol;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t v = i / ncol;
-    dst[i] = src[v * P + c0 + (int)(i - v * ncol)];
-  }
-}
-
 __global__ void k_gather_rows(int64_t n, int ncol, const int* __restrict__ perm, const float* __restrict__ in,
                               float* __restrict__ out) {
   const int64_t total = n * ncol;
@@ -2199,12 +2210,6 @@ void launch_gather_rows(int64_t n, int ncol, const int* perm, const float* in, f
   if (n * ncol == 0) return;
   const int blocks = (int)std::min<int64_t>((n * ncol + 255) / 256, 1 << 16);
   hipLaunchKernelGGL(k_gather_rows, dim3(blocks), dim3(256), 0, st, n, ncol, perm, in, out);
-}
-
-void launch_copy_cols(int64_t n, int P, int c0, int ncol, const float* src, float* dst, hipStream_t st) {
-  if (n == 0 || ncol == 0) return;
-  const int blocks = (int)std::min<int64_t>((n * ncol + 255) / 256, 1 << 16);
-  hipLaunchKernelGGL(k_copy_cols, dim3(blocks), dim3(256), 0, st, n, P, c0, ncol, src, dst);
 }
 
 }  // namespace ac
