@@ -96,8 +96,8 @@ def cpu_baseline(threads, legs=True):
     return out
 
 
-STAGE_OF_KERNEL = {"k_walk_max<true": "edge_walk", "k_vertex<0>": "vertex_a", "k_vertex<1>": "vertex_c",
-                   "k_vertex<2>": "output", "k_walk_max_fixup": "walk_fixup", "k_reduce_q": "reduce_a",
+STAGE_OF_KERNEL = {"k_walk_max<true": "edge_walk", "k_vertex<0,": "vertex_a", "k_vertex<1,": "vertex_c",
+                   "k_vertex<2,": "output", "k_walk_max_fixup": "walk_fixup", "k_reduce_q": "reduce_a",
                    "k_reduce_lse": "reduce_c"}
 
 
