@@ -314,7 +314,7 @@ struct ac_ctx {
   DevBuf<char> pat;
   Part<double> pf_v, pf_e;
   Part<int> d_ps, d_pd, d_inc_off, d_inc, d_sum_off;
-  Part<int2> d_sums;
+  Part<int2> d_inc_at, d_sums;
   int nsum = 0;  // partial sums of the vertex passes
 
   // Work buffers.
@@ -656,11 +656,12 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
     for (int64_t k = 0; k < dE; ++k) pe[((q / 8) * dE + k) * 8 + q % 8] = ef[q * dE + k];
   // Incidence of each pattern vertex in ascending q: the FMax term (q ends at p) before the RMax term (q starts at p).
   std::vector<int> inc_off(nV + 1, 0), inc;
+  std::vector<int2> inc_at((size_t)std::max<int64_t>(1, nE));
   for (int64_t p = 0; p < nV; ++p) {
     inc_off[p] = (int)inc.size();
     for (int64_t q = 0; q < nE; ++q) {
-      if (dst[q] == p) inc.push_back((int)(q << 1));
-      if (src[q] == p) inc.push_back((int)(q << 1) | 1);
+      if (dst[q] == p) inc_at[q].x = (int)inc.size(), inc.push_back((int)(q << 1));
+      if (src[q] == p) inc_at[q].y = (int)inc.size(), inc.push_back((int)(q << 1) | 1);
     }
   }
   inc_off[nV] = (int)inc.size();
@@ -680,7 +681,7 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
   std::vector<int> sum_off(nV + 1);
   (void)ac::vertex_sums((int)nV, inc_off.data(), sums.data(), sum_off.data());
   const size_t o_v = part(pv), o_e = part(pe), o_s = part(ps_pad), o_d = part(pd_pad), o_o = part(inc_off),
-               o_i = part(inc), o_u = part(sums), o_f = part(sum_off);
+               o_i = part(inc), o_a = part(inc_at), o_u = part(sums), o_f = part(sum_off);
   HIPCHK(ctx, ctx->pat.alloc(all.size()));
   if (ctx->stage.ready()) {
     HIPCHK(ctx, ctx->stage.to_device(ctx->pat.p, all.data(), all.size(), st));
@@ -694,6 +695,7 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
   ctx->d_pd.p = reinterpret_cast<int*>(ctx->pat.p + o_d);
   ctx->d_inc_off.p = reinterpret_cast<int*>(ctx->pat.p + o_o);
   ctx->d_inc.p = reinterpret_cast<int*>(ctx->pat.p + o_i);
+  ctx->d_inc_at.p = reinterpret_cast<int2*>(ctx->pat.p + o_a);
   ctx->d_sums.p = reinterpret_cast<int2*>(ctx->pat.p + o_u);
   ctx->d_sum_off.p = reinterpret_cast<int*>(ctx->pat.p + o_f);
   ctx->nsum = nsum;
@@ -1111,7 +1113,7 @@ static ac::VertexArgs vertex_args(ac_ctx* ctx) {
   va.ps = ctx->d_ps.p;
   va.pd = ctx->d_pd.p;
   va.inc_off = ctx->d_inc_off.p;
-  va.inc = ctx->d_inc.p;
+  va.inc_at = ctx->d_inc_at.p;
   va.sums = ctx->d_sums.p;
   va.sum_off = ctx->d_sum_off.p;
   va.nsum = ctx->nsum;

@@ -108,7 +108,8 @@ struct VertexArgs {
   const int* ps;
   const int* pd;
   const int* inc_off;  // [P + 1]
-  const int* inc;      // incidence of each pattern vertex: (q << 1) | (1 if RMax term else 0), ascending q
+  const int2* inc_at;  // [Q] where the FMax and the RMax term of q stand among the incidences, those of each pattern vertex
+                       // together, in ascending q, the FMax term before the RMax term
   const int2* sums;    // [nsum] incidences [x, y) of each partial sum of the MU sums (vertex_sums)
   const int* sum_off;  // [P + 1]
   int nsum;
