@@ -1682,7 +1682,7 @@ void launch_walk_max_fixup(const SplitList& L, const double* carry, int Q, int Q
 // of its partials.  Hence short tiles where there are few (vertex_tile), lanes shared among pattern vertices, and
 // merges that take one exponential however many partials they merge.  Passes A / C per launch, before (a wave per
 // pattern vertex whatever the tile's height, isolated vertices on block 0's way, serial merges, a term at a time) and
-// now: 1,000 vertices with a 10/12 pattern 20.0 / 8.5 -> 9.0 / 5.3 us; 50,001 with 40/70 48.9 / 44.4 -> 29.2 / 20.0 us;
+// now: 1,000 vertices with a 10/12 pattern 20.0 / 8.5 -> 7.5 / 5.1 us; 50,001 with 40/70 48.9 / 44.4 -> 28.1 / 19.7 us;
 // R-MAT 16 slabs of 128 pattern edges 98.5 / 108.3 -> 50 / 35 us; R-MAT 20 with 16/24 105.7 / 58.9 -> 97 / 42 us.
 
 constexpr int kVTMax = 64;
@@ -2095,41 +2095,45 @@ __global__ __launch_bounds__(NT, kMode == kModeA ? (kPFC == 4 ? 4 : 3) : 4) void
   }
   __syncthreads();
 
-  // Block partials, merged in a fixed order: the maxima first, then every accumulator rescaled to them at once (one
-  // exponential each, in parallel), then the sum.
+  // Block partials, merged in a fixed order: the maxima first (every thread of a column finds them, which saves barriers;
+  // a field's values lie together: 1,000 vertices with 10/12 took 9.4 us with whole partials, 7.5 now; R-MAT 18 27.1, 25.9),
+  // then every accumulator rescaled to them at once (one exponential each, in parallel), then the sums.
   if (kA) {
-    QPart* red = reinterpret_cast<QPart*>(lds);
-    if (qthread) red[rq * Q + q] = QPart{vfmax, vrmax, lre, lfe, avf, avr};
-    __syncthreads();
-    QPart acc{-kInf, -kInf, lse_empty(), lse_empty(), -1, -1};
-    if (t < Q)
-      for (int r = 0; r < RQ; ++r) {
-        const QPart x = red[r * Q + t];
-        argmax_merge(acc.vfmax, acc.avf, x.vfmax, x.avf);
-        argmax_merge(acc.vrmax, acc.avr, x.vrmax, x.avr);
-        acc.re.m = fmax(acc.re.m, x.re.m);
-        acc.fe.m = fmax(acc.fe.m, x.fe.m);
-      }
-    __syncthreads();  // every field of red read
-    double* Mx = lds;                // [2][Q] the maxima
-    double* Ts = Mx + 2 * Q;         // [2][RQ][Q] the rescaled sums
-    if (t < Q) {
-      Mx[t] = acc.re.m;
-      Mx[Q + t] = acc.fe.m;
-    }
-    __syncthreads();
+    double* mre = lds;  // [6][NT]: maxima of RE and FE, max VF, max VR, rescaled sums of RE and FE; then the vertices
+    double *mfe = mre + NT, *xvf = mfe + NT, *xvr = xvf + NT, *tre = xvr + NT, *tfe = tre + NT;
+    int *xaf = reinterpret_cast<int*>(tfe + NT), *xar = xaf + NT;
     if (qthread) {
-      Ts[t] = lse_rescaled(lre, Mx[q]);
-      Ts[RQ * Q + t] = lse_rescaled(lfe, Mx[Q + q]);
+      mre[t] = lre.m, mfe[t] = lfe.m;
+      xvf[t] = vfmax, xvr[t] = vrmax;
+      if (kArgMax) xaf[t] = avf, xar[t] = avr;
     }
     __syncthreads();
-    if (t < Q) {
-      // (each rescaled term counts its own maximum; the overall one is left out again)
-      acc.re.t = acc.fe.t = 0.0;
-      bool ore = false, ofe = false;
+    double Mre = -kInf, Mfe = -kInf;
+    if (qthread) {
+#pragma unroll 4
       for (int r = 0; r < RQ; ++r) {
-        lse_sum_step(acc.re.t, ore, Ts[r * Q + t]);
-        lse_sum_step(acc.fe.t, ofe, Ts[RQ * Q + r * Q + t]);
+        Mre = fmax(Mre, mre[r * Q + q]);
+        Mfe = fmax(Mfe, mfe[r * Q + q]);
+      }
+      tre[t] = lse_rescaled(lre, Mre);
+      tfe[t] = lse_rescaled(lfe, Mfe);
+    }
+    __syncthreads();
+    if (t < Q) {  // (q == t)
+      QPart acc{-kInf, -kInf, Lse{Mre, 0.0}, Lse{Mfe, 0.0}, -1, -1};
+      bool ore = false, ofe = false;
+#pragma unroll 4
+      for (int r = 0; r < RQ; ++r) {
+        const int i = r * Q + t;
+        lse_sum_step(acc.re.t, ore, tre[i]);
+        lse_sum_step(acc.fe.t, ofe, tfe[i]);
+        if (kArgMax) {
+          argmax_merge(acc.vfmax, acc.avf, xvf[i], xaf[i]);
+          argmax_merge(acc.vrmax, acc.avr, xvr[i], xar[i]);
+        } else {
+          acc.vfmax = fmax(acc.vfmax, xvf[i]);
+          acc.vrmax = fmax(acc.vrmax, xvr[i]);
+        }
       }
       a.qpart[t * (G + 1) + blk] = acc;
     }
@@ -2171,7 +2175,7 @@ static VertexKernel vertex_kernel_t(int mode, const VertexArgs& a) {
 static VertexKernel vertex_kernel(int mode, const VertexArgs& a, int* nt, size_t* lds) {
   const size_t tiles = vertex_lds_bytes(mode, a.VT, a.P, a.Q, a.Qs, a.nsum);
   *nt = mode == kModeA ? kNA : kNO;
-  *lds = mode == kModeA ? std::max(tiles, sizeof(QPart) * kNA) : tiles;
+  *lds = mode == kModeA ? std::max(tiles, kNA * (6 * sizeof(double) + 2 * sizeof(int))) : tiles;
   return a.VT == 64 ? vertex_kernel_t<true>(mode, a) : vertex_kernel_t<false>(mode, a);
 }
 
