@@ -69,7 +69,9 @@ void launch_bwd_rterms(const BwdGraph& G, const float* gERsum, const int* AO, in
 int bwd_vtx_blocks(const BwdGraph& G);
 void launch_bwd_vtx(const BwdGraph& G, float* gVR, const float* gVF, unsigned long long* gVRfix, const unsigned* gmax,
                     float* gMU, double* part, hipStream_t st);
-void launch_bwd_prep_fill(const BwdGraph& G, const double* red4, const int* am0, float* gMU, hipStream_t st);
+// Also cq[Q], the prep's part of the edge costs' gradients (qs0: the prep state's scalars).
+void launch_bwd_prep_fill(const BwdGraph& G, const double* red4, const QStat* qs0, const int* am0, float* gMU, double* cq,
+                          hipStream_t st);
 void launch_col_argmin(int64_t n, int P, const float* CV, float* pv, int* pi, int nparts, int* am, hipStream_t st);
 void launch_bwd_edge_coef(int64_t nrows, int Q, int Qs, const int* beid, const int* bsrc, const float* CE,
                           const double* cD, const double* cq, float* G, hipStream_t st);

@@ -1991,7 +1991,7 @@ static void launch_mu(ac_ctx* ctx, const ac::BwdState& S, hipStream_t st) {
 
 // Host side of the weight gradient from the outer-product sums A, B (K x dim) and C (K) and the pattern features
 // pf (K x dim): dL/dw_k = sum_q A[q][k] - 2 pf[q][k] B[q][k] + pf[q][k]^2 C[q].
-static void combine_outer(const std::vector<double>& s, const std::vector<float>& pf, int K, int dim, float* out) {
+static void combine_outer(const double* s, const std::vector<float>& pf, int K, int dim, float* out) {
   for (int k = 0; k < dim; ++k) {
     double g = 0.0;
     for (int q = 0; q < K; ++q) {
@@ -2117,24 +2117,13 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
   // Prep (src/main.cu:107-148): FMax0 / RMax0 from -CE normalised by LSE0 = log sum_e exp(-CE), filled from
   // MU0 = LSM(-CV).
   const ac::BwdState S0{ctx->ckF.p, ctx->ckV.p, ctx->ckQ.p, ctx->ckP.p, 1};
-  std::vector<double> cq(Q1, 0.0);
   if (Q > 0) {
     ac::launch_bwd_route(G, S0, nullptr, nullptr, nullptr, nullptr, ctx->gVF.p, ctx->gVR.p, ctx->gEF.p, ctx->gER.p, nullptr, ctx->gERsum.p,
                          ctx->bpart.p, nparts, ctx->red4.p, st);
     ac::launch_bwd_fscatter(G, ctx->gEF.p, ctx->FA0.p, ctx->bs->bsrc.p, brows, ctx->gCE.p, st);
     ac::launch_bwd_rterms(G, ctx->gERsum.p, ctx->AO.p, brows, ctx->gCE.p, st);
-    ac::launch_bwd_prep_fill(G, ctx->red4.p, ctx->am0.p, ctx->gMU.p, st);
-    std::vector<double> red4((size_t)4 * Q);
-    std::vector<QStat> qs0(Q);
-    HIPCHK(ctx, hipMemcpyAsync(red4.data(), ctx->red4.p, red4.size() * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipMemcpyAsync(qs0.data(), ctx->ckQ.p, Q * sizeof(QStat), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    for (int q = 0; q < Q; ++q) {
-      const double lse0 = qs0[q].mFE + qs0[q].lFE;
-      cq[q] = std::isfinite(lse0) ? (red4[q] + red4[Q + q]) * std::exp(-lse0) : 0.0;
-    }
+    ac::launch_bwd_prep_fill(G, ctx->red4.p, ctx->ckQ.p, ctx->am0.p, ctx->gMU.p, ctx->cq.p, st);
   }
-  HIPCHK(ctx, hipMemcpyAsync(ctx->cq.p, cq.data(), Q1 * sizeof(double), hipMemcpyHostToDevice, st));
   if (!have_mu) launch_mu(ctx, S0, st);
   ac::launch_colsum(n, P, ctx->gMU.p, ctx->bpart.p, nparts, ctx->colsum.p, st);
   ac::launch_bwd_out(G, ctx->MUd.p, ctx->colsum.p, ctx->gMU.p, ctx->gCV.p, st);
@@ -2143,33 +2132,30 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
   ac::launch_bwd_vertex_coef((int64_t)np, ctx->CV.p, ctx->gCV.p, st);
   const int dV = (int)ctx->dV, dE = (int)ctx->dE;
   const int onp = 512;
-  std::vector<float> gwv(dV, 0.f), gwe(dE, 0.f);
-  if (dV > 0) {
-    const size_t w = (size_t)2 * P * dV + P;
-    HIPCHK(ctx, ctx->opart.alloc((size_t)onp * w));
-    HIPCHK(ctx, ctx->osum.alloc(w));
-    ac::launch_outer_acc(n, ctx->d_perm.p, ctx->vfeat.p, dV, ctx->gCV.p, P, P, ctx->opart.p, onp, st);
-    ac::launch_sum_parts(onp, (int)w, ctx->opart.p, ctx->osum.p, false, st);
-    std::vector<double> sv(w);
-    HIPCHK(ctx, hipMemcpyAsync(sv.data(), ctx->osum.p, w * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    combine_outer(sv, ctx->pvfeat, P, dV, gwv.data());
+  const bool edges = dE > 0 && Q > 0 && brows > 0;
+  const size_t wV = dV > 0 ? (size_t)2 * P * dV + P : 0, wE = edges ? (size_t)2 * Q * dE + Q : 0;
+  std::vector<double> sums(wV + wE);  // vertices', then edges'
+  if (wV + wE > 0) {
+    HIPCHK(ctx, ctx->opart.alloc((size_t)onp * std::max(wV, wE)));
+    HIPCHK(ctx, ctx->osum.alloc(wV + wE));
   }
-  if (dE > 0 && Q > 0 && brows > 0) {
+  if (wV > 0) {
+    ac::launch_outer_acc(n, ctx->d_perm.p, ctx->vfeat.p, dV, ctx->gCV.p, P, P, ctx->opart.p, onp, st);
+    ac::launch_sum_parts(onp, (int)wV, ctx->opart.p, ctx->osum.p, false, st);
+  }
+  if (edges) {
     ac::launch_bwd_edge_coef(brows, Q, Qs, ctx->bs->beid.p, ctx->bs->bsrc.p, ctx->CE.p, ctx->cD.p, ctx->cq.p,
                              ctx->gCE.p, st);
-    const size_t w = (size_t)2 * Q * dE + Q;
-    HIPCHK(ctx, ctx->opart.alloc((size_t)onp * w));
-    HIPCHK(ctx, ctx->osum.alloc(w));
     ac::launch_outer_acc(brows, ctx->bs->beid.p, ctx->efeat.p, dE, ctx->gCE.p, Qs, Q, ctx->opart.p, onp, st);
-    ac::launch_sum_parts(onp, (int)w, ctx->opart.p, ctx->osum.p, false, st);
-    std::vector<double> se(w);
-    HIPCHK(ctx, hipMemcpyAsync(se.data(), ctx->osum.p, w * sizeof(double), hipMemcpyDeviceToHost, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-    combine_outer(se, ctx->pefeat, Q, dE, gwe.data());
+    ac::launch_sum_parts(onp, (int)wE, ctx->opart.p, ctx->osum.p + wV, false, st);
   }
   HIPCHK(ctx, hipGetLastError());
+  if (wV + wE > 0)
+    HIPCHK(ctx, hipMemcpyAsync(sums.data(), ctx->osum.p, sums.size() * sizeof(double), hipMemcpyDeviceToHost, st));
   HIPCHK(ctx, hipStreamSynchronize(st));
+  std::vector<float> gwv(dV, 0.f), gwe(dE, 0.f);
+  if (wV > 0) combine_outer(sums.data(), ctx->pvfeat, P, dV, gwv.data());
+  if (wE > 0) combine_outer(sums.data() + wV, ctx->pefeat, Q, dE, gwe.data());
   if (grad_wv) std::copy(gwv.begin(), gwv.end(), grad_wv);
   if (grad_we) std::copy(gwe.begin(), gwe.end(), grad_we);
   return AC_OK;
