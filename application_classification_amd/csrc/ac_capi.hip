@@ -1939,10 +1939,8 @@ static int recompute_iteration(ac_ctx* ctx, int it, const StateBufs& In, const S
 // FMaxN rows of vertices without in-edges and in the VFm rows of vertices without out-edges, which no iteration
 // writes (internal order: both, in-edges only, out-edges only, isolated), as the prep sets them in the live state.
 static void fill_constant_rows(ac_ctx* ctx, float* F, float* V, int nslots, hipStream_t st) {
-  const int64_t Qs = ctx->Qs, nq = ctx->dn * Qs;
   const int64_t in_lo = ctx->n_both, in_hi = ctx->n_both + ctx->n_inonly, iso = ctx->n_act, n = ctx->dn;
-  ac::launch_fill_slots(F, V, nslots, nq, in_hi * Qs, (n - in_hi) * Qs, in_lo * Qs, (in_hi - in_lo) * Qs, iso * Qs,
-                        (n - iso) * Qs, st);
+  ac::launch_fill_slots(F, V, nslots, ctx->Qs, n, in_hi, n - in_hi, in_lo, in_hi - in_lo, iso, n - iso, st);
 }
 
 // The iterations of a run with a checkpoint at every iteration (AC_OPT_TAPE = 1): iteration it reads the state in
@@ -2048,16 +2046,18 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
     HIPCHK(ctx, ctx->sgP.alloc((size_t)(K + 1) * P));
     HIPCHK(ctx, ctx->tapeFA.alloc((size_t)K * nq));
   }
-  HIPCHK(ctx, hipMemsetAsync(ctx->gCV.p, 0, np * sizeof(float), st));
-  // gVF / gVR of the state after the last one: zero (k_bwd_route of the first step back reads their negations).
-  HIPCHK(ctx, hipMemsetAsync(ctx->gVF.p, 0, nq * sizeof(float), st));
-  HIPCHK(ctx, hipMemsetAsync(ctx->gVR.p, 0, nq * sizeof(float), st));
-  HIPCHK(ctx, hipMemsetAsync(ctx->gCE.p, 0, ctx->gCE.n * sizeof(float), st));
-  HIPCHK(ctx, hipMemsetAsync(ctx->cD.p, 0, nq * sizeof(double), st));
-  HIPCHK(ctx, hipMemsetAsync(ctx->gERsum.p, 0, nq * sizeof(float), st));
-  // The fixed-point sums start at zero; the vertex kernel of each step clears the ones it adds.
-  HIPCHK(ctx, hipMemsetAsync(ctx->gVRfix.p, 0, nq * sizeof(unsigned long long), st));
-  HIPCHK(ctx, hipMemsetAsync(ctx->gmax.p, 0, ((size_t)n_iter + 1) * sizeof(unsigned), st));
+  // What starts at zero: the gradients that are added to; gVF / gVR of the state after the last one (k_bwd_route of the first
+  // step back reads their negations); the fixed-point sums (the vertex kernel of each step clears the ones it adds).
+  ac::ZeroList zero;
+  zero.add(ctx->gCV.p, np);
+  zero.add(ctx->gVF.p, nq);
+  zero.add(ctx->gVR.p, nq);
+  zero.add(ctx->gCE.p, ctx->gCE.n);
+  zero.add(ctx->cD.p, nq);
+  zero.add(ctx->gERsum.p, nq);
+  zero.add(ctx->gVRfix.p, nq);
+  zero.add(ctx->gmax.p, (size_t)n_iter + 1);
+  ac::launch_zero(zero, st);
 
   int fix_shift = 0;
   while (((int64_t)1 << (23 + fix_shift)) < ctx->max_outdeg) ++fix_shift;

@@ -143,8 +143,22 @@ void launch_prep_scalars(int P, int Q, const int* ps, const int* pd, const Lse2*
                          hipStream_t st, const SplitRows& rows = SplitRows());
 void launch_fill_const(int64_t n, int w, int64_t a0, int64_t a1, int64_t b0, int64_t f0, float* minC, float* ls,
                        float* vfm, float* fmaxn, hipStream_t st);
-void launch_fill_slots(float* A, float* B, int64_t nslots, int64_t stride, int64_t a0, int64_t al, int64_t b0,
-                       int64_t bl, int64_t c0, int64_t cl, hipStream_t st);
+// Rows of w floats (a multiple of four) in slots of `stride` rows.
+void launch_fill_slots(float* A, float* B, int nslots, int w, int64_t stride, int64_t a0, int64_t al, int64_t b0, int64_t bl,
+                       int64_t c0, int64_t cl, hipStream_t st);
+// Buffers that one launch sets to zero.
+struct ZeroList {
+  static constexpr int kMax = 8;
+  unsigned* p[kMax];
+  int64_t words[kMax];
+  int count = 0;
+  template <typename T>
+  void add(T* q, size_t n) {
+    p[count] = reinterpret_cast<unsigned*>(q);
+    words[count++] = (int64_t)(n * (sizeof(T) / 4));
+  }
+};
+void launch_zero(const ZeroList& z, hipStream_t st);
 void launch_walk_src(int64_t nruns, const Run* runs, const int2* ks, const float* CE, int Q, int Qs, float* minCEo,
                      float* lsO, float* VFm, double* carry, Lse* gpart, int nblocks, hipStream_t st, int* AO = nullptr,
                      int* carg = nullptr);
