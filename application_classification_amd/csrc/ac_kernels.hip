@@ -1031,8 +1031,9 @@ __device__ __forceinline__ FixTask fix_task(const SplitList& L, int Qs) {
   int i = b < L.nhub ? b : L.nhub + (b - L.nhub) * kFixWaves + wave, end = L.n - nfew;
   f.active = f.g < G;
   if (f.few) {  // g: unused; j: the thread's pattern edge
-    const int e = (b - bmid) * (64 * kFixWaves) + threadIdx.x;
-    i = L.n - nfew + e / Qs;
+    const int64_t e0 = (int64_t)(b - bmid) * (64 * kFixWaves), v0 = e0 / Qs;  // (the same for the block)
+    const int e = (int)(e0 - v0 * Qs) + threadIdx.x;
+    i = L.n - nfew + (int)v0 + e / Qs;
     end = L.n;
     f.j = e - e / Qs * Qs;
     f.active = true;

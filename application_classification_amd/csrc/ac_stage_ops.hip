@@ -328,10 +328,11 @@ __global__ __launch_bounds__(NT) void k_lsm_row(int64_t n_col, float* __restrict
 int64_t lsm_entries(int64_t n_row, int64_t n_col) { return n_row * (lsm_chunks(n_row, n_col) + 1); }
 
 // The whole operator in one launch where the rows fit: every entry point takes this path first.
-bool lsm_fused(int64_t n_col) { return n_col <= kRowMax; }
+// (The longer ones' blocks of 1024 only while the grid's threads stay below 2^32.)
+bool lsm_fused(int64_t n_row, int64_t n_col) { return n_col <= 16 * kLsmBlock || (n_col <= kRowMax && n_row <= 1 << 20); }
 
 int enqueue_row_lsm(int64_t n_row, int64_t n_col, float* x, ac::Lse* scratch, hipStream_t st, const char* who) {
-  if (lsm_fused(n_col)) {
+  if (lsm_fused(n_row, n_col)) {
     if (n_col <= 16 * kLsmBlock)
       hipLaunchKernelGGL(k_lsm_row<kLsmBlock>, dim3((unsigned)n_row), dim3(kLsmBlock), 0, st, n_col, x);
     else
@@ -393,25 +394,25 @@ __device__ __forceinline__ void atomic_max_float(float* addr, float v) {
 // scratch is needed.  Bound by the one read and by the atomics, which follow each other on the few cache lines of out:
 // as many chunks as fill the chip once with blocks of 1024 threads, and no more (16 x 1,000,003: 37 us with 1968 blocks,
 // 12.5 with 256; 12 x 262,144: 9.9 and 7.3).
-constexpr int kMaxBlock = 256, kRowMaxBlock = 1024;
+constexpr int kMaxBlock = 256;
 constexpr int64_t kRowMaxBlocks = 256;
 
-__global__ __launch_bounds__(kRowMaxBlock) void k_stage_row_max(int64_t n_col, int64_t nchunk,
-                                                                const float* __restrict__ in,
-                                                                float* __restrict__ out) {
-  __shared__ float red[kRowMaxBlock / 64];
+template <int NT>
+__global__ __launch_bounds__(NT) void k_stage_row_max(int64_t n_col, int64_t nchunk, const float* __restrict__ in,
+                                                      float* __restrict__ out) {
+  __shared__ float red[NT / 64];
   const int64_t row = blockIdx.x / nchunk, chunk = blockIdx.x - row * nchunk;
   int64_t c0, c1;
   chunk_range(n_col, nchunk, chunk, c0, c1);
   float m = -INFINITY;
-  stream_chunk<kRowMaxBlock>(in + row * n_col, c0, c1, [&](int64_t, float4 v) {
+  stream_chunk<NT>(in + row * n_col, c0, c1, [&](int64_t, float4 v) {
     m = fmaxf(m, fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
   }, [&](int64_t, float v) { m = fmaxf(m, v); });
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
-    for (int w = 1; w < kRowMaxBlock / 64; ++w) m = fmaxf(m, red[w]);
+    for (int w = 1; w < NT / 64; ++w) m = fmaxf(m, red[w]);
     if (nchunk == 1)
       out[row] = m;
     else
@@ -441,6 +442,9 @@ __global__ void k_stage_fill_rows(int64_t n_row, int64_t n_col, const float* __r
   for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < total; o += (int64_t)gridDim.x * blockDim.x)
     xmax[o] = vymax ? vymax[o / n_col] : -INFINITY;
 }
+// v can raise the entry x (bitwise: +0.0 raises -0.0, as in the atomic's order).
+__device__ __forceinline__ bool above(float v, float x) { return !(v < x) && __float_as_uint(v) != __float_as_uint(x); }
+
 // Bound by the one read of xe.  A value at or below its row's fill can change nothing, so only the others look at
 // their node, and of those only the ones above its present value (read without an atomic: the entries only rise, so a
 // stale value is a low one) issue the atomic.  16 x 3.94 M values into 16 x 262,144, with the fill pass: 47 us where the
@@ -456,8 +460,6 @@ __global__ __launch_bounds__(kMaxBlock) void k_stage_scatter_max(int64_t n_col_i
   chunk_range(n_col_in, nchunk, chunk, c0, c1);
   const float fill = vymax[row];
   float* out = xmax + row * n_col_out;
-  // v can raise the entry x (bitwise: +0.0 raises -0.0, as in the atomic's order).
-  auto above = [](float v, float x) { return !(v < x) && __float_as_uint(v) != __float_as_uint(x); };
   stream_chunk<kMaxBlock>(xe + row * n_col_in, c0, c1, [&](int64_t c, float4 v) {
     if (!(above(v.x, fill) || above(v.y, fill) || above(v.z, fill) || above(v.w, fill))) return;
     const float vv[4] = {v.x, v.y, v.z, v.w};
@@ -471,6 +473,20 @@ __global__ __launch_bounds__(kMaxBlock) void k_stage_scatter_max(int64_t n_col_i
   }, [&](int64_t c, float v) {
     if (above(v, fill)) atomic_max_float(out + nodes[c], v);
   });
+}
+
+// Rows shorter than a block: a thread per value, whatever its row.
+__global__ __launch_bounds__(kMaxBlock) void k_stage_scatter_short(int64_t n_row, int64_t n_col_in, int64_t n_col_out,
+                                                                   const float* __restrict__ vymax,
+                                                                   const float* __restrict__ xe,
+                                                                   float* __restrict__ xmax,
+                                                                   const int* __restrict__ nodes) {
+  const int64_t total = n_row * n_col_in;
+  for (int64_t o = blockIdx.x * (int64_t)kMaxBlock + threadIdx.x; o < total; o += (int64_t)gridDim.x * kMaxBlock) {
+    const int64_t row = o / n_col_in;
+    const float v = xe[o];
+    if (above(v, vymax[row])) atomic_max_float(xmax + row * n_col_out + nodes[o - row * n_col_in], v);
+  }
 }
 
 // ac::ComputeMU2_t (src/ac.hxx:151-186), summed per data vertex in ascending q, FP64, rounded once.  Block (v tile,
@@ -549,31 +565,13 @@ __global__ __launch_bounds__(256) void k_stage_compute_mu(int64_t n_col_in, int6
   }
 }
 
-// ac::transpose (src/ac.hxx:17-31), in tiles of kTr x kTr through LDS, so that both sides move whole runs: one read and
-// one write (262,144 x 12 in 9.3 us).
-constexpr int kTr = 64;
-// `lines` lines of `len` elements over a block of 256 threads, consecutive threads on consecutive elements.
-template <class F>
-__device__ __forceinline__ void tile_walk(int len, int lines, F f) {
-  const int dl = 256 / len, de = 256 - dl * len;
-  int l = threadIdx.x / len, e = threadIdx.x - l * len;
-  while (l < lines) {
-    f(l, e);
-    l += dl, e += de;
-    if (e >= len) e -= len, ++l;
-  }
-}
-__global__ __launch_bounds__(256) void k_stage_transpose(const float* __restrict__ in, float* __restrict__ out,
-                                                         int64_t n_rows, int64_t n_cols) {
-  __shared__ float tile[kTr][kTr + 1];
-  const int64_t tr = (n_rows + kTr - 1) / kTr, tc = (n_cols + kTr - 1) / kTr;
-  for (int64_t b = blockIdx.x; b < tr * tc; b += gridDim.x) {
-    const int64_t r0 = b / tc * kTr, c0 = (b - b / tc * tc) * kTr;
-    const int nr = (int)std::min<int64_t>(kTr, n_rows - r0), nc = (int)std::min<int64_t>(kTr, n_cols - c0);
-    __syncthreads();
-    tile_walk(nc, nr, [&](int r, int c) { tile[r][c] = in[(r0 + r) * n_cols + c0 + c]; });
-    __syncthreads();
-    tile_walk(nr, nc, [&](int c, int r) { out[(c0 + c) * n_rows + r0 + r] = tile[r][c]; });
+// ac::transpose (src/ac.hxx:17-31).  (One side is a pattern's few columns: tiles through LDS took as long.)
+__global__ void k_stage_transpose(const float* __restrict__ in, float* __restrict__ out, int64_t n_rows,
+                                  int64_t n_cols) {
+  const int64_t total = n_rows * n_cols;
+  for (int64_t o = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; o < total; o += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t c = o / n_rows, r = o - c * n_rows;
+    out[o] = in[r * n_cols + c];
   }
 }
 
@@ -621,7 +619,7 @@ extern "C" int ac_row_log_softmax(int64_t n_row, int64_t n_col, float* x, void* 
   if (n_row < 0 || n_col < 0 || n_row > INT32_MAX || (n_row * n_col > 0 && !x)) return bad("ac_row_log_softmax: bad arguments");
   if (n_row * n_col == 0) return AC_OK;
   hipStream_t st = as_stream(stream);
-  if (lsm_fused(n_col)) return enqueue_row_lsm(n_row, n_col, x, nullptr, st, "ac_row_log_softmax");
+  if (lsm_fused(n_row, n_col)) return enqueue_row_lsm(n_row, n_col, x, nullptr, st, "ac_row_log_softmax");
   // Stream-ordered temporary (the reference's RowSoftmax2 allocates its own too, src/ac.hxx:108-113).
   ac::Lse* tmp = nullptr;
   hipError_t e = hipMallocAsync((void**)&tmp, (size_t)lsm_entries(n_row, n_col) * sizeof(ac::Lse), st);
@@ -660,9 +658,12 @@ extern "C" int ac_row_max(int64_t n_row, int64_t n_col, const float* in, float* 
   if (n_col == 0 || nchunk > 1)
     hipLaunchKernelGGL(k_stage_fill_rows, dim3(grid_for(n_row, 256)), dim3(256), 0, st, n_row, (int64_t)1,
                        (const float*)nullptr, out);
-  if (n_col > 0)
-    hipLaunchKernelGGL(k_stage_row_max, dim3((unsigned)(n_row * nchunk)), dim3(kRowMaxBlock), 0, st, n_col, nchunk,
-                       in, out);
+  // The larger block where a row has work for it, and where the grid's threads stay below 2^32.
+  const dim3 grid((unsigned)(n_row * nchunk));
+  if (n_col > kLsmChunkMin && n_row * nchunk <= 1 << 20)
+    hipLaunchKernelGGL(k_stage_row_max<1024>, grid, dim3(1024), 0, st, n_col, nchunk, in, out);
+  else if (n_col > 0)
+    hipLaunchKernelGGL(k_stage_row_max<kMaxBlock>, grid, dim3(kMaxBlock), 0, st, n_col, nchunk, in, out);
   return launch_status("ac_row_max");
 }
 
@@ -673,19 +674,22 @@ extern "C" int ac_edge_max_reduce(int64_t n_col_in, int64_t n_col_out, int64_t n
     return bad("ac_edge_max_reduce: bad arguments");
   hipStream_t st = as_stream(stream);
   const int64_t fchunk = (n_col_out + 4095) / 4096;
-  if (n_col_out >= 4096 && n_row > 0 && n_row <= INT32_MAX / fchunk)
+  if (n_col_out >= 4096 && n_row > 0 && n_row <= (1 << 23) / fchunk)  // (below 2^32 threads)
     hipLaunchKernelGGL(k_stage_fill_long, dim3((unsigned)(n_row * fchunk)), dim3(kMaxBlock), 0, st, n_col_out, fchunk,
                        vymax, xmax);
   else if (n_row * n_col_out > 0)
     hipLaunchKernelGGL(k_stage_fill_rows, dim3(grid_for(n_row * n_col_out, 256)), dim3(256), 0, st, n_row,
                        n_col_out, vymax, xmax);
-  if (n_row * n_col_in > 0) {
+  if (n_col_in < kMaxBlock && n_row * n_col_in > 0) {
+    hipLaunchKernelGGL(k_stage_scatter_short, dim3(grid_for(n_row * n_col_in, kMaxBlock)), dim3(kMaxBlock), 0, st, n_row,
+                       n_col_in, n_col_out, vymax, xe, xmax, nodes);
+  } else if (n_row * n_col_in > 0) {
     // Chunks of 8192 values (32 a thread), shorter ones down to 1024 where fewer than 2048 blocks would result (a
     // block of low-fill values is a chain of dependent reads and atomics: 39 us for 16 x 20,000 values in chunks of
-    // 8192, 15 us in chunks of 1024); rows in slices of at most INT32_MAX blocks.
+    // 8192, 15 us in chunks of 1024); rows in slices of at most 2^23 blocks (2^31 threads).
     const int64_t csize = std::min<int64_t>(8192, std::max<int64_t>(1024, (n_col_in / 2048) * std::min<int64_t>(n_row, 8192)));
-    const int64_t nchunk = std::max<int64_t>(1, std::min<int64_t>((n_col_in + csize - 1) / csize, INT32_MAX));
-    const int64_t slice = INT32_MAX / nchunk;
+    const int64_t nchunk = std::max<int64_t>(1, std::min<int64_t>((n_col_in + csize - 1) / csize, 1 << 23));
+    const int64_t slice = (1 << 23) / nchunk;
     for (int64_t r0 = 0; r0 < n_row; r0 += slice)
       hipLaunchKernelGGL(k_stage_scatter_max, dim3((unsigned)(std::min(slice, n_row - r0) * nchunk)), dim3(kMaxBlock), 0,
                          st, n_col_in, n_col_out, nchunk, vymax + r0, xe + r0 * n_col_in, xmax + r0 * n_col_out, nodes);
@@ -715,8 +719,7 @@ extern "C" int ac_compute_mu(int64_t n_col_in, int64_t n_row_in, int64_t n_col_o
 extern "C" int ac_transpose(const float* in, float* out, int64_t n_rows, int64_t n_cols, void* stream) {
   if (n_rows < 0 || n_cols < 0 || (n_rows * n_cols > 0 && (!in || !out))) return bad("ac_transpose: bad arguments");
   if (n_rows * n_cols == 0) return AC_OK;
-  const int64_t tiles = ((n_rows + kTr - 1) / kTr) * ((n_cols + kTr - 1) / kTr);
-  hipLaunchKernelGGL(k_stage_transpose, dim3((unsigned)std::min<int64_t>(tiles, 1 << 20)), dim3(256), 0, as_stream(stream),
-                     in, out, n_rows, n_cols);
+  hipLaunchKernelGGL(k_stage_transpose, dim3(grid_for(n_rows * n_cols, 256)), dim3(256), 0, as_stream(stream), in,
+                     out, n_rows, n_cols);
   return launch_status("ac_transpose");
 }

@@ -43,7 +43,8 @@ def order_key(x):
 
 @pytest.mark.parametrize("n_row,n_in,n_out,offset", [(1, 1, 1, 0), (3, 7, 2, 1), (5, 1023, 40, 2), (2, 1025, 1, 3),
                                                      (3, 8193, 700, 1), (16, 70_001, 3000, 0), (2, 0, 5, 0),
-                                                     (3, 5, 4099, 1), (0, 5, 5000, 0)])
+                                                     (3, 5, 4099, 1), (0, 5, 5000, 0),
+                                                     (5000, 9, 4, 1), (40, 255, 60, 2), (40, 256, 60, 2)])
 @pytest.mark.parametrize("fill", ["low", "mid", "special"])
 def test_edge_max_reduce_edges(n_row, n_in, n_out, offset, fill):
     """Chunk edges, rows off the 16-byte grid, nodes shared by many and by neighbouring values, fills below, among and
@@ -115,7 +116,8 @@ def test_row_log_softmax_specials(n_col):
     assert np.isnan(got[1:]).all()
 
 
-@pytest.mark.parametrize("n_row,n_col,offset", [(1, 1, 0), (300, 3, 1), (3, 32_768, 1), (3, 32_769, 2), (2, 100_001, 3)])
+@pytest.mark.parametrize("n_row,n_col,offset", [(1, 1, 0), (300, 3, 1), (3, 32_768, 1), (3, 32_769, 2), (2, 100_001, 3),
+                                                (4, 8192, 1), (4, 8193, 1)])
 def test_row_max_edges(n_row, n_col, offset):
     x = -np.abs(np.random.default_rng(n_col).normal(size=(n_row, n_col))).astype(np.float32) - 1.0
     x[0, :] = -np.inf
