@@ -222,6 +222,13 @@ struct HostStage {
   }
 };
 
+// Edges per piece of a vertex of deg > run edges: a run's length, and longer, up to 128, where more than 1024 pieces
+// would result, since the pieces of one vertex are combined on one row (16 pattern columns: a loop's iteration with all
+// 50,000 edges into one vertex 266 us in pieces of 8 edges, now 42).  1024 pieces of 8 edges fill the chip as runs do.
+int64_t piece_edges(int64_t deg, int run) {
+  return std::max<int64_t>(run, std::min<int64_t>(128, (deg + 1023) / 1024));
+}
+
 // Runs over n vertices whose edge lists are the ranges [off[t], off[t + 1]) in sequence: vertex vid[t] (t itself
 // when vid is null).  consecutive: a run may only join vertices whose ids follow each other (the CSC walk steps its
 // destination by one at each new vertex); the CSR walk reads each edge's source and takes any order.
@@ -243,11 +250,12 @@ void build_runs(const std::vector<int64_t>& off, int64_t n, std::vector<Run>& ru
     if (deg == 0) continue;
     if (deg > kRunEdges) {
       close(off[t]);
-      const int pieces = (int)((deg + kRunEdges - 1) / kRunEdges);
+      const int64_t L = piece_edges(deg, kRunEdges);
+      const int pieces = (int)((deg + L - 1) / L);
       splits.push_back(Split{(int)v, nslots, pieces, 0});
       for (int i = 0; i < pieces; ++i) {
-        const int64_t kb = off[t] + (int64_t)i * kRunEdges;
-        runs.push_back(Run{(int)kb, (int)std::min(off[t + 1], kb + kRunEdges), nslots++, 0});
+        const int64_t kb = off[t] + i * L;
+        runs.push_back(Run{(int)kb, (int)std::min(off[t + 1], kb + L), nslots++, pieces});
       }
       continue;
     }
@@ -789,7 +797,9 @@ static int select_bundles(ac_ctx* ctx) {
       if (i >= nr) break;
       const Run& r = R[order[i]];
       brun[i] = order[i];
-      gslot[i] = r.slot;
+      // Atomics on one row follow each other (1.5 ns each): a vertex whose pieces send 8192 values or more (12 us, which
+      // a wave's tail no longer hides) has them look at the row first, which costs each of them a memory latency.
+      gslot[i] = r.slot < 0 || (int64_t)r.pieces * (256 / G) < 8192 ? r.slot : r.slot | ac::kCrowded;
       len = std::max(len, r.ke - r.kb);
     }
     len = (len + Bt - 1) / Bt * Bt;

@@ -53,10 +53,12 @@ struct IsoCol {
 };
 
 // A contiguous run of edges in CSC or CSR order covering whole vertices, or one piece of a vertex whose edge list
-// is longer than a run (slot >= 0 then names its carry slot).
+// is longer than a run (slot >= 0 then names its carry slot, and pieces is the number of the vertex's pieces).
 struct Run {
-  int kb, ke, slot, pad;
+  int kb, ke, slot, pieces;
 };
+// Set in the carry slots of a bundle layout (gslot): the slot's vertex has so many pieces that they crowd its row.
+constexpr int kCrowded = 1 << 30;
 // A vertex split into `count` pieces with carry slots [first, first + count).
 struct Split {
   int v, first, count, pad;

@@ -167,3 +167,29 @@ def test_gradient_tiles(n, m, pn, pe, K, dim):
     _, gv, ge = gpu_grad(data, patt, wv, we, 3, K=K)
     fv, fe = fd_grad(g64(data), g64(patt), patt.vmap, wv.copy(), we.copy(), 3)
     check_grad(np.concatenate([gv, ge]), np.concatenate([fv, fe]), f"dn={n} de={m} pn={pn} pe={pe} dim={dim}")
+
+
+@pytest.mark.parametrize("pe", [3, 17, 70, 130])
+@pytest.mark.parametrize("extra", [0, 500])
+def test_one_vertex_takes_all_edges(pe, extra):
+    """Stars in both directions with more pieces than a vertex is split into at its run length (8 edges): waves whose
+    pieces are all one vertex's, with and without others among them; plain and recorded walks agree bit for bit."""
+    r = np.random.default_rng(pe + extra)
+    n, hub = 90, 12_000
+    src = np.concatenate([r.integers(2, n, hub), np.full(hub, 1), r.integers(0, n, extra)])
+    dst = np.concatenate([np.full(hub, 0), r.integers(2, n, hub), r.integers(0, n, extra)])
+    data = W.Graph(r.normal(size=(n, 5)).astype(np.float32), r.normal(size=(len(src), 5)).astype(np.float32),
+                   src.astype(np.int32), dst.astype(np.int32))
+    patt = random_graph(9, pe, 5, 5, pe)
+    expect = O.run(g64(data), g64(patt), n_iter=4)
+    got = []
+    for tape in (0, 1):
+        with Matcher(0) as m:
+            m.set_option(AC_OPT_TAPE, tape)
+            m.set_data(data)
+            m.set_pattern(patt)
+            got.append([m.run(4) for _ in range(2)])
+        bad, ratio = allclose_report(got[-1][1], expect)
+        assert bad == 0, (tape, ratio)
+    np.testing.assert_array_equal(got[0][0], got[0][1])
+    np.testing.assert_array_equal(got[0][1], got[1][1])
