@@ -193,3 +193,29 @@ def test_one_vertex_takes_all_edges(pe, extra):
         assert bad == 0, (tape, ratio)
     np.testing.assert_array_equal(got[0][0], got[0][1])
     np.testing.assert_array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("n,act,pn,pe", [(17_000, 300, 4, 5), (40_000, 3000, 9, 24), (9000, 60, 33, 40)])
+def test_output_tiles_of_mostly_isolated_graphs(n, act, pn, pe):
+    """Few vertices with edges among many: the iterations' tiles and the output passes' differ in height.  Plain, batched
+    (a pattern's own columns beside another's) and taped runs, and the gradients."""
+    data, patt = random_graph(act, 4 * act, 2, 2, n), random_graph(pn, pe, 2, 2, pn)
+    r = np.random.default_rng(pe)
+    ids = r.permutation(n)[:act].astype(np.int32)
+    data = W.Graph(r.normal(size=(n, 2)).astype(np.float32), data.efeat, ids[data.src], ids[data.dst])
+    expect = O.run(g64(data), g64(patt), n_iter=3)
+    with Matcher(0) as m:
+        m.set_data(data)
+        m.set_pattern(patt)
+        plain = m.run(3)
+        m.batch_set_patterns([random_graph(5, 7, 2, 2, 1), patt])
+        m.batch_run([2, 3])
+        batched = m.batch_mu(1)
+    for mu in (plain, batched):
+        bad, ratio = allclose_report(mu, expect)
+        assert bad == 0, ratio
+    patt.vmap = r.integers(0, n, pn)
+    wv, we = weights(2, 2, 2)
+    _, gv, ge = gpu_grad(data, patt, wv, we, 2, K=1)
+    fv, fe = fd_grad(g64(data), g64(patt), patt.vmap, wv.copy(), we.copy(), 2)
+    check_grad(np.concatenate([gv, ge]), np.concatenate([fv, fe]), f"dn={n} act={act} pn={pn} pe={pe}")
