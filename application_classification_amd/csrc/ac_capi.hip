@@ -19,6 +19,7 @@
 #include "ac_host.hpp"
 #include "ac_internal.hpp"
 #include "ac_select.hpp"
+#include "ac_stage.hpp"
 
 using ac::Lse;
 using ac::Lse2;
@@ -129,99 +130,6 @@ struct DevBuf {
   }
 };
 
-// Pinned host memory through which results and large inputs cross PCIe: slots used in turn, so that the copy engine
-// fills (or drains) one while a thread drains (or fills) another.  A copy straight to or from pageable memory runs at 10
-// GB/s (67 MB of MU: 6.4 ms).  The link takes 57 GB/s; one thread writes a fresh host array, page faults included, at 12
-// GB/s (5.2 ms), so results of 16 MB and more are written by four threads, each with slots of its own (2.4 ms; eight
-// threads 3.3 ms, and at 5-13 MB two or four gain nothing over one).
-// Held by a context from its first copy to its end.
-struct HostStage {
-  static constexpr int kThreads = 4, kSlots = 2 * kThreads;
-  static constexpr size_t kSlot = 1 << 20;
-  static constexpr size_t kDirect = 2 << 20;  // below, a direct copy is as fast (1.5 MB: 93 against 97 us)
-  char* p = nullptr;
-  hipEvent_t ev[kSlots] = {};
-  bool busy[kSlots] = {};  // a copy out of the slot may be in flight
-  HostStage() = default;
-  HostStage(const HostStage&) = delete;
-  HostStage& operator=(const HostStage&) = delete;
-  ~HostStage() {
-    for (auto& e : ev)
-      if (e) (void)hipEventDestroy(e);
-    if (p) (void)hipHostFree(p);
-  }
-  // False where no pinned memory is to be had: the caller copies directly.
-  bool ready() {
-    if (p) return true;
-    for (auto& e : ev)
-      if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) e = nullptr;
-    bool ok = true;
-    for (auto& e : ev) ok = ok && e;
-    if (ok && hipHostMalloc((void**)&p, kSlots * kSlot, hipHostMallocDefault) == hipSuccess) return true;
-    (void)hipGetLastError();
-    p = nullptr;
-    return false;
-  }
-  hipError_t wait(int s) {
-    if (!busy[s]) return hipSuccess;
-    busy[s] = false;
-    return hipEventSynchronize(ev[s]);
-  }
-  // Device to host, complete when it returns.
-  hipError_t to_host(void* dst, const void* src, size_t bytes, hipStream_t st, int device) {
-    const int nt = bytes < (16u << 20) ? 1 : kThreads;
-    const size_t chunk = nt == 1 ? kSlot / 2 : kSlot;  // (one thread: a shorter pipeline to fill)
-    const size_t n = (bytes + chunk - 1) / chunk;
-    hipError_t err[kThreads] = {};
-    // Thread t takes chunks t, t + nt, ... through slots t, t + nt, ...
-    ac::parallel_items(nt, [&](int64_t t) {
-      hipError_t e = t ? hipSetDevice(device) : hipSuccess;
-      const size_t per = (size_t)(kSlots / nt);
-      auto len = [&](size_t i) { return std::min(chunk, bytes - i * chunk); };
-      auto slot = [&](size_t j) { return (int)t + (int)(j % per) * nt; };  // of the thread's j-th chunk, t + j nt
-      auto start = [&](size_t j) {
-        const size_t i = (size_t)t + j * nt;
-        const int s = slot(j);
-        if (i >= n || e != hipSuccess) return;
-        e = wait(s);
-        if (e == hipSuccess)
-          e = hipMemcpyAsync(p + s * kSlot, static_cast<const char*>(src) + i * chunk, len(i), hipMemcpyDeviceToHost, st);
-        if (e == hipSuccess) e = hipEventRecord(ev[s], st);
-        if (e == hipSuccess) busy[s] = true;
-      };
-      for (size_t j = 0; j < per; ++j) start(j);
-      for (size_t j = 0;; ++j) {
-        const size_t i = (size_t)t + j * nt;
-        if (i >= n || e != hipSuccess) break;
-        const int s = slot(j);
-        e = wait(s);
-        if (e != hipSuccess) break;
-        std::memcpy(static_cast<char*>(dst) + i * chunk, p + s * kSlot, len(i));
-        start(j + per);
-      }
-      err[t] = e;
-    }, nt);
-    for (int t = 0; t < nt; ++t)
-      if (err[t] != hipSuccess) return err[t];
-    return hipSuccess;
-  }
-  // Host to device: the source is read when it returns, the copy is ordered on the stream.
-  hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t st) {
-    hipError_t e = hipSuccess;
-    for (size_t o = 0, i = 0; o < bytes && e == hipSuccess; o += kSlot, ++i) {
-      const int s = (int)(i % kSlots);
-      const size_t len = std::min(kSlot, bytes - o);
-      e = wait(s);
-      if (e != hipSuccess) break;
-      std::memcpy(p + s * kSlot, static_cast<const char*>(src) + o, len);
-      e = hipMemcpyAsync(static_cast<char*>(dst) + o, p + s * kSlot, len, hipMemcpyHostToDevice, st);
-      if (e == hipSuccess) e = hipEventRecord(ev[s], st);
-      if (e == hipSuccess) busy[s] = true;
-    }
-    return e;
-  }
-};
-
 // Edges per piece of a vertex of deg > run edges: a run's length, and longer, up to 128, where more than 1024 pieces
 // would result, since the pieces of one vertex are combined on one row (16 pattern columns: a loop's iteration with all
 // 50,000 edges into one vertex 266 us in pieces of 8 edges, now 42).  1024 pieces of 8 edges fill the chip as runs do.
@@ -282,7 +190,7 @@ struct ac_ctx {
   hipStream_t aux = nullptr;
   hipEvent_t xev[4] = {nullptr, nullptr, nullptr, nullptr};
   std::string err;
-  HostStage stage;
+  ac::HostStage stage;
 
   // Data graph (src/main.cu:8-19 / 49-62) plus its CSC and CSR views.
   bool has_data = false;
@@ -691,12 +599,7 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
   const size_t o_v = part(pv), o_e = part(pe), o_s = part(ps_pad), o_d = part(pd_pad), o_o = part(inc_off),
                o_i = part(inc), o_a = part(inc_at), o_u = part(sums), o_f = part(sum_off);
   HIPCHK(ctx, ctx->pat.alloc(all.size()));
-  if (ctx->stage.ready()) {
-    HIPCHK(ctx, ctx->stage.to_device(ctx->pat.p, all.data(), all.size(), st));
-  } else {
-    HIPCHK(ctx, hipMemcpyAsync(ctx->pat.p, all.data(), all.size(), hipMemcpyHostToDevice, st));
-    HIPCHK(ctx, hipStreamSynchronize(st));
-  }
+  HIPCHK(ctx, ctx->stage.to_device(ctx->pat.p, all.data(), all.size(), st));
   ctx->pf_v.p = reinterpret_cast<double*>(ctx->pat.p + o_v);
   ctx->pf_e.p = reinterpret_cast<double*>(ctx->pat.p + o_e);
   ctx->d_ps.p = reinterpret_cast<int*>(ctx->pat.p + o_s);
@@ -1351,22 +1254,13 @@ extern "C" int ac_run(ac_ctx* ctx, int n_iter) {
   return ac_sync(ctx);
 }
 
-// A result to host memory, complete when it returns.
-static int copy_out(ac_ctx* ctx, void* dst, const void* src, size_t bytes) {
-  if (bytes >= HostStage::kDirect && ctx->stage.ready()) {
-    HIPCHK(ctx, ctx->stage.to_host(dst, src, bytes, ctx->stream, ctx->device));
-    return AC_OK;
-  }
-  HIPCHK(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-  HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-  return AC_OK;
-}
-
 extern "C" int ac_get_mu(ac_ctx* ctx, float* host_out) {
   if (!ctx || !host_out) return ctx ? ctx->fail(AC_ERR_ARG, "ac_get_mu: null output") : AC_ERR_ARG;
   if (!ctx->have_result) return ctx->fail(AC_ERR_STATE, "ac_get_mu: no result; call ac_run first");
   HIPCHK(ctx, hipSetDevice(ctx->device));
-  return copy_out(ctx, host_out, ctx->OUT.p, sizeof(float) * (size_t)ctx->dn * ctx->P);
+  HIPCHK(ctx, ctx->stage.to_host(host_out, ctx->OUT.p, sizeof(float) * (size_t)ctx->dn * ctx->P, ctx->stream,
+                                 ctx->device));
+  return AC_OK;
 }
 
 // Each pattern vertex's k best data vertices on the device, if the sizes suit it: out = {idx [P][k], val [P][k]}.
@@ -1805,7 +1699,9 @@ extern "C" int ac_batch_get_mu(ac_ctx* ctx, int i, float* host_out) {
   if (i < 0 || i >= (int)ctx->bp.size()) return ctx->fail(AC_ERR_ARG, "ac_batch_get_mu: no pattern " + std::to_string(i));
   HIPCHK(ctx, hipSetDevice(ctx->device));
   const auto& B = ctx->bp[i];
-  return copy_out(ctx, host_out, ctx->bout.p + B.out_off, sizeof(float) * (size_t)ctx->dn * B.P);
+  HIPCHK(ctx, ctx->stage.to_host(host_out, ctx->bout.p + B.out_off, sizeof(float) * (size_t)ctx->dn * B.P, ctx->stream,
+                                 ctx->device));
+  return AC_OK;
 }
 
 extern "C" int ac_batch_info(const ac_ctx* ctx, int64_t* out4) {
@@ -2034,10 +1930,7 @@ extern "C" int ac_backward(ac_ctx* ctx, const float* grad_mu, float* grad_wv, fl
   const int64_t brows = ctx->bs->brows;
   // grad_mu is in the caller's vertex order; the adjoint works in the internal one.
   HIPCHK(ctx, ctx->gMUin.alloc(np));
-  if (ctx->stage.ready())
-    HIPCHK(ctx, ctx->stage.to_device(ctx->gMUin.p, grad_mu, np * sizeof(float), st));
-  else
-    HIPCHK(ctx, ctx->gMUin.upload(grad_mu, np, st));
+  HIPCHK(ctx, ctx->stage.to_device(ctx->gMUin.p, grad_mu, np * sizeof(float), st));
   HIPCHK(ctx, ctx->gMU.alloc(np));
   ac::launch_gather_rows(ctx->dn, ctx->P, ctx->d_perm.p, ctx->gMUin.p, ctx->gMU.p, st);
   HIPCHK(ctx, ctx->gCV.alloc(np));

@@ -2,7 +2,9 @@
 reference's own tolerance (validate.py:7)."""
 import numpy as np
 import pytest
+import torch
 
+from application_classification_amd import _lib
 from application_classification_amd import workloads as W
 from application_classification_amd.matcher import AC_OPT_PRUNE, AC_OPT_TAPE, Matcher
 from oracle import oracle as O
@@ -219,3 +221,24 @@ def test_output_tiles_of_mostly_isolated_graphs(n, act, pn, pe):
     _, gv, ge = gpu_grad(data, patt, wv, we, 2, K=1)
     fv, fe = fd_grad(g64(data), g64(patt), patt.vmap, wv.copy(), we.copy(), 2)
     check_grad(np.concatenate([gv, ge]), np.concatenate([fv, fe]), f"dn={n} act={act} pn={pn} pe={pe}")
+
+
+@pytest.mark.parametrize("n,pn", [(1000, 10), (70_000, 9), (600_000, 9)])  # a direct copy, one thread's slots, four threads'
+def test_page_locked_results_and_gradients(n, pn):
+    """Results into, and the gradient out of, page-locked memory are those of ordinary memory."""
+    data, patt = random_graph(n, n, 2, 2, n), random_graph(pn, pn, 2, 2, pn)
+    grad = np.zeros((n, pn), np.float32)
+    grad[np.arange(pn) * 7 % n, np.arange(pn)] = -1.0 / pn
+    with Matcher(0) as m:
+        m.set_option(AC_OPT_TAPE, 1)
+        m.set_data(data)
+        m.set_pattern(patt)
+        mu = m.run(1)
+        locked = torch.zeros(n, pn).pin_memory()
+        _lib.check(m._L.ac_get_mu(m._h, locked.data_ptr()), m._h)
+        np.testing.assert_array_equal(locked.numpy(), mu)
+        want = m.backward(grad)
+        locked.copy_(torch.from_numpy(grad))
+        got = m.backward(locked.numpy())
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(a, b)
