@@ -17,11 +17,12 @@ namespace ac {
 // ms, and at 5-13 MB two or four gain nothing over one).
 // Memory that HIP knows (page-locked, managed or the device's) is copied directly, at the link's rate: 50 MB of MU into
 // page-locked memory 0.89 ms, through the slots 1.64 ms.
-// Held by a context from its first copy to its end.
+// Held by a context to its end: the small buffer from its first small input on, the slots from its first large transfer.
 struct HostStage {
   static constexpr int kThreads = 4, kSlots = 2 * kThreads;
   static constexpr size_t kSlot = 1 << 20;
   static constexpr size_t kDirect = 2 << 20;   // below, a direct copy is as fast (1.5 MB: 93 against 97 us)
+  static constexpr size_t kSmall = 256 << 10;  // inputs up to this (a pattern) are not waited for: one buffer, pinned
   // Pinned memory with an event for each slot; a copy into or out of a busy slot may be in flight.
   template <int N>
   struct Slots {
@@ -70,6 +71,7 @@ struct HostStage {
     }
   };
   Slots<kSlots> large;
+  Slots<1> small;
 
   static bool pageable(const void* p) {
     hipPointerAttribute_t a{};
@@ -122,7 +124,8 @@ struct HostStage {
   // Host to device: the source is read when it returns, the copy is ordered on the stream.
   hipError_t to_device(void* dst, const void* src, size_t bytes, hipStream_t st) {
     if (pageable(src)) {
-      if (large.ready(kSlot)) {
+      if (bytes <= kSmall && small.ready(kSmall)) return small.send(0, dst, src, bytes, st);
+      if (bytes >= kDirect && large.ready(kSlot)) {
         hipError_t e = hipSuccess;
         for (size_t o = 0, i = 0; o < bytes && e == hipSuccess; o += kSlot, ++i)
           e = large.send((int)(i % kSlots), static_cast<char*>(dst) + o, static_cast<const char*>(src) + o,

@@ -105,7 +105,7 @@ hipError_t hipStreamSynchronize(hipStream_t) {
 int main() {
   using ac::HostStage;
   device = 1;
-  const size_t sizes[] = {1, 4096, 1 << 18, HostStage::kDirect - 1, HostStage::kDirect,
+  const size_t sizes[] = {1, 4096, HostStage::kSmall, HostStage::kSmall + 1, HostStage::kDirect - 1, HostStage::kDirect,
                           (5 << 20) + 3, (16 << 20) - 1, 16 << 20, (19 << 20) + 7};
   auto fill = [](std::vector<char>& v, int seed) {
     for (size_t i = 0; i < v.size(); ++i) v[i] = (char)(i * 31 + i / 4099 + seed);
@@ -127,6 +127,9 @@ int main() {
       drain(nullptr);
       CHECK(b == first);
       CHECK(c == second);
+      // Small inputs pin a small buffer, ones in between none, large ones the slots.
+      const size_t all = HostStage::kSlots * HostStage::kSlot;
+      CHECK(pinned == (none ? 0 : n <= HostStage::kSmall ? HostStage::kSmall : n < HostStage::kDirect ? 0 : all));
       // Results, into pageable memory: complete on return.
       std::vector<char> d(n, 0);
       copies = selects = 0;
