@@ -91,9 +91,9 @@ struct HostStage {
     const size_t chunk = nt == 1 ? kSlot / 2 : kSlot;  // (one thread: a shorter pipeline to fill)
     const size_t n = (bytes + chunk - 1) / chunk;
     hipError_t err[kThreads] = {};
-    // Item t takes chunks t, t + nt, ... through slots t, t + nt, ....
+    // Item t takes chunks t, t + nt, ... through slots t, t + nt, ..., on whichever thread it falls to.
     parallel_items(nt, [&](int64_t t) {
-      hipError_t e = t ? hipSetDevice(device) : hipSuccess;
+      hipError_t e = hipSetDevice(device);
       const size_t per = (size_t)(kSlots / nt);
       auto slot = [&](size_t j) { return (int)t + (int)(j % per) * nt; };  // of the item's j-th chunk, t + j nt
       auto len = [&](size_t i) { return std::min(chunk, bytes - i * chunk); };

@@ -130,13 +130,15 @@ int main() {
       // Small inputs pin a small buffer, ones in between none, large ones the slots.
       const size_t all = HostStage::kSlots * HostStage::kSlot;
       CHECK(pinned == (none ? 0 : n <= HostStage::kSmall ? HostStage::kSmall : n < HostStage::kDirect ? 0 : all));
-      // Results, into pageable memory: complete on return.
+      // Results, into pageable memory: complete on return, every item of the copy on the context's device.
       std::vector<char> d(n, 0);
       copies = selects = 0;
       CHECK(s.to_host(d.data(), a.data(), n, kStream, 1) == hipSuccess);
       CHECK(d == a);
+      CHECK(wrong_device == 0);
       const bool staged = !none && n >= HostStage::kDirect;
       CHECK(copies == 1 ? !staged : staged);
+      CHECK(!staged || selects == (n < (16u << 20) ? 1 : HostStage::kThreads));
       // Into and out of memory that HIP knows: one copy, complete on return.
       for (auto& x : d) x = 0;
       known = {d.data(), a.data()};
