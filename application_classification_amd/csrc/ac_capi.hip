@@ -520,22 +520,28 @@ static int set_data(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int64_
   ctx->nslots_in = slin;
   ctx->nslots_out = slout;
   {
-    // A radix sort: by first source, 2^11 values a pass, then by decreasing length, every pass stable.
+    // A radix sort: by first source, 2^11 values a pass, then by decreasing length, every pass stable.  Only the runs'
+    // numbers move; their keys stay, read in one sweep of the runs (with the keys looked up through runs and edges in every
+    // pass, R-MAT 18 took 84-87 ms to set, now 81).
     const size_t nr = rin.size();
-    std::vector<int> from(nr), to(nr), cnt;
-    for (size_t i = 0; i < nr; ++i) from[i] = (int)i;
+    std::vector<int> from(nr), to(nr), cnt, first(nr), shorter(nr);
+    int longest = 0;
+    for (const Run& r : rin) longest = std::max(longest, r.ke - r.kb);
+    for (size_t i = 0; i < nr; ++i) {
+      from[i] = (int)i;
+      first[i] = csc_sd[rin[i].kb].x;
+      shorter[i] = longest - (rin[i].ke - rin[i].kb);
+    }
     auto pass = [&](int nkeys, auto key) {
       cnt.assign((size_t)nkeys + 1, 0);
-      for (size_t i = 0; i < nr; ++i) ++cnt[(size_t)key(from[i]) + 1];
+      for (size_t i = 0; i < nr; ++i) ++cnt[(size_t)key((int)i) + 1];
       for (int k = 0; k < nkeys; ++k) cnt[k + 1] += cnt[k];
       for (size_t i = 0; i < nr; ++i) to[(size_t)cnt[key(from[i])]++] = from[i];
       from.swap(to);
     };
     for (int shift = 0; shift < 32 && ((nV - 1) >> shift) > 0; shift += 11)
-      pass(1 << 11, [&](int i) { return (csc_sd[rin[i].kb].x >> shift) & 2047; });
-    int longest = 0;
-    for (const Run& r : rin) longest = std::max(longest, r.ke - r.kb);
-    pass(longest + 1, [&](int i) { return longest - (rin[i].ke - rin[i].kb); });
+      pass(1 << 11, [&](int i) { return (first[i] >> shift) & 2047; });
+    pass(longest + 1, [&](int i) { return shorter[i]; });
     ctx->h_run_order = std::move(from);
   }
   ctx->h_runs_in = std::move(rin);
