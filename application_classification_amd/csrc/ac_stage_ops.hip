@@ -40,8 +40,8 @@ unsigned grid_for(int64_t total, int block) {
 // pair), the root rounded once to FP32.  Both kernels below evaluate exactly that sequence, so they agree bit for bit.
 
 // A thread per output.  Its b row is read element by element (lanes 4 * dim bytes apart) and again for every a row, and
-// every pair converts its own operands: 4.99 ms for 16 x 1,000,003 outputs of 64 features.  Kept for short b (below),
-// where a thread per b row would leave most lanes idle.
+// every pair converts its own operands: 4.99 ms for 16 x 1,000,003 outputs of 64 features.  Kept for short b and small
+// calls of few features (ac_cdist), where a thread per b row would leave lanes or most of the chip idle.
 __global__ void k_stage_cdist(int64_t n_a, int64_t n_b, int64_t dim, const float* __restrict__ a,
                               const float* __restrict__ b, float* __restrict__ out) {
   const int64_t total = n_a * n_b;
@@ -583,17 +583,24 @@ extern "C" int ac_cdist(int64_t n_a, int64_t n_b, int64_t dim, const float* feat
     return bad("ac_cdist: bad arguments");
   if (n_a * n_b == 0) return AC_OK;
   hipStream_t st = as_stream(stream);
-  // A thread per b row from one wave of b rows up: below, a thread per output keeps the lanes busy.
-  if (n_b < 64) {
+  // A thread per output where a wave of b rows would leave lanes idle and the reads cost little: b shorter than a wave,
+  // or small enough as a whole to stay in the cache (50,001 x 65 of 5 features 16.0 against 18.7 us; 50,001 x 80 of 8: 62
+  // against 18.8), and for small calls of few features, a launch's latency (12 x 1,000 of 13: 3.6 against 4.5 us; 24 x
+  // 3,000 of 16: 5.5 against 4.4).
+  if (n_b < 64 || n_b * dim < 384 || (dim <= 24 && n_a * n_b < 1'500'000 / std::max<int64_t>(1, dim))) {
     hipLaunchKernelGGL(k_stage_cdist, dim3(grid_for(n_a * n_b, 256)), dim3(256), 0, st, n_a, n_b, dim, feats_a,
                        feats_b, out);
     return launch_status("ac_cdist");
   }
-  // The a rows in ngroups groups of equal size, at most 16 (a multiple of 4): 24 rows as 2 x 12 rather than 16 + 8.
-  const int64_t ngroups = (n_a + 15) / 16;
+  // The a rows in ngroups groups of equal size, at most 16 (a multiple of 4): 24 rows as 2 x 12 rather than 16 + 8.  Groups
+  // of four where those of 16 would be fewer than two waves for each of the 256 CUs, since a wave takes its rows one after
+  // the other: 16 x 1,000 of 64 features 15.0 -> 6.6 us (a thread per output: 10.0), 16 x 16,000 15.3 -> 7.8 us.
+  const bool few = (n_b + 63) / 64 * ((n_a + 15) / 16) < 512;
+  const int64_t ngroups = few ? (n_a + 3) / 4 : (n_a + 15) / 16;
   const int jp = (int)((n_a + ngroups - 1) / ngroups + 3) / 4 * 4;
-  // Short b takes one wave and one row per thread, so that the tiles reach more of the chip.
-  const bool small = n_b * ngroups < (int64_t)256 * 2048;
+  // Short b takes one wave and one row per thread, so that the tiles reach more of the chip and fewer rows are idle in
+  // the last one (100,000 x 100 of 13 features 65 -> 41 us).
+  const bool small = few || n_b <= 192 || n_b * ngroups < (int64_t)256 * 2048;
   const int64_t ntiles = (n_b + (small ? 63 : 255)) / (small ? 64 : 256);
   const unsigned blocks = (unsigned)std::min<int64_t>(ntiles * ngroups, 1 << 20);
 #define AC_STAGE_CD(JP)                                                                                             \

@@ -35,6 +35,16 @@ def test_cdist_tiles(n_a, n_b, dim, offset):
     np.testing.assert_allclose(got[:n_a * n_b].reshape(n_a, n_b), ref, rtol=2.0**-24 + 2.0**-40, atol=0)
 
 
+@pytest.mark.parametrize("n_a,n_b,dim", [
+    (4, 95, 4), (4, 96, 4), (7, 400, 0),                              # b as a whole on both sides of the cache rule
+    (15, 4166, 24), (15, 4167, 24), (15, 4167, 25), (1200, 50, 25),   # small calls of few features and others
+    (16, 32_704, 25), (16, 32_705, 25), (17, 16_352, 25), (3, 64, 25), (5, 193, 300), (6000, 192, 25), (6000, 193, 25),
+])
+def test_cdist_split_of_small_calls(n_a, n_b, dim):
+    """Both sides of the rules that choose a thread per output, groups of four a rows and short tiles."""
+    test_cdist_tiles(n_a, n_b, dim, 0)
+
+
 def order_key(x):
     """The total order of the scatter's maximum: floats by value, -0.0 below +0.0, NaNs beyond the infinities."""
     b = np.ascontiguousarray(x).view(np.int32).astype(np.int64)
