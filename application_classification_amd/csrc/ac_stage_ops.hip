@@ -333,8 +333,14 @@ bool lsm_fused(int64_t n_row, int64_t n_col) { return n_col <= 16 * kLsmBlock ||
 
 int enqueue_row_lsm(int64_t n_row, int64_t n_col, float* x, ac::Lse* scratch, hipStream_t st, const char* who) {
   if (lsm_fused(n_row, n_col)) {
-    if (n_col <= 16 * kLsmBlock)
+    // The smallest block that holds a row where there are more rows than CUs (256), so that a CU works on several at once:
+    // 4,096 x 4,097 in 31 us with blocks of 256, 82 with 1,024 (three launches: 51); 4,096 x 12,000 69 with 512, 108 with
+    // 1,024 (114).  Few rows take the largest, whose threads have the fewest elements: 256 x 4,097 in 7.6 us.
+    const bool many = n_row > 256;
+    if (n_col <= 16 * kLsmBlock || (many && n_col <= kRowRegs * kLsmBlock))
       hipLaunchKernelGGL(k_lsm_row<kLsmBlock>, dim3((unsigned)n_row), dim3(kLsmBlock), 0, st, n_col, x);
+    else if (many && n_col <= kRowRegs * 512)
+      hipLaunchKernelGGL(k_lsm_row<512>, dim3((unsigned)n_row), dim3(512), 0, st, n_col, x);
     else
       hipLaunchKernelGGL(k_lsm_row<1024>, dim3((unsigned)n_row), dim3(1024), 0, st, n_col, x);
     return launch_status(who);

@@ -126,6 +126,26 @@ def test_row_log_softmax_specials(n_col):
     assert np.isnan(got[1:]).all()
 
 
+@pytest.mark.parametrize("n_row,n_col,offset", [(256, 4097, 1), (257, 4097, 1), (257, 8192, 0), (257, 8193, 3),
+                                                (300, 16_384, 2), (257, 16_385, 1)])
+def test_row_log_softmax_many_rows(n_row, n_col, offset):
+    """More rows than CUs take the smallest block that holds one: both sides of each width."""
+    test_row_log_softmax_edges(n_row, n_col, offset)
+    x = np.random.default_rng(n_col).normal(size=(n_row, n_col)).astype(np.float32)
+    x[0, 7] = np.inf
+    x[1, [3, n_col - 1]] = np.inf
+    x[2] = -np.inf
+    x[3, 9] = np.nan
+    x[n_row - 1, 1:] = -np.inf
+    buf, ptr = at_offset(x, offset)
+    ac.RowSoftmax2(n_row, n_col, ptr)
+    torch.cuda.synchronize()
+    got = buf.cpu().numpy()[offset:offset + x.size].reshape(x.shape)
+    assert np.isnan(got[0, 7]) and (np.delete(got[0], 7) == -np.inf).all()
+    assert np.isnan(got[1:4]).all()
+    assert got[n_row - 1, 0] == 0.0 and (got[n_row - 1, 1:] == -np.inf).all()
+
+
 @pytest.mark.parametrize("n_row,n_col,offset", [(1, 1, 0), (300, 3, 1), (3, 32_768, 1), (3, 32_769, 2), (2, 100_001, 3),
                                                 (4, 8192, 1), (4, 8193, 1)])
 def test_row_max_edges(n_row, n_col, offset):
