@@ -671,9 +671,12 @@ extern "C" int ac_row_max(int64_t n_row, int64_t n_col, const float* in, float* 
   if (n_col == 0 || nchunk > 1)
     hipLaunchKernelGGL(k_stage_fill_rows, dim3(grid_for(n_row, 256)), dim3(256), 0, st, n_row, (int64_t)1,
                        (const float*)nullptr, out);
-  // The larger block where a row has work for it, and where the grid's threads stay below 2^32.
+  // The larger block where a row has work for it, and where the grid's threads stay below 2^32; short rows a wave each
+  // (1,000,000 x 4 223 us, 810 with blocks of 256; 30,000 x 1,000 22.4 and 28.7 us).
   const dim3 grid((unsigned)(n_row * nchunk));
-  if (n_col > kLsmChunkMin && n_row * nchunk <= 1 << 20)
+  if (n_col > 0 && n_col <= 1024)
+    hipLaunchKernelGGL(k_stage_row_max<64>, grid, dim3(64), 0, st, n_col, nchunk, in, out);
+  else if (n_col > kLsmChunkMin && n_row * nchunk <= 1 << 20)
     hipLaunchKernelGGL(k_stage_row_max<1024>, grid, dim3(1024), 0, st, n_col, nchunk, in, out);
   else if (n_col > 0)
     hipLaunchKernelGGL(k_stage_row_max<kMaxBlock>, grid, dim3(kMaxBlock), 0, st, n_col, nchunk, in, out);

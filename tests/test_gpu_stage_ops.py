@@ -159,6 +159,13 @@ def test_row_max_edges(n_row, n_col, offset):
     assert (out.cpu().numpy()[n_row:] == 3.0).all()
 
 
+@pytest.mark.parametrize("n_row,n_col,offset", [(7, 63, 1), (5, 64, 0), (5, 65, 2), (3, 1023, 3), (3, 1024, 1),
+                                                (3, 1025, 1), (70_000, 5, 1)])
+def test_row_max_short_rows(n_row, n_col, offset):
+    """Rows of a wave's and of a block's width."""
+    test_row_max_edges(n_row, n_col, offset)
+
+
 @pytest.mark.parametrize("n_in,n_out,P,Q,offset", [(8, 8, 3, 5, 0), (1028, 2052, 4, 70, 0), (1028, 2052, 4, 70, 1),
                                                    (1027, 1030, 5, 130, 0), (4096, 1000, 2, 64, 0), (40, 44, 2, 700, 0),
                                                    (7, 5, 3, 0, 0)])
