@@ -81,6 +81,14 @@ def test_edge_max_reduce_edges(n_row, n_in, n_out, offset, fill):
     assert (got[n_row * n_out:] == 3.0).all()
 
 
+@pytest.mark.parametrize("n_row,n_in,n_out,offset", [(128, 1024, 300, 1), (129, 1024, 300, 1), (257, 1023, 50, 2),
+                                                     (256, 1023, 50, 2), (1, 131_072, 700, 3), (1, 131_073, 700, 3)])
+@pytest.mark.parametrize("fill", ["low", "mid", "special"])
+def test_edge_max_reduce_small_calls(n_row, n_in, n_out, offset, fill):
+    """Both sides of the number of values up to which each has a thread of its own."""
+    test_edge_max_reduce_edges(n_row, n_in, n_out, offset, fill)
+
+
 def at_offset(x, offset):
     """x on the device, `offset` floats off an aligned start, and room behind it."""
     buf = torch.full((x.size + 8,), 3.0, device="cuda")
