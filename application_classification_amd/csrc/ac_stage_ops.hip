@@ -327,24 +327,33 @@ __global__ __launch_bounds__(NT) void k_lsm_row(int64_t n_col, float* __restrict
 // The three launches on `scratch`, which holds lsm_entries(n_row, n_col) entries.
 int64_t lsm_entries(int64_t n_row, int64_t n_col) { return n_row * (lsm_chunks(n_row, n_col) + 1); }
 
+// Launches over n_row rows with a block of nt threads for each of a row's `per` parts, in slices of rows whose grids
+// stay at 2^31 threads (a grid takes fewer than 2^32): go(first row, rows).
+template <typename Go>
+void for_row_slices(int64_t n_row, int64_t per, int nt, Go go) {
+  const int64_t slice = std::max<int64_t>(1, (int64_t(1) << 31) / (nt * per));
+  for (int64_t r0 = 0; r0 < n_row; r0 += slice) go(r0, (unsigned)std::min(slice, n_row - r0));
+}
+
 // The whole operator in one launch where the rows fit: every entry point takes this path first.
-// (The longer ones' blocks of 1024 only while the grid's threads stay below 2^32.)
-bool lsm_fused(int64_t n_row, int64_t n_col) { return n_col <= 16 * kLsmBlock || (n_col <= kRowMax && n_row <= 1 << 20); }
+bool lsm_fused(int64_t n_col) { return n_col <= kRowMax; }
 
 int enqueue_row_lsm(int64_t n_row, int64_t n_col, float* x, ac::Lse* scratch, hipStream_t st, const char* who) {
-  if (lsm_fused(n_row, n_col)) {
+  if (lsm_fused(n_col)) {
     // The smallest block that holds a row where there are more rows than CUs (256), so that a CU works on several at once:
     // 4,096 x 4,097 in 31 us with blocks of 256, 82 with 1,024 (three launches: 51); 4,096 x 12,000 69 with 512, 108 with
     // 1,024 (114).  Few rows take the largest, whose threads have the fewest elements: 256 x 4,097 in 7.6 us.
     const bool many = n_row > 256;
-    if (n_col <= 16 * kLsmBlock || (many && n_col <= kRowRegs * kLsmBlock))
-      hipLaunchKernelGGL(k_lsm_row<kLsmBlock>, dim3((unsigned)n_row), dim3(kLsmBlock), 0, st, n_col, x);
-    else if (many && n_col <= kRowRegs * 512)
-      hipLaunchKernelGGL(k_lsm_row<512>, dim3((unsigned)n_row), dim3(512), 0, st, n_col, x);
-    else
-      hipLaunchKernelGGL(k_lsm_row<1024>, dim3((unsigned)n_row), dim3(1024), 0, st, n_col, x);
+    const int nt = n_col <= 16 * kLsmBlock || (many && n_col <= kRowRegs * kLsmBlock) ? kLsmBlock
+                   : many && n_col <= kRowRegs * 512                                  ? 512
+                                                                                      : 1024;
+    const auto kernel = nt == kLsmBlock ? k_lsm_row<kLsmBlock> : nt == 512 ? k_lsm_row<512> : k_lsm_row<1024>;
+    for_row_slices(n_row, 1, nt, [&](int64_t r0, unsigned rows) {
+      hipLaunchKernelGGL(kernel, dim3(rows), dim3(nt), 0, st, n_col, x + r0 * n_col);
+    });
     return launch_status(who);
   }
+  // (Rows this long are below 2^24 blocks in any memory.)
   const int64_t nchunk = lsm_chunks(n_row, n_col);
   const int64_t nblk = n_row * nchunk;
   ac::Lse2* fin = reinterpret_cast<ac::Lse2*>(scratch + nblk);
@@ -632,7 +641,7 @@ extern "C" int ac_row_log_softmax(int64_t n_row, int64_t n_col, float* x, void* 
   if (n_row < 0 || n_col < 0 || n_row > INT32_MAX || (n_row * n_col > 0 && !x)) return bad("ac_row_log_softmax: bad arguments");
   if (n_row * n_col == 0) return AC_OK;
   hipStream_t st = as_stream(stream);
-  if (lsm_fused(n_row, n_col)) return enqueue_row_lsm(n_row, n_col, x, nullptr, st, "ac_row_log_softmax");
+  if (lsm_fused(n_col)) return enqueue_row_lsm(n_row, n_col, x, nullptr, st, "ac_row_log_softmax");
   // Stream-ordered temporary (the reference's RowSoftmax2 allocates its own too, src/ac.hxx:108-113).
   ac::Lse* tmp = nullptr;
   hipError_t e = hipMallocAsync((void**)&tmp, (size_t)lsm_entries(n_row, n_col) * sizeof(ac::Lse), st);
@@ -671,15 +680,14 @@ extern "C" int ac_row_max(int64_t n_row, int64_t n_col, const float* in, float* 
   if (n_col == 0 || nchunk > 1)
     hipLaunchKernelGGL(k_stage_fill_rows, dim3(grid_for(n_row, 256)), dim3(256), 0, st, n_row, (int64_t)1,
                        (const float*)nullptr, out);
-  // The larger block where a row has work for it, and where the grid's threads stay below 2^32; short rows a wave each
-  // (1,000,000 x 4 223 us, 810 with blocks of 256; 30,000 x 1,000 22.4 and 28.7 us).
-  const dim3 grid((unsigned)(n_row * nchunk));
-  if (n_col > 0 && n_col <= 1024)
-    hipLaunchKernelGGL(k_stage_row_max<64>, grid, dim3(64), 0, st, n_col, nchunk, in, out);
-  else if (n_col > kLsmChunkMin && n_row * nchunk <= 1 << 20)
-    hipLaunchKernelGGL(k_stage_row_max<1024>, grid, dim3(1024), 0, st, n_col, nchunk, in, out);
-  else if (n_col > 0)
-    hipLaunchKernelGGL(k_stage_row_max<kMaxBlock>, grid, dim3(kMaxBlock), 0, st, n_col, nchunk, in, out);
+  // The larger block where a row has work for it; short rows a wave each (1,000,000 x 4 223 us, 810 with blocks of 256;
+  // 30,000 x 1,000 22.4 and 28.7 us).
+  const int nt = n_col <= 1024 ? 64 : n_col <= kLsmChunkMin ? kMaxBlock : 1024;
+  const auto kernel = nt == 64 ? k_stage_row_max<64> : nt == kMaxBlock ? k_stage_row_max<kMaxBlock> : k_stage_row_max<1024>;
+  if (n_col > 0)
+    for_row_slices(n_row, nchunk, nt, [&](int64_t r0, unsigned rows) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)(rows * nchunk)), dim3(nt), 0, st, n_col, nchunk, in + r0 * n_col, out + r0);
+    });
   return launch_status("ac_row_max");
 }
 
@@ -705,13 +713,13 @@ extern "C" int ac_edge_max_reduce(int64_t n_col_in, int64_t n_col_out, int64_t n
   } else if (n_row * n_col_in > 0) {
     // Chunks of 8192 values (32 a thread), shorter ones down to 1024 where fewer than 2048 blocks would result (a
     // block of low-fill values is a chain of dependent reads and atomics: 39 us for 16 x 20,000 values in chunks of
-    // 8192, 15 us in chunks of 1024); rows in slices of at most 2^23 blocks (2^31 threads).
+    // 8192, 15 us in chunks of 1024).
     const int64_t csize = std::min<int64_t>(8192, std::max<int64_t>(1024, (n_col_in / 2048) * std::min<int64_t>(n_row, 8192)));
     const int64_t nchunk = std::max<int64_t>(1, std::min<int64_t>((n_col_in + csize - 1) / csize, 1 << 23));
-    const int64_t slice = (1 << 23) / nchunk;
-    for (int64_t r0 = 0; r0 < n_row; r0 += slice)
-      hipLaunchKernelGGL(k_stage_scatter_max, dim3((unsigned)(std::min(slice, n_row - r0) * nchunk)), dim3(kMaxBlock), 0,
-                         st, n_col_in, n_col_out, nchunk, vymax + r0, xe + r0 * n_col_in, xmax + r0 * n_col_out, nodes);
+    for_row_slices(n_row, nchunk, kMaxBlock, [&](int64_t r0, unsigned rows) {
+      hipLaunchKernelGGL(k_stage_scatter_max, dim3((unsigned)(rows * nchunk)), dim3(kMaxBlock), 0, st, n_col_in, n_col_out,
+                         nchunk, vymax + r0, xe + r0 * n_col_in, xmax + r0 * n_col_out, nodes);
+    });
   }
   return launch_status("ac_edge_max_reduce");
 }

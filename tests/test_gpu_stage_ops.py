@@ -174,6 +174,25 @@ def test_row_max_short_rows(n_row, n_col, offset):
     test_row_max_edges(n_row, n_col, offset)
 
 
+@pytest.mark.parametrize("n_row", [2**23 + 1, 2**24 + 3, 2**25 + 1])
+def test_more_rows_than_one_grid_takes(n_row):
+    """Row operators on rows of three: beyond 2^23 rows of 256 threads, 2^25 of 64, a launch takes a slice of them.  Maxima
+    bit for bit; the log-softmax against FP64 as in test_row_log_softmax_edges, with values within [-4, 4]."""
+    gen = torch.Generator("cuda").manual_seed(n_row)
+    x = torch.rand(n_row, 3, device="cuda", generator=gen) * 8 - 4
+    top = torch.full((n_row + 4,), 3.0, device="cuda")
+    ac.RowMax2(n_row, 3, x, top)
+    assert torch.equal(top[:n_row], x.amax(1)) and (top[n_row:] == 3.0).all()
+    got = torch.cat([x.flatten(), torch.full((4,), 3.0, device="cuda")])
+    ac.RowSoftmax2(n_row, 3, got)
+    assert (got[3 * n_row:] == 3.0).all()
+    worst = 0.0
+    for a in range(0, n_row, 1 << 22):
+        ref = torch.log_softmax(x[a:a + (1 << 22)].double(), 1)
+        worst = max(worst, (got[3 * a:3 * a + ref.numel()].double().view(-1, 3) - ref).abs().max().item())
+    assert worst <= 9 * 2.0**-23 + 9 * 2.0**-24, worst
+
+
 @pytest.mark.parametrize("n_in,n_out,P,Q,offset", [(8, 8, 3, 5, 0), (1028, 2052, 4, 70, 0), (1028, 2052, 4, 70, 1),
                                                    (1027, 1030, 5, 130, 0), (4096, 1000, 2, 64, 0), (40, 44, 2, 700, 0),
                                                    (7, 5, 3, 0, 0)])
