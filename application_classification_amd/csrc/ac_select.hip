@@ -92,39 +92,56 @@ __global__ __launch_bounds__(256) void k_sel_thresh(int S, int k, const unsigned
   if (threadIdx.x == 0) thr[blockIdx.x] = T;
 }
 
+// A block counts its entries in LDS and reserves their places with one atomic per column: where most of a column ties
+// (and the host selects after all), one per entry made 3.6 M of them follow each other on twelve counters (4.7 ms).
 __global__ __launch_bounds__(256) void k_sel_filter(int64_t n, int P, const float* __restrict__ X,
                                                     const unsigned* __restrict__ thr, int* __restrict__ count,
                                                     unsigned long long* __restrict__ keys, int* __restrict__ flag) {
+  constexpr int kRows = 8;  // a thread's, between barriers
+  __shared__ int own[256], base[256];
   const int t = threadIdx.x, RP = 256 / P;
-  if (t >= RP * P) return;
-  const int p = t % P;
+  const bool active = t < RP * P;
+  const int p = active ? t % P : 0;
   const unsigned lo = thr[p];
-  auto take = [&](int64_t v, float x) {
-    const unsigned b = order_bits(x);
-    if (b < lo) return;
-    const int at = atomicAdd(count + p, 1);
-    if (at < kSelCap)
-      keys[(int64_t)p * kSelCap + at] = ((unsigned long long)b << 32) | (0xFFFFFFFFu - (unsigned)v);
-    else
-      *flag = 1;
-  };
+  own[t] = 0;
   const int64_t step = (int64_t)gridDim.x * RP;
-  int64_t v = (int64_t)blockIdx.x * RP + t / P;
-  for (; v + 3 * step < n; v += 4 * step) {
-    const float a = X[v * P + p], b = X[(v + step) * P + p], c = X[(v + 2 * step) * P + p], d = X[(v + 3 * step) * P + p];
-    take(v, a);
-    take(v + step, b);
-    take(v + 2 * step, c);
-    take(v + 3 * step, d);
+  for (int64_t v0 = (int64_t)blockIdx.x * RP; v0 < n; v0 += kRows * step) {
+    unsigned b[kRows];
+    int hits = 0;
+#pragma unroll
+    for (int u = 0; u < kRows; ++u) {
+      const int64_t v = v0 + u * step + t / P;
+      const float x = X[(v < n ? v : n - 1) * P + p];
+      b[u] = active && v < n ? order_bits(x) : 0u;  // below every value
+      hits += b[u] >= lo && b[u] != 0u;
+    }
+    if (!__syncthreads_or(hits)) continue;
+    int at = hits ? atomicAdd(own + p, hits) : 0;
+    __syncthreads();
+    if (t < P && own[t] > 0) {
+      base[t] = atomicAdd(count + t, own[t]);
+      if (base[t] + own[t] > kSelCap) *flag = 1;
+      own[t] = 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kRows; ++u)
+      if (b[u] >= lo && b[u] != 0u) {
+        const int i = base[p] + at++;
+        if (i < kSelCap)
+          keys[(int64_t)p * kSelCap + i] =
+              ((unsigned long long)b[u] << 32) | (0xFFFFFFFFu - (unsigned)(v0 + u * step + t / P));
+      }
   }
-  for (; v < n; v += step) take(v, X[v * P + p]);
 }
 
 __global__ __launch_bounds__(256) void k_sel_rank(int P, int k, const float* __restrict__ X,
                                                   const int* __restrict__ count,
-                                                  const unsigned long long* __restrict__ keys, int* __restrict__ idx,
+                                                  const unsigned long long* __restrict__ keys,
+                                                  const int* __restrict__ flag, int* __restrict__ idx,
                                                   float* __restrict__ val) {
   __shared__ unsigned long long x[kSelCap];
+  if (*flag) return;  // (1.1 ms for a full column)
   const int p = blockIdx.x, m = min(count[p], kSelCap);
   for (int i = threadIdx.x; i < m; i += 256) x[i] = keys[(int64_t)p * kSelCap + i];
   __syncthreads();
@@ -158,7 +175,7 @@ void launch_select(int64_t n, int P, int k, const SelShape& s, const float* X, c
   const int RP = 256 / P;
   const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((n + 4 * RP - 1) / (4 * RP), 2048));
   hipLaunchKernelGGL(k_sel_filter, dim3(blocks), dim3(256), 0, st, n, P, X, b.thr, b.count, b.keys, b.flag);
-  hipLaunchKernelGGL(k_sel_rank, dim3(P), dim3(256), 0, st, P, k, X, b.count, b.keys, b.idx, b.val);
+  hipLaunchKernelGGL(k_sel_rank, dim3(P), dim3(256), 0, st, P, k, X, b.count, b.keys, b.flag, b.idx, b.val);
 }
 
 }  // namespace ac

@@ -100,6 +100,22 @@ def test_topk_and_match_selection(n, pn, k, kind):
     np.testing.assert_array_equal(match, expect)
 
 
+@pytest.mark.parametrize("n,pn,k,ties", [(65_536, 1, 5, 4000), (65_536, 1, 5, 4200), (120_000, 7, 60, 500), (120_000, 7, 60, 30_000),
+                                         (9000, 256, 3, 4096), (9000, 256, 3, 4097)])
+def test_topk_keeps_up_to_a_limit_of_ties(n, pn, k, ties):
+    """A stretch of vertices that share a column's best value, below and above the number of entries the device keeps."""
+    data, patt = random_graph(n, n, 3, 2, n + k), random_graph(pn, pn, 3, 2, pn)
+    data.vfeat[n // 3:n // 3 + ties] = patt.vfeat[0] + 1e-3
+    with Matcher(0) as m:
+        m.set_data(data)
+        m.set_pattern(patt)
+        mu = m.run(0)
+        idx, val = m.topk(k)
+    want = np.stack([np.lexsort((np.arange(n), -mu[:, p]))[:k] for p in range(pn)])
+    np.testing.assert_array_equal(idx, want)
+    np.testing.assert_array_equal(val, np.take_along_axis(mu.T, want, axis=1))
+
+
 @pytest.mark.parametrize("run_edges", [4, 16, 128])
 def test_gradients_do_not_depend_on_run_lengths(run_edges, monkeypatch):
     """The recorded least-cost out-edges and argmax in-edges of hubs in one to hundreds of pieces, equal costs among
