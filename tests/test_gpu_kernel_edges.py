@@ -116,6 +116,30 @@ def test_topk_keeps_up_to_a_limit_of_ties(n, pn, k, ties):
     np.testing.assert_array_equal(val, np.take_along_axis(mu.T, want, axis=1))
 
 
+@pytest.mark.parametrize("where", ["data", "pattern"])
+def test_selection_with_nan_columns(where):
+    """A NaN is above nothing and nothing is above it: a column of them selects its first vertices, in order, and the other
+    columns are selected as ever."""
+    n, pn, k = 30_000, 4, 5
+    data, patt = random_graph(n, 2 * n, 3, 2, n + k), random_graph(pn, pn, 3, 2, pn)
+    (data if where == "data" else patt).vfeat[1] = np.nan
+    with Matcher(0) as m:
+        m.set_data(data)
+        m.set_pattern(patt)
+        mu = m.run(0)
+        idx, val = m.topk(k)
+        match = m.match(-8.0)
+    expect = np.zeros((n, pn), np.uint8)
+    for p in range(pn):
+        nan = np.isnan(mu[:, p])
+        assert nan.all() == (where == "data" or p == 1) and nan.all() == nan.any()
+        want = np.arange(k) if nan.all() else np.lexsort((np.arange(n), -mu[:, p]))[:k]
+        np.testing.assert_array_equal(idx[p], want)
+        np.testing.assert_array_equal(val[p], mu[want, p])
+        expect[want[0], p] = 2 if mu[want[0], p] >= -8.0 else 1
+    np.testing.assert_array_equal(match, expect)
+
+
 @pytest.mark.parametrize("run_edges", [4, 16, 128])
 def test_gradients_do_not_depend_on_run_lengths(run_edges, monkeypatch):
     """The recorded least-cost out-edges and argmax in-edges of hubs in one to hundreds of pieces, equal costs among
