@@ -558,6 +558,7 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
   if (nV > 256 || nE > 256)
     return ctx->fail(AC_ERR_ARG, "ac_set_graph: patterns are limited to 256 vertices and 256 edges");
   ctx->has_patt = false;
+  ctx->have_result = false;  // from here on the last result's buffers and the pattern's sizes no longer belong together
   ctx->P = (int)nV;
   ctx->Q = (int)nE;
   ctx->Qs = (int)((nE + 3) / 4 * 4);
@@ -618,7 +619,6 @@ static int set_pattern(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int
   ctx->nsum = nsum;
   ctx->cnull_groups.assign({0, (int)nE});
   ctx->has_patt = true;
-  ctx->have_result = false;
   return AC_OK;
 }
 

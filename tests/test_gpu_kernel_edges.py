@@ -6,7 +6,7 @@ import torch
 
 from application_classification_amd import _lib
 from application_classification_amd import workloads as W
-from application_classification_amd.matcher import AC_OPT_PRUNE, AC_OPT_TAPE, Matcher
+from application_classification_amd.matcher import AC_OPT_PRUNE, AC_OPT_TAPE, ACError, Matcher
 from oracle import oracle as O
 from tests.conftest import allclose_report
 from tests.test_gpu_adjoint import check_grad, fd_grad, gpu_grad, weights
@@ -282,3 +282,25 @@ def test_page_locked_results_and_gradients(n, pn):
         got = m.backward(locked.numpy())
     for a, b in zip(got, want):
         np.testing.assert_array_equal(a, b)
+
+
+def test_a_pattern_that_does_not_fit_leaves_no_result(monkeypatch):
+    """A pattern whose upload fails for want of memory takes the last result with it: what reads results says so, and the
+    next pattern runs."""
+    data, small, wide = random_graph(20_000, 40_000, 64, 4, 1), random_graph(4, 5, 64, 4, 2), random_graph(250, 20, 64, 4, 3)
+    with Matcher(0) as m:
+        m.set_option(AC_OPT_TAPE, 1)
+        m.set_data(data)
+        m.set_pattern(small)
+        before = m.run(2)
+        monkeypatch.setenv("AC_MAX_ALLOC_BYTES", "65536")
+        with pytest.raises(ACError) as e:
+            m.set_pattern(wide)
+        assert e.value.code == _lib.AC_ERR_OOM
+        monkeypatch.delenv("AC_MAX_ALLOC_BYTES")
+        for read in (m.mu, m.match, lambda: m.topk(3), lambda: m.backward(np.zeros(m.sizes()[0::2], np.float32))):
+            with pytest.raises(ACError) as e:
+                read()
+            assert e.value.code == _lib.AC_ERR_STATE
+        m.set_pattern(small)
+        np.testing.assert_array_equal(m.run(2), before)
