@@ -762,6 +762,7 @@ static int ensure_work(ac_ctx* ctx) {
   if (rc != AC_OK) return rc;
   const int64_t key[6] = {ctx->dn, ctx->de, ctx->P, ctx->Q, ctx->bs->brows, ctx->nsum};
   if (std::equal(key, key + 6, ctx->work_key)) return AC_OK;
+  ctx->work_key[0] = -1;  // until every buffer is there: a failure below leaves some of the last sizes', some released
   const int64_t n = ctx->dn;
   const int P = ctx->P, Q = ctx->Q, Qs = ctx->Qs;
   // The output passes take every row: where few vertices of many have edges, the iterations' short tiles would leave

@@ -304,3 +304,24 @@ def test_a_pattern_that_does_not_fit_leaves_no_result(monkeypatch):
             assert e.value.code == _lib.AC_ERR_STATE
         m.set_pattern(small)
         np.testing.assert_array_equal(m.run(2), before)
+
+
+def test_work_buffers_after_a_run_that_did_not_fit(monkeypatch):
+    """A run that fails for want of memory leaves buffers of both patterns' sizes behind; the pattern that fitted runs again
+    with the same result."""
+    data, small, wide = random_graph(3000, 9000, 4, 4, 1), random_graph(4, 5, 4, 4, 2), random_graph(60, 90, 4, 4, 3)
+    with Matcher(0) as m:
+        m.set_data(data)
+        m.set_pattern(small)
+        before = m.run(2)
+        m.set_pattern(wide)
+        monkeypatch.setenv("AC_MAX_ALLOC_BYTES", str(600 * 1024))
+        with pytest.raises(ACError) as e:
+            m.run(2)
+        assert e.value.code == _lib.AC_ERR_OOM
+        m.set_pattern(small)
+        np.testing.assert_array_equal(m.run(2), before)
+        monkeypatch.delenv("AC_MAX_ALLOC_BYTES")
+        m.set_pattern(wide)
+        bad, ratio = allclose_report(m.run(2), O.run(g64(data), g64(wide), n_iter=2))
+        assert bad == 0, ratio
