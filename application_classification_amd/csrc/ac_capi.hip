@@ -486,6 +486,7 @@ static int set_data(ac_ctx* ctx, int64_t nV, int64_t dV, const float* vf, int64_
   build_runs(sord_off, (int64_t)sord.size(), rout, sout, slout, sord.data(), false);
 
   ctx->has_data = false;
+  ctx->tape_valid = false;  // a step back reads the graph that the uploads below replace
   hipStream_t st = ctx->stream;
   HIPCHK(ctx, ctx->vfeat.upload(vf, (size_t)(nV * dV), st));
   HIPCHK(ctx, ctx->d_perm.upload(perm.data(), perm.size(), st));

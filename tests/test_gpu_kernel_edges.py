@@ -325,3 +325,21 @@ def test_work_buffers_after_a_run_that_did_not_fit(monkeypatch):
         m.set_pattern(wide)
         bad, ratio = allclose_report(m.run(2), O.run(g64(data), g64(wide), n_iter=2))
         assert bad == 0, ratio
+
+
+def test_no_step_back_over_a_data_graph_that_did_not_fit(monkeypatch):
+    """The graph of a taped run is gone once the next one's upload has failed; the result itself stays readable."""
+    data, big = random_graph(500, 1500, 4, 4, 1), random_graph(20_000, 400, 4, 4, 2)
+    with Matcher(0) as m:
+        m.set_option(AC_OPT_TAPE, 1)
+        m.set_data(data)
+        m.set_pattern(random_graph(4, 5, 4, 4, 3))
+        mu = m.run(2)
+        monkeypatch.setenv("AC_MAX_ALLOC_BYTES", "65536")
+        with pytest.raises(ACError) as e:
+            m.set_data(big)
+        assert e.value.code == _lib.AC_ERR_OOM
+        np.testing.assert_array_equal(m.mu(), mu)
+        with pytest.raises(ACError) as e:
+            m.backward(np.zeros_like(mu))
+        assert e.value.code == _lib.AC_ERR_STATE
