@@ -47,8 +47,8 @@ struct Range {
 // are split into pieces of this length.  A run is walked step by step by one group of lanes, so short runs spread a small
 // graph over the chip, while long ones take fewer bundle headers and leave fewer pieces.  us per call at 8 / 16 / 32 /
 // 64 / 128: 20 K edges 611 / 644 / 692 / 765 / 910; 242 K edges 2283 / 1964 / 1864 / 1974 / 2380; 0.9 M edges 8356 / 6596
-// / 5960 / 5774 / 5876; 3.9 M edges 3341 / 2954 / 2783 / 2786 / 2888; 16 M edges (device time) 10340 / 8277 / 7396 / 7010
-// / 7087.
+// / 5960 / 5774 / 5876; 3.9 M edges 3341 / 2954 / 2783 / 2786 / 2888.  ms of device time at 64 / 128 (R-MAT, 64 features, 16/24
+// pattern): 8 M edges 3.63 / 3.92, 16 M 6.39 / 6.41, 32 M 11.92 / 11.60, 65 M 23.2 / 22.5.
 int run_edges(int64_t nE) {
   if (const char* e = std::getenv("AC_RUN_EDGES")) {
     const int v = std::atoi(e);
@@ -60,7 +60,7 @@ int run_edges(int64_t nE) {
 int round8(int x) { return (x + 7) / 8 * 8; }
 
 // Blocks of a vertex pass.  Each block walks its tiles grid-stride, and passes A and C leave one partial per pattern
-// edge / vertex that is merged serially afterwards: one round of resident blocks (no partly filled last round, few
+// edge / vertex that is merged afterwards: one round of resident blocks (no partly filled last round, few
 // partials) is fastest for them at R-MAT scale 22; the output passes, which leave no partials, use two rounds.
 int vertex_blocks(const char* env, int resident, int rounds, int64_t ntiles) {
   if (const char* e = std::getenv(env)) {  // tuning override
@@ -1690,7 +1690,7 @@ extern "C" int ac_batch_run(ac_ctx* ctx, const int32_t* n_iter) {
     prep += a;
     loop += b;
   }
-  ctx->have_result = false;  // OUT holds the last slab, not a pattern set with ac_set_graph
+  ctx->have_result = false;  // the pattern is the last slab's, and its columns went to the members' results, not to OUT
   ctx->b_info[0] = (int64_t)ctx->bp.size();
   ctx->b_info[1] = (int64_t)slabs.size();
   ctx->b_info[2] = upd;

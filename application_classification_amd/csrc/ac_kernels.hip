@@ -6,7 +6,8 @@
 //   vertex pass A  : MU = LSM(-CV + sum FMax + sum RMax) (recomputed, never stored), VF = MU[pd] - FMax,
 //                    VR = MU[ps] - RMax; stores VR and VFm = VF - minCEo; column maxima and the two edge
 //                    log-sum-exps, using  sum_e exp(X[src e] - CE_e) = sum_v exp(X[v] - minCEo[v] + lsO[v]).
-//   edge walk B    : FMaxN[v] = max over in-edges of (VR[src] - CE) - LSE_FE   (CSC order, no atomics)
+//   edge walk B    : FMaxN[v] = max over in-edges of (VR[src] - CE) - LSE_FE   (CSC order; the pieces of a vertex with a
+//                    long in-edge list raise its row by atomic maxima)
 //   vertex pass C  : column log-sum-exp of MU for the next iteration's normalisation.
 // RMax needs no edge pass: max over out-edges of (VF[v] - CE_e) = VF[v] - min over out-edges of CE_e, exactly.
 // The log-softmax of CE and CV in the reference's prep (src/main.cu:116,118) shift each row by a constant, which
@@ -64,13 +65,6 @@ __device__ __forceinline__ void argmax_merge(double& m, int& a, double x, int b)
     m = x;
     a = b;
   }
-}
-
-__device__ __forceinline__ void qpart_merge(QPart& a, const QPart& b) {
-  argmax_merge(a.vfmax, a.avf, b.vfmax, b.avf);
-  argmax_merge(a.vrmax, a.avr, b.vrmax, b.avr);
-  a.re = lse_merge(a.re, b.re);
-  a.fe = lse_merge(a.fe, b.fe);
 }
 
 }  // namespace
@@ -870,7 +864,8 @@ void launch_zero(const ZeroList& z, hipStream_t st) {
 // ---------------------------------------------------------------------------------------------------------------
 // Edge walks.  A group of Qs/4 lanes walks one run of consecutive edges; lane j owns pattern edges 4j..4j+3 and
 // reads them as one float4 of the edge's cost row (and of the gathered VR row).  Runs cover whole vertices except
-// the pieces of very long edge lists, whose partial results go to carry slots and are combined by a fixup kernel.
+// the pieces of long edge lists: the source statistics' and the taped walks' partial results go to carry slots and are
+// combined by a fixup kernel, a plain walk's raise the vertex's row by atomic maxima.
 
 int walk_blocks(int64_t nruns, int Qs) {
   const int L4 = Qs / 4;

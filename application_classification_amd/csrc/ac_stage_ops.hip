@@ -462,9 +462,11 @@ __device__ __forceinline__ bool above(float v, float x) { return !(v < x) && __f
 
 // Bound by the one read of xe.  A value at or below its row's fill can change nothing, so only the others look at
 // their node, and of those only the ones above its present value (read without an atomic: the entries only rise, so a
-// stale value is a low one) issue the atomic.  16 x 3.94 M values into 16 x 262,144, with the fill pass: 47 us where the
-// fills win, as they nearly all do in a matcher's step (5.4 TB/s; an atomic per value: 9.5 ms by source, 4.9 ms by
-// destination), 0.84 and 1.46 ms where no fill wins.  NaNs pass both comparisons and reach the atomic.
+// stale value is a low one) issue the atomic.  R-MAT 18's 16 x 3.94 M values into 16 x 262,144, with the fill pass, by the
+// share of them above their fill: none 43 us (5.9 TB/s), 0.1 % 55 by source and 59 by destination, 12 % 237 and 478, all 741
+// and 1,473 us; an atomic per value took 8.8-9.2 and 5.6-5.8 ms.  In the iterations of a matcher the share is 0 to 2 % by
+// source and 0 by destination (1,000 vertices, 10/12 pattern), 0 to 12 % and 0 to 0.14 % (R-MAT 14, 24/36), 0 to 0.2 % and
+// 0 (R-MAT 15, 12/16).  NaNs pass both comparisons and reach the atomic.
 __global__ __launch_bounds__(kMaxBlock) void k_stage_scatter_max(int64_t n_col_in, int64_t n_col_out, int64_t nchunk,
                                                                  const float* __restrict__ vymax,
                                                                  const float* __restrict__ xe,
