@@ -1394,32 +1394,37 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_max(int64_t nbundles, const
   } else if (slot >= 0) {
     // A piece of a split vertex: its maximum, normalised and rounded like a finished row, raises the row.  Rounding
     // is monotone, so the maximum over the pieces of the rounded values is the rounded maximum (exact, in any order).
-    float o[4] = {(float)(mx0 - sl[0]), (float)(mx1 - sl[1]), (float)(mx2 - sl[2]), (float)(mx3 - sl[3])};
-    float has[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+    const float o[4] = {(float)(mx0 - sl[0]), (float)(mx1 - sl[1]), (float)(mx2 - sl[2]), (float)(mx3 - sl[3])};
     float* row = FMaxN + (int64_t)cur * Qs + 4 * j;
+    if (!__any(gs & kCrowded)) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (4 * j + u < Q && o[u] != -INFINITY) atomic_raise(row + u, o[u]);
+      return;
+    }
+    // Pieces of a vertex of very many: a wave whose pieces are all one vertex's sends their maximum only, and a value not
+    // above the row's present one (read without an atomic: the row only rises, so a stale value is a low one) is not sent.
+    // With an atomic per piece the walk of 400,000 edges into one vertex, 12/16 pattern, took 354 us, now 33; combined
+    // by two launches of their own (the pieces' maxima stored), the walk and they took 37.  (Apart from the others'
+    // atomics: one sequence for both made a loop of 1,000 vertices, 10/12, 268 us long instead of 263.)
+    float m[4] = {o[0], o[1], o[2], o[3]};
     bool raise = true;
-    if (gs & kCrowded) {
-      // A vertex of very many pieces: a wave whose pieces are all its own sends their maximum only, and a value not above
-      // the row's present one (read without an atomic: the row only rises, so a stale value is a low one) is not sent.
-      // With an atomic per piece the walk of 400,000 edges into one vertex, 12/16 pattern, took 354 us, now 33;
-      // combined by two launches of their own (the pieces' maxima stored), the walk and they took 37.
-      if (__all(cur == __builtin_amdgcn_readfirstlane(cur)) && __popcll(__ballot(1)) == GL4) {
-        float m[4] = {o[0], o[1], o[2], o[3]};
-        for (int d = 1; d < G; ++d) {
-          const int from = (g + d < G ? g + d : g + d - G) * L4 + j;
+    if (__all(cur == __builtin_amdgcn_readfirstlane(cur)) && __popcll(__ballot(1)) == GL4) {
+      for (int d = 1; d < G; ++d) {
+        const int from = (g + d < G ? g + d : g + d - G) * L4 + j;
 #pragma unroll
-          for (int u = 0; u < 4; ++u) m[u] = fmaxf(m[u], __shfl(o[u], from, 64));
-        }
-#pragma unroll
-        for (int u = 0; u < 4; ++u) o[u] = m[u];
-        raise = g == 0;
+        for (int u = 0; u < 4; ++u) m[u] = fmaxf(m[u], __shfl(o[u], from, 64));
       }
+      raise = g == 0;
+    }
+    if (raise) {
+      float has[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) has[u] = __hip_atomic_load(row + u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
-      if (raise && 4 * j + u < Q && !(o[u] <= has[u])) atomic_raise(row + u, o[u]);
+      for (int u = 0; u < 4; ++u)
+        if (4 * j + u < Q && !(m[u] <= has[u])) atomic_raise(row + u, m[u]);
+    }
   } else if (cur >= 0) {
     AC_WK_EMIT(cur);
   }
