@@ -1404,7 +1404,7 @@ __global__ __launch_bounds__(kWalkBlock) void k_walk_max(int64_t nbundles, const
     }
     // Pieces of a vertex of very many: a wave whose pieces are all one vertex's sends their maximum only, and a value not
     // above the row's present one (read without an atomic: the row only rises, so a stale value is a low one) is not sent.
-    // With an atomic per piece the walk of 400,000 edges into one vertex, 12/16 pattern, took 354 us, now 33; combined
+    // With an atomic per piece the walk of 400,000 edges into one vertex, 12/16 pattern, took 354 us, now 31; combined
     // by two launches of their own (the pieces' maxima stored), the walk and they took 37.  (Apart from the others'
     // atomics: one sequence for both made a loop of 1,000 vertices, 10/12, 268 us long instead of 263.)
     float m[4] = {o[0], o[1], o[2], o[3]};
