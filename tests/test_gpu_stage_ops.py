@@ -219,6 +219,13 @@ def test_compute_mu_edges(n_in, n_out, P, Q, offset):
     assert (got[offset + P * n_out:] == 3.0).all() and (got[:offset] == 3.0).all()
 
 
+@pytest.mark.parametrize("n_in,n_out,P,Q,offset", [(40, 44, 1, 192, 0), (40, 44, 1, 256, 1), (40, 44, 1, 257, 0), (1028, 2052, 2, 2100, 0),
+                                                   (300, 300, 4100, 70, 0), (9, 5000, 3, 4000, 2)])
+def test_compute_mu_many_incident_edges(n_in, n_out, P, Q, offset):
+    """Lists that are just full, and several to a pattern vertex; more pattern vertices than the grid has rows."""
+    test_compute_mu_edges(n_in, n_out, P, Q, offset)
+
+
 @pytest.mark.parametrize("n_rows,n_cols", [(1, 1), (64, 64), (63, 65), (3, 1000), (1000, 3), (16, 100_003), (70_001, 12)])
 def test_transpose_tiles(n_rows, n_cols):
     x = np.arange(n_rows * n_cols, dtype=np.float32).reshape(n_rows, n_cols)
